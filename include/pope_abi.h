@@ -43,7 +43,8 @@ enum pope_status {
 };
 
 enum pope_op { POPE_OP_SIM_FWD = 0, POPE_OP_SIM_BWD = 1, POPE_OP_FLASH_FWD = 2,
-               POPE_OP_FLASH_BWD = 3, POPE_OP_FLASH_DECODE = 4, POPE_OP_POLAR_BWD = 5 };
+               POPE_OP_FLASH_BWD = 3, POPE_OP_FLASH_DECODE = 4, POPE_OP_POLAR_BWD = 5,
+               POPE_OP_FLASH_FWD_PARTIALS = 6 /* `partials` of pope_flash_fwd_split */ };
 
 /* pope_desc.flags (flash backward: PREPARED, ZERO_GRADS, DETERMINISTIC; similarity: SPLIT_BF16,
  * DETERMINISTIC; polar transform: COMPLEX, DETERMINISTIC; 0 elsewhere). */
@@ -149,6 +150,19 @@ int pope_sim_bwd(const pope_desc* desc, const void* dsim, const void* q, const v
 int pope_flash_fwd(const pope_desc* desc, const void* q, const void* k, const void* v,
                    const float* freqs, const float* bias, const uint8_t* mask, void* o,
                    float* lse, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * pope_flash_fwd with room for partial results: where the query blocks and heads leave most of
+ * the chip idle (few query rows against many keys), workgroups take splits of the key axis, leave
+ * fp32 partials in `partials` and a second launch merges them.  `partials` is caller-owned device
+ * memory of pope_workspace_bytes(POPE_OP_FLASH_FWD_PARTIALS) bytes (0: the call does not split),
+ * 256-byte aligned, free again once the call's work on the stream is done (the workspace alone is
+ * what the backward reuses); NULL runs unsplit.  No counterpart in the reference.
+ */
+int pope_flash_fwd_split(const pope_desc* desc, const void* q, const void* k, const void* v,
+                         const float* freqs, const float* bias, const uint8_t* mask, void* o,
+                         float* lse, void* workspace, size_t workspace_bytes, void* partials,
+                         size_t partials_bytes, void* stream);
 
 /*
  * Flash attention backward with PoPE.  dq, dk, dv are written (not accumulated);

@@ -26,8 +26,8 @@
 //                  the rows by lane shuffles into one (m, l, o) per (batch, head, split).
 //                  Loads are branch-free (clamped addresses), so each wait covers only
 //                  the rows being computed.
-//   decode_combine : merges the splits of each (batch, head) by their log-sum-exp
-//                  and writes o (input dtype) and lse (natural log, -inf when
+//   flash_merge  : (flash_merge.hip) merges the splits of each (batch, head) by their
+//                  log-sum-exp and writes o (input dtype) and lse (natural log, -inf when
 //                  every key is masked).
 // The query weights use the bias-on-the-query-side form of the score,
 //   a_d c_jd cos((F_q,d - b_d) - F_j,d)
@@ -363,79 +363,6 @@ __global__ __launch_bounds__(kThreads, 2) void decode_split_kernel(DecodeParams 
   }
 }
 
-// One workgroup per (batch, head): merge the splits by log-sum-exp.  Thread = (split group g,
-// 4-dim quad q); group g takes every G-th split, eight splits' (m, l, o) loads in flight at a
-// time, and keeps a running (m, l, o) of its splits (one pass over the partials, no wait for a
-// global maximum first); the groups' states then merge through LDS.
-template <typename T>
-__global__ __launch_bounds__(256) void decode_combine_kernel(DecodeParams p) {
-  __shared__ float4 o_s[256];
-  __shared__ float2 ml_s[256];
-  const int bh = blockIdx.x, tid = threadIdx.x;
-  const int b = bh / p.Hq, h = bh % p.Hq;
-  const int D = p.D, S = p.splits;
-  const float2* pml = reinterpret_cast<const float2*>(p.part_ml) + (int64_t)bh * S;
-  const float* po = p.part_o + (int64_t)bh * S * D;
-  const int qd = D / 4, G = 256 / qd;
-  const int g = tid / qd, q = tid % qd;
-  float m = -INFINITY, l = 0.f;
-  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-  // folds one split into the running state; a split without a visible key has m = -inf, l = 0
-  // and an o the split kernel never wrote, and leaves the state as it is
-  auto fold = [&](float2 ml, float4 v) {
-    if (ml.x == -INFINITY) v = make_float4(0.f, 0.f, 0.f, 0.f);
-    const float mn = fmaxf(m, ml.x);
-    const float mu = mn == -INFINITY ? 0.f : mn;
-    const float a = __builtin_amdgcn_exp2f(m - mu), w = __builtin_amdgcn_exp2f(ml.x - mu);
-    acc.x = fmaf(acc.x, a, v.x * w);
-    acc.y = fmaf(acc.y, a, v.y * w);
-    acc.z = fmaf(acc.z, a, v.z * w);
-    acc.w = fmaf(acc.w, a, v.w * w);
-    l = fmaf(l, a, ml.y * w);
-    m = mn;
-  };
-  if (g < G) {
-    const float4* po4 = reinterpret_cast<const float4*>(po) + q;
-    int s = g;
-    for (; s + 7 * G < S; s += 8 * G) {
-      float2 ml[8];
-      float4 v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        ml[u] = pml[s + u * G];
-        v[u] = po4[(int64_t)(s + u * G) * qd];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) fold(ml[u], v[u]);
-    }
-    for (; s < S; s += G) fold(pml[s], po4[(int64_t)s * qd]);
-  }
-  o_s[tid] = acc;
-  ml_s[tid] = make_float2(m, l);
-  __syncthreads();
-  if (tid < qd) {
-    float M = -INFINITY;
-    for (int g2 = 0; g2 < G; ++g2) M = fmaxf(M, ml_s[g2 * qd + tid].x);
-    const float Mu = M == -INFINITY ? 0.f : M;
-    float L = 0.f;
-    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int g2 = 0; g2 < G; ++g2) {
-      const float2 st = ml_s[g2 * qd + tid];
-      const float w = __builtin_amdgcn_exp2f(st.x - Mu);
-      const float4 v = o_s[g2 * qd + tid];
-      o.x = fmaf(v.x, w, o.x); o.y = fmaf(v.y, w, o.y); o.z = fmaf(v.z, w, o.z); o.w = fmaf(v.w, w, o.w);
-      L = fmaf(st.y, w, L);
-    }
-    const float inv = L > 0.f ? 1.f / L : 0.f;
-    uint16_t* orow = p.o + (int64_t)b * p.o_s[0] + (int64_t)h * p.o_s[1] + 4 * tid;
-    orow[0] = T::bits(o.x * inv);
-    orow[1] = T::bits(o.y * inv);
-    orow[2] = T::bits(o.z * inv);
-    orow[3] = T::bits(o.w * inv);
-    if (tid == 0) p.lse[bh] = L > 0.f ? (M + __builtin_amdgcn_logf(L)) * kLn2 : -INFINITY;
-  }
-}
-
 template <typename T, int LPK, int RMAX>
 hipError_t launch_t(const DecodeParams& p0, hipStream_t s) {
   DecodeParams p = p0;
@@ -443,7 +370,18 @@ hipError_t launch_t(const DecodeParams& p0, hipStream_t s) {
   hipError_t e = launch_named("flash_decode_split", decode_split_kernel<T, LPK, RMAX>,
                               dim3(p.B * p.splits * p.hgroups), dim3(kThreads), s, p);
   if (e != hipSuccess) return e;
-  return launch_named("flash_decode_combine", decode_combine_kernel<T>, dim3(p.B * p.Hq), dim3(256), s, p);
+  FlashMergeParams mp;
+  mp.part_o = p.part_o;
+  mp.part_ml = p.part_ml;
+  mp.o = p.o;
+  mp.lse = p.lse;
+  mp.rows = p.B * p.Hq;
+  mp.Hq = p.Hq;
+  mp.Nq = 1;
+  mp.D = p.D;
+  mp.splits = p.splits;
+  for (int i = 0; i < 3; ++i) mp.o_s[i] = p.o_s[i];
+  return launch_flash_merge(mp, "flash_decode_combine", T::kCode, s);
 }
 
 template <typename T>

@@ -77,7 +77,9 @@ struct FwdCfg {
   static_assert(LDS <= 160 * 1024, "LDS budget");
 };
 
-template <typename T, int EP, int DV>
+// SPLIT: the workgroup takes split `sp` of the key axis (p.split_keys keys, whole pairs of tiles) and
+// leaves its (m, l, O) as fp32 partials for launch_flash_merge instead of writing o and lse.
+template <typename T, int EP, int DV, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashFwdParams p) {
   typedef FwdCfg<EP, DV> C;
   constexpr int BN = C::BN, KB = C::KB, KS = C::KS, NDB = C::NDB;
@@ -89,7 +91,9 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashFwdParams p
   const int grp = wave >> 2, wq = wave & 3;
   const int BH = p.B * p.Hq;
   const int bh = blockIdx.x % BH;
-  const int qb = p.nqb - 1 - (int)(blockIdx.x / BH);
+  const int rest = (int)(blockIdx.x / BH);
+  const int sp = SPLIT ? rest % p.splits : 0;
+  const int qb = p.nqb - 1 - (SPLIT ? rest / p.splits : rest);
   const int b = bh / p.Hq, h = bh % p.Hq, hk = h % p.Hk;
   const int Nk = p.Nk, Nq = p.Nq, D = p.D;
   const int qw0 = qb * kBM + wq * 32;   // first query row of this wave
@@ -111,8 +115,12 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashFwdParams p
   typedef const __attribute__((address_space(4))) int ci32;
   int nkeys = min(((ci32*)p.kend)[b], Nk);
   if (p.causal) nkeys = min(nkeys, min(qb * kBM + kBM, Nq));
+  // this workgroup's pairs: p0, p0 + 1, .. p0 + npair - 1 (pair indices below are relative to p0,
+  // tile and key indices absolute)
+  const int p0 = SPLIT ? sp * (p.split_keys / (2 * BN)) : 0;
+  if (SPLIT) nkeys = min(nkeys, (sp + 1) * p.split_keys);
   const int nt = (nkeys + BN - 1) / BN;
-  const int npair = (nt + 1) / 2;
+  const int npair = max((nt + 1) / 2 - p0, 0);
   cu64* mw = (cu64*)p.mwords + (int64_t)b * p.NW;
 
   // ---- direct-load plan: unit c = m * 512 + tid of a stage slot ---------------------
@@ -142,7 +150,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashFwdParams p
   const int v_last = (Nk - 1) * vs2 + D - 8;   // start of the last chunk of the last row
   auto issue = [&](int pr) {
     char* slot = smem + (pr % C::SLOTS) * C::STAGE;
-    const int j0 = pr * 2 * BN;
+    const int j0 = (p0 + pr) * 2 * BN;
     const uint16_t* kp = khg + j0 * EP;   // K_hat rows are padded to NkP: no clamp
     const int vrow0 = j0 * vs2;
 #pragma unroll
@@ -185,7 +193,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashFwdParams p
   // Visibility of the group's tile of pair pr: true when every key is visible to every row of
   // the wave (no per-element mask needed).
   auto tile_full = [&](int pr, uint64_t& mb) -> bool {
-    const int tile = 2 * pr + grp;
+    const int tile = 2 * (p0 + pr) + grp;
     const int j0 = tile * BN;
     mb = 0;
     if (tile < nt) {
@@ -197,7 +205,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashFwdParams p
   };
   // masked scores -> -inf (cold: diagonal and partially visible tiles)
   auto apply_mask = [&](int pr, uint64_t mb, f32x16* s) {
-    const int j0 = (2 * pr + grp) * BN;
+    const int j0 = (2 * (p0 + pr) + grp) * BN;
     // the lane's keys are 32 kb + 8 (r >> 2) + (r & 3) past 4 hf: compile-time bit positions
     const uint64_t w = mb >> (4 * hf);
     const int lim = p.causal ? qi - j0 - 4 * hf : BN;   // causal: key offset <= lim
@@ -484,6 +492,22 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashFwdParams p
       for (int r = 0; r < 16; ++r) oacc[db][r] = oacc[db][r] * a0 + src[2 + 16 * db + r] * a1;
   }
   const float l = l_run + wave_shfl_xor(l_run, 32);
+  if constexpr (SPLIT) {
+    if (qi >= Nq) return;
+    const int64_t prow = (((int64_t)b * p.Hq + h) * Nq + qi) * p.splits + sp;
+    float* po = p.part_o + prow * D;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int d0 = 32 * db + 8 * g + 4 * hf;
+        if (d0 < D)
+          *reinterpret_cast<float4*>(po + d0) = make_float4(oacc[db][4 * g], oacc[db][4 * g + 1], oacc[db][4 * g + 2],
+                                                            oacc[db][4 * g + 3]);
+      }
+    if (hf == 0) *reinterpret_cast<float2*>(p.part_ml + 2 * prow) = make_float2(m_fin, l);
+    return;
+  }
   const float inv = l > 0.f ? 1.f / l : 0.f;
   if (qi < Nq) {
     uint16_t* orow = p.o + (int64_t)b * p.o_s[0] + (int64_t)h * p.o_s[1] + (int64_t)qi * p.o_s[2];
@@ -508,7 +532,9 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashFwdParams p
 template <typename T, int EP, int DV>
 hipError_t launch_t(const FlashFwdParams& p, hipStream_t s) {
   const int blocks = p.nqb * p.B * p.Hq;
-  return launch_named("flash_fwd", flash_fwd_kernel<T, EP, DV>, dim3(blocks), dim3(kThreads), s, p);
+  if (p.splits > 1)
+    return launch_named("flash_fwd", flash_fwd_kernel<T, EP, DV, true>, dim3(blocks * p.splits), dim3(kThreads), s, p);
+  return launch_named("flash_fwd", flash_fwd_kernel<T, EP, DV, false>, dim3(blocks), dim3(kThreads), s, p);
 }
 
 template <typename T>
@@ -525,6 +551,8 @@ hipError_t dispatch(const FlashFwdParams& p, hipStream_t s) {
 }
 
 }  // namespace
+
+int flash_fwd_step_keys(int EP, int DV) { return EP + DV <= 192 && DV <= 64 ? 128 : 64; }   // 2 FwdCfg::BN
 
 hipError_t launch_flash_fwd(const FlashFwdParams& p, int dtype, hipStream_t s) {
   return dtype == 2 ? dispatch<BF16>(p, s) : dispatch<F16>(p, s);

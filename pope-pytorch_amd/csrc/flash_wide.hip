@@ -107,7 +107,8 @@ __device__ __forceinline__ void tile_fill(const uint16_t* tile, int tid, int wav
 // rows and the V rows go straight from global memory into LDS once for the four waves (unpadded,
 // XOR-swizzled), in three slots: the loads of the next two tiles are in flight while the current
 // tile is computed.
-template <typename T, int EP, int DV>
+// SPLIT: one split of the key axis per workgroup, fp32 partials (as in flash_fwd.hip).
+template <typename T, int EP, int DV, bool SPLIT>
 __global__ __launch_bounds__(256) void wide_fwd_kernel(FlashFwdParams p) {
   constexpr int KS = EP / 16, NDB = DV / 32;
   constexpr int KU = EP / 8, VU = DV / 8;              // 16-byte units per K_hat / V row
@@ -117,15 +118,18 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(FlashFwdParams p) {
   __shared__ __attribute__((aligned(16))) uint16_t vt[kSlots][32 * DV];
 
   const int tid = threadIdx.x, wave = wave_id(), lane = tid & 63, lr = lane & 31, hf = lane >> 5;
-  const int BH = p.B * p.Hq, nqb = p.NqP / 128;
+  const int BH = p.B * p.Hq, nqb = (p.Nq + 127) / 128;
   const int bh = blockIdx.x % BH;
-  const int q0 = 128 * (nqb - 1 - (int)(blockIdx.x / BH));   // heaviest causal blocks first
-  if (q0 >= p.Nq) return;
+  const int rest = (int)(blockIdx.x / BH);
+  const int sp = SPLIT ? rest % p.splits : 0;
+  const int q0 = 128 * (nqb - 1 - (SPLIT ? rest / p.splits : rest));   // heaviest causal blocks first
   const int b = bh / p.Hq, h = bh % p.Hq, hk = h % p.Hk;
   const int Nk = p.Nk, D = p.D, qi = q0 + 32 * wave + lr;
 
   int nkeys = min(((ci32*)p.kend)[b], Nk);
   if (p.causal) nkeys = min(nkeys, q0 + 128);
+  const int t0 = SPLIT ? sp * (p.split_keys / 32) : 0;   // the workgroup's first tile
+  if (SPLIT) nkeys = min(nkeys, (sp + 1) * p.split_keys);
   const uint16_t* khb = p.kh + (int64_t)(b * p.Hk + hk) * p.NkP * EP;   // rows padded to NkP
   const uint16_t* vb = p.v + (int64_t)b * p.v_s[0] + (int64_t)hk * p.v_s[1];
   cu64* mw = (cu64*)p.mwords + (int64_t)b * p.NW;
@@ -136,14 +140,14 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(FlashFwdParams p) {
   // the last one and V units at or past D repeat the row's last unit (they only reach the O rows
   // at or past D, which are not stored)
   auto issue = [&](int t) {
-    const int j0 = 32 * t, slot = t % kSlots;
+    const int j0 = 32 * (t0 + t), slot = t % kSlots;
     const uint16_t* kp = khb + (int64_t)j0 * EP;
     tile_fill<KU>(kt[slot], tid, wave, [&](int r, int u) { return kp + r * EP + 8 * u; });
     tile_fill<VU>(vt[slot], tid, wave, [&](int r, int u) {
       return vb + (int64_t)min(j0 + r, Nk - 1) * p.v_s[2] + min(8 * u, D - 8);
     });
   };
-  const int nt = (nkeys + 31) / 32;
+  const int nt = max((nkeys + 31) / 32 - t0, 0);
   if (nt > 0) issue(0);
   if (nt > 1) issue(1);
 
@@ -163,7 +167,7 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(FlashFwdParams p) {
   float m = -INFINITY, l = 0.f;
   const uint32_t ones = T::pack2(1.f, 1.f);
   for (int t = 0; t < nt; ++t) {
-    const int buf = t % kSlots, j0 = 32 * t;
+    const int buf = t % kSlots, j0 = 32 * (t0 + t);
     if (t + 1 < nt) wait_vmcnt<NL>();   // this thread's loads of tile t landed (t + 1 may be in flight)
     else wait_vmcnt<0>();
     __syncthreads();                    // ... everyone's; and slot (t + 2) % kSlots was last read in step t - 1
@@ -230,6 +234,21 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(FlashFwdParams p) {
     }
   }
   if (qi >= p.Nq) return;
+  if constexpr (SPLIT) {
+    const int64_t prow = (((int64_t)b * p.Hq + h) * p.Nq + qi) * p.splits + sp;
+    float* po = p.part_o + prow * D;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int d0 = 32 * db + 8 * g + 4 * hf;
+        if (d0 < D)
+          *reinterpret_cast<float4*>(po + d0) = make_float4(oacc[db][4 * g], oacc[db][4 * g + 1], oacc[db][4 * g + 2],
+                                                            oacc[db][4 * g + 3]);
+      }
+    if (hf == 0) *reinterpret_cast<float2*>(p.part_ml + 2 * prow) = make_float2(m, l);
+    return;
+  }
   const float inv = l > 0.f ? 1.f / l : 0.f;
   uint16_t* orow = p.o + (int64_t)b * p.o_s[0] + (int64_t)h * p.o_s[1] + (int64_t)qi * p.o_s[2];
 #pragma unroll
@@ -649,7 +668,10 @@ __global__ __launch_bounds__(256) void wide_chain_kernel(FlashBwdParams p, const
 
 template <typename T, int EP, int DV>
 hipError_t fwd_t(const FlashFwdParams& p, hipStream_t s) {
-  return launch_named("flash_wide_fwd", wide_fwd_kernel<T, EP, DV>, dim3((p.NqP / 128) * p.B * p.Hq), dim3(256), s, p);
+  const int blocks = ((p.Nq + 127) / 128) * p.B * p.Hq;
+  if (p.splits > 1)
+    return launch_named("flash_wide_fwd", wide_fwd_kernel<T, EP, DV, true>, dim3(blocks * p.splits), dim3(256), s, p);
+  return launch_named("flash_wide_fwd", wide_fwd_kernel<T, EP, DV, false>, dim3(blocks), dim3(256), s, p);
 }
 
 // Column chunks per row block (each chunk recomputes the scores), as few as measured fastest: with

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -206,6 +207,38 @@ FlashLayout flash_layout(const pope_desc& d) {
 size_t flash_ws(const pope_desc& d, int op) {
   const FlashLayout L = flash_layout(d);
   return L.total + (op == POPE_OP_FLASH_BWD ? L.wide_bytes + det_bytes(d) : 0);
+}
+
+// Splits of the key axis in the flash forward: 1, or as many as bring the grid to one workgroup per
+// CU (256) where query blocks and heads alone leave half of them idle, each split keeping at least
+// kSplitSteps steps of the kernel's loop.  A step takes about 1.3 us at 128 keys, 1.0 us at 64 keys
+// and 2.0 us on the wide path (32 keys); a split call adds the merge launch (4-8 us, and as much on
+// the host), so it has to save kSplitGainUs: at 10 steps of 64 keys (589 keys, D 112, one head)
+// splitting took the kernels from 20.8 to 26.3 us, at 125 steps of 128 keys (16,000 keys, 130
+// queries, 8 heads, D 64) from 187.8 to 39.7.
+constexpr int kCUs = 256, kSplitSteps = 3;
+constexpr float kSplitGainUs = 12.f;
+
+struct FlashSplit {
+  int splits, keys;   // keys per split
+};
+
+FlashSplit flash_split(const pope_desc& d, const FlashLayout& L) {
+  const int step = L.wide ? 32 : pope::flash_fwd_step_keys(L.EP, L.DV);
+  const float step_us = step == 128 ? 1.3f : step == 64 ? 1.0f : 2.0f;
+  const int64_t blocks = (int64_t)((d.Nq + 127) / 128) * d.B * d.Hq;
+  const int steps = ((d.causal ? std::min(d.Nq, d.Nk) : d.Nk) + step - 1) / step;
+  const int want = (int)std::min<int64_t>(kCUs / std::max<int64_t>(blocks, 1), steps / kSplitSteps);
+  if (want < 2) return {1, 0};
+  const int per = (steps + want - 1) / want;
+  if ((steps - per) * step_us < kSplitGainUs) return {1, 0};
+  return {(steps + per - 1) / per, per * step};
+}
+
+size_t flash_partial_bytes(const pope_desc& d, int splits) {
+  if (splits < 2) return 0;
+  const size_t rows = (size_t)d.B * d.Hq * d.Nq;
+  return align_up(rows * splits * d.D * sizeof(float)) + align_up(rows * splits * 2 * sizeof(float));
 }
 
 // The flash kernels address the rows of v and do inside one (batch, head) with 32-bit element
@@ -461,6 +494,9 @@ int pope_workspace_bytes(int op, const pope_desc* desc, size_t* bytes) {
     case POPE_OP_FLASH_BWD: *bytes = flash_ws(*desc, op); return POPE_OK;
     case POPE_OP_FLASH_DECODE: *bytes = decode_ws(*desc); return POPE_OK;
     case POPE_OP_POLAR_BWD: *bytes = det_bytes(*desc); return POPE_OK;
+    case POPE_OP_FLASH_FWD_PARTIALS:
+      *bytes = flash_partial_bytes(*desc, flash_split(*desc, flash_layout(*desc)).splits);
+      return POPE_OK;
     default: return fail(POPE_ERR_INVALID, "unknown op %d", op);
   }
 }
@@ -468,11 +504,22 @@ int pope_workspace_bytes(int op, const pope_desc* desc, size_t* bytes) {
 int pope_flash_fwd(const pope_desc* d, const void* q, const void* k, const void* v, const float* freqs,
                    const float* bias, const uint8_t* mask, void* o, float* lse, void* workspace,
                    size_t workspace_bytes, void* stream) {
+  return pope_flash_fwd_split(d, q, k, v, freqs, bias, mask, o, lse, workspace, workspace_bytes, nullptr, 0, stream);
+}
+
+int pope_flash_fwd_split(const pope_desc* d, const void* q, const void* k, const void* v, const float* freqs,
+                         const float* bias, const uint8_t* mask, void* o, float* lse, void* workspace,
+                         size_t workspace_bytes, void* partials, size_t partials_bytes, void* stream) {
   int rc = check_flash_common(d, q, k, v, freqs, bias, mask, o, lse);
   if (rc) return rc;
   const FlashLayout L = flash_layout(*d);
   if ((rc = check_ws(L.total, workspace, workspace_bytes))) return rc;
   if ((rc = check_row_span("v", L.NkP, d->v_s[2]))) return rc;
+  FlashSplit fs{1, 0};
+  if (partials) {
+    fs = flash_split(*d, L);
+    if ((rc = check_ws(flash_partial_bytes(*d, fs.splits), partials, partials_bytes))) return rc;
+  }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
   hipError_t e = flash_prepare(*d, L, q, k, freqs, bias, mask, ws, s);
@@ -492,10 +539,32 @@ int pope_flash_fwd(const pope_desc* d, const void* q, const void* k, const void*
   p.nqb = (d->Nq + 127) / 128;
   copy3(p.v_s, d->v_s);
   copy3(p.o_s, d->o_s);
+  const size_t rows = (size_t)d->B * d->Hq * d->Nq;
+  p.splits = fs.splits;
+  p.split_keys = fs.keys;
+  if (fs.splits > 1) {
+    p.part_o = static_cast<float*>(partials);
+    p.part_ml = reinterpret_cast<float*>(static_cast<char*>(partials) + align_up(rows * fs.splits * d->D * sizeof(float)));
+  }
   e = L.wide ? pope::launch_flash_wide_fwd(p, d->dtype, s) : pope::launch_flash_fwd(p, d->dtype, s);
   if (e == hipErrorInvalidValue)
     return fail(POPE_ERR_UNSUPPORTED, "no flash forward kernel for head dim %d, rotate dim %d", d->D, d->R);
   if (e != hipSuccess) return hip_fail(e, "flash forward launch");
+  if (fs.splits > 1) {
+    pope::FlashMergeParams m;
+    m.part_o = p.part_o;
+    m.part_ml = p.part_ml;
+    m.o = p.o;
+    m.lse = lse;
+    m.rows = (int)rows;
+    m.Hq = d->Hq;
+    m.Nq = d->Nq;
+    m.D = d->D;
+    m.splits = fs.splits;
+    copy3(m.o_s, d->o_s);
+    e = pope::launch_flash_merge(m, "flash_merge", d->dtype, s);
+    if (e != hipSuccess) return hip_fail(e, "flash merge launch");
+  }
   return POPE_OK;
 }
 

@@ -75,9 +75,26 @@ struct FlashFwdParams {
   uint16_t* o; float* lse;
   int B, Hq, Hk, Nq, Nk, D, EP, DV, NqP, NkP, NW, causal, nqb;
   int64_t v_s[3], o_s[3];
+  // splits > 1: workgroup = (query block, split of split_keys keys); its (m, l, O) go to part_ml
+  // (rows, splits, 2) and part_o (rows, splits, D), row = (b Hq + h) Nq + i, for launch_flash_merge
+  // (a split without a visible key: m = -inf, l = 0)
+  int splits, split_keys;
+  float* part_o; float* part_ml;
 };
 // Returns hipErrorInvalidValue for an uncovered (EP, DV) shape.
 hipError_t launch_flash_fwd(const FlashFwdParams& p, int dtype, hipStream_t s);
+// Keys the workgroups of the forward consume per step (split_keys is a multiple).
+int flash_fwd_step_keys(int EP, int DV);
+
+// Log-sum-exp merge of split partials (flash_merge.hip): o (16-bit, strides o_s, row = (b Hq + h)
+// Nq + i) and lse (natural log, -inf for rows no split has a visible key of).  m in log2 units.
+struct FlashMergeParams {
+  const float* part_o; const float* part_ml;   // (rows, splits, D), (rows, splits, 2)
+  uint16_t* o; float* lse;
+  int rows, Hq, Nq, D, splits;
+  int64_t o_s[3];
+};
+hipError_t launch_flash_merge(const FlashMergeParams& p, const char* name, int dtype, hipStream_t s);
 
 struct FlashBwdParams {
   const uint16_t* q; const uint16_t* k; const uint16_t* v; const uint16_t* o; const uint16_t* dout;

@@ -265,9 +265,10 @@ def _fwd_impl(q, k, v, freqs, bias, mask, causal, softmax_scale):
         # one non-causal query row against a long cache: the split-K decode kernel
         decode = _decode_eligible(q, k, v, freqs, causal)
         dec_bytes = _lib.workspace_bytes(_lib.OP_FLASH_DECODE, d) if decode else -1
-        return d, dec_bytes, _fwd_ws_bytes(d, deterministic)
+        part_bytes = 0 if decode else _lib.workspace_bytes(_lib.OP_FLASH_FWD_PARTIALS, d)
+        return d, dec_bytes, _fwd_ws_bytes(d, deterministic), part_bytes
 
-    d, dec_bytes, fwd_bytes = _plan(key, build)
+    d, dec_bytes, fwd_bytes, part_bytes = _plan(key, build)
     L = _lib.lib()
     args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), _data(freqs), _data(bias), _data(mask),
             o.data_ptr(), lse.data_ptr())
@@ -285,7 +286,10 @@ def _fwd_impl(q, k, v, freqs, bias, mask, causal, softmax_scale):
         return o, lse, q.new_empty(0, dtype=torch.uint8)
     # torch's caching allocator returns 512-byte aligned blocks
     ws = torch.empty(fwd_bytes, dtype=torch.uint8, device=q.device)
-    _lib.check(L.pope_flash_fwd(ctypes.byref(d), *args, ws.data_ptr(), fwd_bytes, stream), "flash forward")
+    # the split forward's partials, apart from the workspace the backward keeps
+    parts = torch.empty(part_bytes, dtype=torch.uint8, device=q.device) if part_bytes else None
+    _lib.check(L.pope_flash_fwd_split(ctypes.byref(d), *args, ws.data_ptr(), fwd_bytes, _data(parts), part_bytes, stream),
+               "flash forward")
     return o, lse, ws
 
 

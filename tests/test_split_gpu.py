@@ -1,0 +1,91 @@
+"""Key splits of the flash forward: few query rows against many keys run as splits of the key axis and a
+log-sum-exp merge.  Against the float64 oracle at the sizes where the splits end unevenly: lengths around tile
+and split edges, splits without a visible key (masks, causal), one row and a partial second query block, every
+step size of the kernels (128 keys: narrow rows; 64: D 96 and 128; 32: heads above 128).
+
+The tolerance is the flash tests' own (2e-2 absolute beyond the rounding of the output format); lse 2e-2.
+"""
+import pytest
+import torch
+
+from gpu_common import excess_over, make_pope_inputs, oracle_attention
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # B, Hq, Hk, Nq, Nk, D, R, mask, causal, dtype
+    (1, 2, 2, 3, 2048, 64, 64, "none", False, torch.bfloat16),
+    (1, 2, 1, 129, 2049, 64, 32, "prefix", False, torch.float16),
+    (1, 1, 1, 2000, 2000, 64, 64, "none", True, torch.bfloat16),
+    (2, 2, 2, 17, 4097, 32, 32, "half", False, torch.bfloat16),
+    (2, 2, 2, 5, 1983, 64, 16, "dead_row", False, torch.float16),
+    (1, 4, 2, 130, 3001, 96, 96, "random", False, torch.bfloat16),
+    (1, 2, 2, 1, 1100, 128, 128, "half", False, torch.float16),
+    (1, 1, 1, 1500, 1500, 128, 64, "prefix", True, torch.bfloat16),
+    (1, 2, 1, 7, 999, 160, 32, "prefix", False, torch.bfloat16),
+    (1, 1, 1, 257, 1025, 256, 256, "half", False, torch.bfloat16),
+    (1, 2, 2, 500, 500, 192, 192, "none", True, torch.float16),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
+def test_split_forward_against_the_oracle(cuda, case):
+    from pope_amd import _lib
+    from pope_amd.hip_pope_flash_attn import flash_attn_head_first, flash_fwd_op
+    B, Hq, Hk, Nq, Nk, D, R, mask, causal, dtype = case
+    inp = make_pope_inputs(8300 + Nk, B, Hq, Hk, Nq, Nk, D, R, dtype, mask)
+    ref = oracle_attention(inp, causal, grads=False)
+    if Nq > 1:   # one non-causal row takes the decode kernel through the public entry point
+        _lib.profile_reset()
+        _lib.profile_enable(True)
+        o, lse, _ = flash_fwd_op(inp["q"], inp["k"], inp["v"], inp["freqs"], inp["bias"], inp["mask"], causal, D ** -0.5)
+        torch.cuda.synchronize()
+        _lib.profile_enable(False)
+        assert "flash_merge" in _lib.profile_read()
+        assert torch.equal(torch.isinf(lse).cpu(), torch.isinf(ref["lse"]))
+        fin = torch.isfinite(ref["lse"])
+        assert (lse.cpu().double()[fin] - ref["lse"][fin]).abs().max().item() <= 2e-2
+    else:
+        o = flash_attn_head_first(inp["q"], inp["k"], inp["v"], inp["freqs"], inp["bias"], mask=inp["mask"], causal=causal)
+    assert excess_over(o, ref["o"], 2e-2) <= 0
+
+
+def test_split_forward_feeds_the_backward(cuda):
+    """Gradients through a split forward (its lse and o are the backward's inputs)."""
+    import pope_amd
+    inp = make_pope_inputs(8400, 1, 2, 1, 70, 3000, 64, 32, torch.bfloat16, "prefix")
+    ref = oracle_attention(inp, False)
+    q, k, v = (inp[n].requires_grad_(True) for n in ("q", "k", "v"))
+    o = pope_amd.flash_attn_with_pope(q, k, v, pos_emb=(inp["freqs"], inp["bias"]), mask=inp["mask"])
+    grads = torch.autograd.grad(o, (q, k, v), inp["do"])
+    for got, name in zip(grads, ("dq", "dk", "dv")):
+        assert excess_over(got, ref[name], 2e-2) <= 0, name
+
+
+def test_partials_are_sized_and_optional(cuda):
+    """pope_flash_fwd (no partials) gives the same result within fp32 merge rounding, and a short buffer is refused."""
+    import ctypes
+
+    from pope_amd import _lib
+    from pope_amd.hip_pope_flash_attn import _desc
+    inp = make_pope_inputs(8500, 1, 2, 2, 40, 2500, 64, 64, torch.bfloat16)
+    q, k, v = inp["q"], inp["k"], inp["v"]
+    d = _desc(q, k, inp["freqs"], inp["bias"], False, 0.125)
+    o = torch.empty_like(q)
+    d.q_s[:], d.k_s[:], d.v_s[:], d.o_s[:] = (_lib.strides3(t) for t in (q, k, v, o))
+    lse = torch.empty(q.shape[:3], device="cuda")
+    nb, pb = _lib.workspace_bytes(_lib.OP_FLASH_FWD, d), _lib.workspace_bytes(_lib.OP_FLASH_FWD_PARTIALS, d)
+    assert pb > 0
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    pt = torch.full((pb,), 0xff, dtype=torch.uint8, device="cuda")   # NaN patterns: nothing unwritten is read
+    args = [t.data_ptr() for t in (q, k, v, inp["freqs"], inp["bias"])] + [None, o.data_ptr(), lse.data_ptr(), ws.data_ptr(), nb]
+    L, s = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    assert L.pope_flash_fwd(ctypes.byref(d), *args, s) == 0
+    torch.cuda.synchronize()
+    o1, lse1 = o.clone(), lse.clone()
+    assert L.pope_flash_fwd_split(ctypes.byref(d), *args, pt.data_ptr(), pb - 256, s) == 3
+    assert L.pope_flash_fwd_split(ctypes.byref(d), *args, pt.data_ptr(), pb, s) == 0
+    torch.cuda.synchronize()
+    # the unsplit kernel rounds P against one reference max, the splits against their own: bf16 P, fp32 sums
+    assert (o1.float() - o.float()).abs().max().item() <= 1e-2
+    assert (lse1 - lse).abs().max().item() <= 1e-3
