@@ -363,10 +363,22 @@ __global__ __launch_bounds__(kThreads, 2) void decode_split_kernel(DecodeParams 
   }
 }
 
+// Query-head groups per split: at least as many as the LDS array of query weights asks for, and as
+// many as bring the grid to two workgroups per CU, down to one head per wave.  A wave takes its
+// heads one after another, so with few batch rows x splits the heads in sequence are the call's
+// time: 1 x 4,001 keys, 32 heads over 8 (D 128): 63 workgroups of 32 heads 56.9 us, 504 of 4 heads 18.8 us.
+// Where the splits alone fill the chip the groups stay few: each computes the split's cos / sin rows.
+int launch_head_groups(const DecodeParams& p) {
+  constexpr int kTarget = 2 * 256, kWavesPerWg = kThreads / 64;
+  int g = decode_head_groups(p.Hq, p.D);
+  while (g > 0 && (int64_t)p.B * p.splits * g < kTarget && p.Hq % (2 * g) == 0 && p.Hq / (2 * g) >= kWavesPerWg) g *= 2;
+  return g;
+}
+
 template <typename T, int LPK, int RMAX>
 hipError_t launch_t(const DecodeParams& p0, hipStream_t s) {
   DecodeParams p = p0;
-  p.hgroups = decode_head_groups(p.Hq, p.D);
+  p.hgroups = launch_head_groups(p);
   hipError_t e = launch_named("flash_decode_split", decode_split_kernel<T, LPK, RMAX>,
                               dim3(p.B * p.splits * p.hgroups), dim3(kThreads), s, p);
   if (e != hipSuccess) return e;

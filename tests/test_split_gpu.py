@@ -89,3 +89,15 @@ def test_partials_are_sized_and_optional(cuda):
     # the unsplit kernel rounds P against one reference max, the splits against their own: bf16 P, fp32 sums
     assert (o1.float() - o.float()).abs().max().item() <= 1e-2
     assert (lse1 - lse).abs().max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("Hq,Hk,D,Nk", [(8, 8, 64, 1025), (12, 4, 128, 1100), (24, 8, 64, 1024), (32, 8, 128, 1333),
+                                        (6, 2, 96, 2000), (64, 8, 128, 1024), (40, 40, 32, 1281)])
+def test_decode_head_groups(cuda, Hq, Hk, D, Nk):
+    """Few batch rows x splits: the decode's workgroups take groups of the query heads (4 to 10 heads per group
+    here, group sizes that are no multiple of the four waves among them)."""
+    import pope_amd
+    inp = make_pope_inputs(8600 + Hq, 1, Hq, Hk, 1, Nk, D, D, torch.bfloat16, "prefix")
+    ref = oracle_attention(inp, False, grads=False)
+    o = pope_amd.flash_attn_with_pope(inp["q"], inp["k"], inp["v"], pos_emb=(inp["freqs"], inp["bias"]), mask=inp["mask"])
+    assert excess_over(o, ref["o"], 2e-2) <= 0
