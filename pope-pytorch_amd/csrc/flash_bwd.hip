@@ -157,6 +157,10 @@ struct BwdCfg {
   // one per SIMD; 128-row steps in a two-slot ring where two such slots fit (C4's E = 192, D = 96:
   // 326 against 331 us with 64-row steps in three slots), else 64-row steps in three.
   static constexpr bool kBig = EP + DV > 160;
+  // The widest rows read their score and dP operands through a ring of eight instead of all at
+  // once: with all of them in registers these kernels spilled, and every reload of a spilled
+  // register waits for the tile loads in flight behind it.
+  static constexpr bool kChunked = EP + DV > 320;
   static constexpr int NW = kBig ? 4 : 8;                    // waves per workgroup
   static constexpr int THREADS = 64 * NW;
   static constexpr int JOB = 32 * NW;                        // keys (dK/dV) or queries (dQ) per job
@@ -218,7 +222,8 @@ __device__ __forceinline__ void dkdv_job(const FlashBwdParams& p, char* smem, fl
 #pragma unroll
     for (int kk = 0; kk < DS; ++kk) {
       const int d0 = 16 * kk + 8 * hf;
-      vreg[kk] = as_vec8<vec8>((kj < Nk && d0 < D) ? ld16(vr + d0) : zero4());
+      const u32x4 x = ld16(vr + min(d0, D - 8));   // no branch: a valid address always, the value selected
+      vreg[kk] = as_vec8<vec8>((kj < Nk && d0 < D) ? x : zero4());
     }
   }
   settle_vector_loads();
@@ -235,11 +240,14 @@ __device__ __forceinline__ void dkdv_job(const FlashBwdParams& p, char* smem, fl
 
   const bool wave_vis = __all(kvis);
   const bool wave_any = __any(kvis);
+  // sub-tiles the wave visits: first rows in [q_lo, q_lo + q_span)
+  const int q_lo = p.causal ? kw0 - 31 : 0;
+  const uint32_t q_span = wave_any ? (uint32_t)max(Nq - q_lo, 0) : 0u;
   const int any_key = __syncthreads_or(kvis ? 1 : 0);
-  const int nqt = NqP / BM;
+  const int nqt = (Nq + BM - 1) / BM;   // steps of padding rows alone are not visited
   const int qt0 = p.causal ? j0 / BM : 0;
   const int groups = p.Hq / p.Hk;
-  const int per_head = nqt - qt0;
+  const int per_head = max(nqt - qt0, 0);
   const int nsteps = any_key ? groups * per_head : 0;
 
   // ---- direct-load plan: unit c = m * 256 + tid of a slot (Q_hat tile | dO tile | -lse | -delta)
@@ -255,14 +263,18 @@ __device__ __forceinline__ void dkdv_job(const FlashBwdParams& p, char* smem, fl
   // those rows only meet P = 0); -lse / -delta offset from the tile's first -lse row (the -delta array
   // follows the -lse array in the workspace)
   const int64_t nd_off = p.nd - p.nl;
+  // The regions begin at multiples of 64 units, so their tests are made on the wave's first unit (a
+  // scalar branch).  Tested per thread they were divergent branches, and in the widest kernel, which
+  // spills, the compiler put the spill store of a live register behind an execz branch, where it
+  // runs with no lane enabled: the reload then read stale memory (NaN in dk, dv and wild addresses).
   int ld_o[C::KV_LPT];
 #pragma unroll
   for (int m = 0; m < C::KV_LPT; ++m) {
-    const int c = m * kThreads + tid;
-    if (c < XU) {
+    const int c = m * kThreads + tid, c0 = m * kThreads + wave * 64;
+    if (c0 < XU) {
       const int r = c / EPU;
       ld_o[m] = r * EP + 8 * ((c % EPU) ^ tile_swz(EPU, r));
-    } else if (c < XU + YU) {
+    } else if (c0 < XU + YU) {
       const int r = (c - XU) / DVU;
       ld_o[m] = r * do_rs + min(8 * (((c - XU) % DVU) ^ tile_swz(DVU, r)), D - 8);
     } else {
@@ -322,8 +334,9 @@ __device__ __forceinline__ void dkdv_job(const FlashBwdParams& p, char* smem, fl
     const uint32_t nla = opaque_u32(sb + 2 * (C::XT + C::YT) + 16 * hf);
 #pragma unroll
     for (int qs = 0; qs < QB; ++qs) {
-      // every query of the sub-tile before every key of the wave (causal), or no visible key
-      if ((p.causal && i0 + 32 * qs + 31 < kw0) || !wave_any) continue;
+      // every query of the sub-tile before every key of the wave (causal) or past the last one, or
+      // no visible key
+      if ((uint32_t)(i0 + 32 * qs - q_lo) >= q_span) continue;
       f32x16 s, dp;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {   // rows 32 qs + 8 q + 4 hf + (0..3)
@@ -335,19 +348,39 @@ __device__ __forceinline__ void dkdv_job(const FlashBwdParams& p, char* smem, fl
           dp[4 * q + x] = d[x];
         }
       }
-      // every operand read of the two products issued before the first product, so one LDS
-      // latency is exposed per sub-tile instead of one per product
-      u32x4 fq[KS], fd[DS];
+      if constexpr (!C::kChunked) {
+        // every operand read of the two products issued before the first product, so one LDS
+        // latency is exposed per sub-tile instead of one per product
+        u32x4 fq[KS], fd[DS];
 #pragma unroll
-      for (int kk = 0; kk < KS; ++kk) fq[kk] = lds_read16_at(qa.row_at(kk) + 2 * 32 * qs * EP);
+        for (int kk = 0; kk < KS; ++kk) fq[kk] = lds_read16_at(qa.row_at(kk) + 2 * 32 * qs * EP);
 #pragma unroll
-      for (int kk = 0; kk < DS; ++kk) fd[kk] = lds_read16_at(da.row_at(kk) + 2 * 32 * qs * DV);
+        for (int kk = 0; kk < DS; ++kk) fd[kk] = lds_read16_at(da.row_at(kk) + 2 * 32 * qs * DV);
 #pragma unroll
-      for (int kk = 0; kk < KS; ++kk) s = T::mfma32(as_vec8<vec8>(fq[kk]), kreg[kk], s);
+        for (int kk = 0; kk < KS; ++kk) s = T::mfma32(as_vec8<vec8>(fq[kk]), kreg[kk], s);
 #pragma unroll
-      for (int kk = 0; kk < DS; ++kk) dp = T::mfma32(as_vec8<vec8>(fd[kk]), vreg[kk], dp);
-      __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 8 + KS + DS, 0);   // with the 8 row-term reads
-      __builtin_amdgcn_sched_group_barrier(kSchedMfma, KS + DS, 0);
+        for (int kk = 0; kk < DS; ++kk) dp = T::mfma32(as_vec8<vec8>(fd[kk]), vreg[kk], dp);
+        __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 8 + KS + DS, 0);   // with the 8 row-term reads
+        __builtin_amdgcn_sched_group_barrier(kSchedMfma, KS + DS, 0);
+      } else {
+        // the widest rows: a ring of eight operands ahead of the products
+        constexpr int NP = KS + DS;
+        u32x4 f[8];
+        auto operand = [&](int i) {
+          return i < KS ? lds_read16_at(qa.row_at(i) + 2 * 32 * qs * EP)
+                        : lds_read16_at(da.row_at(i - KS) + 2 * 32 * qs * DV);
+        };
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = operand(i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+          if (i < KS) s = T::mfma32(as_vec8<vec8>(f[i % 8]), kreg[i < KS ? i : 0], s);
+          else dp = T::mfma32(as_vec8<vec8>(f[i % 8]), vreg[i < KS ? 0 : i - KS], dp);
+          if (i + 8 < NP) f[i % 8] = operand(i + 8);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
       // Partial sub-tile (some key of the wave masked, or on the causal diagonal): masked
       // scores become -inf so that P = 0.
       if (!wave_vis || (p.causal && i0 + 32 * qs < kw0 + 31)) {
@@ -465,7 +498,7 @@ __device__ __forceinline__ void dkdv_job(const FlashBwdParams& p, char* smem, fl
     // general rotate dim: one wave's 32 keys at a time through LDS
     constexpr int BS = EP + 1;
     float* ebuf = reinterpret_cast<float*>(smem);
-    for (int w = 0; w < C::NW; ++w) {
+    for (int w = 0; w < C::NW && j0 + 32 * w < Nk; ++w) {
       __syncthreads();
       if (wave == w) {
   #pragma unroll
@@ -536,18 +569,17 @@ __device__ __forceinline__ void dq_job(const FlashBwdParams& p, char* smem, int 
 #pragma unroll
     for (int kk = 0; kk < DS; ++kk) {
       const int d0 = 16 * kk + 8 * hf;
-      doreg[kk] = as_vec8<vec8>((qi < Nq && d0 < D) ? ld16(dr + d0) : zero4());
+      const u32x4 x = ld16(dr + min(d0, D - 8));
+      doreg[kk] = as_vec8<vec8>((qi < Nq && d0 < D) ? x : zero4());
     }
   }
   // initial accumulators: -lse and -delta of the lane's query in every register
+  const float nl0 = p.nl[(int64_t)bh * p.NqP + qi], nd0 = p.nd[(int64_t)bh * p.NqP + qi];
   f32x16 nlc, ndc;
-  {
-    const float a = p.nl[(int64_t)bh * p.NqP + qi], d = p.nd[(int64_t)bh * p.NqP + qi];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      nlc[r] = a;
-      ndc[r] = d;
-    }
+  for (int r = 0; r < 16; ++r) {
+    nlc[r] = nl0;
+    ndc[r] = nd0;
   }
   settle_vector_loads();
 
@@ -561,6 +593,7 @@ __device__ __forceinline__ void dq_job(const FlashBwdParams& p, char* smem, int 
   int nkeys = min(((ci32*)p.kend)[b], Nk);
   if (p.causal) nkeys = min(nkeys, min(qb * C::JOB + C::JOB, Nq));
   const int nt = (nkeys + BN - 1) / BN;
+  const int k_end = qw0 >= Nq ? 0 : p.causal ? qw0 + 32 : Nk;   // keys the wave visits
 
   // ---- direct-load plan: unit c = m * 256 + tid of a slot (K_hat tile | V tile) --------
   const uint16_t* kh_g = p.kh + (int64_t)bhk * NkP * EP;
@@ -572,7 +605,7 @@ __device__ __forceinline__ void dq_job(const FlashBwdParams& p, char* smem, int 
 #pragma unroll
   for (int m = 0; m < C::Q_LPT; ++m) {
     const int c = m * kThreads + tid;
-    if (c < XU) {
+    if (m * kThreads + wave * 64 < XU) {   // the wave's first unit: a scalar branch, as in dkdv_job
       const int r = c / EPU;
       ld_o[m] = r * EP + 8 * ((c % EPU) ^ tile_swz(EPU, r));
     } else {
@@ -624,20 +657,47 @@ __device__ __forceinline__ void dq_job(const FlashBwdParams& p, char* smem, int 
     for (int ks = 0; ks < NB; ++ks) {
       const int k0 = j0 + 32 * ks;   // first key of the sub-tile
       const uint32_t mb = (uint32_t)(mw[k0 >> 6] >> (k0 & 32));
-      // nothing visible to this wave: every key masked, or (causal) after the wave's last query
-      if (mb == 0 || (p.causal && k0 > qw0 + 31)) continue;
+      // nothing visible to this wave: every key masked, or (causal) after the wave's last query, or
+      // the wave's rows all padding
+      if (mb == 0 || k0 >= k_end) continue;
       // every key visible and (causal) at or before the wave's first query
       const bool full = mb == 0xffffffffu && !(p.causal && k0 + 31 > qw0);
-      f32x16 s = nlc, dp = ndc;
-      u32x4 fk[KS], fv[DS];   // operand reads first (one exposed LDS latency per sub-tile)
+      f32x16 s, dp;
+      if constexpr (!C::kChunked) {
+        s = nlc;
+        dp = ndc;
+        u32x4 fk[KS], fv[DS];   // operand reads first (one exposed LDS latency per sub-tile)
 #pragma unroll
-      for (int kk = 0; kk < KS; ++kk) fk[kk] = lds_read16_at(ka.row_at(kk) + 2 * 32 * ks * EP);
+        for (int kk = 0; kk < KS; ++kk) fk[kk] = lds_read16_at(ka.row_at(kk) + 2 * 32 * ks * EP);
 #pragma unroll
-      for (int kk = 0; kk < DS; ++kk) fv[kk] = lds_read16_at(va.row_at(kk) + 2 * 32 * ks * DV);
+        for (int kk = 0; kk < DS; ++kk) fv[kk] = lds_read16_at(va.row_at(kk) + 2 * 32 * ks * DV);
 #pragma unroll
-      for (int kk = 0; kk < KS; ++kk) s = T::mfma32(as_vec8<vec8>(fk[kk]), qreg[kk], s);
+        for (int kk = 0; kk < KS; ++kk) s = T::mfma32(as_vec8<vec8>(fk[kk]), qreg[kk], s);
 #pragma unroll
-      for (int kk = 0; kk < DS; ++kk) dp = T::mfma32(as_vec8<vec8>(fv[kk]), doreg[kk], dp);
+        for (int kk = 0; kk < DS; ++kk) dp = T::mfma32(as_vec8<vec8>(fv[kk]), doreg[kk], dp);
+      } else {   // as in dkdv_job; the accumulators start from the row terms' scalars
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          s[r] = nl0;
+          dp[r] = nd0;
+        }
+        constexpr int NP = KS + DS;
+        u32x4 f[8];
+        auto operand = [&](int i) {
+          return i < KS ? lds_read16_at(ka.row_at(i) + 2 * 32 * ks * EP)
+                        : lds_read16_at(va.row_at(i - KS) + 2 * 32 * ks * DV);
+        };
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = operand(i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+          if (i < KS) s = T::mfma32(as_vec8<vec8>(f[i % 8]), qreg[i < KS ? i : 0], s);
+          else dp = T::mfma32(as_vec8<vec8>(f[i % 8]), doreg[i < KS ? 0 : i - KS], dp);
+          if (i + 8 < NP) f[i % 8] = operand(i + 8);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
       // the transposed K_hat operands of dQ, read while the products and the exponentials run
       u32x4 ft[2][EB];
 #pragma unroll
@@ -647,9 +707,11 @@ __device__ __forceinline__ void dq_job(const FlashBwdParams& p, char* smem, int 
           const uint32_t r0 = 2 * (32 * ks + 16 * g2) * EP;
           ft[g2][eb] = lds_tr8_at(ka.lo_at(eb) + r0, ka.hi_at(eb) + r0);
         }
-      __builtin_amdgcn_sched_group_barrier(kSchedDsRead, KS + DS, 0);
-      __builtin_amdgcn_sched_group_barrier(kSchedMfma, KS + DS, 0);
-      __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 4 * EB, 0);
+      if constexpr (!C::kChunked) {
+        __builtin_amdgcn_sched_group_barrier(kSchedDsRead, KS + DS, 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedMfma, KS + DS, 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 4 * EB, 0);
+      }
       if (!full) {   // masked scores -> -inf: P = 0
         POPE_COLD_PATH();
         const uint32_t w = mb >> (4 * hf);
@@ -747,7 +809,7 @@ __device__ __forceinline__ void dq_job(const FlashBwdParams& p, char* smem, int 
     // general rotate dim: one wave's 32 queries at a time through LDS
     constexpr int BS = EP + 1;
     float* ebuf = reinterpret_cast<float*>(smem);
-    for (int w = 0; w < C::NW; ++w) {
+    for (int w = 0; w < C::NW && qb * C::JOB + 32 * w < Nq; ++w) {
       __syncthreads();
       if (wave == w) {
   #pragma unroll
@@ -785,7 +847,7 @@ template <typename T, int EP, int DV>
 __global__ __launch_bounds__((BwdCfg<EP, DV>::THREADS), 1) void bwd_main_kernel(FlashBwdParams p) {
   __shared__ __attribute__((aligned(16))) char smem[BwdCfg<EP, DV>::LDS];
   __shared__ float dbias_s[EP];
-  const int nqb = p.NqP / BwdCfg<EP, DV>::JOB;
+  const int nqb = (p.Nq + BwdCfg<EP, DV>::JOB - 1) / BwdCfg<EP, DV>::JOB;   // blocks of padding alone get no job
   const int id = blockIdx.x;
   int kind, blk, head;   // kind 0 = dK/dV job (head = b * Hk + hk), 1 = dQ job (head = b * Hq + h)
   if (p.interleave) {
@@ -827,7 +889,7 @@ hipError_t launch_t(const FlashBwdParams& p0, hipStream_t s) {
                               dim3(256), s, p);
   if (e != hipSuccess) return e;
   typedef BwdCfg<EP, DV> C;
-  const int nkb = p.NkP / C::JOB, nqb = p.NqP / C::JOB;
+  const int nkb = (p.Nk + C::JOB - 1) / C::JOB, nqb = (p.Nq + C::JOB - 1) / C::JOB;
   p.n_kv_jobs = nkb * p.B * p.Hk;
   p.interleave = p.causal && p.Hq == p.Hk && nkb == nqb && p.Nq == p.Nk;
   const int jobs = p.n_kv_jobs + nqb * p.B * p.Hq;

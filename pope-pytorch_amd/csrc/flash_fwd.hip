@@ -136,7 +136,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashFwdParams p
 #pragma unroll
   for (int m = 0; m < C::LPT; ++m) {
     const int c = m * kThreads + tid;
-    if (c < C::KUNITS) {
+    if (m * kThreads + wave * 64 < C::KUNITS) {   // the wave's first unit: a scalar branch
       const int g = c / (BN * C::EPU), rem = c % (BN * C::EPU);
       const int r = rem / C::EPU, u = (rem % C::EPU) ^ tile_swz(C::EPU, r);
       ld_o[m] = (g * BN + r) * EP + 8 * u;
@@ -178,9 +178,15 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashFwdParams p
   for (int db = 0; db < NDB; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[db][r] = 0.f;
-  f32x16 negm;   // -m in every register: the initial accumulator of S
+  // -m in every register: the initial accumulator of S.  The widest rows (Q_hat alone holds 56 or 64
+  // of the 256 registers) write it anew for each tile instead of keeping the 16 copies: with them
+  // these instances spilled 5 to 27 registers.
+  constexpr bool kKeepNegM = EP < 224;
+  f32x16 negm;
+  if constexpr (kKeepNegM) {
 #pragma unroll
-  for (int r = 0; r < 16; ++r) negm[r] = 0.f;
+    for (int r = 0; r < 16; ++r) negm[r] = 0.f;
+  }
   float m_ref = 0.f, l_run = 0.f;
   bool m_set = false;
   f32x16 sacc[KB];
@@ -228,12 +234,17 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashFwdParams p
   // rows keep the compiler's interleave (sched_group_barrier), which was faster there (C4 86.9
   // against 88.5 us).
   constexpr bool kFenced = EP <= 128;
-  constexpr int kPF = 6;   // K_hat operand reads in flight ahead of the products (fenced order)
+  // K_hat operand reads in flight ahead of the products (fenced order; five spill nothing at DV 128)
+  constexpr int kPF = DV < 128 ? 6 : 5;
   auto k_operand = [&](const uint16_t* kt, int i) -> u32x4 {
     return *reinterpret_cast<const u32x4*>(kt + 32 * (i / KS) * EP + ko.row_at(i % KS));
   };
   auto qk = [&](int pr, f32x16* s) {
     const uint16_t* kt = kh_tile(pr);
+    if constexpr (!kKeepNegM) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) negm[r] = -m_ref;
+    }
 #pragma unroll
     for (int i = 0; i < NQK; ++i) {
       const int kb = i / KS, kk = i % KS;
@@ -268,8 +279,10 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_kernel(FlashFwdParams p
       asm("v_mul_f32 %0, %0, %1" : "+v"(l_run) : "v"(alpha));
       m_ref += sh;
       m_set = m_set || need;
+      if constexpr (kKeepNegM) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) asm("v_mov_b32 %0, %1" : "=v"(negm[r]) : "v"(-m_ref));
+        for (int r = 0; r < 16; ++r) asm("v_mov_b32 %0, %1" : "=v"(negm[r]) : "v"(-m_ref));
+      }
     }
   };
   // probabilities (bf16 / fp16 pairs, in B-operand order) and the row sum

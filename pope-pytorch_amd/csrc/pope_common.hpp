@@ -175,7 +175,9 @@ __device__ __forceinline__ int lds_swz(int row, int unit) { return unit ^ ((row 
 //                   (ds_read_b64_tr_b16, lds_read_tr16).
 // Unpadded rows let tiles be filled by direct global-to-LDS loads, which write 64 consecutive
 // units per wave instruction.
-__host__ __device__ constexpr int tile_swz(int U, int r) {
+// (Always inlined: left to its own cost model the compiler kept it a function in the widest backward
+// kernel, called from the per-thread load plans under partial exec masks.)
+__host__ __device__ __forceinline__ constexpr int tile_swz(int U, int r) {
   return (U % 16 == 0) ? (((r & 3) << 2) | ((r >> 2) & 3))
          : (U % 8 == 0) ? ((((r >> 1) & 1) << 2) | ((r >> 2) & 3))
                         : ((r >> 2) & 3);
@@ -217,7 +219,7 @@ __device__ __forceinline__ uint32_t opaque_u32(uint32_t x) {
 // compiler does not add its conservative wait for every outstanding LDS load before each LDS
 // read: the kernel waits for its own loads (vmcnt) before the barrier that publishes a stage.
 __device__ __forceinline__ void load_lds16(const void* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory");
 }
 
 // LDS byte address of a pointer into a __shared__ array.
