@@ -44,7 +44,8 @@ enum pope_status {
 
 enum pope_op { POPE_OP_SIM_FWD = 0, POPE_OP_SIM_BWD = 1, POPE_OP_FLASH_FWD = 2,
                POPE_OP_FLASH_BWD = 3, POPE_OP_FLASH_DECODE = 4, POPE_OP_POLAR_BWD = 5,
-               POPE_OP_FLASH_FWD_PARTIALS = 6 /* `partials` of pope_flash_fwd_split */ };
+               POPE_OP_FLASH_FWD_PARTIALS = 6,  /* `partials` of pope_flash_fwd_split */
+               POPE_OP_FLASH_BWD_PARTIALS = 7   /* `partials` of pope_flash_bwd_split */ };
 
 /* pope_desc.flags (flash backward: PREPARED, ZERO_GRADS, DETERMINISTIC; similarity: SPLIT_BF16,
  * DETERMINISTIC; polar transform: COMPLEX, DETERMINISTIC; 0 elsewhere). */
@@ -177,6 +178,19 @@ int pope_flash_bwd(const pope_desc* desc, const void* dout, const void* q, const
                    const float* bias, const uint8_t* mask, void* dq, void* dk, void* dv,
                    float* dfreqs, float* dbias, void* workspace, size_t workspace_bytes,
                    void* stream);
+
+/*
+ * pope_flash_bwd with room for partial sums: where few, long jobs leave most of the chip idle
+ * (grouped heads, few batches x heads), the jobs' loops are split over workgroups, which leave fp32
+ * partial rows in `partials`; a last launch sums them in a fixed order and applies the chain rule.
+ * `partials`: pope_workspace_bytes(POPE_OP_FLASH_BWD_PARTIALS) bytes (0: the call does not split),
+ * 256-byte aligned, free again once the call's work on the stream is done; NULL runs unsplit.
+ */
+int pope_flash_bwd_split(const pope_desc* desc, const void* dout, const void* q, const void* k,
+                         const void* v, const void* o, const float* lse, const float* freqs,
+                         const float* bias, const uint8_t* mask, void* dq, void* dk, void* dv,
+                         float* dfreqs, float* dbias, void* workspace, size_t workspace_bytes,
+                         void* partials, size_t partials_bytes, void* stream);
 
 /*
  * Bandwidth-bound forward for a single non-causal query row against a long KV

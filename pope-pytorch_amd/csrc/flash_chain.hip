@@ -1,0 +1,167 @@
+// Chain rule of the polar transform on raw expanded-row gradients (gfx950): the last launch of the
+// wide-head backward (one raw row per key / query), and of a narrow backward whose jobs were split
+// (flash_bwd_split: the partial rows of the splits are summed here, in split order, and dV with
+// them).  Bound by HBM: 4 EP bytes per row and split.
+#include "pope_common.hpp"
+#include "pope_kernels.hpp"
+
+namespace pope {
+
+namespace {
+
+// Blocks [0, nk): 32 key rows of one (batch, kv head); blocks [nk, nk + nq): 32 query rows of
+// one (batch, head).  With the raw expanded-row gradients U (cos column e = d, sin column
+// e = R + d, pass-through column e = R + d) and the row's phase (keys F[j]; queries
+// F[q_off + i] - bias, the bias on the query side as in the preparation):
+//   dx = sigmoid(x) (cos U_c + sin U_s),  dphase = softplus(x) (cos U_s - sin U_c)
+// and pass-through dims dx = U.  Key phase derivatives also sum into dbias (per block in LDS,
+// then one atomic per dim).  A thread takes 4 consecutive dims per step (D and R are multiples of
+// 8; the rows of q, k, dq, dk are 16-byte aligned): 16-byte loads of U, 8-byte loads and stores
+// of the bf16 / fp16 rows.
+template <typename T>
+__device__ __forceinline__ void load4(const uint16_t* p, float* x) {
+  const u32x2 w = *reinterpret_cast<const u32x2*>(p);
+  x[0] = T::to_float((uint16_t)(w[0] & 0xffffu));
+  x[1] = T::to_float((uint16_t)(w[0] >> 16));
+  x[2] = T::to_float((uint16_t)(w[1] & 0xffffu));
+  x[3] = T::to_float((uint16_t)(w[1] >> 16));
+}
+template <typename T>
+__device__ __forceinline__ void store4(uint16_t* p, const float* g) {
+  u32x2 w;
+  w[0] = T::pack2(g[0], g[1]);
+  w[1] = T::pack2(g[2], g[3]);
+  *reinterpret_cast<u32x2*>(p) = w;
+}
+// Sum of 4 consecutive floats over S partial rows `stride` floats apart, in order.
+__device__ __forceinline__ float4 sum4(const float* u, int S, int64_t stride) {
+  float4 a = *reinterpret_cast<const float4*>(u);
+#pragma unroll 4
+  for (int s = 1; s < S; ++s) {
+    const float4 b = *reinterpret_cast<const float4*>(u + s * stride);
+    a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+  }
+  return a;
+}
+template <typename T>
+__global__ __launch_bounds__(256) void flash_chain_kernel(FlashBwdParams p, int nk) {
+  const float* wk = p.wk;
+  const float* wq = p.wq;
+  __shared__ float dsum[256];
+  const int tid = threadIdx.x;
+  const int D = p.D, R = p.R, EP = p.EP;
+  if ((int)blockIdx.x < nk) {
+    const int nkb = (p.Nk + 31) / 32;
+    const int k0 = 32 * (blockIdx.x % nkb), bhk = blockIdx.x / nkb;
+    const int b = bhk / p.Hk, hk = bhk % p.Hk;
+    for (int d = tid; d < R; d += 256) dsum[d] = 0.f;
+    __syncthreads();
+    const uint16_t* kb = p.k + (int64_t)b * p.k_s[0] + (int64_t)hk * p.k_s[1];
+    uint16_t* dkb = p.dk + (int64_t)b * p.dk_s[0] + (int64_t)hk * p.dk_s[1];
+    const float2* tb = R ? p.table + (int64_t)b * p.t_sb + (int64_t)hk * p.t_sh : nullptr;
+    float* dfb = p.dfreqs ? p.dfreqs + (int64_t)b * p.df_s[0] + (int64_t)hk * p.df_s[1] : nullptr;
+    float* kpb = p.kpart ? p.kpart + (int64_t)bhk * p.Nk * R : nullptr;
+    const float* wrow = wk + (int64_t)bhk * p.NkP * EP;
+    const int S = p.kv_splits;
+    const int64_t sk = (int64_t)p.B * p.Hk * p.NkP * EP;
+    if (p.wv) {   // dV of the splits
+      const int64_t sv = (int64_t)p.B * p.Hk * p.NkP * p.DV;
+      const float* vrow = p.wv + (int64_t)bhk * p.NkP * p.DV;
+      uint16_t* dvb = p.dv + (int64_t)b * p.dv_s[0] + (int64_t)hk * p.dv_s[1];
+      for (int it = tid; it < 32 * (D / 4); it += 256) {
+        const int key = k0 + it / (D / 4), d = 4 * (it % (D / 4));
+        if (key >= p.Nk) continue;
+        const float4 a = sum4(vrow + (int64_t)key * p.DV + d, S, sv);
+        const float g[4] = {a.x, a.y, a.z, a.w};
+        store4<T>(dvb + (int64_t)key * p.dv_s[2] + d, g);
+      }
+    }
+    const int D4 = D / 4;
+    for (int it = tid; it < 32 * D4; it += 256) {
+      const int key = k0 + it / D4, d = 4 * (it % D4);
+      if (key >= p.Nk) continue;
+      const float* u = wrow + (int64_t)key * EP;
+      float g[4];
+      if (d < R) {   // R % 4 == 0: all four dims rotated
+        float x[4];
+        load4<T>(kb + (int64_t)key * p.k_s[2] + d, x);
+        const float4 c01 = *reinterpret_cast<const float4*>(tb + (int64_t)key * R + d);
+        const float4 c23 = *reinterpret_cast<const float4*>(tb + (int64_t)key * R + d + 2);
+        const float4 uc = sum4(u + d, S, sk), us = sum4(u + R + d, S, sk);
+        const float cs[4] = {c01.x, c01.z, c23.x, c23.z}, sn[4] = {c01.y, c01.w, c23.y, c23.w};
+        const float ucv[4] = {uc.x, uc.y, uc.z, uc.w}, usv[4] = {us.x, us.y, us.z, us.w};
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          g[t] = sigmoid_f(x[t]) * (cs[t] * ucv[t] + sn[t] * usv[t]);
+          const float dpsi = softplus_f(x[t]) * (cs[t] * usv[t] - sn[t] * ucv[t]);
+          if (kpb) {
+            kpb[(int64_t)key * R + d + t] = dpsi;
+          } else {
+            if (dfb) atomicAdd(dfb + (int64_t)key * p.df_s[2] + d + t, dpsi);
+            if (p.dbias) atomicAdd(&dsum[d + t], dpsi);
+          }
+        }
+      } else {
+        const float4 us = sum4(u + R + d, S, sk);
+        g[0] = us.x; g[1] = us.y; g[2] = us.z; g[3] = us.w;
+      }
+      store4<T>(dkb + (int64_t)key * p.dk_s[2] + d, g);
+    }
+    if (p.dbias && !kpb) {
+      __syncthreads();
+      for (int d = tid; d < R; d += 256) atomicAdd(p.dbias + (int64_t)hk * p.bias_sh + d, dsum[d]);
+    }
+    return;
+  }
+  const int nqb = (p.Nq + 31) / 32, blk = blockIdx.x - nk;
+  const int q0 = 32 * (blk % nqb), bh = blk / nqb;
+  const int b = bh / p.Hq, h = bh % p.Hq, hk = h % p.Hk;
+  const int q_off = p.Nk - p.Nq;
+  const uint16_t* qb = p.q + (int64_t)b * p.q_s[0] + (int64_t)h * p.q_s[1];
+  uint16_t* dqb = p.dq + (int64_t)b * p.dq_s[0] + (int64_t)h * p.dq_s[1];
+  const float2* tq = R ? p.table + (int64_t)b * p.t_sb + (int64_t)h * p.t_sh : nullptr;
+  const float2* bq = R ? p.btab + (p.Hb > 1 ? hk : 0) * R : nullptr;
+  float* dfb = p.dfreqs ? p.dfreqs + (int64_t)b * p.df_s[0] + (int64_t)h * p.df_s[1] : nullptr;
+  float* qpb = p.qpart && p.dfreqs ? p.qpart + (int64_t)bh * p.Nq * R : nullptr;
+  const float* wrow = wq + (int64_t)bh * p.NqP * EP;
+  const int S = p.q_splits;
+  const int64_t sq = (int64_t)p.B * p.Hq * p.NqP * EP;
+  const int D4 = D / 4;
+  for (int it = tid; it < 32 * D4; it += 256) {
+    const int i = q0 + it / D4, d = 4 * (it % D4);
+    if (i >= p.Nq) continue;
+    const float* u = wrow + (int64_t)i * EP;
+    float g[4];
+    if (d < R) {   // R % 4 == 0: all four dims rotated
+      float x[4];
+      load4<T>(qb + (int64_t)i * p.q_s[2] + d, x);
+      const float4 uc = sum4(u + d, S, sq), us = sum4(u + R + d, S, sq);
+      const float ucv[4] = {uc.x, uc.y, uc.z, uc.w}, usv[4] = {us.x, us.y, us.z, us.w};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        // cos / sin(F[q_off + i] - bias) from the tables of F and of the bias
+        const float2 tf = tq[(int64_t)(q_off + i) * R + d + t], tbv = bq[d + t];
+        const float cs = fmaf(tf.x, tbv.x, tf.y * tbv.y), sn = fmaf(tf.y, tbv.x, -tf.x * tbv.y);
+        g[t] = sigmoid_f(x[t]) * (cs * ucv[t] + sn * usv[t]);
+        const float dph = softplus_f(x[t]) * (cs * usv[t] - sn * ucv[t]);
+        if (qpb) qpb[(int64_t)i * R + d + t] = dph;
+        else if (dfb) atomicAdd(dfb + (int64_t)(q_off + i) * p.df_s[2] + d + t, dph);
+      }
+    } else {
+      const float4 us = sum4(u + R + d, S, sq);
+      g[0] = us.x; g[1] = us.y; g[2] = us.z; g[3] = us.w;
+    }
+    store4<T>(dqb + (int64_t)i * p.dq_s[2] + d, g);
+  }
+}
+
+}  // namespace
+
+hipError_t launch_flash_chain(const FlashBwdParams& p, const char* name, bool keys, bool queries, int dtype, hipStream_t s) {
+  const int nk = keys ? ((p.Nk + 31) / 32) * p.B * p.Hk : 0, nq = queries ? ((p.Nq + 31) / 32) * p.B * p.Hq : 0;
+  const dim3 grid(nk + nq);
+  return dtype == 2 ? launch_named(name, flash_chain_kernel<BF16>, grid, dim3(256), s, p, nk)
+                    : launch_named(name, flash_chain_kernel<F16>, grid, dim3(256), s, p, nk);
+}
+
+}  // namespace pope

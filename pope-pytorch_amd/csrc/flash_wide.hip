@@ -28,8 +28,8 @@
 //   wide_q     one workgroup per (query blocks, batch * head), wave = (32 queries, column chunk): S^T, dP^T with
 //              the K_hat and V tiles in LDS, dQ_hat^T (its chunk) += K_hat^T dS^T; writes the raw
 //              dQ_hat chunk.
-//   wide_chain the chain rule of the polar transform from the raw rows: dk, dq, dfreqs, dbias
-//              (deterministic mode: the per-row phase derivatives, summed later in a fixed order).
+//   flash_chain (flash_chain.hip) the chain rule of the polar transform from the raw rows: dk, dq,
+//              dfreqs, dbias (deterministic mode: the per-row phase derivatives).
 #include "pope_common.hpp"
 #include "pope_kernels.hpp"
 
@@ -545,127 +545,6 @@ __global__ __launch_bounds__(256) void wide_q_kernel(FlashBwdParams p, float* wq
     for (int r = 0; r < 16; ++r) wqb[32 * (ec * EBC + eb) + res_row(r, hf)] = dqa[eb][r] * p.scale;
 }
 
-// ---- the chain rule of the polar transform -----------------------------------------------
-// Blocks [0, nk): 32 key rows of one (batch, kv head); blocks [nk, nk + nq): 32 query rows of
-// one (batch, head).  With the raw expanded-row gradients U (cos column e = d, sin column
-// e = R + d, pass-through column e = R + d) and the row's phase (keys F[j]; queries
-// F[q_off + i] - bias, the bias on the query side as in the preparation):
-//   dx = sigmoid(x) (cos U_c + sin U_s),  dphase = softplus(x) (cos U_s - sin U_c)
-// and pass-through dims dx = U.  Key phase derivatives also sum into dbias (per block in LDS,
-// then one atomic per dim).  A thread takes 4 consecutive dims per step (D and R are multiples of
-// 8; the rows of q, k, dq, dk are 16-byte aligned): 16-byte loads of U, 8-byte loads and stores
-// of the bf16 / fp16 rows.
-template <typename T>
-__device__ __forceinline__ void load4(const uint16_t* p, float* x) {
-  const u32x2 w = *reinterpret_cast<const u32x2*>(p);
-  x[0] = T::to_float((uint16_t)(w[0] & 0xffffu));
-  x[1] = T::to_float((uint16_t)(w[0] >> 16));
-  x[2] = T::to_float((uint16_t)(w[1] & 0xffffu));
-  x[3] = T::to_float((uint16_t)(w[1] >> 16));
-}
-template <typename T>
-__device__ __forceinline__ void store4(uint16_t* p, const float* g) {
-  u32x2 w;
-  w[0] = T::pack2(g[0], g[1]);
-  w[1] = T::pack2(g[2], g[3]);
-  *reinterpret_cast<u32x2*>(p) = w;
-}
-template <typename T>
-__global__ __launch_bounds__(256) void wide_chain_kernel(FlashBwdParams p, const float* wk, const float* wq, int nk) {
-  __shared__ float dsum[256];
-  const int tid = threadIdx.x;
-  const int D = p.D, R = p.R, EP = p.EP;
-  if ((int)blockIdx.x < nk) {
-    const int nkb = p.NkP / 32;
-    const int k0 = 32 * (blockIdx.x % nkb), bhk = blockIdx.x / nkb;
-    const int b = bhk / p.Hk, hk = bhk % p.Hk;
-    if (k0 >= p.Nk) return;
-    for (int d = tid; d < R; d += 256) dsum[d] = 0.f;
-    __syncthreads();
-    const uint16_t* kb = p.k + (int64_t)b * p.k_s[0] + (int64_t)hk * p.k_s[1];
-    uint16_t* dkb = p.dk + (int64_t)b * p.dk_s[0] + (int64_t)hk * p.dk_s[1];
-    const float2* tb = R ? p.table + (int64_t)b * p.t_sb + (int64_t)hk * p.t_sh : nullptr;
-    float* dfb = p.dfreqs ? p.dfreqs + (int64_t)b * p.df_s[0] + (int64_t)hk * p.df_s[1] : nullptr;
-    float* kpb = p.kpart ? p.kpart + (int64_t)bhk * p.Nk * R : nullptr;
-    const float* wrow = wk + (int64_t)bhk * p.NkP * EP;
-    const int D4 = D / 4;
-    for (int it = tid; it < 32 * D4; it += 256) {
-      const int key = k0 + it / D4, d = 4 * (it % D4);
-      if (key >= p.Nk) continue;
-      const float* u = wrow + (int64_t)key * EP;
-      float g[4];
-      if (d < R) {   // R % 4 == 0: all four dims rotated
-        float x[4];
-        load4<T>(kb + (int64_t)key * p.k_s[2] + d, x);
-        const float4 c01 = *reinterpret_cast<const float4*>(tb + (int64_t)key * R + d);
-        const float4 c23 = *reinterpret_cast<const float4*>(tb + (int64_t)key * R + d + 2);
-        const float4 uc = *reinterpret_cast<const float4*>(u + d), us = *reinterpret_cast<const float4*>(u + R + d);
-        const float cs[4] = {c01.x, c01.z, c23.x, c23.z}, sn[4] = {c01.y, c01.w, c23.y, c23.w};
-        const float ucv[4] = {uc.x, uc.y, uc.z, uc.w}, usv[4] = {us.x, us.y, us.z, us.w};
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          g[t] = sigmoid_f(x[t]) * (cs[t] * ucv[t] + sn[t] * usv[t]);
-          const float dpsi = softplus_f(x[t]) * (cs[t] * usv[t] - sn[t] * ucv[t]);
-          if (kpb) {
-            kpb[(int64_t)key * R + d + t] = dpsi;
-          } else {
-            if (dfb) atomicAdd(dfb + (int64_t)key * p.df_s[2] + d + t, dpsi);
-            if (p.dbias) atomicAdd(&dsum[d + t], dpsi);
-          }
-        }
-      } else {
-        const float4 us = *reinterpret_cast<const float4*>(u + R + d);
-        g[0] = us.x; g[1] = us.y; g[2] = us.z; g[3] = us.w;
-      }
-      store4<T>(dkb + (int64_t)key * p.dk_s[2] + d, g);
-    }
-    if (p.dbias && !kpb) {
-      __syncthreads();
-      for (int d = tid; d < R; d += 256) atomicAdd(p.dbias + (int64_t)hk * p.bias_sh + d, dsum[d]);
-    }
-    return;
-  }
-  const int nqb = p.NqP / 32, blk = blockIdx.x - nk;
-  const int q0 = 32 * (blk % nqb), bh = blk / nqb;
-  const int b = bh / p.Hq, h = bh % p.Hq, hk = h % p.Hk;
-  if (q0 >= p.Nq) return;
-  const int q_off = p.Nk - p.Nq;
-  const uint16_t* qb = p.q + (int64_t)b * p.q_s[0] + (int64_t)h * p.q_s[1];
-  uint16_t* dqb = p.dq + (int64_t)b * p.dq_s[0] + (int64_t)h * p.dq_s[1];
-  const float2* tq = R ? p.table + (int64_t)b * p.t_sb + (int64_t)h * p.t_sh : nullptr;
-  const float2* bq = R ? p.btab + (p.Hb > 1 ? hk : 0) * R : nullptr;
-  float* dfb = p.dfreqs ? p.dfreqs + (int64_t)b * p.df_s[0] + (int64_t)h * p.df_s[1] : nullptr;
-  float* qpb = p.qpart && p.dfreqs ? p.qpart + (int64_t)bh * p.Nq * R : nullptr;
-  const float* wrow = wq + (int64_t)bh * p.NqP * EP;
-  const int D4 = D / 4;
-  for (int it = tid; it < 32 * D4; it += 256) {
-    const int i = q0 + it / D4, d = 4 * (it % D4);
-    if (i >= p.Nq) continue;
-    const float* u = wrow + (int64_t)i * EP;
-    float g[4];
-    if (d < R) {   // R % 4 == 0: all four dims rotated
-      float x[4];
-      load4<T>(qb + (int64_t)i * p.q_s[2] + d, x);
-      const float4 uc = *reinterpret_cast<const float4*>(u + d), us = *reinterpret_cast<const float4*>(u + R + d);
-      const float ucv[4] = {uc.x, uc.y, uc.z, uc.w}, usv[4] = {us.x, us.y, us.z, us.w};
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        // cos / sin(F[q_off + i] - bias) from the tables of F and of the bias
-        const float2 tf = tq[(int64_t)(q_off + i) * R + d + t], tbv = bq[d + t];
-        const float cs = fmaf(tf.x, tbv.x, tf.y * tbv.y), sn = fmaf(tf.y, tbv.x, -tf.x * tbv.y);
-        g[t] = sigmoid_f(x[t]) * (cs * ucv[t] + sn * usv[t]);
-        const float dph = softplus_f(x[t]) * (cs * usv[t] - sn * ucv[t]);
-        if (qpb) qpb[(int64_t)i * R + d + t] = dph;
-        else if (dfb) atomicAdd(dfb + (int64_t)(q_off + i) * p.df_s[2] + d + t, dph);
-      }
-    } else {
-      const float4 us = *reinterpret_cast<const float4*>(u + R + d);
-      g[0] = us.x; g[1] = us.y; g[2] = us.z; g[3] = us.w;
-    }
-    store4<T>(dqb + (int64_t)i * p.dq_s[2] + d, g);
-  }
-}
-
 template <typename T, int EP, int DV>
 hipError_t fwd_t(const FlashFwdParams& p, hipStream_t s) {
   const int blocks = ((p.Nq + 127) / 128) * p.B * p.Hq;
@@ -692,9 +571,12 @@ hipError_t bwd_t(const FlashBwdParams& p, float* wk, float* wq, hipStream_t s) {
   e = launch_named("flash_wide_q", wide_q_kernel<T, EP, DV, CQ>, dim3((p.NqP / (128 / CQ)) * p.B * p.Hq), dim3(256), s,
                    p, wq);
   if (e != hipSuccess) return e;
-  const int nk = (p.NkP / 32) * p.B * p.Hk, nq = (p.NqP / 32) * p.B * p.Hq;
-  return launch_named("flash_wide_chain", wide_chain_kernel<T>, dim3(nk + nq), dim3(256), s, p,
-                      (const float*)wk, (const float*)wq, nk);
+  FlashBwdParams c = p;   // both sides' raw rows, dV written already
+  c.kv_splits = c.q_splits = 1;
+  c.wk = wk;
+  c.wq = wq;
+  c.wv = nullptr;
+  return launch_flash_chain(c, "flash_wide_chain", true, true, T::kCode, s);
 }
 
 }  // namespace

@@ -241,6 +241,28 @@ size_t flash_partial_bytes(const pope_desc& d, int splits) {
   return align_up(rows * splits * d.D * sizeof(float)) + align_up(rows * splits * 2 * sizeof(float));
 }
 
+// Raw rows of a backward whose chain rule runs in its own launch (flash_bwd_split): wk (kv, B, Hk, NkP,
+// EP) | wv (kv, B, Hk, NkP, DV) for the key side, wq (q, B, Hq, NqP, EP) for the query side.  fp32.
+struct BwdPartials {
+  pope::FlashBwdSplit sp;
+  size_t wv, wq, total;
+};
+
+BwdPartials flash_bwd_partials(const pope_desc& d, const FlashLayout& L) {
+  BwdPartials r{{1, 1, false, false}, 0, 0, 0};
+  if (L.wide) return r;
+  r.sp = pope::flash_bwd_split(d.B, d.Hq, d.Hk, d.Nq, d.Nk, d.R, L.EP, L.DV, d.causal != 0);
+  size_t off = 0;
+  const size_t kr = (size_t)r.sp.kv * d.B * d.Hk * L.NkP, qr = (size_t)r.sp.q * d.B * d.Hq * L.NqP;
+  if (r.sp.raw_kv) off += align_up(kr * L.EP * sizeof(float));
+  r.wv = off;
+  if (r.sp.raw_kv) off += align_up(kr * L.DV * sizeof(float));
+  r.wq = off;
+  if (r.sp.raw_q) off += align_up(qr * L.EP * sizeof(float));
+  r.total = off;
+  return r;
+}
+
 // The flash kernels address the rows of v and do inside one (batch, head) with 32-bit element
 // offsets, up to one tile past the padded length.
 int check_row_span(const char* name, int rows_padded, int64_t row_stride) {
@@ -494,6 +516,7 @@ int pope_workspace_bytes(int op, const pope_desc* desc, size_t* bytes) {
     case POPE_OP_FLASH_BWD: *bytes = flash_ws(*desc, op); return POPE_OK;
     case POPE_OP_FLASH_DECODE: *bytes = decode_ws(*desc); return POPE_OK;
     case POPE_OP_POLAR_BWD: *bytes = det_bytes(*desc); return POPE_OK;
+    case POPE_OP_FLASH_BWD_PARTIALS: *bytes = flash_bwd_partials(*desc, flash_layout(*desc)).total; return POPE_OK;
     case POPE_OP_FLASH_FWD_PARTIALS:
       *bytes = flash_partial_bytes(*desc, flash_split(*desc, flash_layout(*desc)).splits);
       return POPE_OK;
@@ -572,6 +595,14 @@ int pope_flash_bwd(const pope_desc* d, const void* dout, const void* q, const vo
                    const void* o, const float* lse, const float* freqs, const float* bias, const uint8_t* mask,
                    void* dq, void* dk, void* dv, float* dfreqs, float* dbias, void* workspace,
                    size_t workspace_bytes, void* stream) {
+  return pope_flash_bwd_split(d, dout, q, k, v, o, lse, freqs, bias, mask, dq, dk, dv, dfreqs, dbias, workspace,
+                              workspace_bytes, nullptr, 0, stream);
+}
+
+int pope_flash_bwd_split(const pope_desc* d, const void* dout, const void* q, const void* k, const void* v,
+                         const void* o, const float* lse, const float* freqs, const float* bias, const uint8_t* mask,
+                         void* dq, void* dk, void* dv, float* dfreqs, float* dbias, void* workspace,
+                         size_t workspace_bytes, void* partials, size_t partials_bytes, void* stream) {
   int rc = check_flash_common(d, q, k, v, freqs, bias, mask, o, lse);
   if (rc) return rc;
   if (!dout || !dq || !dk || !dv) return fail(POPE_ERR_INVALID, "dout, dq, dk, dv must be non-NULL");
@@ -586,6 +617,11 @@ int pope_flash_bwd(const pope_desc* d, const void* dout, const void* q, const vo
   const FlashLayout L = flash_layout(*d);
   if ((rc = check_ws(L.total + L.wide_bytes + det_bytes(*d), workspace, workspace_bytes))) return rc;
   if ((rc = check_row_span("v", L.NkP, d->v_s[2])) || (rc = check_row_span("do", L.NqP, d->do_s[2]))) return rc;
+  BwdPartials bp{{1, 1, false, false}, 0, 0, 0};
+  if (partials) {
+    bp = flash_bwd_partials(*d, L);
+    if ((rc = check_ws(bp.total, partials, partials_bytes))) return rc;
+  }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
   if (!(d->flags & POPE_FLAG_PREPARED)) {
@@ -637,6 +673,15 @@ int pope_flash_bwd(const pope_desc* d, const void* dout, const void* q, const vo
   const DetParts dp = det_parts(*d, ws + L.total + L.wide_bytes, dfreqs, dbias);
   p.kpart = dp.kpart;
   p.qpart = dp.qpart;
+  p.kv_splits = bp.sp.kv;
+  p.q_splits = bp.sp.q;
+  p.raw_kv = bp.sp.raw_kv;
+  p.raw_q = bp.sp.raw_q;
+  if (p.raw_kv) {
+    p.wk = static_cast<float*>(partials);
+    p.wv = reinterpret_cast<float*>(static_cast<char*>(partials) + bp.wv);
+  }
+  if (p.raw_q) p.wq = reinterpret_cast<float*>(static_cast<char*>(partials) + bp.wq);
   hipError_t e;
   if (L.wide) {
     e = pope::launch_flash_bwd_delta(p, d->dtype, s);

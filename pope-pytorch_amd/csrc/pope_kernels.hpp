@@ -114,12 +114,23 @@ struct FlashBwdParams {
   int Bt, Ht, Hb;            // extents of the cos/sin table and of the bias rows
   int zero_grads;            // clear dfreqs / dbias before accumulating
   float* kpart; float* qpart;   // deterministic mode: per-row phase derivatives (PhaseGradParams), else null
+  // split jobs (flash_bwd_split): the steps of a dK/dV job over kv_splits workgroups, of a dQ job over
+  // q_splits; raw sides (every split one): fp32 partial rows wk (kv_splits, B, Hk, NkP, EP), wv (.., DV),
+  // wq (q_splits, B, Hq, NqP, EP), merged by launch_flash_chain
+  int kv_splits, q_splits, raw_kv, raw_q;
+  float* wk; float* wv; float* wq;
   int n_kv_jobs, interleave; // dK/dV jobs of the fused launch; 1 = pair dK/dV and dQ jobs by cost
   float scale;
   int64_t q_s[3], k_s[3], v_s[3], o_s[3], do_s[3], dq_s[3], dk_s[3], dv_s[3], df_s[3];
   int64_t bias_sh, mask_sb, t_sb, t_sh;
 };
 hipError_t launch_flash_bwd(const FlashBwdParams& p, int dtype, hipStream_t s);
+hipError_t launch_flash_bwd_f16(const FlashBwdParams& p, hipStream_t s);
+struct FlashBwdSplit { int kv, q; bool raw_kv, raw_q; };   // raw: the side's rows go through the chain launch
+FlashBwdSplit flash_bwd_split(int B, int Hq, int Hk, int Nq, int Nk, int R, int EP, int DV, bool causal);
+// dk / dq (and dfreqs, dbias) from raw rows wk / wq: the sum of their kv_splits / q_splits partials
+// through the chain rule; dv from wv when non-null.  `keys` / `queries` choose the sides.
+hipError_t launch_flash_chain(const FlashBwdParams& p, const char* name, bool keys, bool queries, int dtype, hipStream_t s);
 // The backward's row terms alone (-lse log2 e and -delta per query row; dfreqs / dbias cleared
 // with zero_grads): the wide path's first launch.
 hipError_t launch_flash_bwd_delta(const FlashBwdParams& p, int dtype, hipStream_t s);

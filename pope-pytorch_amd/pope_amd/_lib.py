@@ -19,7 +19,7 @@ FLAG_PREPARED, FLAG_ZERO_GRADS, FLAG_SPLIT_BF16, FLAG_COMPLEX, FLAG_DETERMINISTI
 
 POPE_F32, POPE_F16, POPE_BF16 = 0, 1, 2
 (OP_SIM_FWD, OP_SIM_BWD, OP_FLASH_FWD, OP_FLASH_BWD, OP_FLASH_DECODE, OP_POLAR_BWD,
- OP_FLASH_FWD_PARTIALS) = range(7)
+ OP_FLASH_FWD_PARTIALS, OP_FLASH_BWD_PARTIALS) = range(8)
 
 _DTYPE_CODE = {torch.float32: POPE_F32, torch.float16: POPE_F16, torch.bfloat16: POPE_BF16}
 
@@ -42,7 +42,7 @@ class PopeDesc(ctypes.Structure):
 
 EXPORTS = (
     "pope_abi_version", "pope_last_error", "pope_workspace_bytes", "pope_sim_fwd", "pope_sim_bwd",
-    "pope_flash_fwd", "pope_flash_fwd_split", "pope_flash_bwd", "pope_flash_decode", "pope_flash_decode_noalloc", "pope_polar_fwd",
+    "pope_flash_fwd", "pope_flash_fwd_split", "pope_flash_bwd", "pope_flash_bwd_split", "pope_flash_decode", "pope_flash_decode_noalloc", "pope_polar_fwd",
     "pope_polar_bwd", "pope_profile_enable", "pope_profile_read", "pope_profile_reset",
 )
 
@@ -69,6 +69,8 @@ def _declare(lib):
     lib.pope_flash_fwd_split.argtypes = [dp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp, sz, vp]
     lib.pope_flash_bwd.restype = i32
     lib.pope_flash_bwd.argtypes = [dp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp]
+    lib.pope_flash_bwd_split.restype = i32
+    lib.pope_flash_bwd_split.argtypes = [dp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp, sz, vp]
     lib.pope_flash_decode.restype = i32
     lib.pope_flash_decode.argtypes = [dp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp]
     lib.pope_flash_decode_noalloc.restype = i32

@@ -354,20 +354,21 @@ def _bwd_impl(do, q, k, v, o, lse, freqs, bias, mask, causal, softmax_scale, nee
         # the same descriptor with PREPARED set, for calls that bring the forward's workspace
         dp = _lib.PopeDesc.from_buffer_copy(d)
         dp.flags |= _lib.FLAG_PREPARED
-        return d, dp, _lib.workspace_bytes(_lib.OP_FLASH_BWD, d)
+        return d, dp, _lib.workspace_bytes(_lib.OP_FLASH_BWD, d), _lib.workspace_bytes(_lib.OP_FLASH_BWD_PARTIALS, d)
 
-    d, dprep, need = _plan(key, build)
+    d, dprep, need, part_bytes = _plan(key, build)
     global _LAST_BWD_PREPARED
     _LAST_BWD_PREPARED = exists(fwd_ws) and fwd_ws.numel() == need
     if _LAST_BWD_PREPARED:
         ws, d = fwd_ws, dprep
     else:
         ws = torch.empty(need, dtype=torch.uint8, device=q.device)
-    st = _lib.lib().pope_flash_bwd(
+    parts = torch.empty(part_bytes, dtype=torch.uint8, device=q.device) if part_bytes else None
+    st = _lib.lib().pope_flash_bwd_split(
         ctypes.byref(d), do.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
         _data(freqs), _data(bias), _data(mask), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
         dfreqs.data_ptr() if need_dfreqs else None, dbias.data_ptr() if need_dbias else None,
-        ws.data_ptr(), need, _stream(q))
+        ws.data_ptr(), need, _data(parts), part_bytes, _stream(q))
     _lib.check(st, "flash backward")
     return dq, dk, dv, dfreqs, dbias
 

@@ -101,3 +101,45 @@ def test_decode_head_groups(cuda, Hq, Hk, D, Nk):
     ref = oracle_attention(inp, False, grads=False)
     o = pope_amd.flash_attn_with_pope(inp["q"], inp["k"], inp["v"], pos_emb=(inp["freqs"], inp["bias"]), mask=inp["mask"])
     assert excess_over(o, ref["o"], 2e-2) <= 0
+
+
+BWD_CASES = [
+    # B, Hq, Hk, Nq, Nk, D, R, mask, causal, dtype: split dK/dV and dQ jobs, or (R % 32 != 0) raw rows alone
+    (1, 8, 1, 700, 700, 64, 64, "prefix", True, torch.bfloat16),
+    (1, 1, 1, 1500, 1500, 64, 32, "half", True, torch.float16),
+    (1, 2, 2, 1300, 1300, 32, 32, "none", False, torch.bfloat16),
+    (1, 4, 1, 641, 900, 128, 64, "random", False, torch.bfloat16),
+    (1, 2, 1, 1025, 1025, 128, 128, "none", True, torch.float16),
+    (1, 4, 2, 33, 1200, 96, 96, "prefix", False, torch.bfloat16),
+    (2, 2, 2, 70, 129, 64, 24, "dead_row", True, torch.bfloat16),
+    (1, 2, 2, 257, 257, 80, 40, "prefix", True, torch.float16),
+]
+
+
+@pytest.mark.parametrize("deterministic", [False, True])
+@pytest.mark.parametrize("case", BWD_CASES, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
+def test_split_backward_against_the_oracle(cuda, case, deterministic):
+    """dq, dk, dv within the flash tests' bound, dbias and dfreqs within 2e-2 max(1, ||ref||_inf), through the
+    partial rows and their merge."""
+    import pope_amd
+    from pope_amd import _lib
+    B, Hq, Hk, Nq, Nk, D, R, mask, causal, dtype = case
+    inp = make_pope_inputs(8700 + Nk, B, Hq, Hk, Nq, Nk, D, R, dtype, mask)
+    ref = oracle_attention(inp, causal)
+    leaves = [inp[n].detach().requires_grad_(True) for n in ("q", "k", "v", "freqs", "bias")]
+    torch.use_deterministic_algorithms(deterministic)
+    try:
+        o = pope_amd.flash_attn_with_pope(*leaves[:3], pos_emb=tuple(leaves[3:]), mask=inp["mask"], causal=causal)
+        _lib.profile_reset()
+        _lib.profile_enable(True)
+        grads = torch.autograd.grad(o, leaves, inp["do"])
+        torch.cuda.synchronize()
+        _lib.profile_enable(False)
+    finally:
+        torch.use_deterministic_algorithms(False)
+    assert "flash_chain" in _lib.profile_read()
+    for got, name in zip(grads, ("dq", "dk", "dv", "dfreqs", "dbias")):
+        if name in ("dfreqs", "dbias"):
+            assert (got.double().cpu() - ref[name]).abs().max().item() <= 2e-2 * max(1.0, ref[name].abs().max().item()), name
+        else:
+            assert excess_over(got, ref[name], 2e-2) <= 0, name
