@@ -250,6 +250,21 @@ int pope_polar_bwd(const pope_desc* desc, const float* dq_hat, const float* dk_h
                    void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * fp32 -> fp16 conversion of up to three (b, h, n, d) tensors (the flash operands of an fp32 call)
+ * with their range check, in one launch.  Any element strides (>= 0).  *flag is set to 1 when some
+ * value is finite and beyond fp16's range (|x| > 65504); it is not cleared, and may be device or
+ * pinned host memory.  The reference runs fp32 inputs at TF32 (triton_pope_flash_attn.py:80).
+ */
+typedef struct pope_cast {
+  const float* src;
+  void* dst;                  /* fp16 */
+  int32_t shape[4];
+  int64_t src_s[4], dst_s[4]; /* element strides */
+} pope_cast;
+
+int pope_cast_f16(const pope_cast* tensors, int n, uint32_t* flag, void* stream);
+
+/*
  * Per-kernel timing.  No counterpart in the reference (its tests print only
  * parity diffs, tests/test_flash_attn.py:61,109).  While enabled, every kernel
  * launch of the library carries a pair of hipEvents that its dispatch stamps with

@@ -699,6 +699,33 @@ int pope_flash_bwd_split(const pope_desc* d, const void* dout, const void* q, co
   return POPE_OK;
 }
 
+int pope_cast_f16(const pope_cast* tensors, int n, uint32_t* flag, void* stream) {
+  if (!tensors || n < 1 || n > 3) return fail(POPE_ERR_INVALID, "cast takes 1 to 3 tensors (got %d)", n);
+  if (!flag) return fail(POPE_ERR_INVALID, "cast flag is NULL");
+  pope::CastParams p;
+  std::memset(&p, 0, sizeof p);
+  p.n = n;
+  p.flag = flag;
+  for (int t = 0; t < n; ++t) {
+    const pope_cast& c = tensors[t];
+    bool empty = false;
+    for (int i = 0; i < 4; ++i) {
+      if (c.shape[i] < 0 || c.src_s[i] < 0 || c.dst_s[i] < 0)
+        return fail(POPE_ERR_INVALID, "cast tensor %d: negative shape or stride", t);
+      empty = empty || c.shape[i] == 0;
+      p.t[t].shape[i] = c.shape[i];
+      p.t[t].src_s[i] = c.src_s[i];
+      p.t[t].dst_s[i] = c.dst_s[i];
+    }
+    if (!empty && (!c.src || !c.dst)) return fail(POPE_ERR_INVALID, "cast tensor %d: NULL data", t);
+    p.t[t].src = c.src;
+    p.t[t].dst = static_cast<uint16_t*>(c.dst);
+  }
+  const hipError_t e = pope::launch_cast_f16(p, 65504.f, reinterpret_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "fp16 cast launch");
+  return POPE_OK;
+}
+
 int pope_flash_decode(const pope_desc* d, const void* q, const void* k, const void* v, const float* freqs,
                       const float* bias, const uint8_t* mask, void* o, float* lse, void* workspace,
                       size_t workspace_bytes, void* stream) {

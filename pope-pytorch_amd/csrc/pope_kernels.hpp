@@ -205,6 +205,22 @@ struct PhaseGradParams {
 size_t phase_grad_slices(int Hb, int R);
 hipError_t launch_phase_grad_reduce(const PhaseGradParams& p, hipStream_t s);
 
+// fp32 -> fp16 copies of up to three (b, h, n, d) tensors with any element strides; *flag = 1 when a
+// finite value exceeds `limit` in magnitude (never cleared here).
+struct CastTensor {
+  const float* src; uint16_t* dst;
+  int shape[4];
+  int64_t src_s[4], dst_s[4];
+  int64_t items;             // set by launch_cast_f16
+};
+struct CastParams {
+  CastTensor t[3];
+  int n;
+  uint32_t* flag;
+  int64_t items;             // set by launch_cast_f16
+};
+hipError_t launch_cast_f16(const CastParams& p, float limit, hipStream_t s);
+
 struct DecodeParams {
   const uint16_t* q; const uint16_t* k; const uint16_t* v;
   const float* freqs; const float* bias; const uint8_t* mask;   // freqs rows 16-byte aligned

@@ -40,10 +40,17 @@ class PopeDesc(ctypes.Structure):
     ]
 
 
+class PopeCast(ctypes.Structure):
+    """Mirror of ``struct pope_cast`` (include/pope_abi.h)."""
+
+    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("shape", ctypes.c_int32 * 4),
+                ("src_s", ctypes.c_int64 * 4), ("dst_s", ctypes.c_int64 * 4)]
+
+
 EXPORTS = (
     "pope_abi_version", "pope_last_error", "pope_workspace_bytes", "pope_sim_fwd", "pope_sim_bwd",
     "pope_flash_fwd", "pope_flash_fwd_split", "pope_flash_bwd", "pope_flash_bwd_split", "pope_flash_decode", "pope_flash_decode_noalloc", "pope_polar_fwd",
-    "pope_polar_bwd", "pope_profile_enable", "pope_profile_read", "pope_profile_reset",
+    "pope_polar_bwd", "pope_cast_f16", "pope_profile_enable", "pope_profile_read", "pope_profile_reset",
 )
 
 _lib = None
@@ -79,6 +86,8 @@ def _declare(lib):
     lib.pope_polar_fwd.argtypes = [dp, vp, vp, vp, vp, vp, vp, vp]
     lib.pope_polar_bwd.restype = i32
     lib.pope_polar_bwd.argtypes = [dp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp]
+    lib.pope_cast_f16.restype = i32
+    lib.pope_cast_f16.argtypes = [ctypes.POINTER(PopeCast), i32, vp, vp]
     lib.pope_profile_enable.restype = i32
     lib.pope_profile_enable.argtypes = [i32]
     lib.pope_profile_read.restype = i32

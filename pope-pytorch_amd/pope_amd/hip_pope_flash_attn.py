@@ -151,23 +151,62 @@ def _check_dtypes(q, *others):
             raise TypeError(f"pope_amd flash: operand of dtype {t.dtype} next to q of dtype {q.dtype}")
 
 
+def _launch_half(ts, flag):
+    """fp16 copies (strides as Tensor.to keeps them) of the fp32 tensors ``ts`` in one launch; the int32
+    ``flag`` (pinned host memory) is set to 1 when a finite value lies beyond fp16's range."""
+    out = tuple(torch.empty_like(t, dtype=torch.float16) for t in ts)
+    c = (_lib.PopeCast * len(ts))()
+    for i, (t, o) in enumerate(zip(ts, out)):
+        c[i].src, c[i].dst = t.data_ptr(), o.data_ptr()
+        c[i].shape[:], c[i].src_s[:], c[i].dst_s[:] = t.shape, t.stride(), o.stride()
+    _lib.check(_lib.lib().pope_cast_f16(c, len(ts), flag.data_ptr(), _stream(ts[0])), "fp16 cast")
+    return out
+
+
+class _HalfOperands(torch.autograd.Function):
+    """q, k, v in fp16; gradients go back in fp32, as through Tensor.to."""
+
+    @staticmethod
+    def forward(ctx, flag, q, k, v):
+        return _launch_half((q, k, v), flag)
+
+    @staticmethod
+    def backward(ctx, dq, dk, dv):
+        return None, *(g.float() if n else None for g, n in zip((dq, dk, dv), ctx.needs_input_grad[1:]))
+
+
 _FP16_MAX = 65504.0
 
 
 def _check_fp16_range(*ts):
-    """fp32 flash inputs run on fp16 operands: a finite value beyond fp16's range would become inf
-    silently, so such inputs raise instead.  The check reads one flag back to the host (fp32 flash
-    is the compatibility path; the bf16 / fp16 paths never synchronise); under torch.compile
-    tracing it is skipped."""
-    if torch.compiler.is_compiling():
-        return
+    """The same check with torch operators, for operands of mixed or other dtypes (reads one flag back)."""
     bad = torch.zeros((), dtype=torch.bool, device=ts[0].device)
     for t in ts:
         bad |= ((t.abs() > _FP16_MAX) & t.isfinite()).any()
     if bool(bad):
-        raise ValueError("pope_amd flash: fp32 q / k / v run on fp16 operands (10-bit mantissa, as the "
-                         "reference's TF32 products) and must stay within fp16's range |x| <= 65504; "
-                         "scale the inputs or pass bf16")
+        raise ValueError(_RANGE_ERROR)
+
+
+_RANGE_ERROR = ("pope_amd flash: fp32 q / k / v run on fp16 operands (10-bit mantissa, as the reference's TF32 "
+                "products) and must stay within fp16's range |x| <= 65504; scale the inputs or pass bf16")
+
+
+class _RangeCheck:
+    """Range check of an fp32 call's operands.  They run on fp16: a finite value beyond fp16's range would
+    become inf silently, so such inputs raise instead.  The conversion kernel writes the flag into pinned host memory and
+    an event after it is waited for once the call's other kernels are on the stream, so the one
+    readback of fp32 flash (the compatibility path; the bf16 / fp16 paths never synchronise) does not
+    leave the GPU idle."""
+
+    def __init__(self):
+        self.flag = torch.empty(1, dtype=torch.int32, pin_memory=True)
+        self.flag[0] = 0
+        self.event = torch.cuda.Event()
+
+    def raise_if_out_of_range(self):
+        """After ``event.synchronize()``."""
+        if int(self.flag[0]):
+            raise ValueError(_RANGE_ERROR)
 
 
 _INT32_MAX = 2 ** 31 - 1
@@ -470,24 +509,41 @@ def flash_attn_head_first(q: Tensor, k: Tensor, v: Tensor, freqs: Optional[Tenso
     freqs, pope_bias = _prep_pope(freqs, pope_bias)
     mask = _prep_mask(mask, q.shape[0])
     out_dtype = q.dtype
+    check = None
     if q.dtype not in _MFMA_DTYPES:
         # fp32 inputs: fp16 operands keep 10 significant bits, as the TF32 products of the
         # reference's fp32 path do (triton_pope_flash_attn.py:80), but not TF32's exponent range
-        _check_fp16_range(q, k, v)
-        q, k, v = q.to(torch.float16), k.to(torch.float16), v.to(torch.float16)
-    if k.dtype != q.dtype:
-        k = k.to(q.dtype)
-    if v.dtype != q.dtype:
-        v = v.to(q.dtype)
-    # head / rotate dims that are not multiples of 8: padded on the device (pope_amd._pad)
-    plan = pad_plan(q.shape[-1], freqs.shape[-1] if exists(freqs) else 0)
-    if plan is not None:
-        q, k, v = pad_qk(q, plan), pad_qk(k, plan), pad_last(v, plan.Dp)
-        freqs, pope_bias = pad_last(freqs, plan.R8), pad_last(pope_bias, plan.R8)
-    o = _flash(q, k, v, freqs, pope_bias, mask, causal, float(scale))
-    if plan is not None:
-        o = o[..., :plan.D]
-    return o.to(out_dtype) if o.dtype != out_dtype else o
+        # (under torch.compile tracing, and for other dtypes than fp32, plain conversions)
+        if not torch.compiler.is_compiling() and q.dtype == k.dtype == v.dtype == torch.float32:
+            check = _RangeCheck()
+            q, k, v = _HalfOperands.apply(check.flag, q, k, v)
+            check.event.record(torch.cuda.current_stream(q.device))
+        else:
+            if not torch.compiler.is_compiling():
+                _check_fp16_range(q, k, v)
+            q, k, v = q.to(torch.float16), k.to(torch.float16), v.to(torch.float16)
+    try:
+        if k.dtype != q.dtype:
+            k = k.to(q.dtype)
+        if v.dtype != q.dtype:
+            v = v.to(q.dtype)
+        # head / rotate dims that are not multiples of 8: padded on the device (pope_amd._pad)
+        plan = pad_plan(q.shape[-1], freqs.shape[-1] if exists(freqs) else 0)
+        if plan is not None:
+            q, k, v = pad_qk(q, plan), pad_qk(k, plan), pad_last(v, plan.Dp)
+            freqs, pope_bias = pad_last(freqs, plan.R8), pad_last(pope_bias, plan.R8)
+        o = _flash(q, k, v, freqs, pope_bias, mask, causal, float(scale))
+        if plan is not None:
+            o = o[..., :plan.D]
+        if o.dtype != out_dtype:
+            o = o.to(out_dtype)
+    finally:
+        # also when the call fails: the flag's memory is not given back before the kernel that may write it is done
+        if exists(check):
+            check.event.synchronize()
+    if exists(check):
+        check.raise_if_out_of_range()
+    return o
 
 
 # ------------------------------------------------- reference-named (b, n, h, d) API
