@@ -1,6 +1,6 @@
 // Per-call cos/sin table of the PoPE phases.
 //
-// tab[((bt * Ht + ht) * rows + n) * R + d] = (cos th, sin th), fp32 pairs or fp16 pairs,
+// tab[((bt * Ht + ht) * rows + n) * R + d] = (cos th, sin th), fp32 pairs,
 //   th = fl(F[bt, ht, n, d] + bias[ht, d])   (bias optional)
 // The sum is rounded to fp32 before the trig call, as the reference does
 // (freqs_with_bias = freqs + bias, pope.py:56; theta_k = fk + bias,
@@ -11,7 +11,10 @@
 
 namespace pope {
 
-__global__ __launch_bounds__(256) void phase_table_kernel(TableParams p) {
+// blockIdx.y: the table (the fp32 similarity's key and query tables go in one launch: 2 x 4.4 -> 4.6 us
+// at 1,024 rows of 64).
+__global__ __launch_bounds__(256) void phase_table_kernel(TableParams p0, TableParams p1) {
+  const TableParams& p = blockIdx.y ? p1 : p0;
   // four consecutive entries of one row per thread (R is a multiple of 8): four independent
   // loads, 16-byte stores; the index is decomposed in 32 bits when the table allows
   const int64_t total = (int64_t)p.Bt * p.Ht * p.rows * p.R;
@@ -44,25 +47,19 @@ __global__ __launch_bounds__(256) void phase_table_kernel(TableParams p) {
     }
 #pragma unroll
     for (int t = 0; t < 4; ++t) sincos_acc(th[t], &sn[t], &cs[t]);
-    if (p.out16) {
-      u32x4 w;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) w[t] = __builtin_bit_cast(uint32_t, f16x2{(_Float16)cs[t], (_Float16)sn[t]});
-      *reinterpret_cast<u32x4*>(p.out16 + i4) = w;
-    } else {
-      float4* dst = reinterpret_cast<float4*>(p.out + i4);
-      dst[0] = make_float4(cs[0], sn[0], cs[1], sn[1]);
-      dst[1] = make_float4(cs[2], sn[2], cs[3], sn[3]);
-    }
+    float4* dst = reinterpret_cast<float4*>(p.out + i4);
+    dst[0] = make_float4(cs[0], sn[0], cs[1], sn[1]);
+    dst[1] = make_float4(cs[2], sn[2], cs[3], sn[3]);
   }
 }
 
-hipError_t launch_phase_table(const TableParams& p, hipStream_t s) {
-  const int64_t total = (int64_t)p.Bt * p.Ht * p.rows * p.R;
-  if (total == 0) return hipSuccess;
-  int64_t blocks = (total / 4 + 255) / 256;   // four entries per thread
+hipError_t launch_phase_tables(const TableParams& p0, const TableParams& p1, hipStream_t s) {
+  const auto total = [](const TableParams& p) { return (int64_t)p.Bt * p.Ht * p.rows * p.R; };
+  const int64_t most = total(p0) > total(p1) ? total(p0) : total(p1);
+  if (most == 0) return hipSuccess;
+  int64_t blocks = (most / 4 + 255) / 256;   // four entries per thread
   if (blocks > 4096) blocks = 4096;
-  return launch_named("phase_table", phase_table_kernel, dim3((unsigned)blocks), dim3(256), s, p);
+  return launch_named("phase_table", phase_table_kernel, dim3((unsigned)blocks, 2), dim3(256), s, p0, p1);
 }
 
 }  // namespace pope

@@ -315,14 +315,21 @@ size_t sim_table_q(const pope_desc& d) {
   const int Hqt = d.f_s[1] != 0 ? d.Hq : 1;
   return d.R > 0 ? align_up((size_t)Bt * Hqt * d.Nk * d.R * sizeof(float2)) : 0;
 }
-// Similarity workspace: [key table | query table | (backward) U | W | (split) Q_hat hi | lo |
+// Partial buffers of U and W in the backward (the split-bf16 path has its second ones elsewhere).
+pope::SimBwdSplit sim_splits(const pope_desc& d, int EP) {
+  if (d.flags & POPE_FLAG_SPLIT_BF16) return {1, 1};
+  return pope::sim_bwd_split(d.B, d.Hq, d.Hk, d.Nq, d.Nk, EP);
+}
+
+// Similarity workspace: [key table | query table | (backward) partial sums of U | of W | (split) Q_hat hi | lo |
 // K_hat hi | lo planes, rows padded to 128].
 size_t sim_ws(const pope_desc& d, int op) {
   const int EP = round_up(d.D + d.R, 32);
   size_t n = sim_table_k(d) + sim_table_q(d);
   if (op == POPE_OP_SIM_BWD) {
-    n += align_up((size_t)d.B * d.Hq * d.Nq * EP * sizeof(float));
-    n += align_up((size_t)d.B * d.Hk * d.Nk * EP * sizeof(float));
+    const pope::SimBwdSplit sp = sim_splits(d, EP);
+    n += sp.u * align_up((size_t)d.B * d.Hq * d.Nq * EP * sizeof(float));
+    n += sp.w * align_up((size_t)d.B * d.Hk * d.Nk * EP * sizeof(float));
   }
   if (d.flags & POPE_FLAG_SPLIT_BF16) {
     n += 2 * align_up((size_t)d.B * d.Hq * round_up(d.Nq, 128) * EP * sizeof(uint16_t));
@@ -374,10 +381,8 @@ size_t decode_ws(const pope_desc& d) {
   return align_up(rows * splits * d.D * sizeof(float)) + align_up(rows * splits * 2 * sizeof(float));
 }
 
-hipError_t build_table(const pope_desc& d, const float* freqs, const float* bias, int Bt, int Ht,
-                       float2* out, hipStream_t s, uint32_t* out16 = nullptr) {
+pope::TableParams phase_table(const pope_desc& d, const float* freqs, const float* bias, int Bt, int Ht, float2* out) {
   pope::TableParams t;
-  t.out16 = out16;
   t.freqs = freqs;
   t.f_sb = d.f_s[0];
   t.f_sh = d.f_s[1];
@@ -389,7 +394,7 @@ hipError_t build_table(const pope_desc& d, const float* freqs, const float* bias
   t.rows = d.Nk;
   t.R = d.R;
   t.out = out;
-  return pope::launch_phase_table(t, s);
+  return t;
 }
 
 void copy3(int64_t* dst, const int64_t* src) {
@@ -448,9 +453,8 @@ hipError_t sim_setup(const pope_desc& d, const void* q, const void* k, const flo
   // the fp32 kernels read the phases from tables; the split-bf16 kernels compute them in place
   const bool tables = d.R > 0 && !(d.flags & POPE_FLAG_SPLIT_BF16);
   if (tables) {
-    hipError_t e = build_table(d, freqs, bias, Bt, d.Hk, ktab, s);
-    if (e != hipSuccess) return e;
-    e = build_table(d, freqs, nullptr, Bt, Hqt, qtab, s);  // query phases never carry the bias
+    const hipError_t e = pope::launch_phase_tables(phase_table(d, freqs, bias, Bt, d.Hk, ktab),
+                                                   phase_table(d, freqs, nullptr, Bt, Hqt, qtab), s);   // query phases never carry the bias
     if (e != hipSuccess) return e;
   }
   p.q = static_cast<const float*>(q);
@@ -853,7 +857,10 @@ int pope_sim_bwd(const pope_desc* d, const void* dsim, const void* q, const void
   copy3(p.df_s, d->df_s);
   const size_t off_u = sim_table_k(*d) + sim_table_q(*d);
   float* U = reinterpret_cast<float*>(ws + off_u);
-  float* W = reinterpret_cast<float*>(ws + off_u + align_up((size_t)d->B * d->Hq * d->Nq * p.EP * sizeof(float)));
+  const pope::SimBwdSplit sp = sim_splits(*d, p.EP);
+  const size_t ub = align_up((size_t)d->B * d->Hq * d->Nq * p.EP * sizeof(float));
+  const size_t wb = align_up((size_t)d->B * d->Hk * d->Nk * p.EP * sizeof(float));
+  float* W = reinterpret_cast<float*>(ws + off_u + sp.u * ub);
   const DetParts dp = det_parts(*d, ws + sim_ws(*d, POPE_OP_SIM_BWD) - det_bytes(*d), dfreqs, dbias);
   p.kpart = dp.kpart;
   p.qpart = dp.qpart;
@@ -866,7 +873,8 @@ int pope_sim_bwd(const pope_desc* d, const void* dsim, const void* q, const void
   if (d->flags & POPE_FLAG_SPLIT_BF16)
     e = pope::launch_sim_split_bwd(p, sim_split_planes(*d, ws, POPE_OP_SIM_BWD), U, W, s);
   else
-    e = pope::launch_sim_bwd_ws(p, U, W, s);
+    e = pope::launch_sim_bwd_ws(p, pope::SimAcc{U, sp.u, (int64_t)(ub / sizeof(float))},
+                                pope::SimAcc{W, sp.w, (int64_t)(wb / sizeof(float))}, s);
   if (e != hipSuccess) return hip_fail(e, "similarity backward launch");
   e = det_reduce(*d, dp, dfreqs, dbias, zero, s);
   if (e != hipSuccess) return hip_fail(e, "phase gradient reduction launch");

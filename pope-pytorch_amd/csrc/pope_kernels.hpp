@@ -38,10 +38,9 @@ struct TableParams {
   const float* freqs; int64_t f_sb, f_sh, f_sn;
   const float* bias; int64_t bias_sh;  // may be null
   int Bt, Ht, rows, R;
-  float2* out;               // fp32 (cos, sin), or
-  uint32_t* out16;           // fp16 (cos, sin) pairs packed per 32-bit word when non-null
+  float2* out;               // fp32 (cos, sin)
 };
-hipError_t launch_phase_table(const TableParams& p, hipStream_t s);
+hipError_t launch_phase_tables(const TableParams& p0, const TableParams& p1, hipStream_t s);
 
 // Shared preparation of the flash forward and backward (flash_prep.hip, one launch), written
 // into the caller's workspace once per forward call and reused by the backward: K_hat and the
@@ -156,12 +155,18 @@ struct SimParams {
   int64_t bias_sh, kt_sb, kt_sh, qt_sb, qt_sh;
 };
 hipError_t launch_sim_fwd(const SimParams& p, hipStream_t s);
-// U: (B, Hq, Nq, EP) and W: (B, Hk, Nk, EP) fp32 workspace.
-hipError_t launch_sim_bwd_ws(const SimParams& p, float* U, float* W, hipStream_t s);
-// Chain rule of the polar transform on U (queries) and W (keys) (sim.hip); U2 / W2 are second
-// partial sums added to them, or null.
-hipError_t launch_sim_finalize(const SimParams& p, const float* U, const float* U2, const float* W, const float* W2,
-                               hipStream_t s);
+// Partial sums of U and W: n buffers of (B, Hq, Nq, EP) / (B, Hk, Nk, EP) fp32, `stride` floats apart.
+struct SimAcc {
+  float* p;
+  int n;
+  int64_t stride;
+};
+// Splits of the reductions of U (over keys) and W (over query rows) in the fp32 backward.
+struct SimBwdSplit { int u, w; };
+SimBwdSplit sim_bwd_split(int B, int Hq, int Hk, int Nq, int Nk, int EP);
+hipError_t launch_sim_bwd_ws(const SimParams& p, const SimAcc& U, const SimAcc& W, hipStream_t s);
+// Chain rule of the polar transform on the sums of U (queries) and W (keys) (sim.hip).
+hipError_t launch_sim_finalize(const SimParams& p, const SimAcc& U, const SimAcc& W, hipStream_t s);
 
 // Split-bf16 similarity (sim_split.hip): hi / lo bf16 planes of Q_hat and K_hat, rows padded
 // to 128, row-major (heads, NP, EP) for the forward or transposed (heads, EP, NP) for the

@@ -19,6 +19,8 @@
 //   dpsi = c (cos psi W_s - sin psi W_c)  -> dfreqs rows j and dbias (sum over j).
 // dbias = sum_j dpsi replaces the reference's third pass over dS
 // (_bwd_kernel_dbias_optimized): both are the derivative of S by the key phase.
+#include <algorithm>
+
 #include "pope_common.hpp"
 #include "pope_kernels.hpp"
 #include "sim_phase.hpp"
@@ -150,13 +152,14 @@ __global__ __launch_bounds__(kThreads, 2) void sim_fwd_kernel(SimParams p, int n
 constexpr int kBJ = 64;
 constexpr int kKtRow = 128 + 1;   // fp32 row stride of the K_hat tile (keys x 128 cols)
 
-__global__ __launch_bounds__(kThreads, 2) void sim_bwd_u_kernel(SimParams p, float* U, int nib, int nec) {
+// Split sp of the reduction takes the key blocks [nb sp / n, nb (sp + 1) / n) into partial buffer sp.
+__global__ __launch_bounds__(kThreads, 2) void sim_bwd_u_kernel(SimParams p, SimAcc U, int nib, int nec) {
   __shared__ float kt[kBJ * kKtRow];
   if (p.zero_grads)   // the backward's first launch
     sim_clear_grads(p, (int64_t)blockIdx.x * kThreads + threadIdx.x, (int64_t)gridDim.x * kThreads);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 31, hf = lane >> 5;
   const int id = xcd_remap(blockIdx.x, gridDim.x);
-  const int ec = id % nec, ib = (id / nec) % nib, bh = id / (nec * nib);
+  const int ec = id % nec, ib = (id / nec) % nib, bs = id / (nec * nib), sp = bs % U.n, bh = bs / U.n;
   const int b = bh / p.Hq, h = bh % p.Hq, hk = h % p.Hk;
   const int R = p.R, E = p.E, Nq = p.Nq, Nk = p.Nk;
   const int i = ib * 128 + wave * 32 + lr;
@@ -174,7 +177,9 @@ __global__ __launch_bounds__(kThreads, 2) void sim_bwd_u_kernel(SimParams p, flo
   const float* kb = p.k + (int64_t)b * p.k_s[0] + (int64_t)hk * p.k_s[1];
   const float2* tb = R ? p.ktab + (int64_t)b * p.kt_sb + (int64_t)hk * p.kt_sh : nullptr;
 
-  for (int j0 = 0; j0 < Nk; j0 += kBJ) {
+  const int nb = (Nk + kBJ - 1) / kBJ;
+  for (int jb = nb * sp / U.n; jb < nb * (sp + 1) / U.n; ++jb) {
+    const int j0 = jb * kBJ;
     __syncthreads();
     {
       const int kj = j0 + trow;
@@ -232,7 +237,7 @@ __global__ __launch_bounds__(kThreads, 2) void sim_bwd_u_kernel(SimParams p, flo
     }
   }
   // result lane <-> column e (B operand lane), regs <-> row i
-  float* ub = U + ((int64_t)b * p.Hq + h) * Nq * p.EP;
+  float* ub = U.p + sp * U.stride + ((int64_t)b * p.Hq + h) * Nq * p.EP;
 #pragma unroll
   for (int y = 0; y < 4; ++y) {
     const int e = e_base + 32 * y + lr;
@@ -253,11 +258,11 @@ __global__ __launch_bounds__(kThreads, 2) void sim_bwd_u_kernel(SimParams p, flo
 // The B operand (Q_hat row i, column e) comes from the transformed tile in LDS.
 constexpr int kBI = 64;
 
-__global__ __launch_bounds__(kThreads, 2) void sim_bwd_w_kernel(SimParams p, float* W, int njb, int nec) {
+__global__ __launch_bounds__(kThreads, 2) void sim_bwd_w_kernel(SimParams p, SimAcc W, int njb, int nec) {
   __shared__ float qt[kBI * kKtRow];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 31, hf = lane >> 5;
   const int id = xcd_remap(blockIdx.x, gridDim.x);
-  const int ec = id % nec, jb = (id / nec) % njb, bhk = id / (nec * njb);
+  const int ec = id % nec, jb = (id / nec) % njb, bs = id / (nec * njb), sp = bs % W.n, bhk = bs / W.n;
   const int b = bhk / p.Hk, hk = bhk % p.Hk;
   const int R = p.R, E = p.E, Nq = p.Nq, Nk = p.Nk, q_off = Nk - Nq;
   const int j4 = jb * 128 + 4 * lr;   // the lane's four keys
@@ -274,12 +279,15 @@ __global__ __launch_bounds__(kThreads, 2) void sim_bwd_w_kernel(SimParams p, flo
     for (int r = 0; r < 16; ++r) acc[y][r] = 0.f;
 
   const int trow = tid >> 2, tq = tid & 3;
-  for (int g = 0; g < groups; ++g) {
-    const int h = hk + g * p.Hk;
+  // the steps (query head g of the group, 64-row block), flattened; split sp takes its share
+  const int nib = (Nq + kBI - 1) / kBI, nst = groups * nib;
+  for (int st = (int)((int64_t)nst * sp / W.n), st1 = (int)((int64_t)nst * (sp + 1) / W.n); st < st1;) {
+    const int g = st / nib, h = hk + g * p.Hk;
+    const int i_end = min((st % nib + st1 - st) * kBI, Nq);
     const float* gb = p.dsim + (int64_t)b * p.sim_s[0] + (int64_t)h * p.sim_s[1];
     const float* qb = p.q + (int64_t)b * p.q_s[0] + (int64_t)h * p.q_s[1];
     const float2* tb = R ? p.qtab + (int64_t)b * p.qt_sb + (int64_t)h * p.qt_sh : nullptr;
-    for (int i0 = 0; i0 < Nq; i0 += kBI) {
+    for (int i0 = (st % nib) * kBI; i0 < i_end; i0 += kBI) {
       __syncthreads();
       {
         const int qi = i0 + trow;
@@ -339,12 +347,13 @@ __global__ __launch_bounds__(kThreads, 2) void sim_bwd_w_kernel(SimParams p, flo
         acc[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(g4.w, bq, acc[3], 0, 0, 0);
       }
     }
+    st = (g + 1) * nib;   // the next head's first block (or past the share)
   }
   // result lane <-> column e, register r <-> row 8 (r / 4) + 4 hf + r % 4 of block s, i.e. key
   // 4 row + s
   const int e = e_base + 32 * wave + lr;
   if (e < p.EP) {
-    float* wb = W + ((int64_t)b * p.Hk + hk) * Nk * p.EP;
+    float* wb = W.p + sp * W.stride + ((int64_t)b * p.Hk + hk) * Nk * p.EP;
 #pragma unroll
     for (int s4 = 0; s4 < 4; ++s4)
 #pragma unroll
@@ -364,13 +373,11 @@ __global__ __launch_bounds__(kThreads, 2) void sim_bwd_w_kernel(SimParams p, flo
 // load and store of the pass moves 16 bytes per lane (29.1 -> 22.3 us at C2 against one float per
 // lane: the pass is bound by its loads in flight, not by its arithmetic).  The phases come from the
 // tables when present, else are computed in place (sim_phase).
-__global__ __launch_bounds__(kThreads) void sim_bwd_finalize_kernel(SimParams p, const float* U, const float* U2,
-                                                                     const float* W, const float* W2, int nqb) {
+__global__ __launch_bounds__(kThreads) void sim_bwd_finalize_kernel(SimParams p, SimAcc U, SimAcc W, int nqb) {
   __shared__ float red[16][64];
   const int tid = threadIdx.x;
   const int side = (int)blockIdx.x < nqb ? 0 : 1;
-  const float* acc = side == 0 ? U : W;
-  const float* acc2 = side == 0 ? U2 : W2;
+  const SimAcc acc = side == 0 ? U : W;
   const int nrb = side == 0 ? (p.Nq + 31) / 32 : (p.Nk + 31) / 32;
   const int blk = side == 0 ? (int)blockIdx.x : (int)blockIdx.x - nqb;
   const int rb = blk % nrb, bh = blk / nrb;
@@ -389,9 +396,7 @@ __global__ __launch_bounds__(kThreads) void sim_bwd_finalize_kernel(SimParams p,
   if (R && (side == 0 ? p.qtab : p.ktab))
     tab = side == 0 ? p.qtab + (int64_t)b * p.qt_sb + (int64_t)hh * p.qt_sh
                     : p.ktab + (int64_t)b * p.kt_sb + (int64_t)hh * p.kt_sh;
-  const float* ab = acc + (int64_t)bh * rows * EP;
-  // a second partial sum (split reduction of the split-bf16 path), added when present
-  const float* ab2 = acc2 ? acc2 + (int64_t)bh * rows * EP : nullptr;
+  const float* ab = acc.p + (int64_t)bh * rows * EP;
   float* part = side == 0 ? p.qpart : p.kpart;   // deterministic mode: written once, summed later
   // thread = (4-dim quad dq4 of a 64-dim chunk, row group rg of 16); every load and store moves 16 bytes
   const int dq4 = tid & 15, rg = tid >> 4;
@@ -402,6 +407,16 @@ __global__ __launch_bounds__(kThreads) void sim_bwd_finalize_kernel(SimParams p,
     return __builtin_bit_cast(float4, __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(a)));
   };
 
+  // the partial sums of a quad, added in order
+  auto sum = [&](const float* a) {
+    float4 v = ldnt(a);
+    for (int x = 1; x < acc.n; ++x) {
+      const float4 w = ldnt(a + x * acc.stride);
+      v.x += w.x; v.y += w.y; v.z += w.z; v.w += w.w;
+    }
+    return v;
+  };
+
   for (int d0 = 0; d0 < D; d0 += 64) {
     const int d = d0 + 4 * dq4;
     float4 dps = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -410,7 +425,6 @@ __global__ __launch_bounds__(kThreads) void sim_bwd_finalize_kernel(SimParams p,
         const int n = rb * 32 + rr;
         if (n >= rows) continue;
         const float* arow = ab + (int64_t)n * EP;
-        const float* arow2 = ab2 ? ab2 + (int64_t)n * EP : nullptr;
         float* orow = out + (int64_t)n * os + d;
         if (d < R) {   // R is a multiple of 8: a quad is all rotated or all pass-through
           const int prow = side == 0 ? q_off + n : n;
@@ -428,12 +442,7 @@ __global__ __launch_bounds__(kThreads) void sim_bwd_finalize_kernel(SimParams p,
             }
           }
           const float4 xv = ld4(x + (int64_t)n * xs + d);
-          float4 uc = ldnt(arow + d), us = ldnt(arow + R + d);
-          if (arow2) {
-            const float4 uc2 = ldnt(arow2 + d), us2 = ldnt(arow2 + R + d);
-            uc.x += uc2.x; uc.y += uc2.y; uc.z += uc2.z; uc.w += uc2.w;
-            us.x += us2.x; us.y += us2.y; us.z += us2.z; us.w += us2.w;
-          }
+          const float4 uc = sum(arow + d), us = sum(arow + R + d);
           const float xa[4] = {xv.x, xv.y, xv.z, xv.w};
           const float ca[4] = {uc.x, uc.y, uc.z, uc.w}, sa[4] = {us.x, us.y, us.z, us.w};
           float g[4], dph[4];
@@ -452,11 +461,7 @@ __global__ __launch_bounds__(kThreads) void sim_bwd_finalize_kernel(SimParams p,
           }
           dps.x += dph[0]; dps.y += dph[1]; dps.z += dph[2]; dps.w += dph[3];
         } else {
-          float4 v = ldnt(arow + R + d);
-          if (arow2) {
-            const float4 v2 = ldnt(arow2 + R + d);
-            v.x += v2.x; v.y += v2.y; v.z += v2.z; v.w += v2.w;
-          }
+          const float4 v = sum(arow + R + d);
           __builtin_nontemporal_store(f32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4*>(orow));
         }
       }
@@ -483,25 +488,36 @@ hipError_t launch_sim_fwd(const SimParams& p, hipStream_t s) {
   return launch_named("sim_fwd", sim_fwd_kernel, dim3(blocks), dim3(kThreads), s, p, nib, njb);
 }
 
-// Workspace for U and W follows the two tables; the ABI passes it through SimParams::dsim-adjacent
-// pointers set by the caller (see launch_sim_bwd_ws).
-hipError_t launch_sim_bwd_ws(const SimParams& p, float* U, float* W, hipStream_t s) {
-  const int nec = (p.EP + 127) / 128;
-  const int nib = (p.Nq + 127) / 128, njb = (p.Nk + 127) / 128;
-  hipError_t e = launch_named("sim_bwd_u", sim_bwd_u_kernel, dim3(nib * nec * p.B * p.Hq), dim3(kThreads), s, p, U,
-                              nib, nec);
-  if (e != hipSuccess) return e;
-  e = launch_named("sim_bwd_w", sim_bwd_w_kernel, dim3(njb * nec * p.B * p.Hk), dim3(kThreads), s, p, W, njb, nec);
-  if (e != hipSuccess) return e;
-  return launch_sim_finalize(p, U, nullptr, W, nullptr, s);
+// One 128-row block of one head is a workgroup's output, two workgroups per CU: with few heads and
+// rows (1,024 x 8 heads: 64 workgroups) the reduction is split until every CU has one, at most four
+// ways (each partial is written and read once) and at least four blocks of 64 each.  1,024 rows, 8 heads,
+// D 64, R 64: U 111 -> 36 us, W 126 -> 37, the finalize 5.7 -> 9.5.
+SimBwdSplit sim_bwd_split(int B, int Hq, int Hk, int Nq, int Nk, int EP) {
+  const int nec = (EP + 127) / 128;
+  const auto split = [](int64_t blocks, int64_t steps) {
+    return (int)std::max<int64_t>(1, std::min<int64_t>({4, 256 / std::max<int64_t>(blocks, 1), steps / 4}));
+  };
+  return {split((int64_t)((Nq + 127) / 128) * nec * B * Hq, (Nk + kBJ - 1) / kBJ),
+          split((int64_t)((Nk + 127) / 128) * nec * B * Hk, (int64_t)(Hq / Hk) * ((Nq + kBI - 1) / kBI))};
 }
 
-hipError_t launch_sim_finalize(const SimParams& p, const float* U, const float* U2, const float* W, const float* W2,
-                               hipStream_t s) {
+hipError_t launch_sim_bwd_ws(const SimParams& p, const SimAcc& U, const SimAcc& W, hipStream_t s) {
+  const int nec = (p.EP + 127) / 128;
+  const int nib = (p.Nq + 127) / 128, njb = (p.Nk + 127) / 128;
+  hipError_t e = launch_named("sim_bwd_u", sim_bwd_u_kernel, dim3(nib * nec * p.B * p.Hq * U.n), dim3(kThreads), s, p,
+                              U, nib, nec);
+  if (e != hipSuccess) return e;
+  e = launch_named("sim_bwd_w", sim_bwd_w_kernel, dim3(njb * nec * p.B * p.Hk * W.n), dim3(kThreads), s, p, W, njb,
+                   nec);
+  if (e != hipSuccess) return e;
+  return launch_sim_finalize(p, U, W, s);
+}
+
+hipError_t launch_sim_finalize(const SimParams& p, const SimAcc& U, const SimAcc& W, hipStream_t s) {
   const int nrq = (p.Nq + 31) / 32, nrk = (p.Nk + 31) / 32;
   const int nqb = nrq * p.B * p.Hq;
   return launch_named("sim_bwd_finalize", sim_bwd_finalize_kernel, dim3(nqb + nrk * p.B * p.Hk), dim3(kThreads), s,
-                      p, U, U2, W, W2, nqb);
+                      p, U, W, nqb);
 }
 
 }  // namespace pope

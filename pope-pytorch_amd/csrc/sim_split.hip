@@ -642,7 +642,7 @@ hipError_t launch_sim_split_bwd(const SimParams& p, const SimSplit& sp, float* U
           : launch_named("sim_split_uw", sim_split_uw_kernel<false>, grid, dim3(kThreads), s, p, sp, U, W, nib, njb, nec,
                          nsplit);
   if (e != hipSuccess) return e;
-  return launch_sim_finalize(p, U, nsplit == 2 ? sp.U2 : nullptr, W, nsplit == 2 ? sp.W2 : nullptr, s);
+  return launch_sim_finalize(p, SimAcc{U, nsplit, sp.U2 - U}, SimAcc{W, nsplit, sp.W2 - W}, s);
 }
 
 }  // namespace pope

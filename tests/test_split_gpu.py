@@ -9,6 +9,7 @@ import pytest
 import torch
 
 from gpu_common import excess_over, make_pope_inputs, oracle_attention
+from oracle import pope_oracle as orc
 
 pytestmark = pytest.mark.gpu
 
@@ -143,3 +144,21 @@ def test_split_backward_against_the_oracle(cuda, case, deterministic):
             assert (got.double().cpu() - ref[name]).abs().max().item() <= 2e-2 * max(1.0, ref[name].abs().max().item()), name
         else:
             assert excess_over(got, ref[name], 2e-2) <= 0, name
+
+
+@pytest.mark.parametrize("B,Hq,Hk,Nq,Nk,D,R", [(1, 1, 1, 512, 512, 64, 64), (1, 4, 1, 257, 300, 32, 16), (1, 2, 2, 1000, 1023, 64, 32),
+                                               (1, 2, 1, 64, 1025, 128, 128), (2, 1, 1, 700, 701, 48, 8)])
+def test_fp32_backward_with_split_reductions(cuda, B, Hq, Hk, Nq, Nk, D, R):
+    """allow_tf32=False with few heads: U and W reduced in up to four parts, whose last ones are shorter and, for
+    grouped heads, end inside a head.  Tolerance of the fp32 similarity: 1e-4 of ||ref||_inf."""
+    import pope_amd
+    inp = make_pope_inputs(8900 + Nk, B, Hq, Hk, Nq, Nk, D, R, torch.float32)
+    leaves = [inp[n].detach().requires_grad_(True) for n in ("q", "k", "freqs", "bias")]
+    sim = pope_amd.compute_attn_similarity(leaves[0], leaves[1], tuple(leaves[2:]), allow_tf32=False)
+    G = torch.randn(sim.shape, generator=torch.Generator().manual_seed(1))
+    got = [sim.detach()] + list(torch.autograd.grad(sim, leaves, G.to(sim.device)))
+    refs = [t.detach().double().cpu().requires_grad_(True) for t in leaves]
+    S = orc.sim_nonfused(*refs)
+    want = [S.detach()] + list(torch.autograd.grad(S, refs, G.double()))
+    for a, r in zip(got, want):
+        assert (a.double().cpu() - r).abs().max().item() <= 1e-4 * r.abs().max().item()
