@@ -20,8 +20,11 @@
 // sign(q_d) times the real part of the pair's gradient (torch.polar's backward for a possibly
 // negative magnitude, which the reference's torch path differentiates).
 //
-// One thread per (row, 4 input dims); a workgroup covers 256 / (D / 4) rows of one (batch, head)
-// (grid y), so the dbias partial sums reduce in LDS.
+// One thread per (row, 4 input dims); a workgroup covers 256 / (D / 4) rows at a time of one (batch,
+// head), `iters` row groups one after another, so the dbias partial sums reduce in registers and LDS
+// before one atomic per dim; both sides (q and k) in one launch.  Bound by HBM.  With one row group per
+// workgroup the key side's 2,048 workgroups (2 x 8 heads x 2,048 rows, D 64, R 64) each added 64
+// atomics to the same 512 floats: backward 2 x 21.7 us, now 17.9 for both; forward 2 x 8.9, now 12.3.
 #include <type_traits>
 
 #include "pope_common.hpp"
@@ -85,80 +88,102 @@ __device__ __forceinline__ void phases(const PolarParams& p, const Side& sd, int
   }
 }
 
+struct Task {
+  int u, r, rpb, b, h, bh, n0;   // 4-dim unit, row of a group, rows per group, head, first row
+};
+// The workgroup's side and rows: blocks [0, nq) the q side's, then the k side's.
+__device__ __forceinline__ Task task_of(const PolarParams& p, const Side& sd, int blk, int iters) {
+  Task t;
+  const int U = p.D / 4;
+  t.rpb = kThreads / U;
+  t.u = threadIdx.x % U;
+  t.r = threadIdx.x / U;
+  const int per = (sd.N + t.rpb * iters - 1) / (t.rpb * iters);
+  t.bh = blk / per;
+  t.n0 = (blk % per) * t.rpb * iters;
+  t.b = t.bh / sd.H;
+  t.h = t.bh % sd.H;
+  return t;
+}
+
 template <typename T>
-__global__ __launch_bounds__(kThreads) void polar_fwd_kernel(PolarParams p, Side sd) {
-  const int U = p.D / 4, rpb = kThreads / U;
-  const int u = threadIdx.x % U, r = threadIdx.x / U;
-  const int bh = blockIdx.y, n = blockIdx.x * rpb + r;
-  if (r >= rpb || n >= sd.N) return;
-  const int b = bh / sd.H, h = bh % sd.H;
-  const int d0 = 4 * u, E = p.cplx ? 2 * p.D : p.D + p.R;
-  float x[4];
-  load4<T>(sd.x, (int64_t)b * sd.xs0 + (int64_t)h * sd.xs1 + (int64_t)n * sd.xs2 + d0, x);
-  float* orow = sd.out + ((int64_t)bh * sd.N + n) * E;
-  if (d0 < p.R) {
-    float ph[4];
-    int frow;
-    phases(p, sd, b, h, n, d0, ph, frow);
-    float o[8];
+__global__ __launch_bounds__(kThreads) void polar_fwd_kernel(PolarParams p, Side sq, Side sk, int nq, int iters) {
+  const bool key = (int)blockIdx.x >= nq;
+  const Side& sd = key ? sk : sq;
+  const Task t = task_of(p, sd, key ? (int)blockIdx.x - nq : (int)blockIdx.x, iters);
+  const int d0 = 4 * t.u, E = p.cplx ? 2 * p.D : p.D + p.R;
+  if (t.r >= t.rpb) return;
+  for (int it = 0; it < iters; ++it) {
+    const int n = t.n0 + it * t.rpb + t.r;
+    if (n >= sd.N) return;
+    float x[4];
+    load4<T>(sd.x, (int64_t)t.b * sd.xs0 + (int64_t)t.h * sd.xs1 + (int64_t)n * sd.xs2 + d0, x);
+    float* orow = sd.out + ((int64_t)t.bh * sd.N + n) * E;
+    if (d0 < p.R) {
+      float ph[4];
+      int frow;
+      phases(p, sd, t.b, t.h, n, d0, ph, frow);
+      float o[8];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      float sn, cs;
-      sincos_acc(ph[t], &sn, &cs);
-      const float a = round_to<T>(softplus_f(x[t]));
-      o[2 * t] = a * cs;
-      o[2 * t + 1] = a * sn;
+      for (int c = 0; c < 4; ++c) {
+        float sn, cs;
+        sincos_acc(ph[c], &sn, &cs);
+        const float a = round_to<T>(softplus_f(x[c]));
+        o[2 * c] = a * cs;
+        o[2 * c + 1] = a * sn;
+      }
+      *reinterpret_cast<float4*>(orow + 2 * d0) = make_float4(o[0], o[1], o[2], o[3]);
+      *reinterpret_cast<float4*>(orow + 2 * d0 + 4) = make_float4(o[4], o[5], o[6], o[7]);
+    } else if (p.cplx) {
+      *reinterpret_cast<float4*>(orow + 2 * d0) = make_float4(x[0], 0.f, x[1], 0.f);
+      *reinterpret_cast<float4*>(orow + 2 * d0 + 4) = make_float4(x[2], 0.f, x[3], 0.f);
+    } else {
+      *reinterpret_cast<float4*>(orow + p.R + d0) = make_float4(x[0], x[1], x[2], x[3]);
     }
-    *reinterpret_cast<float4*>(orow + 2 * d0) = make_float4(o[0], o[1], o[2], o[3]);
-    *reinterpret_cast<float4*>(orow + 2 * d0 + 4) = make_float4(o[4], o[5], o[6], o[7]);
-  } else if (p.cplx) {
-    *reinterpret_cast<float4*>(orow + 2 * d0) = make_float4(x[0], 0.f, x[1], 0.f);
-    *reinterpret_cast<float4*>(orow + 2 * d0 + 4) = make_float4(x[2], 0.f, x[3], 0.f);
-  } else {
-    *reinterpret_cast<float4*>(orow + p.R + d0) = make_float4(x[0], x[1], x[2], x[3]);
   }
 }
 
 template <typename T>
-__global__ __launch_bounds__(kThreads) void polar_bwd_kernel(PolarParams p, Side sd) {
+__global__ __launch_bounds__(kThreads) void polar_bwd_kernel(PolarParams p, Side sq, Side sk, int nq, int iters) {
   __shared__ float red[kThreads][4];
-  const int U = p.D / 4, rpb = kThreads / U;
-  const int u = threadIdx.x % U, r = threadIdx.x / U;
-  const int bh = blockIdx.y, n = blockIdx.x * rpb + r;
-  const bool live = r < rpb && n < sd.N;
-  const int b = bh / sd.H, h = bh % sd.H;
-  const int d0 = 4 * u, E = p.cplx ? 2 * p.D : p.D + p.R;
-  float dph[4] = {0.f, 0.f, 0.f, 0.f};
-  if (live) {
+  const bool key = (int)blockIdx.x >= nq;
+  const Side& sd = key ? sk : sq;
+  const Task t = task_of(p, sd, key ? (int)blockIdx.x - nq : (int)blockIdx.x, iters);
+  const int U = p.D / 4, d0 = 4 * t.u, E = p.cplx ? 2 * p.D : p.D + p.R;
+  float dsum[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int it = 0; it < iters; ++it) {
+    const int n = t.n0 + it * t.rpb + t.r;
+    if (t.r >= t.rpb || n >= sd.N) break;
     float x[4];
-    load4<T>(sd.x, (int64_t)b * sd.xs0 + (int64_t)h * sd.xs1 + (int64_t)n * sd.xs2 + d0, x);
-    const float* grow = sd.gout + ((int64_t)bh * sd.N + n) * E;
-    const int64_t doff = (int64_t)b * sd.ds0 + (int64_t)h * sd.ds1 + (int64_t)n * sd.ds2 + d0;
+    load4<T>(sd.x, (int64_t)t.b * sd.xs0 + (int64_t)t.h * sd.xs1 + (int64_t)n * sd.xs2 + d0, x);
+    const float* grow = sd.gout + ((int64_t)t.bh * sd.N + n) * E;
+    const int64_t doff = (int64_t)t.b * sd.ds0 + (int64_t)t.h * sd.ds1 + (int64_t)n * sd.ds2 + d0;
     float dx[4];
     if (d0 < p.R) {
-      float ph[4];
+      float ph[4], dph[4];
       int frow;
-      phases(p, sd, b, h, n, d0, ph, frow);
+      phases(p, sd, t.b, t.h, n, d0, ph, frow);
       const float4 g0 = *reinterpret_cast<const float4*>(grow + 2 * d0);
       const float4 g1 = *reinterpret_cast<const float4*>(grow + 2 * d0 + 4);
       const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
+      for (int c = 0; c < 4; ++c) {
         float sn, cs;
-        sincos_acc(ph[t], &sn, &cs);
-        const float a = round_to<T>(softplus_f(x[t]));
-        dx[t] = sigmoid_f(x[t]) * (cs * g[2 * t] + sn * g[2 * t + 1]);
-        dph[t] = a * (cs * g[2 * t + 1] - sn * g[2 * t]);
+        sincos_acc(ph[c], &sn, &cs);
+        const float a = round_to<T>(softplus_f(x[c]));
+        dx[c] = sigmoid_f(x[c]) * (cs * g[2 * c] + sn * g[2 * c + 1]);
+        dph[c] = a * (cs * g[2 * c + 1] - sn * g[2 * c]);
+        dsum[c] += dph[c];
       }
       float* part = sd.key ? p.kpart : p.qpart;   // deterministic mode: written once, summed later
       if (part) {
-        float* dst = part + (((int64_t)b * sd.H + h) * sd.N + n) * p.R + d0;
+        float* dst = part + (((int64_t)t.b * sd.H + t.h) * sd.N + n) * p.R + d0;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) dst[t] = dph[t];
+        for (int c = 0; c < 4; ++c) dst[c] = dph[c];
       } else if (p.dfreqs) {
-        float* df = p.dfreqs + (int64_t)b * p.df_s[0] + (int64_t)h * p.df_s[1] + (int64_t)frow * p.df_s[2] + d0;
+        float* df = p.dfreqs + (int64_t)t.b * p.df_s[0] + (int64_t)t.h * p.df_s[1] + (int64_t)frow * p.df_s[2] + d0;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) atomicAdd(df + t, dph[t]);
+        for (int c = 0; c < 4; ++c) atomicAdd(df + c, dph[c]);
       }
     } else if (p.cplx) {
       // real parts of the (re, im) gradient pairs, times sign(x): the reference builds the pair
@@ -167,7 +192,7 @@ __global__ __launch_bounds__(kThreads) void polar_bwd_kernel(PolarParams p, Side
       const float4 g1 = *reinterpret_cast<const float4*>(grow + 2 * d0 + 4);
       const float gr[4] = {g0.x, g0.z, g1.x, g1.z};
 #pragma unroll
-      for (int t = 0; t < 4; ++t) dx[t] = x[t] > 0.f ? gr[t] : x[t] < 0.f ? -gr[t] : 0.f;
+      for (int c = 0; c < 4; ++c) dx[c] = x[c] > 0.f ? gr[c] : x[c] < 0.f ? -gr[c] : 0.f;
     } else {
       const float4 g = *reinterpret_cast<const float4*>(grow + p.R + d0);
       dx[0] = g.x; dx[1] = g.y; dx[2] = g.z; dx[3] = g.w;
@@ -176,26 +201,18 @@ __global__ __launch_bounds__(kThreads) void polar_bwd_kernel(PolarParams p, Side
   }
   if (sd.key && p.dbias && !p.kpart) {   // sum the workgroup's rows per dim, one atomic per dim
 #pragma unroll
-    for (int t = 0; t < 4; ++t) red[threadIdx.x][t] = dph[t];
+    for (int c = 0; c < 4; ++c) red[threadIdx.x][c] = dsum[c];
     __syncthreads();
-    if (r == 0 && d0 < p.R) {
+    if (t.r == 0 && d0 < p.R) {
       float s4[4] = {0.f, 0.f, 0.f, 0.f};
-      for (int r2 = 0; r2 < rpb; ++r2)
+      for (int r2 = 0; r2 < t.rpb; ++r2)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) s4[t] += red[r2 * U + u][t];
-      float* db = p.dbias + (int64_t)h * p.bias_sh + d0;
+        for (int c = 0; c < 4; ++c) s4[c] += red[r2 * U + t.u][c];
+      float* db = p.dbias + (int64_t)t.h * p.bias_sh + d0;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) atomicAdd(db + t, s4[t]);
+      for (int c = 0; c < 4; ++c) atomicAdd(db + c, s4[c]);
     }
   }
-}
-
-template <typename T>
-hipError_t launch_side(const PolarParams& p, const Side& sd, bool bwd, hipStream_t s) {
-  const int U = p.D / 4, rpb = kThreads / U;
-  const dim3 grid((unsigned)((sd.N + rpb - 1) / rpb), (unsigned)(p.B * sd.H));
-  if (bwd) return launch_named("polar_bwd", polar_bwd_kernel<T>, grid, dim3(kThreads), s, p, sd);
-  return launch_named("polar_fwd", polar_fwd_kernel<T>, grid, dim3(kThreads), s, p, sd);
 }
 
 template <typename T>
@@ -204,9 +221,18 @@ hipError_t launch_t(const PolarParams& p, bool bwd, hipStream_t s) {
          p.Hq, p.Nq, p.Nk - p.Nq, 0};
   Side k{p.k, p.k_s[0], p.k_s[1], p.k_s[2], p.kh, p.gk, p.dk, p.dk_s[0], p.dk_s[1], p.dk_s[2],
          p.Hk, p.Nk, 0, 1};
-  hipError_t e = launch_side<T>(p, q, bwd, s);
-  if (e != hipSuccess) return e;
-  return launch_side<T>(p, k, bwd, s);
+  const int rpb = kThreads / (p.D / 4);
+  const auto blocks = [&](const Side& sd, int iters) {
+    return (int64_t)((sd.N + rpb * iters - 1) / (rpb * iters)) * p.B * sd.H;
+  };
+  // row groups per workgroup: up to 8 while about eight workgroups per CU remain
+  int iters = 1;
+  while (iters < 8 && blocks(q, 2 * iters) + blocks(k, 2 * iters) >= 1024) iters *= 2;
+  const int64_t nq = blocks(q, iters), nk = blocks(k, iters);
+  if (nq + nk > INT32_MAX) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(nq + nk));
+  if (bwd) return launch_named("polar_bwd", polar_bwd_kernel<T>, grid, dim3(kThreads), s, p, q, k, (int)nq, iters);
+  return launch_named("polar_fwd", polar_fwd_kernel<T>, grid, dim3(kThreads), s, p, q, k, (int)nq, iters);
 }
 
 }  // namespace
