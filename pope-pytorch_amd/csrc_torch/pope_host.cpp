@@ -1,0 +1,430 @@
+// Native call layer of pope_amd's eager calls: descriptor, workspaces, launch and autograd node of the
+// flash attention, the similarity and the polar transform on libpope_hip.so (include/pope_abi.h).
+//
+// A small call is bound by the host: a (1, 4, 257, 64) training step spent 75-150 us (by host) in
+// Python between kernels of 45 us, a similarity step 115-175 us in the custom-op dispatch layers.  The
+// Python modules keep the argument checks that raise, the padding and the torch.library ops
+// (torch.compile tracing, opcheck); what is here is their forward / backward, with the same
+// workspaces, flags and entry points, under torch::autograd::Function.  Nothing is kept between calls.
+#include <torch/extension.h>
+
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+
+#include <algorithm>
+#include <atomic>
+#include <climits>
+
+#include "../../include/pope_abi.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// whether the last flash backward reused its forward's preparation (read by tests)
+std::atomic<bool> g_last_bwd_prepared{false};
+
+void check(int status, const char* what) {
+  if (status == POPE_OK) return;
+  char msg[512];
+  pope_last_error(msg, sizeof msg);
+  TORCH_CHECK(false, "pope_amd ", what, " failed (status ", status, "): ", msg);
+}
+
+size_t workspace_bytes(int op, const pope_desc& d) {
+  size_t n = 0;
+  check(pope_workspace_bytes(op, &d, &n), "workspace query");
+  return n;
+}
+
+// torch's caching allocator returns 512-byte aligned blocks
+Tensor bytes_like(const Tensor& t, size_t n) {
+  return n ? at::empty({(int64_t)n}, t.options().dtype(at::kByte).requires_grad(false)) : Tensor();
+}
+Tensor fp32_like(const Tensor& t, at::IntArrayRef shape) {
+  return at::empty(shape, t.options().dtype(at::kFloat).requires_grad(false));
+}
+
+void* data(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+int deterministic_flag() { return at::globalContext().deterministicAlgorithms() ? POPE_FLAG_DETERMINISTIC : 0; }
+
+void strides3(int64_t* dst, const Tensor& t) {
+  for (int i = 0; i < 3; ++i) dst[i] = t.stride(i);
+}
+
+// (b, h, n) element strides of a freqs table; an extent of 1 broadcasts (stride 0).
+void freqs_strides(int64_t* dst, const Tensor& f) {
+  const auto st = [&](int64_t i) { return f.size(i) == 1 ? (int64_t)0 : f.stride(i); };
+  const int64_t n = f.dim();
+  TORCH_CHECK_VALUE(n >= 2 && n <= 4, "freqs must be 2-D, 3-D or 4-D, got ", f.sizes());
+  dst[0] = n >= 3 ? st(0) : 0;
+  dst[1] = n == 4 ? st(1) : 0;
+  dst[2] = st(n - 2);
+}
+
+int dtype_code(const Tensor& t) {
+  switch (t.scalar_type()) {
+    case at::kFloat: return POPE_F32;
+    case at::kHalf: return POPE_F16;
+    case at::kBFloat16: return POPE_BF16;
+    default: TORCH_CHECK_TYPE(false, "pope_amd: unsupported dtype ", t.scalar_type());
+  }
+}
+
+pope_desc desc_of(const Tensor& q, const Tensor& k, const Tensor& freqs, const Tensor& bias) {
+  pope_desc d{};
+  d.B = q.size(0);
+  d.Hq = q.size(1);
+  d.Nq = q.size(2);
+  d.D = q.size(3);
+  d.Hk = k.size(1);
+  d.Nk = k.size(2);
+  d.R = freqs.defined() ? freqs.size(-1) : 0;
+  d.dtype = dtype_code(q);
+  strides3(d.q_s, q);
+  strides3(d.k_s, k);
+  if (freqs.defined()) {
+    freqs_strides(d.f_s, freqs);
+    d.bias_sh = bias.size(0) > 1 ? bias.stride(0) : 0;
+  }
+  return d;
+}
+
+// Every operand on q's GPU: the kernels read raw pointers.
+void check_device(const Tensor& q, std::initializer_list<const Tensor*> ts) {
+  TORCH_CHECK(q.is_cuda(), "pope_amd runs on GPU tensors only");
+  for (const Tensor* t : ts)
+    TORCH_CHECK(!t->defined() || t->device() == q.device(), "pope_amd: operand on ", t->device(), " next to q on ", q.device());
+}
+
+// ---------------------------------------------------------------- flash attention
+
+Tensor unit_feature(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
+
+void check_flash(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& freqs, const Tensor& bias,
+                 const Tensor& mask) {
+  check_device(q, {&k, &v, &freqs, &bias, &mask});
+  TORCH_CHECK_VALUE(q.dim() == 4 && k.dim() == 4 && v.dim() == 4, "q, k, v must be 4-D, got ", q.sizes(), ", ", k.sizes(),
+                    ", ", v.sizes());
+  TORCH_CHECK_VALUE(v.sizes() == k.sizes(), "v ", v.sizes(), " must match k ", k.sizes());
+  TORCH_CHECK_VALUE(!mask.defined() || (mask.dim() == 2 && mask.size(0) == q.size(0) && mask.size(1) == k.size(2)), "mask ",
+                    mask.defined() ? mask.sizes() : at::IntArrayRef(), " must be (batch, seq_k) = (", q.size(0), ", ", k.size(2), ")");
+  for (const Tensor* t : {&k, &v})
+    TORCH_CHECK_TYPE(t->scalar_type() == q.scalar_type(), "pope_amd flash: operand of dtype ", t->scalar_type(),
+                     " next to q of dtype ", q.scalar_type());
+  TORCH_CHECK_VALUE(k.size(0) == q.size(0) && k.size(3) == q.size(3) && k.size(1) > 0 && q.size(1) % k.size(1) == 0,
+                    "incompatible q ", q.sizes(), " and k ", k.sizes());
+  if (freqs.defined()) {
+    TORCH_CHECK_VALUE(freqs.size(-2) >= k.size(2), "freqs has ", freqs.size(-2), " positions, keys need ", k.size(2));
+    TORCH_CHECK_VALUE(bias.size(-1) == freqs.size(-1) && (bias.size(0) == 1 || bias.size(0) == k.size(1)), "bias ",
+                      bias.sizes(), " must be (1 or ", k.size(1), ", ", freqs.size(-1), ")");
+  }
+}
+
+// decode_head_groups() of the library: whether some power-of-two group of the query heads fits.
+bool decode_groups(int64_t Hq, int64_t D) {
+  for (int64_t g = 1; g <= Hq; g *= 2)
+    if (Hq % g == 0 && Hq / g * D <= 4096) return true;
+  return false;
+}
+
+// The same decision as hip_pope_flash_attn._decode_eligible.
+bool decode_eligible(const pope_desc& d, int64_t min_keys) {
+  if (d.Nq != 1 || d.causal || d.Nk < min_keys || d.D > 128 || !decode_groups(d.Hq, d.D)) return false;
+  if (d.R && (d.f_s[1] != 0 || d.f_s[0] % 4 || d.f_s[2] % 4)) return false;
+  return (int64_t)(d.Nk - 1) * std::max(d.k_s[2], d.v_s[2]) + d.D < INT_MAX;
+}
+
+struct FlashOut {
+  Tensor o, lse, ws;
+};
+
+FlashOut flash_forward(const Tensor& q0, const Tensor& k0, const Tensor& v0, Tensor freqs, const Tensor& bias,
+                       const Tensor& mask, bool causal, double scale, int64_t decode_min_keys) {
+  const Tensor q = unit_feature(q0), k = unit_feature(k0), v = unit_feature(v0);
+  check_flash(q, k, v, freqs, bias, mask);
+  FlashOut r;
+  r.o = at::empty_like(q);
+  r.lse = fp32_like(q, q.sizes().slice(0, 3));
+  pope_desc d = desc_of(q, k, freqs, bias);
+  d.causal = causal;
+  d.softmax_scale = (float)scale;
+  strides3(d.v_s, v);
+  strides3(d.o_s, r.o);
+  if (mask.defined()) d.mask_sb = mask.stride(0);
+  const auto* mp = static_cast<const uint8_t*>(data(mask));
+  auto* lse = static_cast<float*>(r.lse.data_ptr());
+  void* s = stream_of(q);
+  if (decode_eligible(d, decode_min_keys)) {
+    if (freqs.defined() && reinterpret_cast<uintptr_t>(freqs.data_ptr()) % 16) {
+      // a table in memory torch did not allocate: an aligned dense copy, with its strides
+      freqs = freqs.clone(at::MemoryFormat::Contiguous);
+      freqs_strides(d.f_s, freqs);
+    }
+    const size_t n = workspace_bytes(POPE_OP_FLASH_DECODE, d);
+    const Tensor ws = bytes_like(q, n);
+    check(pope_flash_decode(&d, q.data_ptr(), k.data_ptr(), v.data_ptr(), static_cast<const float*>(data(freqs)),
+                            static_cast<const float*>(data(bias)), mp, r.o.data_ptr(), lse, data(ws), n, s), "flash decode");
+    return r;
+  }
+  // the workspace holds the preparation the backward reuses and, under deterministic mode, the
+  // backward's phase-derivative region after it
+  pope_desc dd = d;
+  dd.flags = deterministic_flag();
+  const size_t n = workspace_bytes(dd.flags ? POPE_OP_FLASH_BWD : POPE_OP_FLASH_FWD, dd);
+  const size_t np = workspace_bytes(POPE_OP_FLASH_FWD_PARTIALS, d);
+  r.ws = bytes_like(q, n);
+  const Tensor parts = bytes_like(q, np);
+  check(pope_flash_fwd_split(&d, q.data_ptr(), k.data_ptr(), v.data_ptr(), static_cast<const float*>(data(freqs)),
+                             static_cast<const float*>(data(bias)), mp, r.o.data_ptr(), lse, data(r.ws), n, data(parts), np, s),
+        "flash forward");
+  return r;
+}
+
+Tensor opt(const std::optional<Tensor>& t) { return t.has_value() ? *t : Tensor(); }
+
+struct FlashFn : torch::autograd::Function<FlashFn> {
+  // freqs and bias come together, so the node's inputs 3 and 4 are theirs where they exist
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
+                        const std::optional<Tensor>& freqs_, const std::optional<Tensor>& bias_,
+                        const std::optional<Tensor>& mask_, bool causal, double scale, int64_t decode_min_keys, bool reuse) {
+    const Tensor freqs = opt(freqs_), bias = opt(bias_), mask = opt(mask_);
+    FlashOut r = flash_forward(q, k, v, freqs, bias, mask, causal, scale, decode_min_keys);
+    ctx->save_for_backward({q, k, v, freqs, bias, mask, r.o, r.lse, reuse ? r.ws : Tensor()});
+    ctx->saved_data["causal"] = causal;
+    ctx->saved_data["scale"] = scale;
+    return r.o;
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list sv = ctx->get_saved_variables();
+    const Tensor q = unit_feature(sv[0]), k = unit_feature(sv[1]), v = unit_feature(sv[2]), freqs = sv[3], bias = sv[4],
+                 mask = sv[5], o = unit_feature(sv[6]), fwd_ws = sv[8];
+    const Tensor lse = sv[7].contiguous();
+    Tensor dout = unit_feature(grads[0]);
+    if (dout.scalar_type() != q.scalar_type()) dout = dout.to(q.scalar_type());
+    check_flash(q, k, v, freqs, bias, mask);
+    TORCH_CHECK_VALUE(dout.sizes() == q.sizes(), "do ", dout.sizes(), " must match q ", q.sizes());
+    const bool need_df = freqs.defined() && ctx->needs_input_grad(3);
+    const bool need_db = bias.defined() && ctx->needs_input_grad(4);
+    const Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+    Tensor dfreqs, dbias;
+    // the library clears the gradients over the key positions n < Nk it addresses; rows of a longer
+    // table get none, so such a table's gradient starts from zeros
+    if (need_df)
+      dfreqs = freqs.size(-2) > k.size(2) ? at::zeros(freqs.sizes(), freqs.options().dtype(at::kFloat).requires_grad(false))
+                                          : fp32_like(freqs, freqs.sizes());
+    if (need_db) dbias = fp32_like(bias, bias.sizes());
+    pope_desc d = desc_of(q, k, freqs, bias);
+    d.causal = ctx->saved_data["causal"].toBool();
+    d.softmax_scale = (float)ctx->saved_data["scale"].toDouble();
+    strides3(d.v_s, v);
+    strides3(d.o_s, o);
+    strides3(d.do_s, dout);
+    strides3(d.dq_s, dq);
+    strides3(d.dk_s, dk);
+    strides3(d.dv_s, dv);
+    if (need_df) freqs_strides(d.df_s, dfreqs);
+    if (mask.defined()) d.mask_sb = mask.stride(0);
+    d.flags = POPE_FLAG_ZERO_GRADS | deterministic_flag();
+    const size_t n = workspace_bytes(POPE_OP_FLASH_BWD, d), np = workspace_bytes(POPE_OP_FLASH_BWD_PARTIALS, d);
+    const bool prepared = fwd_ws.defined() && (size_t)fwd_ws.numel() == n;
+    g_last_bwd_prepared = prepared;
+    if (prepared) d.flags |= POPE_FLAG_PREPARED;
+    const Tensor ws = prepared ? fwd_ws : bytes_like(q, n);
+    const Tensor parts = bytes_like(q, np);
+    check(pope_flash_bwd_split(&d, dout.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+                               static_cast<const float*>(lse.data_ptr()), static_cast<const float*>(data(freqs)),
+                               static_cast<const float*>(data(bias)), static_cast<const uint8_t*>(data(mask)),
+                               dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), static_cast<float*>(data(dfreqs)),
+                               static_cast<float*>(data(dbias)), data(ws), n, data(parts), np, stream_of(q)),
+          "flash backward");
+    return {dq, dk, dv, dfreqs, dbias, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+// Whether a call has to go through the autograd node (which also refuses forward-mode tangents).
+bool tracked(std::initializer_list<Tensor> ts) {
+  for (const Tensor& t : ts)
+    if (t.defined() && ((at::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(0).defined())) return true;
+  return false;
+}
+
+Tensor flash(const Tensor& q, const Tensor& k, const Tensor& v, const std::optional<Tensor>& freqs,
+             const std::optional<Tensor>& bias, const std::optional<Tensor>& mask, bool causal, double scale,
+             int64_t decode_min_keys, bool reuse) {
+  const Tensor f = opt(freqs), b = opt(bias), m = opt(mask);
+  if (!tracked({q, k, v, f, b})) return flash_forward(q, k, v, f, b, m, causal, scale, decode_min_keys).o;
+  TORCH_CHECK_VALUE(f.defined() == b.defined(), "freqs and bias come together");
+  return FlashFn::apply(q, k, v, freqs, bias, mask, causal, scale, decode_min_keys, reuse);
+}
+
+// ---------------------------------------------------------------- similarity and polar transform
+
+// Gradients under create_graph: differentiating them again raises, as it does through the torch.library
+// ops (whose backward ops have no autograd formula), instead of treating them as constants.
+variable_list once_differentiable(variable_list grads, const char* what) {
+  if (!at::GradMode::is_enabled()) return grads;
+  variable_list in;
+  for (const Tensor& g : grads)
+    if (g.defined()) in.push_back(g.detach().requires_grad_(true));
+  auto err = std::make_shared<torch::autograd::DelayedError>(
+      std::string("pope_amd ") + what + ": the gradient is not differentiable a second time", (int64_t)in.size());
+  const variable_list out = (*err)(std::move(in));
+  size_t i = 0;
+  for (Tensor& g : grads)
+    if (g.defined()) g = out[i++];
+  return grads;
+}
+
+// Views the kernels read in 16-byte vectors: unit feature stride, other strides multiples of 4
+// elements, 16-byte aligned start.
+Tensor rows4(Tensor t) {
+  const auto off = [](const Tensor& x) { return reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 != 0; };
+  bool bad = t.stride(-1) != 1 || off(t);
+  for (int64_t i = 0; i + 1 < t.dim(); ++i) bad = bad || t.stride(i) % 4 != 0;
+  if (bad) {
+    t = t.contiguous();
+    if (off(t)) t = t.clone();
+  }
+  return t;
+}
+
+struct SimFn : torch::autograd::Function<SimFn> {
+  static Tensor run(const Tensor& q0, const Tensor& k0, const Tensor& freqs, const Tensor& bias, bool split) {
+    check_device(q0, {&k0, &freqs, &bias});
+    const Tensor q = rows4(q0), k = rows4(k0);
+    pope_desc d = desc_of(q, k, freqs, bias);
+    d.flags = split ? POPE_FLAG_SPLIT_BF16 : 0;
+    const Tensor sim = fp32_like(q, {q.size(0), q.size(1), q.size(2), k.size(2)});
+    strides3(d.sim_s, sim);
+    const size_t n = workspace_bytes(POPE_OP_SIM_FWD, d);
+    const Tensor ws = bytes_like(q, n);
+    check(pope_sim_fwd(&d, q.data_ptr(), k.data_ptr(), static_cast<const float*>(freqs.data_ptr()),
+                       static_cast<const float*>(bias.data_ptr()), sim.data_ptr(), data(ws), n, stream_of(q)),
+          "similarity forward");
+    return sim;
+  }
+
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& freqs, const Tensor& bias,
+                        bool split) {
+    ctx->save_for_backward({q, k, freqs, bias});
+    ctx->saved_data["split"] = split;
+    return run(q, k, freqs, bias, split);
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list sv = ctx->get_saved_variables();
+    const Tensor q = rows4(sv[0]), k = rows4(sv[1]), freqs = sv[2], bias = sv[3];
+    const Tensor dsim = rows4(grads[0].to(at::kFloat));
+    TORCH_CHECK_VALUE(dsim.dim() == 4 && dsim.size(0) == q.size(0) && dsim.size(1) == q.size(1) &&
+                          dsim.size(2) == q.size(2) && dsim.size(3) == k.size(2), "dsim ", dsim.sizes(), " does not fit the similarity");
+    const bool need_df = ctx->needs_input_grad(2) && freqs.size(-1) > 0;
+    const bool need_db = ctx->needs_input_grad(3) && bias.size(-1) > 0;
+    pope_desc d = desc_of(q, k, freqs, bias);
+    d.flags = (ctx->saved_data["split"].toBool() ? POPE_FLAG_SPLIT_BF16 : 0) | deterministic_flag() | POPE_FLAG_ZERO_GRADS;
+    strides3(d.sim_s, dsim);
+    const Tensor dq = at::empty_like(q), dk = at::empty_like(k);
+    strides3(d.dq_s, dq);
+    strides3(d.dk_s, dk);
+    Tensor dfreqs, dbias;
+    if (need_df) {
+      dfreqs = freqs.size(-2) > k.size(2) ? at::zeros(freqs.sizes(), freqs.options().dtype(at::kFloat).requires_grad(false))
+                                          : fp32_like(freqs, freqs.sizes());
+      freqs_strides(d.df_s, dfreqs);
+    }
+    if (need_db) dbias = fp32_like(bias, bias.sizes());
+    const size_t n = workspace_bytes(POPE_OP_SIM_BWD, d);
+    const Tensor ws = bytes_like(q, n);
+    check(pope_sim_bwd(&d, dsim.data_ptr(), q.data_ptr(), k.data_ptr(), static_cast<const float*>(freqs.data_ptr()),
+                       static_cast<const float*>(bias.data_ptr()), dq.data_ptr(), dk.data_ptr(),
+                       static_cast<float*>(data(dfreqs)), static_cast<float*>(data(dbias)), data(ws), n, stream_of(q)),
+          "similarity backward");
+    return once_differentiable({dq, dk, dfreqs, dbias, Tensor()}, "similarity");
+  }
+};
+
+Tensor sim(const Tensor& q, const Tensor& k, const Tensor& freqs, const Tensor& bias, bool split) {
+  if (!tracked({q, k, freqs, bias})) return SimFn::run(q, k, freqs, bias, split);
+  return SimFn::apply(q, k, freqs, bias, split);
+}
+
+struct PolarFn : torch::autograd::Function<PolarFn> {
+  // fp32 columns per output row: D + R, or D (re, im) pairs
+  static int64_t width(const Tensor& q, const Tensor& freqs, bool cplx) {
+    return cplx ? 2 * q.size(-1) : q.size(-1) + freqs.size(-1);
+  }
+
+  static variable_list run(const Tensor& q0, const Tensor& k0, const Tensor& freqs, const Tensor& bias, bool cplx) {
+    check_device(q0, {&k0, &freqs, &bias});
+    const Tensor q = rows4(q0), k = rows4(k0);
+    pope_desc d = desc_of(q, k, freqs, bias);
+    d.flags = cplx ? POPE_FLAG_COMPLEX : 0;
+    const int64_t E = width(q, freqs, cplx);
+    const Tensor qh = fp32_like(q, {q.size(0), q.size(1), q.size(2), E});
+    const Tensor kh = fp32_like(k, {k.size(0), k.size(1), k.size(2), E});
+    check(pope_polar_fwd(&d, q.data_ptr(), k.data_ptr(), static_cast<const float*>(freqs.data_ptr()),
+                         static_cast<const float*>(bias.data_ptr()), static_cast<float*>(qh.data_ptr()),
+                         static_cast<float*>(kh.data_ptr()), stream_of(q)), "polar transform");
+    return {qh, kh};
+  }
+
+  static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& freqs,
+                               const Tensor& bias, bool cplx) {
+    ctx->save_for_backward({q, k, freqs, bias});
+    ctx->saved_data["cplx"] = cplx;
+    return run(q, k, freqs, bias, cplx);
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list sv = ctx->get_saved_variables();
+    const Tensor q = rows4(sv[0]), k = rows4(sv[1]), freqs = sv[2], bias = sv[3];
+    const bool cplx = ctx->saved_data["cplx"].toBool();
+    const int64_t E = width(q, freqs, cplx);
+    const auto grad = [&](const Tensor& g, const Tensor& x) {
+      return g.defined() ? g.to(at::kFloat).contiguous()
+                         : at::zeros({x.size(0), x.size(1), x.size(2), E}, x.options().dtype(at::kFloat).requires_grad(false));
+    };
+    const Tensor gq = grad(grads[0], q), gk = grad(grads[1], k);
+    const bool need_df = ctx->needs_input_grad(2), need_db = ctx->needs_input_grad(3);
+    pope_desc d = desc_of(q, k, freqs, bias);
+    d.flags = (cplx ? POPE_FLAG_COMPLEX : 0) | deterministic_flag();
+    const Tensor dq = at::empty_like(q), dk = at::empty_like(k);
+    strides3(d.dq_s, dq);
+    strides3(d.dk_s, dk);
+    Tensor dfreqs, dbias;   // accumulated into
+    if (need_df) {
+      dfreqs = at::zeros(freqs.sizes(), freqs.options().dtype(at::kFloat).requires_grad(false));
+      freqs_strides(d.df_s, dfreqs);
+    }
+    if (need_db) dbias = at::zeros(bias.sizes(), bias.options().dtype(at::kFloat).requires_grad(false));
+    const size_t n = workspace_bytes(POPE_OP_POLAR_BWD, d);
+    const Tensor ws = bytes_like(q, n);
+    check(pope_polar_bwd(&d, static_cast<const float*>(gq.data_ptr()), static_cast<const float*>(gk.data_ptr()),
+                         q.data_ptr(), k.data_ptr(), static_cast<const float*>(freqs.data_ptr()),
+                         static_cast<const float*>(bias.data_ptr()), dq.data_ptr(), dk.data_ptr(),
+                         static_cast<float*>(data(dfreqs)), static_cast<float*>(data(dbias)), data(ws), n, stream_of(q)),
+          "polar transform backward");
+    return once_differentiable({dq, dk, dfreqs, dbias, Tensor()}, "polar transform");
+  }
+};
+
+std::pair<Tensor, Tensor> polar(const Tensor& q, const Tensor& k, const Tensor& freqs, const Tensor& bias, bool cplx) {
+  const variable_list r =
+      tracked({q, k, freqs, bias}) ? PolarFn::apply(q, k, freqs, bias, cplx) : PolarFn::run(q, k, freqs, bias, cplx);
+  return {r[0], r[1]};
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_pope_host, m) {
+  const auto nogil = py::call_guard<py::gil_scoped_release>();
+  m.def("flash", &flash, nogil);
+  m.def("sim", &sim, nogil);
+  m.def("polar", &polar, nogil);
+  m.def("last_bwd_prepared", [] { return g_last_bwd_prepared.load(); });
+  m.def("abi_version", [] { return POPE_ABI_VERSION; });
+}

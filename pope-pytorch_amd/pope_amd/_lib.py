@@ -119,6 +119,37 @@ def lib():
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The native call layer (pope_amd/_pope_host.so, csrc_torch/pope_host.cpp); raises RuntimeError
+    when it or the library is missing."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _pope_host
+        except ImportError as e:
+            raise RuntimeError(f"pope_amd: cannot load the native call layer: {e}; "
+                               "build it with `python pope-pytorch_amd/build.py`") from e
+        if _pope_host.abi_version() != ABI_VERSION:
+            raise RuntimeError(f"pope_amd: call layer ABI {_pope_host.abi_version()} != expected {ABI_VERSION}")
+        _host = _pope_host
+    return _host
+
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter, type(None))
+
+
+def eager(*ts) -> bool:
+    """Whether a call on these tensors can take the native call layer in place of the torch.library ops: no
+    tracing, no dispatch mode (fake tensors, make_fx, operator-recording checkpointing), no functorch
+    transform and no tensor subclass, each of which works on the ops."""
+    return (not torch.compiler.is_compiling() and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._functorch.peek_interpreter_stack() is None and all(type(t) in _PLAIN for t in ts))
+
+
 def last_error() -> str:
     buf = ctypes.create_string_buffer(512)
     lib().pope_last_error(buf, 512)

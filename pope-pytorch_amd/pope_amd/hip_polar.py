@@ -157,7 +157,10 @@ def polar(q: Tensor, k: Tensor, freqs: Tensor, bias: Tensor, return_complex: boo
         # rows padded on the device (pope_amd._pad); the padded dims' output columns are dropped
         q, k = pad_qk(q, plan), pad_qk(k, plan)
         freqs, bias = pad_last(freqs, plan.R8), pad_last(bias, plan.R8)
-    qh, kh = polar_fwd_op(q, k, freqs, bias, return_complex)
+    if _lib.eager(q, k, freqs, bias):   # the same forward / backward without the custom-op dispatch
+        qh, kh = _lib.host().polar(q, k, freqs, bias, return_complex)
+    else:
+        qh, kh = polar_fwd_op(q, k, freqs, bias, return_complex)
     if return_complex:
         W = q.shape[-1]
         qh = torch.view_as_complex(qh.view(*qh.shape[:-1], W, 2))

@@ -181,5 +181,8 @@ def hip_compute_qk_similarity(q, k, freqs, bias, rotate_dim=None, allow_tf32=Tru
     if plan is not None:
         qf, kf = pad_qk(qf, plan), pad_qk(kf, plan)
         freqs, bias = pad_last(freqs, plan.R8), pad_last(bias, plan.R8)
-    sim = sim_fwd_op(qf, kf, freqs, bias, bool(allow_tf32))
+    if _lib.eager(qf, kf, freqs, bias):   # the same forward / backward without the custom-op dispatch
+        sim = _lib.host().sim(qf, kf, freqs, bias, bool(allow_tf32))
+    else:
+        sim = sim_fwd_op(qf, kf, freqs, bias, bool(allow_tf32))
     return sim.to(out_dtype) if out_dtype != torch.float32 else sim

@@ -11,9 +11,10 @@ arguments, (batch, seq, heads, dim) layout and return values.  Underneath, two
                       need_dfreqs, need_dbias) -> (dq, dk, dv, dfreqs, dbias)
 
 with ``flash_fwd`` differentiable through ``register_autograd``.  Eager calls of
-``flash_attn`` / ``flash_attn_head_first`` run the same forward and backward through a
-plain ``autograd.Function`` (no custom-op dispatch, which costs more host time than a
-launch); torch.compile tracing records the ops.  The ops take
+``flash_attn`` / ``flash_attn_head_first`` run the same forward and backward in the native
+call layer (csrc_torch/pope_host.cpp: no custom-op dispatch and no Python between the
+launches, which cost more host time than small calls' kernels); torch.compile tracing
+records the ops.  The ops take
 head-first logical views (B, H, N, D) with any batch/head/seq strides and a unit
 feature stride, so the (b n h d) <-> (b h n d) permutes of the reference cost no
 copies.  Query head h reads kv head h % Hk (the reference's torch-path GQA
@@ -210,6 +211,7 @@ class _RangeCheck:
 
 
 _INT32_MAX = 2 ** 31 - 1
+_DECODE_MIN_KEYS = 1024      # shortest cache the decode kernel takes
 _DECODE_QUERY_WORDS = 4096   # query-weight words a decode workgroup stages in LDS
 
 
@@ -232,7 +234,7 @@ def _decode_eligible(q, k, v, freqs, causal) -> bool:
     B, Hq, Nq, D = q.shape
     Nk = k.shape[2]
     R = freqs.shape[-1] if exists(freqs) else 0
-    if Nq != 1 or causal or Nk < 1024 or D > 128:
+    if Nq != 1 or causal or Nk < _DECODE_MIN_KEYS or D > 128:
         return False
     if _decode_head_groups(Hq, D) == 0:
         return False   # a workgroup stages its group's query weights in LDS
@@ -332,8 +334,13 @@ def _fwd_impl(q, k, v, freqs, bias, mask, causal, softmax_scale):
     return o, lse, ws
 
 
-# whether the last backward reused its forward's preparation (read by tests)
-_LAST_BWD_PREPARED = False
+
+def __getattr__(name):
+    # whether the last eager backward reused its forward's preparation (read by tests)
+    if name == "_LAST_BWD_PREPARED":
+        return _lib.host().last_bwd_prepared()
+    raise AttributeError(f"module {__name__!r} has no attribute {name!r}")
+
 
 # whether the forward's workspace is kept for the backward (set_flash_workspace_reuse)
 _REUSE_FWD_WORKSPACE = True
@@ -396,9 +403,7 @@ def _bwd_impl(do, q, k, v, o, lse, freqs, bias, mask, causal, softmax_scale, nee
         return d, dp, _lib.workspace_bytes(_lib.OP_FLASH_BWD, d), _lib.workspace_bytes(_lib.OP_FLASH_BWD_PARTIALS, d)
 
     d, dprep, need, part_bytes = _plan(key, build)
-    global _LAST_BWD_PREPARED
-    _LAST_BWD_PREPARED = exists(fwd_ws) and fwd_ws.numel() == need
-    if _LAST_BWD_PREPARED:
+    if exists(fwd_ws) and fwd_ws.numel() == need:
         ws, d = fwd_ws, dprep
     else:
         ws = torch.empty(need, dtype=torch.uint8, device=q.device)
@@ -469,32 +474,14 @@ def _fwd_backward(ctx, do, dlse, dws):
 flash_fwd_op.register_autograd(_fwd_backward, setup_context=_fwd_setup)
 
 
-class _FlashAttnEager(torch.autograd.Function):
-    """The same forward / backward as the registered ops, called without the custom-op
-    dispatch layers (about 20-30 us of host time per call).  Used outside torch.compile
-    tracing; under tracing the ops above are used so the graph records them."""
-
-    @staticmethod
-    def forward(ctx, q, k, v, freqs, bias, mask, causal, scale):
-        o, lse, ws = _fwd_impl(q, k, v, freqs, bias, mask, causal, scale)
-        ctx.save_for_backward(q, k, v, freqs, bias, mask, o, lse, _kept(ws))
-        ctx.causal, ctx.scale = causal, scale
-        return o
-
-    @staticmethod
-    def backward(ctx, do):
-        q, k, v, freqs, bias, mask, o, lse, ws = ctx.saved_tensors
-        need_df = bool(ctx.needs_input_grad[3]) and exists(freqs)
-        need_db = bool(ctx.needs_input_grad[4]) and exists(bias)
-        dq, dk, dv, df, db = _bwd_impl(do, q, k, v, o, lse, freqs, bias, mask, ctx.causal, ctx.scale,
-                                       need_df, need_db, ws)
-        return dq, dk, dv, df if need_df else None, db if need_db else None, None, None, None
-
-
 def _flash(q, k, v, freqs, bias, mask, causal, scale) -> Tensor:
-    if torch.compiler.is_compiling():
+    """The native call layer (csrc_torch/pope_host.cpp), or the ops above, with the same forward / backward,
+    where tracing, a dispatch mode or a transform works on the call."""
+    if not _lib.eager(q, k, v, freqs, bias, mask):
         return flash_fwd_op(q, k, v, freqs, bias, mask, causal, scale)[0]
-    return _FlashAttnEager.apply(q, k, v, freqs, bias, mask, causal, scale)
+    if exists(freqs) and freqs.shape[-1] > q.shape[-1]:
+        raise AssertionError(f"rotate dim {freqs.shape[-1]} exceeds head dim {q.shape[-1]}")
+    return _lib.host().flash(q, k, v, freqs, bias, mask, bool(causal), scale, _DECODE_MIN_KEYS, _REUSE_FWD_WORKSPACE)
 
 
 # ------------------------------------------------------------ head-first entry point

@@ -1,0 +1,105 @@
+"""Eager calls through the native call layer against the torch.library ops they stand beside: the same kernels on
+the same inputs, so the same bits (dbias, summed by atomics, within fp32 rounding); and the tracing and transform
+machinery that works on the ops still sees them."""
+import pytest
+import torch
+
+from gpu_common import make_pope_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def _grads(fn, leaves, up):
+    out = fn(*leaves)
+    outs = out if isinstance(out, tuple) else (out,)
+    return [o.detach() for o in outs] + list(torch.autograd.grad(outs, leaves, up))
+
+
+def _same(a, b):
+    for x, y in zip(a, b):
+        assert torch.equal(x, y) or torch.allclose(x, y, rtol=1e-5, atol=1e-5 * y.abs().max().item())
+
+
+@pytest.mark.parametrize("layout", ["dense", "seq_first", "offset_freqs", "batch_freqs", "one_bias_row", "no_pope", "decode"])
+def test_flash_matches_the_op(cuda, layout):
+    from pope_amd import _lib
+    from pope_amd.hip_pope_flash_attn import flash_fwd_op
+    B, Hq, Hk, Nq, Nk, R = 2, 4, 2, 70, 90, 32
+    if layout == "decode":
+        Nq, Nk = 1, 1500
+    inp = make_pope_inputs(61, B, Hq, Hk, Nq, Nk, 64, R, torch.bfloat16, "prefix")
+    q, k, v, f, b = (inp[n] for n in ("q", "k", "v", "freqs", "bias"))
+    if layout == "seq_first":
+        q, k, v = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v))
+    if layout == "offset_freqs":   # a table longer than the cache, viewed at an offset that keeps its alignment
+        f = torch.cat([f, f])[4:]
+    if layout == "batch_freqs":
+        f = torch.stack([f, f * 0.5])
+    if layout == "one_bias_row":
+        b = b[:1]
+    names = [q, k, v] if layout == "no_pope" else [q, k, v, f, b]
+    leaves = [t.detach().requires_grad_(True) for t in names]
+    pad = [None] * (5 - len(leaves))
+    scale = 0.125
+    native = _grads(lambda *t: _lib.host().flash(*t, *pad, inp["mask"], False, scale, 1024, True), leaves, inp["do"])
+    ops = _grads(lambda *t: flash_fwd_op(*t, *pad, inp["mask"], False, scale)[0], leaves, inp["do"])
+    _same(native, ops)
+
+
+@pytest.mark.parametrize("split", [False, True])
+def test_similarity_and_polar_match_the_ops(cuda, split):
+    from pope_amd import _lib
+    from pope_amd.hip_polar import polar_fwd_op
+    from pope_amd.hip_pope import sim_fwd_op
+    inp = make_pope_inputs(62, 2, 4, 2, 40, 75, 64, 24, torch.float32)
+    leaves = [inp[n].detach().requires_grad_(True) for n in ("q", "k", "freqs", "bias")]
+    leaves[0] = inp["q"].transpose(1, 2).contiguous().transpose(1, 2).requires_grad_(True)
+    up = torch.randn(2, 4, 40, 75, device="cuda")
+    _same(_grads(lambda *t: _lib.host().sim(*t, split), leaves, up), _grads(lambda *t: sim_fwd_op(*t, split), leaves, up))
+    E = 128 if split else 64 + 24
+    ups = (torch.randn(2, 4, 40, E, device="cuda"), torch.randn(2, 2, 75, E, device="cuda"))
+    _same(_grads(lambda *t: _lib.host().polar(*t, split), leaves, ups), _grads(lambda *t: polar_fwd_op(*t, split), leaves, ups))
+
+
+def test_transforms_and_modes_still_work_on_the_ops(cuda):
+    import pope_amd
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    inp = make_pope_inputs(63, 1, 2, 2, 16, 16, 32, 16, torch.float32)
+    q, k, f, b = (inp[n] for n in ("q", "k", "freqs", "bias"))
+    sim = lambda q, k: pope_amd.compute_attn_similarity(q, k, (f, b))
+    want = sim(q, k)
+    assert torch.equal(make_fx(sim)(q, k)(q, k), want)
+    leaf = q.detach().requires_grad_(True)
+    flash = lambda q: pope_amd.flash_attn_with_pope(q, k.bfloat16(), k.bfloat16(), pos_emb=(f, b))
+    for fn in (lambda t: sim(t, k).sum(), lambda t: flash(t.bfloat16()).float().sum()):
+        with pytest.raises(RuntimeError):   # functorch transforms: refused, by the ops' autograd functions
+            torch.func.grad(fn)(q)
+    traced = make_fx(flash)(q.bfloat16())
+    assert torch.equal(traced(q.bfloat16()), flash(q.bfloat16()))
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+        fq, fk = mode.from_tensor(q), mode.from_tensor(k)
+        assert sim(fq, fk).shape == want.shape
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t)[1], lambda t: t):
+        s = sim(leaf, k)
+        o = flash(leaf.bfloat16())
+    assert len(packed) >= 8
+    (s.sum() + o.float().sum()).backward()
+
+
+def test_second_derivative_of_the_similarity_raises(cuda):
+    import pope_amd
+    inp = make_pope_inputs(64, 1, 1, 1, 8, 8, 32, 16, torch.float32)
+    q = inp["q"].detach().requires_grad_(True)
+    s = pope_amd.compute_attn_similarity(q, inp["k"], (inp["freqs"], inp["bias"]))
+    (g,) = torch.autograd.grad(s.square().sum(), q, create_graph=True)
+    with pytest.raises(RuntimeError):
+        g.sum().backward()
+
+
+def test_operands_on_another_device_are_refused(cuda):
+    import pope_amd
+    inp = make_pope_inputs(65, 1, 1, 1, 8, 8, 32, 16, torch.bfloat16)
+    with pytest.raises(RuntimeError):
+        pope_amd.flash_attn_with_pope(inp["q"], inp["k"], inp["v"], pos_emb=(inp["freqs"].cpu(), inp["bias"]))
