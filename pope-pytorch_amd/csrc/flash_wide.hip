@@ -14,7 +14,14 @@
 // pass.  The streamed tiles go straight from global memory into LDS (global_load_lds_dwordx4) in
 // three slots, two steps ahead of the step computed: a step's products take less time than the
 // tile's fetch, and tiles staged through registers would hold registers these kernels do not
-// have.  Memory stays linear in the sequence length: no score matrix is stored.  Same workspace preparation as the narrow path
+// have.  Each step's operand reads run as one ring over its products, with the addresses formed by an
+// exclusive or from one base per tile, masks are applied on a side branch, and a head's jobs stay on
+// one XCD.  What bounds the kernels: one operand read from LDS per product (1 KB per 32 cycles and
+// SIMD), and the softmax of a wave's only row block, which nothing overlaps.  At (2, 8, 2048, 256),
+// R 256, causal bf16 (two chunks): forward 205 -> 117 us, dK/dV 649 -> 168 (921 TFLOP/s of products),
+// dQ 510 -> 167; before, every product group waited on reloads of spilled registers behind tile
+// loads that missed the XCD's L2.
+// Memory stays linear in the sequence length: no score matrix is stored.  Same workspace preparation as the narrow path
 // (flash_prep.hip: K_hat, Q_hat pre-scaled by softmax_scale * log2 e, key visibility words,
 // phase tables), with EP = E rounded up to 128 and DV = 256.
 //   wide_fwd   one workgroup per (128 queries, batch * head): S^T = K_hat Q_hat^T, online softmax
@@ -71,36 +78,81 @@ constexpr float kLazyMax = 8.f;
 // t + 2 load, so each tile has two steps of compute to arrive in.
 constexpr int kSlots = 3;
 
-// Transpose-read offsets (lo, hi) of column block nb of a tile, nb known only at run time: the
-// entry of the swizzle period is picked by selects rather than by indexing the offset arrays,
-// which would place them in scratch memory (vector loads that would wait on the tile loads).
-template <int U>
-__device__ __forceinline__ int2 tr_offsets(const TileOffsets<U>& o, int nb) {
-  constexpr int TP = TileOffsets<U>::TP;
-  const int k = nb % TP;
-  int lo = o.lo[0], hi = o.hi[0];
-#pragma unroll
-  for (int i = 1; i < TP; ++i) {
-    lo = k == i ? o.lo[i] : lo;
-    hi = k == i ? o.hi[i] : hi;
-  }
-  return make_int2(lo + 32 * (nb - k), hi + 32 * (nb - k));
+// Job of a workgroup: (block, head) of nb blocks per head and `heads` heads.  Workgroup ids go
+// round-robin over the 8 XCDs, each with its own 4 MB L2, and one head's streamed tiles are 3 MB at
+// N 2048: where the heads divide over the XCDs, an XCD takes its heads one after the other, heaviest
+// blocks first.  Otherwise the head index is fastest, so that a head stays on few XCDs.
+__device__ __forceinline__ int2 wide_job(int id, int nb, int heads) {
+  if (heads % 8 == 0) return make_int2(id / 8 % nb, id % 8 + 8 * (id / 8 / nb));
+  return make_int2(id / heads, id % heads);
 }
 
 // Direct global -> LDS fill of one tile of 32 rows x U 16-byte units, stored unpadded with
-// tile_swz (unit u of row r at position u ^ tile_swz(U, r)).  Load i of the thread fills
-// position c = 256 i + tid (a wave's 64 lanes write 64 consecutive positions), in row c / U,
-// with unit (c % U) ^ tile_swz(U, c / U) of that row; src(r, u) is its global address.
-template <int U, typename Src>
-__device__ __forceinline__ void tile_fill(const uint16_t* tile, int tid, int wave, Src src) {
+// tile_swz (unit u of row r at position u ^ tile_swz(U, r)).  Load i of the thread fills position
+// c = 64 (wave + 4 i) + lane (a wave's 64 lanes write 64 consecutive positions), in row c / U, with
+// unit (c % U) ^ tile_swz(U, c / U) of that row.
+//   dense rows of 8 U elements; U = 64: one row per wave load, so the row is scalar
+template <int U>
+__device__ __forceinline__ void fill_dense(uint32_t tile, int wave, int lane, const uint16_t* rows) {
   static_assert(32 * U % 256 == 0, "whole loads per thread");
-  const uint32_t base = lds_addr(tile) + 1024 * wave;
 #pragma unroll
   for (int i = 0; i < 32 * U / 256; ++i) {
-    const int c = tid + 256 * i, r = c / U;
-    load_lds16(src(r, (c % U) ^ tile_swz(U, r)), base + 4096 * i);
+    const int w = wave + 4 * i;
+    if constexpr (U == 64) {
+      load_lds16(rows + w * 8 * U, 16 * (lane ^ tile_swz(U, w)), tile + 1024 * w);
+    } else {
+      const int c = 64 * w + lane, r = c / U;
+      load_lds16(rows, 16 * (r * U + ((c % U) ^ tile_swz(U, r))), tile + 1024 * w);
+    }
   }
 }
+//   rows of a strided tensor from its row 0 of the tile: rows at or past `left` repeat the last one,
+//   units at or past D the row's last unit
+template <int U>
+__device__ __forceinline__ void fill_strided(uint32_t tile, int wave, int lane, const uint16_t* rows, uint32_t row_bytes,
+                                             int left, int D) {
+  static_assert(64 % U == 0, "whole rows per wave load");
+#pragma unroll
+  for (int i = 0; i < 32 * U / 256; ++i) {
+    const int w = wave + 4 * i, r = w * (64 / U) + lane / U;
+    const uint32_t col = 2 * min(8 * ((lane % U) ^ tile_swz(U, r)), D - 8);
+    load_lds16(rows, (uint32_t)min(r, left - 1) * row_bytes + col, tile + 1024 * w);
+  }
+}
+
+// LDS byte addresses of a tile's operand reads, from one row-read and one transpose-read base per
+// lane: with U % 16 == 0 and tiles on 256-byte boundaries, the swizzle turns the k step or column
+// block within 256 bytes into an exclusive or on the base (TileOffsets has the layout).  The bases
+// are opaque per step, so a step holds these two registers per tile and not one per address.
+template <int U>
+struct WideAddr {
+  static_assert(U % 16 == 0, "rows of whole 256-byte groups");
+  uint32_t row, tr;
+  static __device__ __forceinline__ uint32_t lane_row(int lane) {
+    const int lr = lane & 31, hf = lane >> 5;
+    return 16 * (lr * U + (hf ^ tile_swz(U, lr)));
+  }
+  // of column blocks CH nb + ec
+  static __device__ __forceinline__ uint32_t lane_tr(int lane, int ec) {
+    const int j = lane & 15, hf = lane >> 5, u = 2 * ((lane >> 4) & 1) + ((j >> 1) & 1), r = 4 * hf + (j >> 2);
+    return 16 * (r * U + ((u ^ tile_swz(U, r)) ^ (4 * ec))) + 8 * (j & 1);
+  }
+  __device__ __forceinline__ WideAddr(uint32_t tile, uint32_t lrow, uint32_t ltr)
+      : row(opaque_u32(tile + lrow)), tr(opaque_u32(tile + ltr)) {}
+  __device__ __forceinline__ u32x4 row_at(int kk) const { return lds_read16_at((row ^ (32 * (kk % 8))) + 256 * (kk / 8)); }
+  // rows 16 g + (4 hf .. + 3) and + 8 of column block nb of the lane's chunk
+  template <int CH>
+  __device__ __forceinline__ u32x4 tr_at(int x, int g) const {
+    const uint32_t nb = CH * x, o = 256 * (nb / 4) + 256 * U * g, lo = 64 * (nb % 4);
+    return lds_tr8_at((tr ^ lo) + o, (tr ^ (lo ^ 32)) + o + 128 * U);
+  }
+};
+
+// Operand reads kept in flight ahead of the product that takes them: as many of eight as leave the
+// kernel without spills (a reload waits for every tile load in flight behind it).
+template <int EP>
+constexpr int fwd_ring() { return EP >= 512 ? 6 : 8; }
+constexpr int kKvRing = 4, kQRing = 8;
 
 // ---- forward ---------------------------------------------------------------------------
 // Four waves per workgroup, 128 query rows (wave w: rows q0 + 32 w ..); per 32-key tile the K_hat
@@ -110,21 +162,20 @@ __device__ __forceinline__ void tile_fill(const uint16_t* tile, int tid, int wav
 // SPLIT: one split of the key axis per workgroup, fp32 partials (as in flash_fwd.hip).
 template <typename T, int EP, int DV, bool SPLIT>
 __global__ __launch_bounds__(256) void wide_fwd_kernel(FlashFwdParams p) {
-  constexpr int KS = EP / 16, NDB = DV / 32;
+  constexpr int KS = EP / 16, NDB = DV / 32, kRing = fwd_ring<EP>();
   constexpr int KU = EP / 8, VU = DV / 8;              // 16-byte units per K_hat / V row
   constexpr int NL = 32 * (KU + VU) / 256;             // loads per thread and tile
+  constexpr uint32_t KT = 64 * EP, SLOT = 64 * (EP + DV);   // bytes of the K_hat tile and of a slot
   typedef typename T::vec8 vec8;
-  __shared__ __attribute__((aligned(16))) uint16_t kt[kSlots][32 * EP];
-  __shared__ __attribute__((aligned(16))) uint16_t vt[kSlots][32 * DV];
+  __shared__ __attribute__((aligned(256))) char smem[kSlots * SLOT];
 
   const int tid = threadIdx.x, wave = wave_id(), lane = tid & 63, lr = lane & 31, hf = lane >> 5;
-  const int BH = p.B * p.Hq, nqb = (p.Nq + 127) / 128;
-  const int bh = blockIdx.x % BH;
-  const int rest = (int)(blockIdx.x / BH);
-  const int sp = SPLIT ? rest % p.splits : 0;
-  const int q0 = 128 * (nqb - 1 - (SPLIT ? rest / p.splits : rest));   // heaviest causal blocks first
+  const int BH = p.B * p.Hq, nqb = (p.Nq + 127) / 128, splits = SPLIT ? p.splits : 1;
+  const int2 job = wide_job(blockIdx.x, nqb * splits, BH);
+  const int bh = job.y, sp = SPLIT ? job.x % splits : 0;
+  const int q0 = 128 * (nqb - 1 - (SPLIT ? job.x / splits : job.x));   // heaviest causal blocks first
   const int b = bh / p.Hq, h = bh % p.Hq, hk = h % p.Hk;
-  const int Nk = p.Nk, D = p.D, qi = q0 + 32 * wave + lr;
+  const int Nk = p.Nk, D = p.D, qw = q0 + 32 * wave, qi = qw + lr;
 
   int nkeys = min(((ci32*)p.kend)[b], Nk);
   if (p.causal) nkeys = min(nkeys, q0 + 128);
@@ -133,19 +184,18 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(FlashFwdParams p) {
   const uint16_t* khb = p.kh + (int64_t)(b * p.Hk + hk) * p.NkP * EP;   // rows padded to NkP
   const uint16_t* vb = p.v + (int64_t)b * p.v_s[0] + (int64_t)hk * p.v_s[1];
   cu64* mw = (cu64*)p.mwords + (int64_t)b * p.NW;
-  const TileOffsets<KU> ko(lane);
-  const TileOffsets<VU> vo(lane);
+  const uint32_t lds0 = lds_addr(smem);
+  const uint32_t krow = WideAddr<KU>::lane_row(lane), vtr = WideAddr<VU>::lane_tr(lane, 0);
+  const uint32_t v_row = 2 * (uint32_t)p.v_s[2];
 
   // tile t into slot t % kSlots: K_hat rows are padded to NkP (no clamp); V rows past Nk repeat
   // the last one and V units at or past D repeat the row's last unit (they only reach the O rows
   // at or past D, which are not stored)
   auto issue = [&](int t) {
-    const int j0 = 32 * (t0 + t), slot = t % kSlots;
-    const uint16_t* kp = khb + (int64_t)j0 * EP;
-    tile_fill<KU>(kt[slot], tid, wave, [&](int r, int u) { return kp + r * EP + 8 * u; });
-    tile_fill<VU>(vt[slot], tid, wave, [&](int r, int u) {
-      return vb + (int64_t)min(j0 + r, Nk - 1) * p.v_s[2] + min(8 * u, D - 8);
-    });
+    const int j0 = 32 * (t0 + t);
+    const uint32_t slot = lds0 + (t % kSlots) * SLOT;
+    fill_dense<KU>(slot, wave, lane, khb + (int64_t)j0 * EP);
+    fill_strided<VU>(slot + KT, wave, lane, vb + (int64_t)j0 * p.v_s[2], v_row, Nk - j0, D);
   };
   const int nt = max((nkeys + 31) / 32 - t0, 0);
   if (nt > 0) issue(0);
@@ -164,53 +214,65 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(FlashFwdParams p) {
   f32x16 oacc[NDB];
 #pragma unroll
   for (int db = 0; db < NDB; ++db) oacc[db] = splat16(0.f);
-  float m = -INFINITY, l = 0.f;
+  float m = -INFINITY, l = 0.f;   // l: the lane half's share of the row sum
   const uint32_t ones = T::pack2(1.f, 1.f);
+  uint32_t word = nt > 0 ? (uint32_t)(mw[t0 >> 1] >> (32 * (t0 & 1))) : 0u;   // visibility of the step's keys
   for (int t = 0; t < nt; ++t) {
-    const int buf = t % kSlots, j0 = 32 * (t0 + t);
+    const int j0 = 32 * (t0 + t);
     if (t + 1 < nt) wait_vmcnt<NL>();   // this thread's loads of tile t landed (t + 1 may be in flight)
     else wait_vmcnt<0>();
     __syncthreads();                    // ... everyone's; and slot (t + 2) % kSlots was last read in step t - 1
     if (t + 2 < nt) issue(t + 2);
-    // S^T (rows = keys, lane = query), log2 units
+    const uint32_t wv = word;
+    if (t + 1 < nt) word = (uint32_t)(mw[(t0 + t + 1) >> 1] >> (32 * ((t0 + t + 1) & 1)));
+    const uint32_t slot = lds0 + (t % kSlots) * SLOT;
+    const WideAddr<KU> ka(slot, krow, 0);
+    const WideAddr<VU> va(slot + KT, 0, vtr);
+    // one ring of operand reads over both products: S^T = K_hat Q_hat^T (rows = keys, lane = query,
+    // log2 units), then O^T += V^T P^T; the first V operands arrive during the softmax
+    constexpr int NP = KS + 2 * NDB;
+    u32x4 f[kRing];
+    auto operand = [&](int i) { return i < KS ? ka.row_at(i) : va.template tr_at<1>((i - KS) % NDB, (i - KS) / NDB); };
+#pragma unroll
+    for (int i = 0; i < kRing; ++i) f[i] = operand(i);
+    __builtin_amdgcn_sched_barrier(0);
     f32x16 s = splat16(0.f);
 #pragma unroll
-    for (int kk = 0; kk < KS; ++kk)
-      s = T::mfma32(as_vec8<vec8>(*reinterpret_cast<const u32x4*>(kt[buf] + ko.row_at(kk))), qreg[kk], s);
-    const uint32_t wv = (uint32_t)(mw[j0 >> 6] >> (j0 & 32));
-    float mt = -INFINITY;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int kr_ = res_row(r, hf);
-      const bool ok = ((wv >> kr_) & 1u) && (!p.causal || j0 + kr_ <= qi);
-      s[r] = ok ? s[r] : -INFINITY;
-      mt = fmaxf(mt, s[r]);
+    for (int i = 0; i < KS; ++i) {
+      s = T::mfma32(as_vec8<vec8>(f[i % kRing]), qreg[i], s);
+      f[i % kRing] = operand(i + kRing);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-    float alpha = 1.f;
-    if constexpr (EP < 512) {
-      // lazy rescale: a row's reference max m moves only when the tile's max exceeds it by more
-      // than kLazyMax (log2 units), so the probabilities stay below 2^kLazyMax and most steps skip
-      // rescaling the O accumulators (the branch is taken when any row of the wave moves).  At
-      // 512 features the branch costs more than it saves: the rescale stays in every step.
-      const bool grow = mt > m + kLazyMax;
-      if (__ballot(grow)) {
-        const float mn = grow ? mt : m;
-        alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+    if (wv != 0xffffffffu || (p.causal && j0 + 31 > qw)) {   // a masked key, or the causal diagonal
+      POPE_COLD_PATH();
+      const int lim = qi - j0 - 4 * hf;   // causal: row offset <= lim
 #pragma unroll
-        for (int db = 0; db < NDB; ++db)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
-        m = mn;   // l takes alpha below
+      for (int r = 0; r < 16; ++r) {
+        const int kr_ = 8 * (r >> 2) + (r & 3);
+        s[r] = ((wv >> (4 * hf + kr_)) & 1u) && (!p.causal || kr_ <= lim) ? s[r] : -INFINITY;
       }
-    } else {
-      const float mn = fmaxf(m, mt);
-      alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+    }
+    float mt = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mt = fmaxf(mt, s[r]);
+    mt = half_swap_max(mt);
+    // lazy rescale: a row's reference max m moves only when the tile's max exceeds it by more than
+    // kLazyMax (log2 units), so the probabilities stay below 2^kLazyMax and most steps skip
+    // rescaling the O accumulators (the branch is taken when any row of the wave moves)
+    const bool grow = mt > m + kLazyMax;
+    if (__ballot(grow)) {
+      POPE_COLD_PATH();
+      const float mn = grow ? mt : m;
+      const float alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
+      l *= alpha;
       m = mn;
     }
     const float mu = m == -INFINITY ? 0.f : m;
     u32x4 pw[2];
-    float ls = 0.f;
 #pragma unroll
     for (int g = 0; g < 2; ++g)
 #pragma unroll
@@ -218,21 +280,17 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(FlashFwdParams p) {
         const uint32_t w = T::pack2(__builtin_amdgcn_exp2f(s[8 * g + 2 * q] - mu),
                                     __builtin_amdgcn_exp2f(s[8 * g + 2 * q + 1] - mu));
         pw[g][q] = w;
-        ls = T::dot2(w, ones, ls);   // the row sum of the probabilities the products use
-      }
-    l = l * alpha + ls + __shfl_xor(ls, 32, 64);
-#pragma unroll
-    for (int db = 0; db < NDB; ++db) {
-      if constexpr (EP >= 512) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
+        l = T::dot2(w, ones, l);   // the row sum of the probabilities the products use
       }
 #pragma unroll
-      for (int g = 0; g < 2; ++g)
-        oacc[db] = T::mfma32(as_vec8<vec8>(lds_tr8(vt[buf], vo.lo_at(db) + 16 * g * DV, vo.hi_at(db) + 16 * g * DV)),
-                             as_vec8<vec8>(pw[g]), oacc[db]);
+    for (int i = KS; i < NP; ++i) {
+      const int db = (i - KS) % NDB;
+      oacc[db] = T::mfma32(as_vec8<vec8>(f[i % kRing]), as_vec8<vec8>(pw[(i - KS) / NDB]), oacc[db]);
+      if (i + kRing < NP) f[i % kRing] = operand(i + kRing);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
+  l += __shfl_xor(l, 32, 64);
   if (qi >= p.Nq) return;
   if constexpr (SPLIT) {
     const int64_t prow = (((int64_t)b * p.Hq + h) * p.Nq + qi) * p.splits + sp;
@@ -277,16 +335,16 @@ template <typename T, int EP, int DV, int CH>
 __global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p, float* wk) {
   constexpr int KS = EP / 16, DS = DV / 16, EBC = EP / 32 / CH, DBC = DV / 32 / CH, RB = 4 / CH;
   constexpr int QU = EP / 8, OU = DV / 8, NL = 32 * (QU + OU) / 256;
+  constexpr uint32_t QT = 64 * EP, RT = 64 * (EP + DV), SLOT = RT + 1024;   // byte offsets in a slot: dO tile, row terms
   typedef typename T::vec8 vec8;
-  __shared__ __attribute__((aligned(16))) uint16_t qt[kSlots][32 * EP];
-  __shared__ __attribute__((aligned(16))) uint16_t dt[kSlots][32 * DV];
-  __shared__ __attribute__((aligned(16))) float rt[kSlots][256];   // [0, 32) -lse, [32, 64) -delta
+  __shared__ __attribute__((aligned(256))) char smem[kSlots * SLOT];
 
   const int tid = threadIdx.x, wave = wave_id(), lane = tid & 63, lr = lane & 31, hf = lane >> 5;
   const int nkb = p.NkP / (32 * RB);
-  const int ec = (tid >> 6) % CH;   // the wave's column chunk
-  const int kb0 = 32 * RB * ((int)blockIdx.x % nkb), bhk = (int)blockIdx.x / nkb;   // key block 0 (the heaviest causal one) first
-  const int k0 = kb0 + 32 * ((tid >> 6) / CH);   // the wave's keys
+  const int ec = wave % CH;   // the wave's column chunk
+  const int2 job = wide_job(blockIdx.x, nkb, p.B * p.Hk);
+  const int kb0 = 32 * RB * job.x, bhk = job.y;   // key block 0 (the heaviest causal one) first
+  const int k0 = kb0 + 32 * (wave / CH);   // the wave's keys
   const int b = bhk / p.Hk, hk = bhk % p.Hk;
   const int Nk = p.Nk, Nq = p.Nq, D = p.D, NqP = p.NqP;
   if (kb0 >= Nk) return;
@@ -299,33 +357,32 @@ __global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p, float* w
   const int qstart = p.causal ? kb0 : 0;   // the workgroup's first key block
   const int nsq = Nq > qstart ? (Nq - qstart + 31) / 32 : 0;
   const int nsteps = __syncthreads_or(kvis) ? groups * nsq : 0;   // uniform over the workgroup
-  auto step_at = [&](int st, int& h, int& q0) {
-    h = (st / nsq) * p.Hk + hk;
-    q0 = qstart + 32 * (st % nsq);
-  };
-  // step st's tiles into slot st % kSlots: Q_hat rows padded to NqP (no clamp); dO rows past Nq
+  const uint32_t lds0 = lds_addr(smem), do_row = 2 * (uint32_t)p.do_s[2];
+  // the next step's tiles into the next slot: Q_hat rows padded to NqP (no clamp); dO rows past Nq
   // repeat the last one and dO units at or past D repeat the row's last unit (they meet zero V
   // columns in dP and reach only the dV columns at or past D, which are not stored)
-  auto issue = [&](int st) {
-    int h, q0;
-    step_at(st, h, q0);
-    const int slot = st % kSlots;
-    const uint16_t* qhb = p.qh + ((int64_t)(b * p.Hq + h) * NqP + q0) * EP;
-    const uint16_t* dob = p.dout + (int64_t)b * p.do_s[0] + (int64_t)h * p.do_s[1];
-    tile_fill<QU>(qt[slot], tid, wave, [&](int r, int u) { return qhb + r * EP + 8 * u; });
-    tile_fill<OU>(dt[slot], tid, wave, [&](int r, int u) {
-      return dob + (int64_t)min(q0 + r, Nq - 1) * p.do_s[2] + min(8 * u, D - 8);
-    });
-    // the row terms of queries q0 .. q0 + 31: lane units 0-7 -lse, 8-15 -delta (lanes past 15
-    // repeat them past float 64, unread)
+  int ih = hk, iq = qstart, islot = 0;
+  auto issue = [&]() {
+    const uint32_t slot = lds0 + islot * SLOT;
+    const int64_t row = (int64_t)(b * p.Hq + ih) * NqP + iq;
+    fill_dense<QU>(slot, wave, lane, p.qh + row * EP);
+    fill_strided<OU>(slot + QT, wave, lane,
+                     p.dout + (int64_t)b * p.do_s[0] + (int64_t)ih * p.do_s[1] + (int64_t)iq * p.do_s[2], do_row, Nq - iq, D);
+    // the row terms of the step's queries: lane units 0-7 -lse, 8-15 -delta (lanes past 15 repeat
+    // them past float 64, unread)
     if (wave == 0) {
       const int u = lane & 15;
-      const float* src = (u < 8 ? p.nl : p.nd) + (int64_t)(b * p.Hq + h) * NqP + q0 + 4 * (u & 7);
-      load_lds16(src, lds_addr(rt[slot]));
+      load_lds16((u < 8 ? p.nl : p.nd) + row + 4 * (u & 7), slot + RT);
     }
+    iq += 32;
+    if (iq >= Nq) {
+      iq = qstart;
+      ih += p.Hk;
+    }
+    islot = islot == kSlots - 1 ? 0 : islot + 1;
   };
-  if (nsteps > 0) issue(0);
-  if (nsteps > 1) issue(1);
+  if (nsteps > 0) issue();
+  if (nsteps > 1) issue();
 
   vec8 kreg[KS], vreg[DS];
   {
@@ -336,7 +393,8 @@ __global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p, float* w
 #pragma unroll
     for (int kk = 0; kk < DS; ++kk) {
       const int d0 = 16 * kk + 8 * hf;
-      vreg[kk] = as_vec8<vec8>((kj < Nk && d0 < D) ? ld16(vr + d0) : zero4());
+      const u32x4 x = ld16(vr + min(d0, D - 8));   // no branch: a valid address always, the value selected
+      vreg[kk] = as_vec8<vec8>((kj < Nk && d0 < D) ? x : zero4());
     }
   }
   // the K_hat / V rows as loads the compiler sees complete: no use of them in the loop waits on
@@ -347,20 +405,12 @@ __global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p, float* w
   for (int x = 0; x < EBC; ++x) dka[x] = splat16(0.f);
 #pragma unroll
   for (int x = 0; x < DBC; ++x) dva[x] = splat16(0.f);
-  // the tiles' row-read offsets, and the wave's transpose-read offsets: its dV column blocks of
-  // the dO tile, its dK_hat column blocks of the Q_hat tile
-  const TileOffsets<QU> qo(lane);
-  const TileOffsets<OU> dO(lane);
-  int2 dof[DBC], qof[EBC];
-#pragma unroll
-  for (int db = 0; db < DBC; ++db) dof[db] = tr_offsets(dO, ec * DBC + db);
-#pragma unroll
-  for (int eb = 0; eb < EBC; ++eb) qof[eb] = tr_offsets(qo, ec * EBC + eb);
+  const uint32_t qrow = WideAddr<QU>::lane_row(lane), qtr = WideAddr<QU>::lane_tr(lane, ec);
+  const uint32_t orow = WideAddr<OU>::lane_row(lane), otr = WideAddr<OU>::lane_tr(lane, ec);
+  const bool wave_vis = __all(kvis);
 
+  int q0 = qstart, buf = 0;
   for (int st = 0; st < nsteps; ++st) {
-    const int buf = st % kSlots;
-    int h, q0;
-    step_at(st, h, q0);
     // this thread's loads of step st landed (st + 1 may be in flight; wave 0 has one more per step)
     if (st + 1 < nsteps) {
       if (wave == 0) wait_vmcnt<NL + 1>();
@@ -369,59 +419,79 @@ __global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p, float* w
       wait_vmcnt<0>();
     }
     __syncthreads();                         // ... everyone's; and slot (st + 2) % kSlots was last read in step st - 1
-    if (st + 2 < nsteps) issue(st + 2);
+    if (st + 2 < nsteps) issue();
+    const uint32_t slot = lds0 + buf * SLOT;
+    const WideAddr<QU> qa(slot, qrow, qtr);
+    const WideAddr<OU> oa(slot + QT, orow, otr);
     // -lse and -delta of the result rows (queries q0 + res_row(r, hf); padded rows give P = 0)
+    const uint32_t ra = slot + RT + 16 * hf;
     f32x16 s, dp;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const f32x4 a = *reinterpret_cast<const f32x4*>(&rt[buf][8 * q + 4 * hf]);
-      const f32x4 c = *reinterpret_cast<const f32x4*>(&rt[buf][32 + 8 * q + 4 * hf]);
+      const f32x4 a = lds_read_f4_at(ra + 32 * q), c = lds_read_f4_at(ra + 128 + 32 * q);
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         s[4 * q + x] = a[x];
         dp[4 * q + x] = c[x];
       }
     }
-    // S = Q_hat K_hat^T - lse and dP = dO V^T - delta (rows = queries, lane = key)
+    // one ring of operand reads over the step's products: S = Q_hat K_hat^T - lse and
+    // dP = dO V^T - delta (rows = queries, lane = key), then dV += P^T dO and dK_hat += dS^T Q_hat
+    // by 16 queries; the first transposed operands arrive during the exponentials
+    constexpr int N1 = KS + DS, NX = DBC + EBC, NP = N1 + 2 * NX;
+    u32x4 f[kKvRing];
+    auto operand = [&](int i) {
+      if (i < KS) return qa.row_at(i);
+      if (i < N1) return oa.row_at(i - KS);
+      const int g = (i - N1) / NX, x = (i - N1) % NX;
+      return x < DBC ? oa.template tr_at<CH>(x, g) : qa.template tr_at<CH>(x - DBC, g);
+    };
 #pragma unroll
-    for (int kg = 0; kg < KS; kg += 8) {
+    for (int i = 0; i < kKvRing; ++i) f[i] = operand(i);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int kk = kg; kk < kg + 8; ++kk)
-        s = T::mfma32(as_vec8<vec8>(*reinterpret_cast<const u32x4*>(qt[buf] + qo.row_at(kk))), kreg[kk], s);
-      __builtin_amdgcn_sched_barrier(0);   // eight operand reads in flight, not all of them
-    }
-#pragma unroll
-    for (int kg = 0; kg < DS; kg += 8) {
-#pragma unroll
-      for (int kk = kg; kk < kg + 8; ++kk)
-        dp = T::mfma32(as_vec8<vec8>(*reinterpret_cast<const u32x4*>(dt[buf] + dO.row_at(kk))), vreg[kk], dp);
+    for (int i = 0; i < N1; ++i) {
+      if (i < KS) s = T::mfma32(as_vec8<vec8>(f[i % kKvRing]), kreg[i < KS ? i : 0], s);
+      else dp = T::mfma32(as_vec8<vec8>(f[i % kKvRing]), vreg[i < KS ? 0 : i - KS], dp);
+      f[i % kKvRing] = operand(i + kKvRing);
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!wave_vis || (p.causal && q0 < k0 + 31)) {   // a masked key, or the causal diagonal
+      POPE_COLD_PATH();
+      const int lim = q0 + 4 * hf - kj;   // causal: row offset >= -lim
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        s[r] = (kvis && (!p.causal || 8 * (r >> 2) + (r & 3) + lim >= 0)) ? s[r] : -INFINITY;
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const bool ok = kvis && (!p.causal || kj <= q0 + res_row(r, hf));
-      const float pv = ok ? __builtin_amdgcn_exp2f(s[r]) : 0.f;
+      const float pv = __builtin_amdgcn_exp2f(s[r]);
       s[r] = pv;
       dp[r] = pv * dp[r];
     }
+    vec8 ap[2], ads[2];
 #pragma unroll
-    for (int g2 = 0; g2 < 2; ++g2) {
-      const vec8 ap = as_vec8<vec8>(pack8w<T>(s, g2)), ads = as_vec8<vec8>(pack8w<T>(dp, g2));
-#pragma unroll
-      for (int db = 0; db < DBC; ++db)
-        dva[db] = T::mfma32(
-            ap, as_vec8<vec8>(lds_tr8(dt[buf], dof[db].x + 16 * g2 * DV, dof[db].y + 16 * g2 * DV)), dva[db]);
-#pragma unroll
-      for (int eb = 0; eb < EBC; ++eb)
-        dka[eb] = T::mfma32(
-            ads, as_vec8<vec8>(lds_tr8(qt[buf], qof[eb].x + 16 * g2 * EP, qof[eb].y + 16 * g2 * EP)), dka[eb]);
+    for (int g = 0; g < 2; ++g) {
+      ap[g] = as_vec8<vec8>(pack8w<T>(s, g));
+      ads[g] = as_vec8<vec8>(pack8w<T>(dp, g));
     }
+#pragma unroll
+    for (int i = N1; i < NP; ++i) {
+      const int g = (i - N1) / NX, x = (i - N1) % NX;
+      if (x < DBC) dva[x < DBC ? x : 0] = T::mfma32(ap[g], as_vec8<vec8>(f[i % kKvRing]), dva[x < DBC ? x : 0]);
+      else dka[x < DBC ? 0 : x - DBC] = T::mfma32(ads[g], as_vec8<vec8>(f[i % kKvRing]), dka[x < DBC ? 0 : x - DBC]);
+      if (i + kKvRing < NP) f[i % kKvRing] = operand(i + kKvRing);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    q0 += 32;
+    if (q0 >= Nq) q0 = qstart;
+    buf = buf == kSlots - 1 ? 0 : buf + 1;
   }
   // dV (lane = d column, registers = keys); the raw dK_hat chunk, times ln 2 (Q_hat carries log2 e)
   uint16_t* dvb = p.dv + (int64_t)b * p.dv_s[0] + (int64_t)hk * p.dv_s[1];
 #pragma unroll
   for (int db = 0; db < DBC; ++db) {
-    const int d = 32 * (ec * DBC + db) + lr;
+    const int d = 32 * (CH * db + ec) + lr;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int key = k0 + res_row(r, hf);
@@ -431,7 +501,7 @@ __global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p, float* w
   float* wkb = wk + (int64_t)bhk * p.NkP * EP;
 #pragma unroll
   for (int eb = 0; eb < EBC; ++eb) {
-    const int e = 32 * (ec * EBC + eb) + lr;
+    const int e = 32 * (CH * eb + ec) + lr;
 #pragma unroll
     for (int r = 0; r < 16; ++r) wkb[(int64_t)(k0 + res_row(r, hf)) * EP + e] = dka[eb][r] * kLn2;
   }
@@ -445,15 +515,16 @@ template <typename T, int EP, int DV, int CH>
 __global__ __launch_bounds__(256) void wide_q_kernel(FlashBwdParams p, float* wq) {
   constexpr int KS = EP / 16, DS = DV / 16, EBC = EP / 32 / CH, RB = 4 / CH;
   constexpr int KU = EP / 8, VU = DV / 8, NL = 32 * (KU + VU) / 256;
+  constexpr uint32_t KT = 64 * EP, SLOT = 64 * (EP + DV);   // bytes of the K_hat tile and of a slot
   typedef typename T::vec8 vec8;
-  __shared__ __attribute__((aligned(16))) uint16_t kt[kSlots][32 * EP];
-  __shared__ __attribute__((aligned(16))) uint16_t vt[kSlots][32 * DV];
+  __shared__ __attribute__((aligned(256))) char smem[kSlots * SLOT];
 
   const int tid = threadIdx.x, wave = wave_id(), lane = tid & 63, lr = lane & 31, hf = lane >> 5;
   const int nqb = p.NqP / (32 * RB);
-  const int ec = (tid >> 6) % CH;   // the wave's column chunk
-  const int qb0 = 32 * RB * (nqb - 1 - (int)blockIdx.x % nqb), bh = (int)blockIdx.x / nqb;   // heaviest causal blocks first
-  const int q0 = qb0 + 32 * ((tid >> 6) / CH);   // the wave's queries
+  const int ec = wave % CH;   // the wave's column chunk
+  const int2 job = wide_job(blockIdx.x, nqb, p.B * p.Hq);
+  const int qb0 = 32 * RB * (nqb - 1 - job.x), bh = job.y;   // heaviest causal blocks first
+  const int q0 = qb0 + 32 * (wave / CH);   // the wave's queries
   const int b = bh / p.Hq, h = bh % p.Hq, hk = h % p.Hk;
   const int Nk = p.Nk, Nq = p.Nq, D = p.D;
   if (qb0 >= Nq) return;
@@ -462,15 +533,14 @@ __global__ __launch_bounds__(256) void wide_q_kernel(FlashBwdParams p, float* wq
   if (p.causal) nkeys = min(nkeys, qb0 + 32 * RB);   // the workgroup's last query block
   const uint16_t* khb = p.kh + (int64_t)(b * p.Hk + hk) * p.NkP * EP;   // rows padded to NkP
   const uint16_t* vb = p.v + (int64_t)b * p.v_s[0] + (int64_t)hk * p.v_s[1];
+  const uint32_t lds0 = lds_addr(smem), v_row = 2 * (uint32_t)p.v_s[2];
   // tile t into slot t % kSlots: K_hat rows padded to NkP (no clamp); V rows past Nk repeat the
   // last one and V units at or past D repeat the row's last unit (they meet zero dO columns)
   auto issue = [&](int t) {
-    const int j0 = 32 * t, slot = t % kSlots;
-    const uint16_t* kp = khb + (int64_t)j0 * EP;
-    tile_fill<KU>(kt[slot], tid, wave, [&](int r, int u) { return kp + r * EP + 8 * u; });
-    tile_fill<VU>(vt[slot], tid, wave, [&](int r, int u) {
-      return vb + (int64_t)min(j0 + r, Nk - 1) * p.v_s[2] + min(8 * u, D - 8);
-    });
+    const int j0 = 32 * t;
+    const uint32_t slot = lds0 + (t % kSlots) * SLOT;
+    fill_dense<KU>(slot, wave, lane, khb + (int64_t)j0 * EP);
+    fill_strided<VU>(slot + KT, wave, lane, vb + (int64_t)j0 * p.v_s[2], v_row, Nk - j0, D);
   };
   const int nt = (nkeys + 31) / 32;
   if (nt > 0) issue(0);
@@ -485,7 +555,8 @@ __global__ __launch_bounds__(256) void wide_q_kernel(FlashBwdParams p, float* wq
 #pragma unroll
     for (int kk = 0; kk < DS; ++kk) {
       const int d0 = 16 * kk + 8 * hf;
-      doreg[kk] = as_vec8<vec8>((qi < Nq && d0 < D) ? ld16(dr + d0) : zero4());
+      const u32x4 x = ld16(dr + min(d0, D - 8));   // no branch: a valid address always, the value selected
+      doreg[kk] = as_vec8<vec8>((qi < Nq && d0 < D) ? x : zero4());
     }
   }
   const float nls = p.nl[(int64_t)bh * p.NqP + qi], nds = p.nd[(int64_t)bh * p.NqP + qi];
@@ -496,45 +567,60 @@ __global__ __launch_bounds__(256) void wide_q_kernel(FlashBwdParams p, float* wq
 #pragma unroll
   for (int x = 0; x < EBC; ++x) dqa[x] = splat16(0.f);
   cu64* mw = (cu64*)p.mwords + (int64_t)b * p.NW;
-  const TileOffsets<KU> ko(lane);
-  const TileOffsets<VU> vo(lane);
+  const uint32_t krow = WideAddr<KU>::lane_row(lane), ktr = WideAddr<KU>::lane_tr(lane, ec);
+  const uint32_t vrow = WideAddr<VU>::lane_row(lane);
+  uint32_t word = nt > 0 ? (uint32_t)mw[0] : 0u;   // visibility of the step's keys
   for (int t = 0; t < nt; ++t) {
-    const int buf = t % kSlots, j0 = 32 * t;
+    const int j0 = 32 * t;
     if (t + 1 < nt) wait_vmcnt<NL>();   // this thread's loads of tile t landed (t + 1 may be in flight)
     else wait_vmcnt<0>();
     __syncthreads();                    // ... everyone's; and slot (t + 2) % kSlots was last read in step t - 1
     if (t + 2 < nt) issue(t + 2);
-    // S^T = K_hat Q_hat^T - lse and dP^T = V dO^T - delta (rows = keys, lane = query)
+    const uint32_t wv = word;
+    if (t + 1 < nt) word = (uint32_t)(mw[(t + 1) >> 1] >> (32 * ((t + 1) & 1)));
+    const uint32_t slot = lds0 + (t % kSlots) * SLOT;
+    const WideAddr<KU> ka(slot, krow, ktr);
+    const WideAddr<VU> va(slot + KT, vrow, 0);
+    // one ring of operand reads: S^T = K_hat Q_hat^T - lse and dP^T = V dO^T - delta (rows = keys,
+    // lane = query), then dQ_hat^T += K_hat^T dS^T by 16 keys
+    constexpr int N1 = KS + DS, NP = N1 + 2 * EBC;
+    u32x4 f[kQRing];
+    auto operand = [&](int i) {
+      if (i < KS) return ka.row_at(i);
+      if (i < N1) return va.row_at(i - KS);
+      return ka.template tr_at<CH>((i - N1) % EBC, (i - N1) / EBC);
+    };
+#pragma unroll
+    for (int i = 0; i < kQRing; ++i) f[i] = operand(i);
+    __builtin_amdgcn_sched_barrier(0);
     f32x16 s = splat16(nls), dp = splat16(nds);
 #pragma unroll
-    for (int kg = 0; kg < KS; kg += 8) {
-#pragma unroll
-      for (int kk = kg; kk < kg + 8; ++kk)
-        s = T::mfma32(as_vec8<vec8>(*reinterpret_cast<const u32x4*>(kt[buf] + ko.row_at(kk))), qreg[kk], s);
-      __builtin_amdgcn_sched_barrier(0);   // eight operand reads in flight, not all of them
-    }
-#pragma unroll
-    for (int kg = 0; kg < DS; kg += 8) {
-#pragma unroll
-      for (int kk = kg; kk < kg + 8; ++kk)
-        dp = T::mfma32(as_vec8<vec8>(*reinterpret_cast<const u32x4*>(vt[buf] + vo.row_at(kk))), doreg[kk], dp);
+    for (int i = 0; i < N1; ++i) {
+      if (i < KS) s = T::mfma32(as_vec8<vec8>(f[i % kQRing]), qreg[i < KS ? i : 0], s);
+      else dp = T::mfma32(as_vec8<vec8>(f[i % kQRing]), doreg[i < KS ? 0 : i - KS], dp);
+      f[i % kQRing] = operand(i + kQRing);
       __builtin_amdgcn_sched_barrier(0);
     }
-    const uint32_t wv = (uint32_t)(mw[j0 >> 6] >> (j0 & 32));
+    if (wv != 0xffffffffu || (p.causal && j0 + 31 > q0)) {   // a masked key, or the causal diagonal
+      POPE_COLD_PATH();
+      const int lim = qi - j0 - 4 * hf;   // causal: row offset <= lim
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int kr_ = res_row(r, hf);
-      const bool ok = ((wv >> kr_) & 1u) && (!p.causal || j0 + kr_ <= qi);
-      dp[r] = ok ? __builtin_amdgcn_exp2f(s[r]) * dp[r] : 0.f;
+      for (int r = 0; r < 16; ++r) {
+        const int kr_ = 8 * (r >> 2) + (r & 3);
+        s[r] = ((wv >> (4 * hf + kr_)) & 1u) && (!p.causal || kr_ <= lim) ? s[r] : -INFINITY;
+      }
     }
 #pragma unroll
-    for (int g2 = 0; g2 < 2; ++g2) {
-      const vec8 bds = as_vec8<vec8>(pack8w<T>(dp, g2));
+    for (int r = 0; r < 16; ++r) dp[r] = __builtin_amdgcn_exp2f(s[r]) * dp[r];
+    vec8 bds[2];
 #pragma unroll
-      for (int eb = 0; eb < EBC; ++eb)
-        dqa[eb] = T::mfma32(
-            as_vec8<vec8>(lds_tr8(kt[buf], ko.lo_at(ec * EBC + eb) + 16 * g2 * EP, ko.hi_at(ec * EBC + eb) + 16 * g2 * EP)),
-            bds, dqa[eb]);
+    for (int g = 0; g < 2; ++g) bds[g] = as_vec8<vec8>(pack8w<T>(dp, g));
+#pragma unroll
+    for (int i = N1; i < NP; ++i) {
+      const int g = (i - N1) / EBC, x = (i - N1) % EBC;
+      dqa[x] = T::mfma32(as_vec8<vec8>(f[i % kQRing]), bds[g], dqa[x]);
+      if (i + kQRing < NP) f[i % kQRing] = operand(i + kQRing);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
   // the raw dQ_hat chunk (rows = e, lane = query), times softmax_scale
@@ -542,7 +628,7 @@ __global__ __launch_bounds__(256) void wide_q_kernel(FlashBwdParams p, float* wq
 #pragma unroll
   for (int eb = 0; eb < EBC; ++eb)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) wqb[32 * (ec * EBC + eb) + res_row(r, hf)] = dqa[eb][r] * p.scale;
+    for (int r = 0; r < 16; ++r) wqb[32 * (CH * eb + ec) + res_row(r, hf)] = dqa[eb][r] * p.scale;
 }
 
 template <typename T, int EP, int DV>
@@ -553,10 +639,8 @@ hipError_t fwd_t(const FlashFwdParams& p, hipStream_t s) {
   return launch_named("flash_wide_fwd", wide_fwd_kernel<T, EP, DV, false>, dim3(blocks), dim3(256), s, p);
 }
 
-// Column chunks per row block (each chunk recomputes the scores), as few as measured fastest: with
-// the tiles loaded straight into LDS, one dK/dV chunk at 256 features and two at 384 / 512, one
-// dQ chunk at 256 and two at 384 / 512 (some of these spill a few registers, which still beats
-// recomputing the scores more often).
+// Column chunks per row block (each chunk recomputes the scores), as few as the registers hold: one
+// at 256 features, two at 384 / 512.
 template <int EP>
 constexpr int kv_chunks() { return EP <= 256 ? 1 : 2; }
 template <int EP>

@@ -1,0 +1,38 @@
+"""Wide heads (head dims above 128) where their kernels' jobs and tiles end unevenly: head counts that divide over the
+eight dies and ones that do not, lengths around the 32-row tiles and the 64- and 128-row jobs, columns past the head
+dim, every expanded width (256, 384, 512).  Against the float64 oracle with the flash tests' tolerance (2e-2 absolute
+beyond the rounding of the output format); dk and dv sum the independent 16-bit operand roundings of their group's G
+query heads, which grow as sqrt(G)."""
+import pytest
+import torch
+
+from gpu_common import excess_over, make_pope_inputs, oracle_attention
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # B, Hq, Hk, Nq, Nk, D, R, mask, causal, dtype
+    (1, 8, 8, 65, 65, 256, 256, "none", True, torch.bfloat16),
+    (2, 8, 4, 33, 97, 136, 104, "prefix", False, torch.float16),
+    (1, 3, 3, 159, 159, 144, 144, "half", True, torch.bfloat16),
+    (1, 16, 2, 31, 129, 200, 200, "random", True, torch.bfloat16),
+    (4, 2, 2, 1, 63, 256, 64, "dead_row", False, torch.float16),
+    (1, 5, 1, 96, 225, 192, 64, "none", False, torch.bfloat16),
+    (2, 4, 4, 128, 128, 160, 96, "prefix", True, torch.float16),
+    (1, 1, 1, 257, 289, 248, 136, "none", True, torch.bfloat16),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
+def test_wide_jobs_against_the_oracle(cuda, case):
+    import pope_amd
+    B, Hq, Hk, Nq, Nk, D, R, mask, causal, dtype = case
+    inp = make_pope_inputs(8800 + Nk, B, Hq, Hk, Nq, Nk, D, R, dtype, mask)
+    ref = oracle_attention(inp, causal)
+    q, k, v = (inp[n].requires_grad_(True) for n in ("q", "k", "v"))
+    o = pope_amd.flash_attn_with_pope(q, k, v, pos_emb=(inp["freqs"], inp["bias"]), mask=inp["mask"], causal=causal)
+    assert excess_over(o.detach(), ref["o"], 2e-2) <= 0
+    grads = torch.autograd.grad(o, (q, k, v), inp["do"])
+    for got, name in zip(grads, ("dq", "dk", "dv")):
+        tol = 2e-2 if name == "dq" else 2e-2 * (Hq / Hk) ** 0.5
+        assert excess_over(got, ref[name], tol) <= 0, name
