@@ -185,6 +185,8 @@ int pope_flash_bwd(const pope_desc* desc, const void* dout, const void* q, const
  * partial rows in `partials`; a last launch sums them in a fixed order and applies the chain rule.
  * `partials`: pope_workspace_bytes(POPE_OP_FLASH_BWD_PARTIALS) bytes (0: the call does not split),
  * 256-byte aligned, free again once the call's work on the stream is done; NULL runs unsplit.
+ * Head dims above 128 put their raw gradient rows there (outside deterministic mode), so that with
+ * partials the workspace is the forward's, pope_workspace_bytes(POPE_OP_FLASH_FWD), for every head dim.
  */
 int pope_flash_bwd_split(const pope_desc* desc, const void* dout, const void* q, const void* k,
                          const void* v, const void* o, const float* lse, const float* freqs,

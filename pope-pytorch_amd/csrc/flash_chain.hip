@@ -1,7 +1,9 @@
 // Chain rule of the polar transform on raw expanded-row gradients (gfx950): the last launch of the
 // wide-head backward (one raw row per key / query), and of a narrow backward whose jobs were split
 // (flash_bwd_split: the partial rows of the splits are summed here, in split order, and dV with
-// them).  Bound by HBM: 4 EP bytes per row and split.
+// them).  Bound by HBM: 4 EP bytes per row and split, 4.2 TB/s at 32,768 rows each side of EP 512 (44.6 us).
+// A thread keeps its four dims over the block's rows, so that dbias adds up in registers: with an LDS
+// atomic per element the LDS was busy 80% of the time (64.7 us there).
 #include "pope_common.hpp"
 #include "pope_kernels.hpp"
 
@@ -50,11 +52,12 @@ __global__ __launch_bounds__(256) void flash_chain_kernel(FlashBwdParams p, int 
   __shared__ float dsum[256];
   const int tid = threadIdx.x;
   const int D = p.D, R = p.R, EP = p.EP;
+  const int D4 = D / 4, rpp = 256 / D4, r0 = tid / D4, d = 4 * (tid % D4);   // rpp rows per pass, threads past them idle
   if ((int)blockIdx.x < nk) {
     const int nkb = (p.Nk + 31) / 32;
     const int k0 = 32 * (blockIdx.x % nkb), bhk = blockIdx.x / nkb;
     const int b = bhk / p.Hk, hk = bhk % p.Hk;
-    for (int d = tid; d < R; d += 256) dsum[d] = 0.f;
+    for (int e = tid; e < R; e += 256) dsum[e] = 0.f;
     __syncthreads();
     const uint16_t* kb = p.k + (int64_t)b * p.k_s[0] + (int64_t)hk * p.k_s[1];
     uint16_t* dkb = p.dk + (int64_t)b * p.dk_s[0] + (int64_t)hk * p.dk_s[1];
@@ -68,48 +71,53 @@ __global__ __launch_bounds__(256) void flash_chain_kernel(FlashBwdParams p, int 
       const int64_t sv = (int64_t)p.B * p.Hk * p.NkP * p.DV;
       const float* vrow = p.wv + (int64_t)bhk * p.NkP * p.DV;
       uint16_t* dvb = p.dv + (int64_t)b * p.dv_s[0] + (int64_t)hk * p.dv_s[1];
-      for (int it = tid; it < 32 * (D / 4); it += 256) {
-        const int key = k0 + it / (D / 4), d = 4 * (it % (D / 4));
-        if (key >= p.Nk) continue;
-        const float4 a = sum4(vrow + (int64_t)key * p.DV + d, S, sv);
-        const float g[4] = {a.x, a.y, a.z, a.w};
-        store4<T>(dvb + (int64_t)key * p.dv_s[2] + d, g);
+      if (r0 < rpp) {
+#pragma unroll 2
+        for (int key = k0 + r0; key < min(k0 + 32, p.Nk); key += rpp) {
+          const float4 a = sum4(vrow + (int64_t)key * p.DV + d, S, sv);
+          const float g[4] = {a.x, a.y, a.z, a.w};
+          store4<T>(dvb + (int64_t)key * p.dv_s[2] + d, g);
+        }
       }
     }
-    const int D4 = D / 4;
-    for (int it = tid; it < 32 * D4; it += 256) {
-      const int key = k0 + it / D4, d = 4 * (it % D4);
-      if (key >= p.Nk) continue;
-      const float* u = wrow + (int64_t)key * EP;
-      float g[4];
-      if (d < R) {   // R % 4 == 0: all four dims rotated
-        float x[4];
-        load4<T>(kb + (int64_t)key * p.k_s[2] + d, x);
-        const float4 c01 = *reinterpret_cast<const float4*>(tb + (int64_t)key * R + d);
-        const float4 c23 = *reinterpret_cast<const float4*>(tb + (int64_t)key * R + d + 2);
-        const float4 uc = sum4(u + d, S, sk), us = sum4(u + R + d, S, sk);
-        const float cs[4] = {c01.x, c01.z, c23.x, c23.z}, sn[4] = {c01.y, c01.w, c23.y, c23.w};
-        const float ucv[4] = {uc.x, uc.y, uc.z, uc.w}, usv[4] = {us.x, us.y, us.z, us.w};
+    float db[4] = {0.f, 0.f, 0.f, 0.f};
+    if (r0 < rpp) {
+#pragma unroll 2
+      for (int r = r0; r < 32; r += rpp) {
+        const int key = k0 + r;
+        if (key >= p.Nk) break;
+        const float* u = wrow + (int64_t)key * EP;
+        float g[4];
+        if (d < R) {   // R % 4 == 0: all four dims rotated
+          float x[4];
+          load4<T>(kb + (int64_t)key * p.k_s[2] + d, x);
+          const float4 c01 = *reinterpret_cast<const float4*>(tb + (int64_t)key * R + d);
+          const float4 c23 = *reinterpret_cast<const float4*>(tb + (int64_t)key * R + d + 2);
+          const float4 uc = sum4(u + d, S, sk), us = sum4(u + R + d, S, sk);
+          const float cs[4] = {c01.x, c01.z, c23.x, c23.z}, sn[4] = {c01.y, c01.w, c23.y, c23.w};
+          const float ucv[4] = {uc.x, uc.y, uc.z, uc.w}, usv[4] = {us.x, us.y, us.z, us.w};
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          g[t] = sigmoid_f(x[t]) * (cs[t] * ucv[t] + sn[t] * usv[t]);
-          const float dpsi = softplus_f(x[t]) * (cs[t] * usv[t] - sn[t] * ucv[t]);
-          if (kpb) {
-            kpb[(int64_t)key * R + d + t] = dpsi;
-          } else {
-            if (dfb) atomicAdd(dfb + (int64_t)key * p.df_s[2] + d + t, dpsi);
-            if (p.dbias) atomicAdd(&dsum[d + t], dpsi);
+          for (int t = 0; t < 4; ++t) {
+            g[t] = sigmoid_f(x[t]) * (cs[t] * ucv[t] + sn[t] * usv[t]);
+            const float dpsi = softplus_f(x[t]) * (cs[t] * usv[t] - sn[t] * ucv[t]);
+            db[t] += dpsi;
+            if (kpb) kpb[(int64_t)key * R + d + t] = dpsi;
+            else if (dfb) atomicAdd(dfb + (int64_t)key * p.df_s[2] + d + t, dpsi);
           }
+        } else {
+          const float4 us = sum4(u + R + d, S, sk);
+          g[0] = us.x; g[1] = us.y; g[2] = us.z; g[3] = us.w;
         }
-      } else {
-        const float4 us = sum4(u + R + d, S, sk);
-        g[0] = us.x; g[1] = us.y; g[2] = us.z; g[3] = us.w;
+        store4<T>(dkb + (int64_t)key * p.dk_s[2] + d, g);
       }
-      store4<T>(dkb + (int64_t)key * p.dk_s[2] + d, g);
     }
     if (p.dbias && !kpb) {
+      if (r0 < rpp && d < R) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) atomicAdd(&dsum[d + t], db[t]);
+      }
       __syncthreads();
-      for (int d = tid; d < R; d += 256) atomicAdd(p.dbias + (int64_t)hk * p.bias_sh + d, dsum[d]);
+      for (int e = tid; e < R; e += 256) atomicAdd(p.dbias + (int64_t)hk * p.bias_sh + e, dsum[e]);
     }
     return;
   }
@@ -126,22 +134,30 @@ __global__ __launch_bounds__(256) void flash_chain_kernel(FlashBwdParams p, int 
   const float* wrow = wq + (int64_t)bh * p.NqP * EP;
   const int S = p.q_splits;
   const int64_t sq = (int64_t)p.B * p.Hq * p.NqP * EP;
-  const int D4 = D / 4;
-  for (int it = tid; it < 32 * D4; it += 256) {
-    const int i = q0 + it / D4, d = 4 * (it % D4);
-    if (i >= p.Nq) continue;
+  if (r0 >= rpp) return;
+  float2 tbv[4];
+  if (d < R) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) tbv[t] = bq[d + t];
+  }
+#pragma unroll 2
+  for (int r = r0; r < 32; r += rpp) {
+    const int i = q0 + r;
+    if (i >= p.Nq) break;
     const float* u = wrow + (int64_t)i * EP;
     float g[4];
     if (d < R) {   // R % 4 == 0: all four dims rotated
       float x[4];
       load4<T>(qb + (int64_t)i * p.q_s[2] + d, x);
+      const float4 f01 = *reinterpret_cast<const float4*>(tq + (int64_t)(q_off + i) * R + d);
+      const float4 f23 = *reinterpret_cast<const float4*>(tq + (int64_t)(q_off + i) * R + d + 2);
       const float4 uc = sum4(u + d, S, sq), us = sum4(u + R + d, S, sq);
+      const float tc[4] = {f01.x, f01.z, f23.x, f23.z}, ts[4] = {f01.y, f01.w, f23.y, f23.w};
       const float ucv[4] = {uc.x, uc.y, uc.z, uc.w}, usv[4] = {us.x, us.y, us.z, us.w};
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         // cos / sin(F[q_off + i] - bias) from the tables of F and of the bias
-        const float2 tf = tq[(int64_t)(q_off + i) * R + d + t], tbv = bq[d + t];
-        const float cs = fmaf(tf.x, tbv.x, tf.y * tbv.y), sn = fmaf(tf.y, tbv.x, -tf.x * tbv.y);
+        const float cs = fmaf(tc[t], tbv[t].x, ts[t] * tbv[t].y), sn = fmaf(ts[t], tbv[t].x, -tc[t] * tbv[t].y);
         g[t] = sigmoid_f(x[t]) * (cs * ucv[t] + sn * usv[t]);
         const float dph = softplus_f(x[t]) * (cs * usv[t] - sn * ucv[t]);
         if (qpb) qpb[(int64_t)i * R + d + t] = dph;

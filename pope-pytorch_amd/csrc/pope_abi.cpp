@@ -250,7 +250,12 @@ struct BwdPartials {
 
 BwdPartials flash_bwd_partials(const pope_desc& d, const FlashLayout& L) {
   BwdPartials r{{1, 1, false, false}, 0, 0, 0};
-  if (L.wide) return r;
+  // Wide heads: the raw rows, out of the workspace, which is then the forward's and brings its
+  // preparation (a second one took 25 us of 573 at (2, 8, 2048, 256)).
+  if (L.wide) {
+    if (!(d.flags & POPE_FLAG_DETERMINISTIC)) r.total = L.wide_bytes;
+    return r;
+  }
   r.sp = pope::flash_bwd_split(d.B, d.Hq, d.Hk, d.Nq, d.Nk, d.R, L.EP, L.DV, d.causal != 0);
   size_t off = 0;
   const size_t kr = (size_t)r.sp.kv * d.B * d.Hk * L.NkP, qr = (size_t)r.sp.q * d.B * d.Hq * L.NqP;
@@ -619,13 +624,14 @@ int pope_flash_bwd_split(const pope_desc* d, const void* dout, const void* q, co
   if (d->flags & ~(POPE_FLAG_PREPARED | POPE_FLAG_ZERO_GRADS | POPE_FLAG_DETERMINISTIC))
     return fail(POPE_ERR_INVALID, "unknown flags 0x%x", (unsigned)d->flags);
   const FlashLayout L = flash_layout(*d);
-  if ((rc = check_ws(L.total + L.wide_bytes + det_bytes(*d), workspace, workspace_bytes))) return rc;
-  if ((rc = check_row_span("v", L.NkP, d->v_s[2])) || (rc = check_row_span("do", L.NqP, d->do_s[2]))) return rc;
   BwdPartials bp{{1, 1, false, false}, 0, 0, 0};
   if (partials) {
     bp = flash_bwd_partials(*d, L);
     if ((rc = check_ws(bp.total, partials, partials_bytes))) return rc;
   }
+  const bool wide_parts = L.wide && bp.total > 0;
+  if ((rc = check_ws(L.total + (wide_parts ? 0 : L.wide_bytes + det_bytes(*d)), workspace, workspace_bytes))) return rc;
+  if ((rc = check_row_span("v", L.NkP, d->v_s[2])) || (rc = check_row_span("do", L.NqP, d->do_s[2]))) return rc;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
   if (!(d->flags & POPE_FLAG_PREPARED)) {
@@ -689,8 +695,9 @@ int pope_flash_bwd_split(const pope_desc* d, const void* dout, const void* q, co
   hipError_t e;
   if (L.wide) {
     e = pope::launch_flash_bwd_delta(p, d->dtype, s);
+    char* raw = wide_parts ? static_cast<char*>(partials) : ws + L.wk;
     if (e == hipSuccess)
-      e = pope::launch_flash_wide_bwd(p, reinterpret_cast<float*>(ws + L.wk), reinterpret_cast<float*>(ws + L.wq),
+      e = pope::launch_flash_wide_bwd(p, reinterpret_cast<float*>(raw), reinterpret_cast<float*>(raw + (L.wq - L.wk)),
                                       d->dtype, s);
   } else {
     e = pope::launch_flash_bwd(p, d->dtype, s);

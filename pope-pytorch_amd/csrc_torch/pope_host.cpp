@@ -138,6 +138,12 @@ bool decode_eligible(const pope_desc& d, int64_t min_keys) {
   return (int64_t)(d.Nk - 1) * std::max(d.k_s[2], d.v_s[2]) + d.D < INT_MAX;
 }
 
+// One size for a forward and its backward, which reuses the preparation in it.
+size_t flash_workspace_bytes(pope_desc d) {
+  d.flags = deterministic_flag();
+  return workspace_bytes(d.flags ? POPE_OP_FLASH_BWD : POPE_OP_FLASH_FWD, d);
+}
+
 struct FlashOut {
   Tensor o, lse, ws;
 };
@@ -172,9 +178,7 @@ FlashOut flash_forward(const Tensor& q0, const Tensor& k0, const Tensor& v0, Ten
   }
   // the workspace holds the preparation the backward reuses and, under deterministic mode, the
   // backward's phase-derivative region after it
-  pope_desc dd = d;
-  dd.flags = deterministic_flag();
-  const size_t n = workspace_bytes(dd.flags ? POPE_OP_FLASH_BWD : POPE_OP_FLASH_FWD, dd);
+  const size_t n = flash_workspace_bytes(d);
   const size_t np = workspace_bytes(POPE_OP_FLASH_FWD_PARTIALS, d);
   r.ws = bytes_like(q, n);
   const Tensor parts = bytes_like(q, np);
@@ -230,7 +234,8 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
     if (need_df) freqs_strides(d.df_s, dfreqs);
     if (mask.defined()) d.mask_sb = mask.stride(0);
     d.flags = POPE_FLAG_ZERO_GRADS | deterministic_flag();
-    const size_t n = workspace_bytes(POPE_OP_FLASH_BWD, d), np = workspace_bytes(POPE_OP_FLASH_BWD_PARTIALS, d);
+    // with the partials the workspace is the forward's
+    const size_t n = flash_workspace_bytes(d), np = workspace_bytes(POPE_OP_FLASH_BWD_PARTIALS, d);
     const bool prepared = fwd_ws.defined() && (size_t)fwd_ws.numel() == n;
     g_last_bwd_prepared = prepared;
     if (prepared) d.flags |= POPE_FLAG_PREPARED;

@@ -400,7 +400,9 @@ def _bwd_impl(do, q, k, v, o, lse, freqs, bias, mask, causal, softmax_scale, nee
         # the same descriptor with PREPARED set, for calls that bring the forward's workspace
         dp = _lib.PopeDesc.from_buffer_copy(d)
         dp.flags |= _lib.FLAG_PREPARED
-        return d, dp, _lib.workspace_bytes(_lib.OP_FLASH_BWD, d), _lib.workspace_bytes(_lib.OP_FLASH_BWD_PARTIALS, d)
+        # with the partials the workspace is the forward's (deterministic mode: the larger one it took)
+        op = _lib.OP_FLASH_BWD if deterministic else _lib.OP_FLASH_FWD
+        return d, dp, _lib.workspace_bytes(op, d), _lib.workspace_bytes(_lib.OP_FLASH_BWD_PARTIALS, d)
 
     d, dprep, need, part_bytes = _plan(key, build)
     if exists(fwd_ws) and fwd_ws.numel() == need:

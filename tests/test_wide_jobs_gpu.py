@@ -33,6 +33,8 @@ def test_wide_jobs_against_the_oracle(cuda, case):
     o = pope_amd.flash_attn_with_pope(q, k, v, pos_emb=(inp["freqs"], inp["bias"]), mask=inp["mask"], causal=causal)
     assert excess_over(o.detach(), ref["o"], 2e-2) <= 0
     grads = torch.autograd.grad(o, (q, k, v), inp["do"])
+    from pope_amd import hip_pope_flash_attn
+    assert hip_pope_flash_attn._LAST_BWD_PREPARED   # the forward's preparation, reused
     for got, name in zip(grads, ("dq", "dk", "dv")):
         tol = 2e-2 if name == "dq" else 2e-2 * (Hq / Hk) ** 0.5
         assert excess_over(got, ref[name], tol) <= 0, name
