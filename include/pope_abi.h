@@ -267,6 +267,27 @@ typedef struct pope_cast {
 int pope_cast_f16(const pope_cast* tensors, int n, uint32_t* flag, void* stream);
 
 /*
+ * Rows moved between a caller's width and a padded width, up to six (b, h, n, d) tensors in one
+ * launch (head and rotate dims that are not multiples of 8; the reference masks such dims inside its
+ * kernels, triton_pope.py:58-60).  `cols` real columns, of which the first `split` stay in place and
+ * the others are `gap` columns further on in the padded row:
+ *   pad = 1   dst (padded, dst_cols >= cols + gap): the gap holds `fill`, columns past the real ones 0
+ *   pad = 0   src padded, dst real (dst_cols = cols)
+ * Any source element strides (>= 0); destination rows have unit feature stride.
+ */
+typedef struct pope_pad {
+  const void* src;
+  void* dst;
+  int32_t shape[3];           /* b, h, n */
+  int32_t pad, elem;          /* elem: bytes per element, 2 or 4 */
+  int32_t split, gap, cols, dst_cols;
+  uint32_t fill;              /* element bits */
+  int64_t src_s[4], dst_s[3]; /* element strides */
+} pope_pad;
+
+int pope_pad_rows(const pope_pad* tensors, int n, void* stream);
+
+/*
  * Per-kernel timing.  No counterpart in the reference (its tests print only
  * parity diffs, tests/test_flash_attn.py:61,109).  While enabled, every kernel
  * launch of the library carries a pair of hipEvents that its dispatch stamps with

@@ -737,6 +737,46 @@ int pope_cast_f16(const pope_cast* tensors, int n, uint32_t* flag, void* stream)
   return POPE_OK;
 }
 
+int pope_pad_rows(const pope_pad* tensors, int n, void* stream) {
+  if (!tensors || n < 1 || n > 6) return fail(POPE_ERR_INVALID, "pad takes 1 to 6 tensors (got %d)", n);
+  pope::PadParams p;
+  std::memset(&p, 0, sizeof p);
+  p.n = n;
+  for (int t = 0; t < n; ++t) {
+    const pope_pad& c = tensors[t];
+    pope::PadTensor& x = p.t[t];
+    bool empty = c.dst_cols == 0;
+    for (int i = 0; i < 3; ++i) {
+      if (c.shape[i] < 0 || c.src_s[i] < 0 || c.dst_s[i] < 0)
+        return fail(POPE_ERR_INVALID, "pad tensor %d: negative shape or stride", t);
+      empty = empty || c.shape[i] == 0;
+      x.shape[i] = c.shape[i];
+      x.src_s[i] = c.src_s[i];
+      x.dst_s[i] = c.dst_s[i];
+    }
+    if (c.src_s[3] < 0) return fail(POPE_ERR_INVALID, "pad tensor %d: negative shape or stride", t);
+    if (c.elem != 2 && c.elem != 4) return fail(POPE_ERR_INVALID, "pad tensor %d: %d-byte elements", t, (int)c.elem);
+    if (c.split < 0 || c.gap < 0 || c.split > c.cols ||
+        (c.pad ? (int64_t)c.dst_cols < (int64_t)c.cols + c.gap : c.dst_cols != c.cols))
+      return fail(POPE_ERR_INVALID, "pad tensor %d: columns split %d, gap %d, real %d, destination %d", t, (int)c.split,
+                  (int)c.gap, (int)c.cols, (int)c.dst_cols);
+    if (!empty && (!c.src || !c.dst)) return fail(POPE_ERR_INVALID, "pad tensor %d: NULL data", t);
+    x.src_s[3] = c.src_s[3];
+    x.src = c.src;
+    x.dst = c.dst;
+    x.pad = c.pad != 0;
+    x.elem = c.elem;
+    x.split = c.split;
+    x.gap = c.gap;
+    x.cols = c.cols;
+    x.dst_cols = c.dst_cols;
+    x.fill = c.fill;
+  }
+  const hipError_t e = pope::launch_pad_rows(p, reinterpret_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "pad launch");
+  return POPE_OK;
+}
+
 int pope_flash_decode(const pope_desc* d, const void* q, const void* k, const void* v, const float* freqs,
                       const float* bias, const uint8_t* mask, void* o, float* lse, void* workspace,
                       size_t workspace_bytes, void* stream) {

@@ -226,6 +226,23 @@ struct CastParams {
 };
 hipError_t launch_cast_f16(const CastParams& p, float limit, hipStream_t s);
 
+// Rows between the caller's width and the padded width (pad.hip); `cols`: real columns.
+struct PadTensor {
+  const void* src; void* dst;
+  int shape[3];              // b, h, n
+  int pad, elem, split, gap, cols, dst_cols;   // pad: 1 pads, 0 unpads; elem: bytes per element (2 or 4)
+  uint32_t fill;
+  int64_t src_s[4], dst_s[3];
+  int64_t items;             // set by launch_pad_rows
+  int vec;                   // likewise: 16-byte stores
+};
+struct PadParams {
+  PadTensor t[6];
+  int n;
+  int64_t items;             // set by launch_pad_rows
+};
+hipError_t launch_pad_rows(const PadParams& p, hipStream_t s);
+
 struct DecodeParams {
   const uint16_t* q; const uint16_t* k; const uint16_t* v;
   const float* freqs; const float* bias; const uint8_t* mask;   // freqs rows 16-byte aligned

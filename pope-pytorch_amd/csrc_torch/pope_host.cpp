@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <atomic>
 #include <climits>
+#include <cstring>
 
 #include "../../include/pope_abi.h"
 
@@ -98,6 +99,104 @@ void check_device(const Tensor& q, std::initializer_list<const Tensor*> ts) {
   TORCH_CHECK(q.is_cuda(), "pope_amd runs on GPU tensors only");
   for (const Tensor* t : ts)
     TORCH_CHECK(!t->defined() || t->device() == q.device(), "pope_amd: operand on ", t->device(), " next to q on ", q.device());
+}
+
+// ---------------------------------------------------------------- padded rows
+
+// Columns of a padded tensor: `cols` real ones, the first `split` in place, the others `gap` further on,
+// `width` in all; `fill`: element bits of the gap.
+struct PadCols {
+  int64_t split, gap, cols, width;
+  uint32_t fill;
+};
+
+// Widths of a call whose head dim D or rotate dim R is no multiple of 8 (pope_amd/_pad.py has the plan
+// and the reasons): rotate dims R -> R8, head dims D -> Dp.
+struct PadPlan {
+  int64_t D, R, R8, Dp;
+  PadCols qk(const Tensor& t) const {   // the gap: a logit whose softplus and sigmoid are 0
+    const float logit = -1.0e4f;
+    uint32_t bits = 0;
+    if (t.scalar_type() == at::kFloat) std::memcpy(&bits, &logit, 4);
+    else if (t.scalar_type() == at::kHalf) bits = c10::Half(logit).x;
+    else bits = c10::BFloat16(logit).x;
+    return {R, R8 - R, D, Dp, bits};
+  }
+  PadCols v() const { return {D, 0, D, Dp, 0}; }
+  PadCols phase() const { return {R, 0, R, R8, 0}; }
+};
+
+// Every tensor padded or unpadded, in one launch.
+variable_list pad_rows(at::TensorList ts, const std::vector<PadCols>& cols, bool pad) {
+  std::vector<pope_pad> d(ts.size());
+  variable_list out;
+  for (size_t i = 0; i < ts.size(); ++i) {
+    const Tensor& t = ts[i];
+    const PadCols& c = cols[i];
+    const int64_t n = t.dim(), lead = n - 1;
+    check_device(ts[0], {&t});
+    TORCH_CHECK_VALUE(n >= 1 && n <= 4 && t.size(-1) == (pad ? c.cols : c.width), "pope_amd: ", t.sizes(),
+                      " does not have rows of ", pad ? c.cols : c.width);
+    std::vector<int64_t> shape = t.sizes().vec();
+    shape.back() = pad ? c.width : c.cols;
+    out.push_back(at::empty(shape, t.options().requires_grad(false)));
+    pope_pad& p = d[i];
+    p = pope_pad{};
+    p.src = t.data_ptr();
+    p.dst = out.back().data_ptr();
+    for (int64_t j = 0; j < 3; ++j) {
+      const int64_t x = lead - 3 + j;   // right-aligned leading dims
+      TORCH_CHECK_VALUE(x < 0 || t.size(x) <= INT_MAX, "pope_amd: tensor too large to pad");
+      p.shape[j] = x < 0 ? 1 : (int32_t)t.size(x);
+      p.src_s[j] = x < 0 ? 0 : t.stride(x);
+      p.dst_s[j] = x < 0 ? 0 : out.back().stride(x);
+    }
+    p.src_s[3] = t.stride(-1);
+    p.pad = pad;
+    p.elem = (int32_t)t.element_size();
+    p.split = (int32_t)c.split;
+    p.gap = (int32_t)c.gap;
+    p.cols = (int32_t)c.cols;
+    p.dst_cols = (int32_t)shape.back();
+    p.fill = c.fill;
+  }
+  check(pope_pad_rows(d.data(), (int)d.size(), stream_of(ts[0])), "padding");
+  return out;
+}
+
+bool tracked(at::TensorList ts);
+
+// pad_rows under autograd: the gradients take the inverse move (the gap's gradient is dropped, or zero).
+struct PadFn : torch::autograd::Function<PadFn> {
+  static variable_list forward(AutogradContext* ctx, at::TensorList ts, const std::vector<PadCols>& cols, bool pad) {
+    std::vector<int64_t> flat;
+    for (const PadCols& c : cols) flat.insert(flat.end(), {c.split, c.gap, c.cols, c.width});
+    ctx->saved_data["cols"] = flat;
+    ctx->saved_data["pad"] = pad;
+    return pad_rows(ts, cols, pad);
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const std::vector<int64_t> flat = ctx->saved_data["cols"].toIntVector();
+    variable_list ts;
+    std::vector<PadCols> cols;
+    std::vector<size_t> at_;
+    for (size_t i = 0; i < grads.size(); ++i)
+      if (grads[i].defined() && ctx->needs_input_grad(i)) {
+        ts.push_back(grads[i]);
+        cols.push_back({flat[4 * i], flat[4 * i + 1], flat[4 * i + 2], flat[4 * i + 3], 0});
+        at_.push_back(i);
+      }
+    variable_list r(grads.size() + 2);
+    if (ts.empty()) return r;
+    const variable_list out = pad_rows(ts, cols, !ctx->saved_data["pad"].toBool());
+    for (size_t j = 0; j < out.size(); ++j) r[at_[j]] = out[j];
+    return r;
+  }
+};
+
+variable_list padded(at::TensorList ts, const std::vector<PadCols>& cols, bool pad) {
+  return tracked(ts) ? PadFn::apply(ts, cols, pad) : pad_rows(ts, cols, pad);
 }
 
 // ---------------------------------------------------------------- flash attention
@@ -194,13 +293,28 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
   // freqs and bias come together, so the node's inputs 3 and 4 are theirs where they exist
   static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
                         const std::optional<Tensor>& freqs_, const std::optional<Tensor>& bias_,
-                        const std::optional<Tensor>& mask_, bool causal, double scale, int64_t decode_min_keys, bool reuse) {
+                        const std::optional<Tensor>& mask_, bool causal, double scale, int64_t decode_min_keys, bool reuse,
+                        int64_t cols) {
     const Tensor freqs = opt(freqs_), bias = opt(bias_), mask = opt(mask_);
     FlashOut r = flash_forward(q, k, v, freqs, bias, mask, causal, scale, decode_min_keys);
     ctx->save_for_backward({q, k, v, freqs, bias, mask, r.o, r.lse, reuse ? r.ws : Tensor()});
     ctx->saved_data["causal"] = causal;
+    ctx->saved_data["cols"] = cols;
     ctx->saved_data["scale"] = scale;
-    return r.o;
+    return leading_columns(r.o, cols);
+  }
+
+  // The first `cols` columns of o (all: o itself) as an output of the node: no autograd view of o, but with
+  // its version counter, so that an in-place change of the output is seen by the saved o.
+  static Tensor leading_columns(const Tensor& o, int64_t cols) {
+    if (cols == o.size(3)) return o;
+    Tensor x;
+    {
+      at::AutoDispatchBelowADInplaceOrView plain;
+      x = o.narrow(3, 0, cols);
+    }
+    torch::autograd::impl::set_version_counter(x, torch::autograd::impl::version_counter(o));
+    return x;
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
@@ -210,6 +324,8 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
     const Tensor lse = sv[7].contiguous();
     Tensor dout = unit_feature(grads[0]);
     if (dout.scalar_type() != q.scalar_type()) dout = dout.to(q.scalar_type());
+    if (const int64_t cols = ctx->saved_data["cols"].toInt(); cols < q.size(3))
+      dout = pad_rows({dout}, {{cols, 0, cols, q.size(3), 0}}, true)[0];
     check_flash(q, k, v, freqs, bias, mask);
     TORCH_CHECK_VALUE(dout.sizes() == q.sizes(), "do ", dout.sizes(), " must match q ", q.sizes());
     const bool need_df = freqs.defined() && ctx->needs_input_grad(3);
@@ -247,12 +363,12 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
                                dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), static_cast<float*>(data(dfreqs)),
                                static_cast<float*>(data(dbias)), data(ws), n, data(parts), np, stream_of(q)),
           "flash backward");
-    return {dq, dk, dv, dfreqs, dbias, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    return {dq, dk, dv, dfreqs, dbias, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
 
 // Whether a call has to go through the autograd node (which also refuses forward-mode tangents).
-bool tracked(std::initializer_list<Tensor> ts) {
+bool tracked(at::TensorList ts) {
   for (const Tensor& t : ts)
     if (t.defined() && ((at::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(0).defined())) return true;
   return false;
@@ -264,7 +380,29 @@ Tensor flash(const Tensor& q, const Tensor& k, const Tensor& v, const std::optio
   const Tensor f = opt(freqs), b = opt(bias), m = opt(mask);
   if (!tracked({q, k, v, f, b})) return flash_forward(q, k, v, f, b, m, causal, scale, decode_min_keys).o;
   TORCH_CHECK_VALUE(f.defined() == b.defined(), "freqs and bias come together");
-  return FlashFn::apply(q, k, v, freqs, bias, mask, causal, scale, decode_min_keys, reuse);
+  return FlashFn::apply(q, k, v, freqs, bias, mask, causal, scale, decode_min_keys, reuse, q.size(-1));
+}
+
+// The same on unpadded rows: q, k, v, freqs and bias padded in one launch, o's real columns.
+Tensor flash_padded(const Tensor& q, const Tensor& k, const Tensor& v, const std::optional<Tensor>& freqs,
+                    const std::optional<Tensor>& bias, const std::optional<Tensor>& mask, bool causal, double scale,
+                    int64_t decode_min_keys, bool reuse, int64_t R, int64_t R8, int64_t Dp) {
+  const Tensor f = opt(freqs), b = opt(bias), m = opt(mask);
+  TORCH_CHECK_VALUE(f.defined() == b.defined(), "freqs and bias come together");
+  const PadPlan plan{q.size(-1), R, R8, Dp};
+  variable_list ts{q, k, v};
+  std::vector<PadCols> cols{plan.qk(q), plan.qk(k), plan.v()};
+  if (f.defined() && R8 != R) {
+    ts.insert(ts.end(), {f, b});
+    cols.insert(cols.end(), {plan.phase(), plan.phase()});
+  }
+  variable_list p = padded(ts, cols, true);
+  if (f.defined() && p.size() == 3) p.insert(p.end(), {f, b});
+  p.resize(5);
+  if (!tracked({p[0], p[1], p[2], p[3], p[4]}))
+    return flash_forward(p[0], p[1], p[2], p[3], p[4], m, causal, scale, decode_min_keys).o.narrow(3, 0, plan.D);
+  const auto maybe = [](const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
+  return FlashFn::apply(p[0], p[1], p[2], maybe(p[3]), maybe(p[4]), mask, causal, scale, decode_min_keys, reuse, plan.D);
 }
 
 // ---------------------------------------------------------------- similarity and polar transform
@@ -357,6 +495,22 @@ Tensor sim(const Tensor& q, const Tensor& k, const Tensor& freqs, const Tensor& 
   return SimFn::apply(q, k, freqs, bias, split);
 }
 
+// q, k, freqs and bias of a similarity or polar call, padded in one launch.
+variable_list pad_operands(const Tensor& q, const Tensor& k, const Tensor& freqs, const Tensor& bias, const PadPlan& plan) {
+  if (plan.R == plan.R8) {
+    variable_list p = padded({q, k}, {plan.qk(q), plan.qk(k)}, true);
+    p.insert(p.end(), {freqs, bias});
+    return p;
+  }
+  return padded({q, k, freqs, bias}, {plan.qk(q), plan.qk(k), plan.phase(), plan.phase()}, true);
+}
+
+Tensor sim_padded(const Tensor& q, const Tensor& k, const Tensor& freqs, const Tensor& bias, bool split, int64_t R,
+                  int64_t R8, int64_t Dp) {
+  const variable_list p = pad_operands(q, k, freqs, bias, {q.size(-1), R, R8, Dp});
+  return sim(p[0], p[1], p[2], p[3], split);
+}
+
 struct PolarFn : torch::autograd::Function<PolarFn> {
   // fp32 columns per output row: D + R, or D (re, im) pairs
   static int64_t width(const Tensor& q, const Tensor& freqs, bool cplx) {
@@ -423,13 +577,27 @@ std::pair<Tensor, Tensor> polar(const Tensor& q, const Tensor& k, const Tensor& 
   return {r[0], r[1]};
 }
 
+// Real output on unpadded rows: 2 R interleaved (cos, sin) columns, then the D - R pass-through ones.
+std::pair<Tensor, Tensor> polar_padded(const Tensor& q, const Tensor& k, const Tensor& freqs, const Tensor& bias, int64_t R,
+                                       int64_t R8, int64_t Dp) {
+  const int64_t D = q.size(-1);
+  const variable_list p = pad_operands(q, k, freqs, bias, {D, R, R8, Dp});
+  const auto [qh, kh] = polar(p[0], p[1], p[2], p[3], false);
+  const PadCols c{2 * R, 2 * (R8 - R), D + R, Dp + R8, 0};
+  const variable_list r = padded({qh, kh}, {c, c}, false);
+  return {r[0], r[1]};
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_pope_host, m) {
   const auto nogil = py::call_guard<py::gil_scoped_release>();
   m.def("flash", &flash, nogil);
+  m.def("flash_padded", &flash_padded, nogil);
   m.def("sim", &sim, nogil);
+  m.def("sim_padded", &sim_padded, nogil);
   m.def("polar", &polar, nogil);
+  m.def("polar_padded", &polar_padded, nogil);
   m.def("last_bwd_prepared", [] { return g_last_bwd_prepared.load(); });
   m.def("abi_version", [] { return POPE_ABI_VERSION; });
 }

@@ -50,7 +50,7 @@ class PopeCast(ctypes.Structure):
 EXPORTS = (
     "pope_abi_version", "pope_last_error", "pope_workspace_bytes", "pope_sim_fwd", "pope_sim_bwd",
     "pope_flash_fwd", "pope_flash_fwd_split", "pope_flash_bwd", "pope_flash_bwd_split", "pope_flash_decode", "pope_flash_decode_noalloc", "pope_polar_fwd",
-    "pope_polar_bwd", "pope_cast_f16", "pope_profile_enable", "pope_profile_read", "pope_profile_reset",
+    "pope_polar_bwd", "pope_cast_f16", "pope_pad_rows", "pope_profile_enable", "pope_profile_read", "pope_profile_reset",
 )
 
 _lib = None

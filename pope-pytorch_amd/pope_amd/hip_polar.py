@@ -153,11 +153,14 @@ def fits(q: Tensor, k: Tensor, freqs: Tensor, bias: Tensor, to_magnitude, return
 def polar(q: Tensor, k: Tensor, freqs: Tensor, bias: Tensor, return_complex: bool = False) -> tuple[Tensor, Tensor]:
     D, R = q.shape[-1], freqs.shape[-1]
     plan = pad_plan(D, R)
+    eager = _lib.eager(q, k, freqs, bias)
+    if plan is not None and eager and not return_complex:
+        return _lib.host().polar_padded(q, k, freqs, bias, plan.R, plan.R8, plan.Dp)
     if plan is not None:
         # rows padded on the device (pope_amd._pad); the padded dims' output columns are dropped
         q, k = pad_qk(q, plan), pad_qk(k, plan)
         freqs, bias = pad_last(freqs, plan.R8), pad_last(bias, plan.R8)
-    if _lib.eager(q, k, freqs, bias):   # the same forward / backward without the custom-op dispatch
+    if eager:   # the same forward / backward without the custom-op dispatch
         qh, kh = _lib.host().polar(q, k, freqs, bias, return_complex)
     else:
         qh, kh = polar_fwd_op(q, k, freqs, bias, return_complex)

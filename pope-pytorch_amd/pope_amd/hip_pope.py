@@ -178,10 +178,14 @@ def hip_compute_qk_similarity(q, k, freqs, bias, rotate_dim=None, allow_tf32=Tru
     qf, kf = q.float(), k.float()
     # head / rotate dims that are not multiples of 8: padded on the device (pope_amd._pad)
     plan = pad_plan(q.shape[-1], R)
+    eager = _lib.eager(qf, kf, freqs, bias)
+    if plan is not None and eager and qf.ndim == kf.ndim == 4 and kf.shape[-1] == plan.D and bias.shape[-1] == R:
+        sim = _lib.host().sim_padded(qf, kf, freqs, bias, bool(allow_tf32), plan.R, plan.R8, plan.Dp)
+        return sim.to(out_dtype) if out_dtype != torch.float32 else sim
     if plan is not None:
         qf, kf = pad_qk(qf, plan), pad_qk(kf, plan)
         freqs, bias = pad_last(freqs, plan.R8), pad_last(bias, plan.R8)
-    if _lib.eager(qf, kf, freqs, bias):   # the same forward / backward without the custom-op dispatch
+    if eager:   # the same forward / backward without the custom-op dispatch
         sim = _lib.host().sim(qf, kf, freqs, bias, bool(allow_tf32))
     else:
         sim = sim_fwd_op(qf, kf, freqs, bias, bool(allow_tf32))

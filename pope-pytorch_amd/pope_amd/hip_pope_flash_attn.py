@@ -486,6 +486,13 @@ def _flash(q, k, v, freqs, bias, mask, causal, scale) -> Tensor:
     return _lib.host().flash(q, k, v, freqs, bias, mask, bool(causal), scale, _DECODE_MIN_KEYS, _REUSE_FWD_WORKSPACE)
 
 
+def _pads_natively(plan, q, k, v, freqs, bias, mask) -> bool:
+    """Whether the native call layer pads this call: eager, and rows that pad_qk's plan describes (a rotate
+    dim above the head dim, and operands of other widths, keep the torch ops and what they answer)."""
+    return (plan.R <= plan.D and q.ndim == k.ndim == v.ndim == 4 and k.shape[-1] == v.shape[-1] == plan.D
+            and (not exists(freqs) or bias.shape[-1] == plan.R) and _lib.eager(q, k, v, freqs, bias, mask))
+
+
 # ------------------------------------------------------------ head-first entry point
 
 def flash_attn_head_first(q: Tensor, k: Tensor, v: Tensor, freqs: Optional[Tensor] = None,
@@ -518,12 +525,15 @@ def flash_attn_head_first(q: Tensor, k: Tensor, v: Tensor, freqs: Optional[Tenso
             v = v.to(q.dtype)
         # head / rotate dims that are not multiples of 8: padded on the device (pope_amd._pad)
         plan = pad_plan(q.shape[-1], freqs.shape[-1] if exists(freqs) else 0)
-        if plan is not None:
+        if plan is None:
+            o = _flash(q, k, v, freqs, pope_bias, mask, causal, float(scale))
+        elif _pads_natively(plan, q, k, v, freqs, pope_bias, mask):
+            o = _lib.host().flash_padded(q, k, v, freqs, pope_bias, mask, bool(causal), float(scale), _DECODE_MIN_KEYS,
+                                         _REUSE_FWD_WORKSPACE, plan.R, plan.R8, plan.Dp)
+        else:
             q, k, v = pad_qk(q, plan), pad_qk(k, plan), pad_last(v, plan.Dp)
             freqs, pope_bias = pad_last(freqs, plan.R8), pad_last(pope_bias, plan.R8)
-        o = _flash(q, k, v, freqs, pope_bias, mask, causal, float(scale))
-        if plan is not None:
-            o = o[..., :plan.D]
+            o = _flash(q, k, v, freqs, pope_bias, mask, causal, float(scale))[..., :plan.D]
         if o.dtype != out_dtype:
             o = o.to(out_dtype)
     finally:
