@@ -173,7 +173,13 @@ struct PadFn : torch::autograd::Function<PadFn> {
     for (const PadCols& c : cols) flat.insert(flat.end(), {c.split, c.gap, c.cols, c.width});
     ctx->saved_data["cols"] = flat;
     ctx->saved_data["pad"] = pad;
-    return pad_rows(ts, cols, pad);
+    ctx->set_materialize_grads(false);
+    variable_list out = pad_rows(ts, cols, pad), constant;
+    // what needs no gradient stays a constant for the node after this one (freqs, mostly)
+    for (size_t i = 0; i < out.size(); ++i)
+      if (!ts[i].requires_grad()) constant.push_back(out[i]);
+    ctx->mark_non_differentiable(constant);
+    return out;
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
