@@ -11,7 +11,7 @@ namespace pope {
 
 namespace {
 
-// Blocks [0, nk): 32 key rows of one (batch, kv head); blocks [nk, nk + nq): 32 query rows of
+// Blocks [0, nk): krows key rows of one (batch, kv head); blocks [nk, nk + nq): qrows query rows of
 // one (batch, head).  With the raw expanded-row gradients U (cos column e = d, sin column
 // e = R + d, pass-through column e = R + d) and the row's phase (keys F[j]; queries
 // F[q_off + i] - bias, the bias on the query side as in the preparation):
@@ -46,7 +46,7 @@ __device__ __forceinline__ float4 sum4(const float* u, int S, int64_t stride) {
   return a;
 }
 template <typename T>
-__global__ __launch_bounds__(256) void flash_chain_kernel(FlashBwdParams p, int nk) {
+__global__ __launch_bounds__(256) void flash_chain_kernel(FlashBwdParams p, int nk, int krows, int qrows) {
   const float* wk = p.wk;
   const float* wq = p.wq;
   __shared__ float dsum[256];
@@ -54,8 +54,8 @@ __global__ __launch_bounds__(256) void flash_chain_kernel(FlashBwdParams p, int 
   const int D = p.D, R = p.R, EP = p.EP;
   const int D4 = D / 4, rpp = 256 / D4, r0 = tid / D4, d = 4 * (tid % D4);   // rpp rows per pass, threads past them idle
   if ((int)blockIdx.x < nk) {
-    const int nkb = (p.Nk + 31) / 32;
-    const int k0 = 32 * (blockIdx.x % nkb), bhk = blockIdx.x / nkb;
+    const int nkb = (p.Nk + krows - 1) / krows;
+    const int k0 = krows * (blockIdx.x % nkb), bhk = blockIdx.x / nkb;
     const int b = bhk / p.Hk, hk = bhk % p.Hk;
     for (int e = tid; e < R; e += 256) dsum[e] = 0.f;
     __syncthreads();
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256) void flash_chain_kernel(FlashBwdParams p, int 
       uint16_t* dvb = p.dv + (int64_t)b * p.dv_s[0] + (int64_t)hk * p.dv_s[1];
       if (r0 < rpp) {
 #pragma unroll 2
-        for (int key = k0 + r0; key < min(k0 + 32, p.Nk); key += rpp) {
+        for (int key = k0 + r0; key < min(k0 + krows, p.Nk); key += rpp) {
           const float4 a = sum4(vrow + (int64_t)key * p.DV + d, S, sv);
           const float g[4] = {a.x, a.y, a.z, a.w};
           store4<T>(dvb + (int64_t)key * p.dv_s[2] + d, g);
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(256) void flash_chain_kernel(FlashBwdParams p, int 
     float db[4] = {0.f, 0.f, 0.f, 0.f};
     if (r0 < rpp) {
 #pragma unroll 2
-      for (int r = r0; r < 32; r += rpp) {
+      for (int r = r0; r < krows; r += rpp) {
         const int key = k0 + r;
         if (key >= p.Nk) break;
         const float* u = wrow + (int64_t)key * EP;
@@ -121,8 +121,8 @@ __global__ __launch_bounds__(256) void flash_chain_kernel(FlashBwdParams p, int 
     }
     return;
   }
-  const int nqb = (p.Nq + 31) / 32, blk = blockIdx.x - nk;
-  const int q0 = 32 * (blk % nqb), bh = blk / nqb;
+  const int nqb = (p.Nq + qrows - 1) / qrows, blk = blockIdx.x - nk;
+  const int q0 = qrows * (blk % nqb), bh = blk / nqb;
   const int b = bh / p.Hq, h = bh % p.Hq, hk = h % p.Hk;
   const int q_off = p.Nk - p.Nq;
   const uint16_t* qb = p.q + (int64_t)b * p.q_s[0] + (int64_t)h * p.q_s[1];
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) void flash_chain_kernel(FlashBwdParams p, int 
     for (int t = 0; t < 4; ++t) tbv[t] = bq[d + t];
   }
 #pragma unroll 2
-  for (int r = r0; r < 32; r += rpp) {
+  for (int r = r0; r < qrows; r += rpp) {
     const int i = q0 + r;
     if (i >= p.Nq) break;
     const float* u = wrow + (int64_t)i * EP;
@@ -174,10 +174,20 @@ __global__ __launch_bounds__(256) void flash_chain_kernel(FlashBwdParams p, int 
 }  // namespace
 
 hipError_t launch_flash_chain(const FlashBwdParams& p, const char* name, bool keys, bool queries, int dtype, hipStream_t s) {
-  const int nk = keys ? ((p.Nk + 31) / 32) * p.B * p.Hk : 0, nq = queries ? ((p.Nq + 31) / 32) * p.B * p.Hq : 0;
-  const dim3 grid(nk + nq);
-  return dtype == 2 ? launch_named(name, flash_chain_kernel<BF16>, grid, dim3(256), s, p, nk)
-                    : launch_named(name, flash_chain_kernel<F16>, grid, dim3(256), s, p, nk);
+  const auto nkey = [&](int rows) { return keys ? ((p.Nk + rows - 1) / rows) * p.B * p.Hk : 0; };
+  const auto nquery = [&](int rows) { return queries ? ((p.Nq + rows - 1) / rows) * p.B * p.Hq : 0; };
+  // A block's rows come one after another, a memory latency and one per split each: 8 rows a block where
+  // blocks of 32 leave the chip idle (8 heads of 413 rows, D 250, R 62: 28 -> 12.5 us).  Every key block
+  // adds to the same dbias row, 10 ns apiece: 3,410 keys of 4 batches on one row took 15.5 us at 32 and
+  // 31.8 at 8, 2,999 keys of one batch 19 and 25, so keys keep 32 beyond kBiasAdds of them.
+  constexpr int kBiasAdds = 192;
+  const bool few = nkey(32) + nquery(32) < 1024;
+  const int64_t adds = p.dbias ? (int64_t)((p.Nk + 7) / 8) * p.B * (p.Hb > 1 ? 1 : p.Hk) : 0;
+  const int krows = few && adds <= kBiasAdds ? 8 : 32, qrows = few ? 8 : 32;
+  const int nk = nkey(krows);
+  const dim3 grid(nk + nquery(qrows));
+  return dtype == 2 ? launch_named(name, flash_chain_kernel<BF16>, grid, dim3(256), s, p, nk, krows, qrows)
+                    : launch_named(name, flash_chain_kernel<F16>, grid, dim3(256), s, p, nk, krows, qrows);
 }
 
 }  // namespace pope

@@ -37,6 +37,8 @@
 //              dQ_hat chunk.
 //   flash_chain (flash_chain.hip) the chain rule of the polar transform from the raw rows: dk, dq,
 //              dfreqs, dbias (deterministic mode: the per-row phase derivatives).
+#include <algorithm>
+
 #include "pope_common.hpp"
 #include "pope_kernels.hpp"
 
@@ -331,8 +333,10 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(FlashFwdParams p) {
 // registers allow).  The Q_hat and dO tiles of each 32-query step go straight from global memory
 // into LDS once for the four waves, in three slots (two steps ahead of the step computed), with
 // the step's -lse and -delta rows (one more load, wave 0).
-template <typename T, int EP, int DV, int CH>
-__global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p, float* wk) {
+// SPLIT: the workgroup takes one of kv_splits shares of the steps and leaves raw dV rows too (a run-time
+// split count cost the unsplit kernels 5%).
+template <typename T, int EP, int DV, int CH, bool SPLIT>
+__global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p) {
   constexpr int KS = EP / 16, DS = DV / 16, EBC = EP / 32 / CH, DBC = DV / 32 / CH, RB = 4 / CH;
   constexpr int QU = EP / 8, OU = DV / 8, NL = 32 * (QU + OU) / 256;
   constexpr uint32_t QT = 64 * EP, RT = 64 * (EP + DV), SLOT = RT + 1024;   // byte offsets in a slot: dO tile, row terms
@@ -342,8 +346,10 @@ __global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p, float* w
   const int tid = threadIdx.x, wave = wave_id(), lane = tid & 63, lr = lane & 31, hf = lane >> 5;
   const int nkb = p.NkP / (32 * RB);
   const int ec = wave % CH;   // the wave's column chunk
-  const int2 job = wide_job(blockIdx.x, nkb, p.B * p.Hk);
-  const int kb0 = 32 * RB * job.x, bhk = job.y;   // key block 0 (the heaviest causal one) first
+  const int S = SPLIT ? p.kv_splits : 1;
+  const int2 job = wide_job(blockIdx.x, nkb * S, p.B * p.Hk);
+  const int kb0 = 32 * RB * (SPLIT ? job.x / S : job.x), bhk = job.y;   // key block 0 (the heaviest causal one) first
+  const int sp = SPLIT ? job.x % S : 0;
   const int k0 = kb0 + 32 * (wave / CH);   // the wave's keys
   const int b = bhk / p.Hk, hk = bhk % p.Hk;
   const int Nk = p.Nk, Nq = p.Nq, D = p.D, NqP = p.NqP;
@@ -356,12 +362,16 @@ __global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p, float* w
   const int groups = p.Hq / p.Hk;
   const int qstart = p.causal ? kb0 : 0;   // the workgroup's first key block
   const int nsq = Nq > qstart ? (Nq - qstart + 31) / 32 : 0;
-  const int nsteps = __syncthreads_or(kvis) ? groups * nsq : 0;   // uniform over the workgroup
+  const int nall = __syncthreads_or(kvis) ? groups * nsq : 0;   // uniform over the workgroup
+  // the workgroup's share of the steps (split sp of kv_splits)
+  const int st_lo = SPLIT ? (int)((int64_t)nall * sp / S) : 0;
+  const int nsteps = SPLIT ? (int)((int64_t)nall * (sp + 1) / S) - st_lo : nall;
   const uint32_t lds0 = lds_addr(smem), do_row = 2 * (uint32_t)p.do_s[2];
   // the next step's tiles into the next slot: Q_hat rows padded to NqP (no clamp); dO rows past Nq
   // repeat the last one and dO units at or past D repeat the row's last unit (they meet zero V
   // columns in dP and reach only the dV columns at or past D, which are not stored)
-  int ih = hk, iq = qstart, islot = 0;
+  const int q_first = SPLIT && nall > 0 ? qstart + 32 * (st_lo % nsq) : qstart;
+  int ih = hk + (SPLIT && nall > 0 ? p.Hk * (st_lo / nsq) : 0), iq = q_first, islot = 0;
   auto issue = [&]() {
     const uint32_t slot = lds0 + islot * SLOT;
     const int64_t row = (int64_t)(b * p.Hq + ih) * NqP + iq;
@@ -409,7 +419,7 @@ __global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p, float* w
   const uint32_t orow = WideAddr<OU>::lane_row(lane), otr = WideAddr<OU>::lane_tr(lane, ec);
   const bool wave_vis = __all(kvis);
 
-  int q0 = qstart, buf = 0;
+  int q0 = q_first, buf = 0;
   for (int st = 0; st < nsteps; ++st) {
     // this thread's loads of step st landed (st + 1 may be in flight; wave 0 has one more per step)
     if (st + 1 < nsteps) {
@@ -487,18 +497,28 @@ __global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p, float* w
     if (q0 >= Nq) q0 = qstart;
     buf = buf == kSlots - 1 ? 0 : buf + 1;
   }
-  // dV (lane = d column, registers = keys); the raw dK_hat chunk, times ln 2 (Q_hat carries log2 e)
-  uint16_t* dvb = p.dv + (int64_t)b * p.dv_s[0] + (int64_t)hk * p.dv_s[1];
+  // dV (lane = d column, registers = keys; a split's as raw fp32 rows); the raw dK_hat chunk, times
+  // ln 2 (Q_hat carries log2 e)
+  const int64_t row0 = ((int64_t)sp * p.B * p.Hk + bhk) * p.NkP;
+  if constexpr (SPLIT) {
+    float* wvb = p.wv + row0 * DV;
 #pragma unroll
-  for (int db = 0; db < DBC; ++db) {
-    const int d = 32 * (CH * db + ec) + lr;
+    for (int db = 0; db < DBC; ++db)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int key = k0 + res_row(r, hf);
-      if (key < Nk && d < D) dvb[(int64_t)key * p.dv_s[2] + d] = T::bits(dva[db][r]);
+      for (int r = 0; r < 16; ++r) wvb[(int64_t)(k0 + res_row(r, hf)) * DV + 32 * (CH * db + ec) + lr] = dva[db][r];
+  } else {
+    uint16_t* dvb = p.dv + (int64_t)b * p.dv_s[0] + (int64_t)hk * p.dv_s[1];
+#pragma unroll
+    for (int db = 0; db < DBC; ++db) {
+      const int d = 32 * (CH * db + ec) + lr;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = k0 + res_row(r, hf);
+        if (key < Nk && d < D) dvb[(int64_t)key * p.dv_s[2] + d] = T::bits(dva[db][r]);
+      }
     }
   }
-  float* wkb = wk + (int64_t)bhk * p.NkP * EP;
+  float* wkb = p.wk + row0 * EP;
 #pragma unroll
   for (int eb = 0; eb < EBC; ++eb) {
     const int e = 32 * (CH * eb + ec) + lr;
@@ -511,8 +531,8 @@ __global__ __launch_bounds__(256) void wide_kv_kernel(FlashBwdParams p, float* w
 // One workgroup per (4 / CH blocks of 32 queries, batch * head); wave w takes query block w / CH
 // and column chunk w % CH of the accumulator.  The K_hat and V tiles of each 32-key step go
 // straight from global memory into LDS once for the four waves, in three slots (two steps ahead).
-template <typename T, int EP, int DV, int CH>
-__global__ __launch_bounds__(256) void wide_q_kernel(FlashBwdParams p, float* wq) {
+template <typename T, int EP, int DV, int CH, bool SPLIT>
+__global__ __launch_bounds__(256) void wide_q_kernel(FlashBwdParams p) {
   constexpr int KS = EP / 16, DS = DV / 16, EBC = EP / 32 / CH, RB = 4 / CH;
   constexpr int KU = EP / 8, VU = DV / 8, NL = 32 * (KU + VU) / 256;
   constexpr uint32_t KT = 64 * EP, SLOT = 64 * (EP + DV);   // bytes of the K_hat tile and of a slot
@@ -522,8 +542,10 @@ __global__ __launch_bounds__(256) void wide_q_kernel(FlashBwdParams p, float* wq
   const int tid = threadIdx.x, wave = wave_id(), lane = tid & 63, lr = lane & 31, hf = lane >> 5;
   const int nqb = p.NqP / (32 * RB);
   const int ec = wave % CH;   // the wave's column chunk
-  const int2 job = wide_job(blockIdx.x, nqb, p.B * p.Hq);
-  const int qb0 = 32 * RB * (nqb - 1 - job.x), bh = job.y;   // heaviest causal blocks first
+  const int S = SPLIT ? p.q_splits : 1;
+  const int2 job = wide_job(blockIdx.x, nqb * S, p.B * p.Hq);
+  const int qb0 = 32 * RB * (nqb - 1 - (SPLIT ? job.x / S : job.x)), bh = job.y;   // heaviest causal blocks first
+  const int sp = SPLIT ? job.x % S : 0;
   const int q0 = qb0 + 32 * (wave / CH);   // the wave's queries
   const int b = bh / p.Hq, h = bh % p.Hq, hk = h % p.Hk;
   const int Nk = p.Nk, Nq = p.Nq, D = p.D;
@@ -533,16 +555,18 @@ __global__ __launch_bounds__(256) void wide_q_kernel(FlashBwdParams p, float* wq
   if (p.causal) nkeys = min(nkeys, qb0 + 32 * RB);   // the workgroup's last query block
   const uint16_t* khb = p.kh + (int64_t)(b * p.Hk + hk) * p.NkP * EP;   // rows padded to NkP
   const uint16_t* vb = p.v + (int64_t)b * p.v_s[0] + (int64_t)hk * p.v_s[1];
+  // the workgroup's share of the tiles (split sp of q_splits): local tile t is tile t_lo + t
+  const int nall = (nkeys + 31) / 32, t_lo = SPLIT ? (int)((int64_t)nall * sp / S) : 0;
+  const int nt = SPLIT ? (int)((int64_t)nall * (sp + 1) / S) - t_lo : nall;
   const uint32_t lds0 = lds_addr(smem), v_row = 2 * (uint32_t)p.v_s[2];
   // tile t into slot t % kSlots: K_hat rows padded to NkP (no clamp); V rows past Nk repeat the
   // last one and V units at or past D repeat the row's last unit (they meet zero dO columns)
   auto issue = [&](int t) {
-    const int j0 = 32 * t;
+    const int j0 = 32 * (t_lo + t);
     const uint32_t slot = lds0 + (t % kSlots) * SLOT;
     fill_dense<KU>(slot, wave, lane, khb + (int64_t)j0 * EP);
     fill_strided<VU>(slot + KT, wave, lane, vb + (int64_t)j0 * p.v_s[2], v_row, Nk - j0, D);
   };
-  const int nt = (nkeys + 31) / 32;
   if (nt > 0) issue(0);
   if (nt > 1) issue(1);
 
@@ -569,15 +593,15 @@ __global__ __launch_bounds__(256) void wide_q_kernel(FlashBwdParams p, float* wq
   cu64* mw = (cu64*)p.mwords + (int64_t)b * p.NW;
   const uint32_t krow = WideAddr<KU>::lane_row(lane), ktr = WideAddr<KU>::lane_tr(lane, ec);
   const uint32_t vrow = WideAddr<VU>::lane_row(lane);
-  uint32_t word = nt > 0 ? (uint32_t)mw[0] : 0u;   // visibility of the step's keys
+  uint32_t word = nt > 0 ? (uint32_t)(mw[t_lo >> 1] >> (32 * (t_lo & 1))) : 0u;   // visibility of the step's keys
   for (int t = 0; t < nt; ++t) {
-    const int j0 = 32 * t;
+    const int j0 = 32 * (t_lo + t);
     if (t + 1 < nt) wait_vmcnt<NL>();   // this thread's loads of tile t landed (t + 1 may be in flight)
     else wait_vmcnt<0>();
     __syncthreads();                    // ... everyone's; and slot (t + 2) % kSlots was last read in step t - 1
     if (t + 2 < nt) issue(t + 2);
     const uint32_t wv = word;
-    if (t + 1 < nt) word = (uint32_t)(mw[(t + 1) >> 1] >> (32 * ((t + 1) & 1)));
+    if (t + 1 < nt) word = (uint32_t)(mw[(t_lo + t + 1) >> 1] >> (32 * ((t_lo + t + 1) & 1)));
     const uint32_t slot = lds0 + (t % kSlots) * SLOT;
     const WideAddr<KU> ka(slot, krow, ktr);
     const WideAddr<VU> va(slot + KT, vrow, 0);
@@ -624,7 +648,7 @@ __global__ __launch_bounds__(256) void wide_q_kernel(FlashBwdParams p, float* wq
     }
   }
   // the raw dQ_hat chunk (rows = e, lane = query), times softmax_scale
-  float* wqb = wq + ((int64_t)bh * p.NqP + qi) * EP;
+  float* wqb = p.wq + (((int64_t)sp * p.B * p.Hq + bh) * p.NqP + qi) * EP;
 #pragma unroll
   for (int eb = 0; eb < EBC; ++eb)
 #pragma unroll
@@ -647,23 +671,40 @@ template <int EP>
 constexpr int q_chunks() { return EP <= 256 ? 1 : 2; }
 
 template <typename T, int EP, int DV>
-hipError_t bwd_t(const FlashBwdParams& p, float* wk, float* wq, hipStream_t s) {
+hipError_t bwd_t(const FlashBwdParams& p, hipStream_t s) {
   constexpr int CK = kv_chunks<EP>(), CQ = q_chunks<EP>();
-  hipError_t e = launch_named("flash_wide_kv", wide_kv_kernel<T, EP, DV, CK>, dim3((p.NkP / (128 / CK)) * p.B * p.Hk),
-                              dim3(256), s, p, wk);
+  const dim3 gk((p.NkP / (128 / CK)) * p.B * p.Hk * p.kv_splits), gq((p.NqP / (128 / CQ)) * p.B * p.Hq * p.q_splits);
+  hipError_t e = p.kv_splits > 1 ? launch_named("flash_wide_kv", wide_kv_kernel<T, EP, DV, CK, true>, gk, dim3(256), s, p)
+                                 : launch_named("flash_wide_kv", wide_kv_kernel<T, EP, DV, CK, false>, gk, dim3(256), s, p);
   if (e != hipSuccess) return e;
-  e = launch_named("flash_wide_q", wide_q_kernel<T, EP, DV, CQ>, dim3((p.NqP / (128 / CQ)) * p.B * p.Hq), dim3(256), s,
-                   p, wq);
+  e = p.q_splits > 1 ? launch_named("flash_wide_q", wide_q_kernel<T, EP, DV, CQ, true>, gq, dim3(256), s, p)
+                     : launch_named("flash_wide_q", wide_q_kernel<T, EP, DV, CQ, false>, gq, dim3(256), s, p);
   if (e != hipSuccess) return e;
-  FlashBwdParams c = p;   // both sides' raw rows, dV written already
-  c.kv_splits = c.q_splits = 1;
-  c.wk = wk;
-  c.wq = wq;
-  c.wv = nullptr;
+  FlashBwdParams c = p;   // both sides' raw rows; dV from the splits, or written already
+  if (c.kv_splits == 1) c.wv = nullptr;
   return launch_flash_chain(c, "flash_wide_chain", true, true, T::kCode, s);
 }
 
+// Splits of n jobs with `steps` steps of 32 rows each (2.4 us a step) over the CUs they leave idle, one
+// workgroup per CU, each split keeping kWideSplitSteps steps and the longest job losing kWideSplitGainUs
+// (the chain rule reads a row per split).
+constexpr int kWideSplitSteps = 4;
+constexpr float kWideStepUs = 2.4f, kWideSplitGainUs = 8.f;
+int wide_splits(int64_t n, int steps) {
+  const int s = (int)std::min<int64_t>(256 / std::max<int64_t>(n, 1), steps / kWideSplitSteps);
+  return s > 1 && (steps - (steps + s - 1) / s) * kWideStepUs >= kWideSplitGainUs ? s : 1;
+}
+
 }  // namespace
+
+// Job splits of a wide backward (raw rows in any case: raw_kv and raw_q stay false).
+FlashBwdSplit flash_wide_bwd_split(int B, int Hq, int Hk, int Nq, int Nk, int EP, bool causal) {
+  const int jk = EP <= 256 ? 128 : 64, jq = jk;   // rows per workgroup: 128 / chunks
+  FlashBwdSplit r{1, 1, false, false};
+  r.kv = wide_splits((int64_t)((Nk + jk - 1) / jk) * B * Hk, Hq / Hk * ((Nq + 31) / 32));
+  r.q = wide_splits((int64_t)((Nq + jq - 1) / jq) * B * Hq, ((causal ? std::min(Nq, Nk) : Nk) + 31) / 32);
+  return r;
+}
 
 bool flash_wide_shape(int EP, int DV) { return DV == 256 && (EP == 256 || EP == 384 || EP == 512); }
 
@@ -679,16 +720,16 @@ hipError_t launch_flash_wide_fwd(const FlashFwdParams& p, int dtype, hipStream_t
   return fwd_t<F16, 512, 256>(p, s);
 }
 
-hipError_t launch_flash_wide_bwd(const FlashBwdParams& p, float* wk, float* wq, int dtype, hipStream_t s) {
+hipError_t launch_flash_wide_bwd(const FlashBwdParams& p, int dtype, hipStream_t s) {
   if (!flash_wide_shape(p.EP, p.DV)) return hipErrorInvalidValue;
   if (dtype == 2) {
-    if (p.EP == 256) return bwd_t<BF16, 256, 256>(p, wk, wq, s);
-    if (p.EP == 384) return bwd_t<BF16, 384, 256>(p, wk, wq, s);
-    return bwd_t<BF16, 512, 256>(p, wk, wq, s);
+    if (p.EP == 256) return bwd_t<BF16, 256, 256>(p, s);
+    if (p.EP == 384) return bwd_t<BF16, 384, 256>(p, s);
+    return bwd_t<BF16, 512, 256>(p, s);
   }
-  if (p.EP == 256) return bwd_t<F16, 256, 256>(p, wk, wq, s);
-  if (p.EP == 384) return bwd_t<F16, 384, 256>(p, wk, wq, s);
-  return bwd_t<F16, 512, 256>(p, wk, wq, s);
+  if (p.EP == 256) return bwd_t<F16, 256, 256>(p, s);
+  if (p.EP == 384) return bwd_t<F16, 384, 256>(p, s);
+  return bwd_t<F16, 512, 256>(p, s);
 }
 
 }  // namespace pope

@@ -252,13 +252,19 @@ BwdPartials flash_bwd_partials(const pope_desc& d, const FlashLayout& L) {
   BwdPartials r{{1, 1, false, false}, 0, 0, 0};
   // Wide heads: the raw rows, out of the workspace, which is then the forward's and brings its
   // preparation (a second one took 25 us of 573 at (2, 8, 2048, 256)).
-  if (L.wide) {
-    if (!(d.flags & POPE_FLAG_DETERMINISTIC)) r.total = L.wide_bytes;
-    return r;
-  }
-  r.sp = pope::flash_bwd_split(d.B, d.Hq, d.Hk, d.Nq, d.Nk, d.R, L.EP, L.DV, d.causal != 0);
+  if (L.wide && (d.flags & POPE_FLAG_DETERMINISTIC)) return r;
+  r.sp = L.wide ? pope::flash_wide_bwd_split(d.B, d.Hq, d.Hk, d.Nq, d.Nk, L.EP, d.causal != 0)
+                : pope::flash_bwd_split(d.B, d.Hq, d.Hk, d.Nq, d.Nk, d.R, L.EP, L.DV, d.causal != 0);
   size_t off = 0;
   const size_t kr = (size_t)r.sp.kv * d.B * d.Hk * L.NkP, qr = (size_t)r.sp.q * d.B * d.Hq * L.NqP;
+  if (L.wide) {
+    off += align_up(kr * L.EP * sizeof(float));
+    r.wv = off;
+    if (r.sp.kv > 1) off += align_up(kr * L.DV * sizeof(float));
+    r.wq = off;
+    r.total = off + align_up(qr * L.EP * sizeof(float));
+    return r;
+  }
   if (r.sp.raw_kv) off += align_up(kr * L.EP * sizeof(float));
   r.wv = off;
   if (r.sp.raw_kv) off += align_up(kr * L.DV * sizeof(float));
@@ -694,11 +700,12 @@ int pope_flash_bwd_split(const pope_desc* d, const void* dout, const void* q, co
   if (p.raw_q) p.wq = reinterpret_cast<float*>(static_cast<char*>(partials) + bp.wq);
   hipError_t e;
   if (L.wide) {
-    e = pope::launch_flash_bwd_delta(p, d->dtype, s);
     char* raw = wide_parts ? static_cast<char*>(partials) : ws + L.wk;
-    if (e == hipSuccess)
-      e = pope::launch_flash_wide_bwd(p, reinterpret_cast<float*>(raw), reinterpret_cast<float*>(raw + (L.wq - L.wk)),
-                                      d->dtype, s);
+    p.wk = reinterpret_cast<float*>(raw);
+    p.wv = reinterpret_cast<float*>(raw + bp.wv);   // read and written by splits only
+    p.wq = reinterpret_cast<float*>(raw + (wide_parts ? bp.wq : L.wq - L.wk));
+    e = pope::launch_flash_bwd_delta(p, d->dtype, s);
+    if (e == hipSuccess) e = pope::launch_flash_wide_bwd(p, d->dtype, s);
   } else {
     e = pope::launch_flash_bwd(p, d->dtype, s);
   }

@@ -138,7 +138,8 @@ hipError_t launch_flash_bwd_delta(const FlashBwdParams& p, int dtype, hipStream_
 // workspaces for the raw expanded-row gradients, wk (B, Hk, NkP, EP) and wq (B, Hq, NqP, EP).
 bool flash_wide_shape(int EP, int DV);
 hipError_t launch_flash_wide_fwd(const FlashFwdParams& p, int dtype, hipStream_t s);
-hipError_t launch_flash_wide_bwd(const FlashBwdParams& p, float* wk, float* wq, int dtype, hipStream_t s);
+hipError_t launch_flash_wide_bwd(const FlashBwdParams& p, int dtype, hipStream_t s);
+FlashBwdSplit flash_wide_bwd_split(int B, int Hq, int Hk, int Nq, int Nk, int EP, bool causal);
 
 struct SimParams {
   const float* q; const float* k; const float* dsim; float* sim;

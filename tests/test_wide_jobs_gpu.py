@@ -20,6 +20,11 @@ CASES = [
     (1, 5, 1, 96, 225, 192, 64, "none", False, torch.bfloat16),
     (2, 4, 4, 128, 128, 160, 96, "prefix", True, torch.float16),
     (1, 1, 1, 257, 289, 248, 136, "none", True, torch.bfloat16),
+    # job splits in the backward: ragged shares, grouped heads, splits without a visible row
+    (1, 1, 1, 700, 700, 160, 32, "none", False, torch.bfloat16),
+    (2, 4, 1, 301, 333, 256, 256, "prefix", True, torch.float16),
+    (1, 2, 2, 513, 900, 144, 144, "half", True, torch.bfloat16),
+    (1, 8, 1, 130, 130, 192, 64, "dead_row", False, torch.bfloat16),
 ]
 
 
