@@ -238,7 +238,7 @@ bool decode_groups(int64_t Hq, int64_t D) {
 
 // The same decision as hip_pope_flash_attn._decode_eligible.
 bool decode_eligible(const pope_desc& d, int64_t min_keys) {
-  if (d.Nq != 1 || d.causal || d.Nk < min_keys || d.D > 128 || !decode_groups(d.Hq, d.D)) return false;
+  if (d.Nq != 1 || d.causal || (d.Nk < min_keys && (int64_t)d.Nk * d.D < 36 * min_keys) || d.D > 128 || !decode_groups(d.Hq, d.D)) return false;
   if (d.R && (d.f_s[1] != 0 || d.f_s[0] % 4 || d.f_s[2] % 4)) return false;
   return (int64_t)(d.Nk - 1) * std::max(d.k_s[2], d.v_s[2]) + d.D < INT_MAX;
 }

@@ -211,7 +211,11 @@ class _RangeCheck:
 
 
 _INT32_MAX = 2 ** 31 - 1
-_DECODE_MIN_KEYS = 1024      # shortest cache the decode kernel takes
+# Shortest cache the decode kernel takes, or Nk * D >= 36 of it (576 keys at D 64, 288 at D 128).  A decode
+# call is 14-16 us at any of these lengths; the general forward grows with a head's rows: 1 x 8 heads of D 64
+# 13.5 us at 512 keys, 16.9 at 768; 8 x 16 heads of D 64 21.7 at 512; 1 x 32 heads of D 128 15.6 at 256, 23 at
+# 768; 8 x 32 heads of D 128 33 at 256 (decode 15.4); 2 x 16 heads of D 32 10.8 at 512, 14.6 at 1000 (14.1).
+_DECODE_MIN_KEYS = 1024
 _DECODE_QUERY_WORDS = 4096   # query-weight words a decode workgroup stages in LDS
 
 
@@ -228,13 +232,14 @@ def _decode_head_groups(Hq: int, D: int) -> int:
 
 def _decode_eligible(q, k, v, freqs, causal) -> bool:
     """Whether the forward runs the split-K decode kernel (pope_flash_decode): one non-causal query
-    row against a cache of at least 1024 keys, within the decode kernel's head-dim and 32-bit index
+    row against a cache of at least _DECODE_MIN_KEYS keys (fewer for wider heads), within the decode kernel's head-dim and 32-bit index
     limits.  The forward op and its fake implementation both decide with this predicate, so the
     workspace they return has the same size (empty for decode)."""
     B, Hq, Nq, D = q.shape
     Nk = k.shape[2]
     R = freqs.shape[-1] if exists(freqs) else 0
-    if Nq != 1 or causal or Nk < _DECODE_MIN_KEYS or D > 128:
+    short = Nk < _DECODE_MIN_KEYS and Nk * D < 36 * _DECODE_MIN_KEYS
+    if Nq != 1 or causal or short or D > 128:
         return False
     if _decode_head_groups(Hq, D) == 0:
         return False   # a workgroup stages its group's query weights in LDS
