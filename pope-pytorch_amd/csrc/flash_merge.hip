@@ -30,9 +30,11 @@ __global__ __launch_bounds__(kThreads) void flash_merge_kernel(FlashMergeParams 
   float m = -INFINITY, l = 0.f;
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
   // folds one split into the running state; a split without a visible key has m = -inf, l = 0
-  // and possibly an o that was never written, and leaves the state as it is
+  // and possibly an o that was never written, and leaves the state as it is.  One whose visible
+  // scores are all NaN has m = -inf too (the maximum drops NaN) but l = NaN, and its NaN o counts:
+  // the row is NaN, as in an unsplit kernel
   auto fold = [&](float2 ml, float4 v) {
-    if (ml.x == -INFINITY) v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (ml.x == -INFINITY && ml.y == 0.f) v = make_float4(0.f, 0.f, 0.f, 0.f);
     const float mn = fmaxf(m, ml.x);
     const float mu = mn == -INFINITY ? 0.f : mn;
     const float a = __builtin_amdgcn_exp2f(m - mu), w = __builtin_amdgcn_exp2f(ml.x - mu);

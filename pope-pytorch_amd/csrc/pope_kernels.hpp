@@ -76,7 +76,7 @@ struct FlashFwdParams {
   int64_t v_s[3], o_s[3];
   // splits > 1: workgroup = (query block, split of split_keys keys); its (m, l, O) go to part_ml
   // (rows, splits, 2) and part_o (rows, splits, D), row = (b Hq + h) Nq + i, for launch_flash_merge
-  // (a split without a visible key: m = -inf, l = 0)
+  // (a split without a visible key: m = -inf, l = 0; one whose visible scores are all NaN: m = -inf, l = NaN)
   int splits, split_keys;
   float* part_o; float* part_ml;
 };
