@@ -284,8 +284,8 @@ __global__ __launch_bounds__(kThreads, 2) void decode_split_kernel(DecodeParams 
     for (int u = 0; u < kLoads; ++u) {
       float part = 0.f;
       if (R == D || rot) {
-        // softplus(x) = max(x, 0) + ln 2 log2(1 + 2^(-|x| log2 e)), the max taken on the bit
-        // pattern (x >= 0 iff its signed bits are)
+        // softplus(x) = max(x, 0) + ln 2 log2(1 + 2^(-|x| log2 e)); the maximum that propagates NaN
+        // (the table's clamp and fmaxf drop it)
         const uint32_t ta = tab_lane + 4 * TS * RPI * u;
         const u32x4 t0 = lds_read16_at(ta), t1 = lds_read16_at(ta + 16);
 #pragma unroll
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(kThreads, 2) void decode_split_kernel(DecodeParams 
           } else {
             lt = __builtin_amdgcn_logf(1.f + __builtin_amdgcn_exp2f(-fabsf(__builtin_bit_cast(float, xb)) * kLog2e));
           }
-          const float sp = fmaf(lt, kLn2, __builtin_bit_cast(float, max((int)xb, 0)));
+          const float sp = fmaf(lt, kLn2, __builtin_elementwise_maximum(__builtin_bit_cast(float, xb), 0.f));
           const f16x2 cs = __builtin_bit_cast(f16x2, q < 4 ? t0[q] : t1[q - 4]);
           part = fmaf(sp, __builtin_amdgcn_fdot2(cs, __builtin_bit_cast(f16x2, wq[q]), 0.f, false), part);
         }

@@ -98,7 +98,7 @@ def test_split_forward_keeps_nan(cuda, case, what):
 
 @pytest.mark.parametrize("Hq,Hk,D,R,Nk,dtype", [(2, 2, 64, 64, 576, torch.bfloat16), (4, 2, 128, 64, 300, torch.float16),
                                                 (2, 1, 96, 96, 1500, torch.bfloat16), (8, 8, 64, 32, 2048, torch.bfloat16)])
-@pytest.mark.parametrize("what", ["query", "key", "lone_key", "value"])
+@pytest.mark.parametrize("what", ["query", "key", "negative_key", "lone_key", "negative_lone_key", "value"])
 def test_decode_keeps_nan(cuda, Hq, Hk, D, R, Nk, dtype, what):
     import pope_amd
     from pope_amd import _lib
