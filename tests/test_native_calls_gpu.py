@@ -103,3 +103,36 @@ def test_operands_on_another_device_are_refused(cuda):
     inp = make_pope_inputs(65, 1, 1, 1, 8, 8, 32, 16, torch.bfloat16)
     with pytest.raises(RuntimeError):
         pope_amd.flash_attn_with_pope(inp["q"], inp["k"], inp["v"], pos_emb=(inp["freqs"].cpu(), inp["bias"]))
+
+
+def _flash(dtype):
+    import pope_amd
+    return lambda q, k, f, b: pope_amd.flash_attn_with_pope(q.to(dtype), k.to(dtype), k.to(dtype), pos_emb=(f, b), causal=True)
+
+
+def _sim(q, k, f, b):
+    from pope_amd.hip_pope import hip_compute_qk_similarity
+    return hip_compute_qk_similarity(q, k, f, b)
+
+
+def _polar(q, k, f, b):
+    import pope_amd
+    return pope_amd.apply_pope_to_qk(pope_amd.PolarEmbedReturn(f, b), q, k)
+
+
+@pytest.mark.parametrize("R", [16, 12])   # 12: padded operands
+@pytest.mark.parametrize("name", ["sim", "polar", "flash_bf16"])
+@pytest.mark.parametrize("tracer", ["torch.jit.trace", "make_fx", "make_fx_pre_dispatch"])
+def test_traced_calls_replay_on_other_inputs(cuda, name, R, tracer):
+    """Tracers that are neither torch.compile nor a dispatch mode record the ops as well: a trace on one input gives the
+    eager result on another."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    fn = {"sim": _sim, "polar": _polar, "flash_bf16": _flash(torch.bfloat16)}[name]
+    a, b = (tuple(make_pope_inputs(s, 1, 2, 1, 16, 16, 32, R, torch.float32)[n] for n in ("q", "k", "freqs", "bias")) for s in (66, 67))
+    if tracer == "torch.jit.trace":
+        traced = torch.jit.trace(fn, a, check_trace=False)
+    else:
+        traced = make_fx(fn, pre_dispatch=tracer != "make_fx")(*a)
+    got, want = traced(*b), fn(*b)
+    for x, y in zip(*((t if isinstance(t, tuple) else (t,)) for t in (got, want))):
+        assert torch.equal(x, y)
