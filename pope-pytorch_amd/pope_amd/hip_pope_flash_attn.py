@@ -180,7 +180,8 @@ _FP16_MAX = 65504.0
 
 
 def _check_fp16_range(*ts):
-    """The same check with torch operators, for operands of mixed or other dtypes (reads one flag back)."""
+    """The same check with torch operators, for operands of mixed or other dtypes, tracers and modes (reads one
+    flag back: torch.jit.trace records the check as it went, make_fx and fake tensors refuse it)."""
     bad = torch.zeros((), dtype=torch.bool, device=ts[0].device)
     for t in ts:
         bad |= ((t.abs() > _FP16_MAX) & t.isfinite()).any()
@@ -514,8 +515,8 @@ def flash_attn_head_first(q: Tensor, k: Tensor, v: Tensor, freqs: Optional[Tenso
     if q.dtype not in _MFMA_DTYPES:
         # fp32 inputs: fp16 operands keep 10 significant bits, as the TF32 products of the
         # reference's fp32 path do (triton_pope_flash_attn.py:80), but not TF32's exponent range
-        # (under torch.compile tracing, and for other dtypes than fp32, plain conversions)
-        if not torch.compiler.is_compiling() and q.dtype == k.dtype == v.dtype == torch.float32:
+        # (under tracing, modes and transforms, and for other dtypes than fp32, plain conversions)
+        if _lib.eager(q, k, v) and q.dtype == k.dtype == v.dtype == torch.float32:
             check = _RangeCheck()
             q, k, v = _HalfOperands.apply(check.flag, q, k, v)
             check.event.record(torch.cuda.current_stream(q.device))

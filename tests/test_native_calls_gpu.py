@@ -121,18 +121,43 @@ def _polar(q, k, f, b):
 
 
 @pytest.mark.parametrize("R", [16, 12])   # 12: padded operands
-@pytest.mark.parametrize("name", ["sim", "polar", "flash_bf16"])
+@pytest.mark.parametrize("name", ["sim", "polar", "flash_bf16", "flash_fp32"])
 @pytest.mark.parametrize("tracer", ["torch.jit.trace", "make_fx", "make_fx_pre_dispatch"])
 def test_traced_calls_replay_on_other_inputs(cuda, name, R, tracer):
     """Tracers that are neither torch.compile nor a dispatch mode record the ops as well: a trace on one input gives the
-    eager result on another."""
+    eager result on another.  (fp32 flash reads its range check back, which make_fx cannot record: it refuses.)"""
     from torch.fx.experimental.proxy_tensor import make_fx
-    fn = {"sim": _sim, "polar": _polar, "flash_bf16": _flash(torch.bfloat16)}[name]
+    fn = {"sim": _sim, "polar": _polar, "flash_bf16": _flash(torch.bfloat16), "flash_fp32": _flash(torch.float32)}[name]
     a, b = (tuple(make_pope_inputs(s, 1, 2, 1, 16, 16, 32, R, torch.float32)[n] for n in ("q", "k", "freqs", "bias")) for s in (66, 67))
     if tracer == "torch.jit.trace":
         traced = torch.jit.trace(fn, a, check_trace=False)
+    elif name == "flash_fp32":
+        with pytest.raises(RuntimeError):
+            make_fx(fn, pre_dispatch=tracer != "make_fx")(*a)
+        return
     else:
         traced = make_fx(fn, pre_dispatch=tracer != "make_fx")(*a)
     got, want = traced(*b), fn(*b)
     for x, y in zip(*((t if isinstance(t, tuple) else (t,)) for t in (got, want))):
         assert torch.equal(x, y)
+
+
+def test_fp32_flash_refuses_fake_tensors_and_runs_under_modes(cuda):
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Count(TorchDispatchMode):
+        ops = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.ops += "pope_amd" in str(func) or "_to_copy" in str(func)
+            return func(*args, **(kwargs or {}))
+
+    inp = make_pope_inputs(68, 1, 2, 1, 16, 16, 32, 16, torch.float32)
+    q, k, f, b = (inp[n] for n in ("q", "k", "freqs", "bias"))
+    want = _flash(torch.float32)(q, k, f, b)
+    with Count() as mode:
+        assert torch.equal(_flash(torch.float32)(q, k, f, b), want)
+    assert mode.ops >= 5   # q, k, v and o converted where the mode sees it, and the op
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode, pytest.raises(RuntimeError):
+        _flash(torch.float32)(mode.from_tensor(q), mode.from_tensor(k), f, b)
