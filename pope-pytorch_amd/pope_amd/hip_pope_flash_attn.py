@@ -155,6 +155,9 @@ def _check_dtypes(q, *others):
 def _launch_half(ts, flag):
     """fp16 copies (strides as Tensor.to keeps them) of the fp32 tensors ``ts`` in one launch; the int32
     ``flag`` (pinned host memory) is set to 1 when a finite value lies beyond fp16's range."""
+    for t in ts[1:]:   # before the launch: the kernel reads raw pointers
+        if t.device != ts[0].device:
+            raise RuntimeError(f"pope_amd: operand on {t.device} next to q on {ts[0].device}")
     out = tuple(torch.empty_like(t, dtype=torch.float16) for t in ts)
     c = (_lib.PopeCast * len(ts))()
     for i, (t, o) in enumerate(zip(ts, out)):
