@@ -166,6 +166,22 @@ variable_list pad_rows(at::TensorList ts, const std::vector<PadCols>& cols, bool
 
 bool tracked(at::TensorList ts);
 
+// Gradients under create_graph: differentiating them again raises, as it does through the torch.library
+// ops (whose backward ops have no autograd formula), instead of treating them as constants.
+variable_list once_differentiable(variable_list grads, const char* what) {
+  if (!at::GradMode::is_enabled()) return grads;
+  variable_list in;
+  for (const Tensor& g : grads)
+    if (g.defined()) in.push_back(g.detach().requires_grad_(true));
+  auto err = std::make_shared<torch::autograd::DelayedError>(
+      std::string("pope_amd ") + what + ": the gradient is not differentiable a second time", (int64_t)in.size());
+  const variable_list out = (*err)(std::move(in));
+  size_t i = 0;
+  for (Tensor& g : grads)
+    if (g.defined()) g = out[i++];
+  return grads;
+}
+
 // pad_rows under autograd: the gradients take the inverse move (the gap's gradient is dropped, or zero).
 struct PadFn : torch::autograd::Function<PadFn> {
   static variable_list forward(AutogradContext* ctx, at::TensorList ts, const std::vector<PadCols>& cols, bool pad) {
@@ -195,7 +211,10 @@ struct PadFn : torch::autograd::Function<PadFn> {
       }
     variable_list r(grads.size() + 2);
     if (ts.empty()) return r;
-    const variable_list out = pad_rows(ts, cols, !ctx->saved_data["pad"].toBool());
+    variable_list out = pad_rows(ts, cols, !ctx->saved_data["pad"].toBool());
+    // the node before this one may have marked its gradients as not differentiable: so are the moved ones
+    if (std::any_of(ts.begin(), ts.end(), [](const Tensor& t) { return t.requires_grad(); }))
+      out = once_differentiable(std::move(out), "padding");
     for (size_t j = 0; j < out.size(); ++j) r[at_[j]] = out[j];
     return r;
   }
@@ -412,22 +431,6 @@ Tensor flash_padded(const Tensor& q, const Tensor& k, const Tensor& v, const std
 }
 
 // ---------------------------------------------------------------- similarity and polar transform
-
-// Gradients under create_graph: differentiating them again raises, as it does through the torch.library
-// ops (whose backward ops have no autograd formula), instead of treating them as constants.
-variable_list once_differentiable(variable_list grads, const char* what) {
-  if (!at::GradMode::is_enabled()) return grads;
-  variable_list in;
-  for (const Tensor& g : grads)
-    if (g.defined()) in.push_back(g.detach().requires_grad_(true));
-  auto err = std::make_shared<torch::autograd::DelayedError>(
-      std::string("pope_amd ") + what + ": the gradient is not differentiable a second time", (int64_t)in.size());
-  const variable_list out = (*err)(std::move(in));
-  size_t i = 0;
-  for (Tensor& g : grads)
-    if (g.defined()) g = out[i++];
-  return grads;
-}
 
 // Views the kernels read in 16-byte vectors: unit feature stride, other strides multiples of 4
 // elements, 16-byte aligned start.

@@ -161,3 +161,15 @@ def test_fp32_flash_refuses_fake_tensors_and_runs_under_modes(cuda):
     assert mode.ops >= 5   # q, k, v and o converted where the mode sees it, and the op
     with FakeTensorMode(allow_non_fake_inputs=True) as mode, pytest.raises(RuntimeError):
         _flash(torch.float32)(mode.from_tensor(q), mode.from_tensor(k), f, b)
+
+
+@pytest.mark.parametrize("R", [16, 12])   # 12: padded operands
+@pytest.mark.parametrize("fn", [_sim, _polar])
+def test_a_gradient_penalty_raises_instead_of_counting_as_constant(cuda, fn, R):
+    inp = make_pope_inputs(69, 1, 1, 1, 8, 8, 32, R, torch.float32)
+    q = inp["q"].detach().requires_grad_(True)
+    out = fn(q, inp["k"], inp["freqs"], inp["bias"])
+    loss = (out[0] if isinstance(out, tuple) else out).square().sum()
+    (g,) = torch.autograd.grad(loss, q, create_graph=True)
+    with pytest.raises(RuntimeError, match="second time|not differentiable"):
+        (loss + g.square().sum()).backward()
