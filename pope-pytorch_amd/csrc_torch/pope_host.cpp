@@ -183,19 +183,18 @@ variable_list once_differentiable(variable_list grads, const char* what) {
 }
 
 // pad_rows under autograd: the gradients take the inverse move (the gap's gradient is dropped, or zero).
+// Its inputs are the tensors that need a gradient and its outputs their moved copies, made before, so
+// that what needs no gradient (freqs, mostly) stays a constant for the node after this one.
+// (mark_non_differentiable would do that too, but compiled autograd asserts that no node has any.)
 struct PadFn : torch::autograd::Function<PadFn> {
-  static variable_list forward(AutogradContext* ctx, at::TensorList ts, const std::vector<PadCols>& cols, bool pad) {
+  static variable_list forward(AutogradContext* ctx, at::TensorList ts, const variable_list& moved,
+                               const std::vector<PadCols>& cols, bool pad) {
     std::vector<int64_t> flat;
     for (const PadCols& c : cols) flat.insert(flat.end(), {c.split, c.gap, c.cols, c.width});
     ctx->saved_data["cols"] = flat;
     ctx->saved_data["pad"] = pad;
     ctx->set_materialize_grads(false);
-    variable_list out = pad_rows(ts, cols, pad), constant;
-    // what needs no gradient stays a constant for the node after this one (freqs, mostly)
-    for (size_t i = 0; i < out.size(); ++i)
-      if (!ts[i].requires_grad()) constant.push_back(out[i]);
-    ctx->mark_non_differentiable(constant);
-    return out;
+    return moved;
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
@@ -209,7 +208,7 @@ struct PadFn : torch::autograd::Function<PadFn> {
         cols.push_back({flat[4 * i], flat[4 * i + 1], flat[4 * i + 2], flat[4 * i + 3], 0});
         at_.push_back(i);
       }
-    variable_list r(grads.size() + 2);
+    variable_list r(grads.size() + 3);
     if (ts.empty()) return r;
     variable_list out = pad_rows(ts, cols, !ctx->saved_data["pad"].toBool());
     // the node before this one may have marked its gradients as not differentiable: so are the moved ones
@@ -221,7 +220,20 @@ struct PadFn : torch::autograd::Function<PadFn> {
 };
 
 variable_list padded(at::TensorList ts, const std::vector<PadCols>& cols, bool pad) {
-  return tracked(ts) ? PadFn::apply(ts, cols, pad) : pad_rows(ts, cols, pad);
+  variable_list out = pad_rows(ts, cols, pad), in, moved;
+  std::vector<PadCols> in_cols;
+  std::vector<size_t> at_;
+  for (size_t i = 0; i < ts.size(); ++i)
+    if (tracked(ts[i])) {
+      in.push_back(ts[i]);
+      moved.push_back(out[i]);
+      in_cols.push_back(cols[i]);
+      at_.push_back(i);
+    }
+  if (in.empty()) return out;
+  const variable_list r = PadFn::apply(at::TensorList(in), moved, in_cols, pad);
+  for (size_t j = 0; j < r.size(); ++j) out[at_[j]] = r[j];
+  return out;
 }
 
 // ---------------------------------------------------------------- flash attention

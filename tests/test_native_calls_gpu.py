@@ -173,3 +173,25 @@ def test_a_gradient_penalty_raises_instead_of_counting_as_constant(cuda, fn, R):
     (g,) = torch.autograd.grad(loss, q, create_graph=True)
     with pytest.raises(RuntimeError, match="second time|not differentiable"):
         (loss + g.square().sum()).backward()
+
+
+@pytest.mark.parametrize("R", [16, 12])   # 12: padded operands
+@pytest.mark.parametrize("name", ["sim", "polar", "flash_bf16", "flash_fp32"])
+def test_compiled_autograd_takes_the_nodes(cuda, name, R):
+    """A backward under compiled autograd (eager backend) gives the eager gradients."""
+    from torch._dynamo import compiled_autograd
+    fn = {"sim": _sim, "polar": _polar, "flash_bf16": _flash(torch.bfloat16), "flash_fp32": _flash(torch.float32)}[name]
+    inp = make_pope_inputs(70, 1, 2, 1, 16, 16, 32, R, torch.float32)
+    grads = []
+    for compiled in (False, True):
+        leaves = [inp["q"].clone().requires_grad_(True), inp["k"], inp["freqs"], inp["bias"].clone().requires_grad_(True)]
+        out = fn(*leaves)
+        loss = sum(t.float().square().sum() for t in (out if isinstance(out, tuple) else (out,)))
+        if compiled:
+            with compiled_autograd._enable(torch.compile(backend="eager")):
+                loss.backward()
+            torch._dynamo.reset()
+        else:
+            loss.backward()
+        grads.append((leaves[0].grad, leaves[3].grad))
+    _same(grads[1], grads[0])
