@@ -73,8 +73,10 @@ __device__ __forceinline__ f32x16 splat16(float x) {
 __device__ __forceinline__ int res_row(int r, int hf) { return 8 * (r >> 2) + 4 * hf + (r & 3); }
 
 // Growth of a row's running max (log2 units) that the forward absorbs without rescaling its
-// accumulators: probabilities reach at most 2^kLazyMax.
-constexpr float kLazyMax = 8.f;
+// accumulators: probabilities reach at most 2^lazy_max.  None at 512 features: the row's largest
+// probability is exactly 1 there and adds no 16-bit rounding of its own.
+template <int EP>
+constexpr float lazy_max() { return EP < 512 ? 8.f : 0.f; }
 
 // LDS slots of the streamed tiles: tile t is computed from slot t % kSlots while tiles t + 1 and
 // t + 2 load, so each tile has two steps of compute to arrive in.
@@ -259,9 +261,9 @@ __global__ __launch_bounds__(256) void wide_fwd_kernel(FlashFwdParams p) {
     for (int r = 1; r < 16; ++r) mt = fmaxf(mt, s[r]);
     mt = half_swap_max(mt);
     // lazy rescale: a row's reference max m moves only when the tile's max exceeds it by more than
-    // kLazyMax (log2 units), so the probabilities stay below 2^kLazyMax and most steps skip
+    // lazy_max (log2 units), so the probabilities stay below 2^lazy_max and most steps skip
     // rescaling the O accumulators (the branch is taken when any row of the wave moves)
-    const bool grow = mt > m + kLazyMax;
+    const bool grow = mt > m + lazy_max<EP>();
     if (__ballot(grow)) {
       POPE_COLD_PATH();
       const float mn = grow ? mt : m;

@@ -3,6 +3,8 @@ eight dies and ones that do not, lengths around the 32-row tiles and the 64- and
 dim, every expanded width (256, 384, 512).  Against the float64 oracle with the flash tests' tolerance (2e-2 absolute
 beyond the rounding of the output format); dk and dv sum the independent 16-bit operand roundings of their group's G
 query heads, which grow as sqrt(G)."""
+import math
+
 import pytest
 import torch
 
@@ -43,3 +45,39 @@ def test_wide_jobs_against_the_oracle(cuda, case):
     for got, name in zip(grads, ("dq", "dk", "dv")):
         tol = 2e-2 if name == "dq" else 2e-2 * (Hq / Hk) ** 0.5
         assert excess_over(got, ref[name], tol) <= 0, name
+
+
+def test_wide_forward_at_512_features_keeps_the_exact_maximum(cuda):
+    """The row's largest probability is exactly 1 there, so its 16-bit rounding adds nothing: the running maximum moves
+    with every growth, however small.  A row whose first tile holds a score x below its maximum (x < 8), then two keys in
+    the ratio 4 : 3 whose probabilities 2^x and 0.75 2^x round apart in bf16 (1 and 0.75 do not): o = (1 - 0.75) / sum,
+    within the rounding of the output."""
+    import pope_amd
+    from pope_amd import _lib
+    D, R, Nk = 256, 136, 64
+    xs = torch.linspace(6.5, 7.9, 2000, dtype=torch.float64)
+    err = lambda p: (p.to(torch.bfloat16).double() - p) / p
+    x = xs[(err(2 ** xs) - err(0.75 * 2 ** xs)).abs().argmax()].item()
+    s = torch.full((Nk,), -60.0, dtype=torch.float64)
+    s[0], s[32], s[33] = 0.0, x, x + torch.tensor(0.75).log2().item()
+    q = torch.full((1, 1, 1, D), -30.0)   # softplus of the rotated dims: 1e-13
+    k = torch.full((1, 1, Nk, D), -30.0)
+    q[..., R:], k[..., R:] = 0.0, 0.0
+    left = s.clone()
+    for i in range(3):                    # the score in three bf16 parts, times q = 1
+        q[..., R + i] = 1.0
+        k[0, 0, :, R + i] = left.float().to(torch.bfloat16).float()
+        left -= k[0, 0, :, R + i].double()
+    v = torch.zeros(1, 1, Nk, D)
+    v[:, :, 32], v[:, :, 33] = 1.0, -1.0
+    w = 2.0 ** (s - left)
+    ref = (w[32] - w[33]) / w.sum()
+    q, k, v = (t.to(torch.bfloat16).cuda() for t in (q, k, v))
+    freqs, bias = torch.zeros(Nk, R, device="cuda"), torch.zeros(1, R, device="cuda")
+    _lib.profile_reset()
+    _lib.profile_enable(True)
+    o = pope_amd.flash_attn_with_pope(q, k, v, pos_emb=(freqs, bias), softmax_scale=math.log(2.0))
+    torch.cuda.synchronize()
+    _lib.profile_enable(False)
+    assert "flash_wide_fwd" in _lib.profile_read()
+    assert excess_over(o, ref.expand(o.shape), 1e-4) <= 0
