@@ -81,9 +81,9 @@ def polar_bwd_op(gq: Tensor, gk: Tensor, q: Tensor, k: Tensor, freqs: Tensor, bi
     d.flags |= _lib.deterministic_flag()   # torch.use_deterministic_algorithms(True): no fp32 atomics
     dq, dk = torch.empty_like(q), torch.empty_like(k)
     d.dq_s[:], d.dk_s[:] = _lib.strides3(dq), _lib.strides3(dk)
-    empty = q.new_empty(0, dtype=torch.float32)
-    dfreqs = torch.zeros(freqs.shape, device=q.device, dtype=torch.float32) if need_dfreqs else empty
-    dbias = torch.zeros(bias.shape, device=q.device, dtype=torch.float32) if need_dbias else empty
+    # two empty tensors where neither is wanted: an op's outputs must not alias
+    dfreqs = torch.zeros(freqs.shape, device=q.device, dtype=torch.float32) if need_dfreqs else q.new_empty(0, dtype=torch.float32)
+    dbias = torch.zeros(bias.shape, device=q.device, dtype=torch.float32) if need_dbias else q.new_empty(0, dtype=torch.float32)
     if need_dfreqs:
         d.df_s[:] = _freqs_strides(dfreqs)
     ws = _lib.workspace(_lib.OP_POLAR_BWD, d, q.device)

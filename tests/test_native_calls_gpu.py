@@ -195,3 +195,19 @@ def test_compiled_autograd_takes_the_nodes(cuda, name, R):
             loss.backward()
         grads.append((leaves[0].grad, leaves[3].grad))
     _same(grads[1], grads[0])
+
+
+@pytest.mark.parametrize("wanted", [(), ("bias",), ("freqs",), ("freqs", "bias")])
+def test_the_ops_give_only_the_wanted_gradients(cuda, wanted):
+    from pope_amd import _lib
+    from pope_amd.hip_polar import polar_fwd_op
+    from pope_amd.hip_pope import sim_fwd_op
+    inp = make_pope_inputs(71, 1, 2, 2, 8, 12, 32, 16, torch.float32)
+    leaves = [inp[n].detach().requires_grad_(n in ("q", "k", *wanted)) for n in ("q", "k", "freqs", "bias")]
+    for op, native in ((polar_fwd_op, _lib.host().polar), (sim_fwd_op, _lib.host().sim)):
+        grads = []
+        for fn in (op, native):
+            out = fn(*leaves, False)
+            loss = sum(t.square().sum() for t in (out if isinstance(out, tuple) else (out,)))
+            grads.append(torch.autograd.grad(loss, [t for t in leaves if t.requires_grad]))
+        _same(*grads)
