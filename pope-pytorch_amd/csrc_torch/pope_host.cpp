@@ -66,6 +66,23 @@ void freqs_strides(int64_t* dst, const Tensor& f) {
   dst[2] = st(n - 2);
 }
 
+// The gradient of freqs, and its strides for d.  The library clears and fills the positions n < Nk of one table per
+// batch and head the descriptor tells apart: any other entry (a longer table, more batches, a broadcast extent)
+// stays zero, and a broadcast extent's gradient is summed into its first entry, not written past the tensor
+// (grouped heads: more query heads than entries).
+Tensor phase_grad(const Tensor& freqs, pope_desc& d) {
+  const int64_t n = freqs.dim();
+  bool whole = freqs.size(-2) == d.Nk;
+  if (n >= 3) whole = whole && freqs.size(0) == (d.f_s[0] ? d.B : 1);
+  if (n == 4) whole = whole && freqs.size(1) == (d.f_s[1] ? d.Hq : 1);
+  const Tensor g = whole ? fp32_like(freqs, freqs.sizes())
+                         : at::zeros(freqs.sizes(), freqs.options().dtype(at::kFloat).requires_grad(false));
+  freqs_strides(d.df_s, g);
+  for (int i = 0; i < 2; ++i)
+    if (d.f_s[i] == 0) d.df_s[i] = 0;
+  return g;
+}
+
 int dtype_code(const Tensor& t) {
   switch (t.scalar_type()) {
     case at::kFloat: return POPE_F32;
@@ -369,11 +386,6 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
     const bool need_db = bias.defined() && ctx->needs_input_grad(4);
     const Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     Tensor dfreqs, dbias;
-    // the library clears the gradients over the key positions n < Nk it addresses; rows of a longer
-    // table get none, so such a table's gradient starts from zeros
-    if (need_df)
-      dfreqs = freqs.size(-2) > k.size(2) ? at::zeros(freqs.sizes(), freqs.options().dtype(at::kFloat).requires_grad(false))
-                                          : fp32_like(freqs, freqs.sizes());
     if (need_db) dbias = fp32_like(bias, bias.sizes());
     pope_desc d = desc_of(q, k, freqs, bias);
     d.causal = ctx->saved_data["causal"].toBool();
@@ -384,7 +396,7 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
     strides3(d.dq_s, dq);
     strides3(d.dk_s, dk);
     strides3(d.dv_s, dv);
-    if (need_df) freqs_strides(d.df_s, dfreqs);
+    if (need_df) dfreqs = phase_grad(freqs, d);
     if (mask.defined()) d.mask_sb = mask.stride(0);
     d.flags = POPE_FLAG_ZERO_GRADS | deterministic_flag();
     // with the partials the workspace is the forward's
@@ -495,11 +507,7 @@ struct SimFn : torch::autograd::Function<SimFn> {
     strides3(d.dq_s, dq);
     strides3(d.dk_s, dk);
     Tensor dfreqs, dbias;
-    if (need_df) {
-      dfreqs = freqs.size(-2) > k.size(2) ? at::zeros(freqs.sizes(), freqs.options().dtype(at::kFloat).requires_grad(false))
-                                          : fp32_like(freqs, freqs.sizes());
-      freqs_strides(d.df_s, dfreqs);
-    }
+    if (need_df) dfreqs = phase_grad(freqs, d);
     if (need_db) dbias = fp32_like(bias, bias.sizes());
     const size_t n = workspace_bytes(POPE_OP_SIM_BWD, d);
     const Tensor ws = bytes_like(q, n);

@@ -30,7 +30,7 @@ from torch import Tensor
 
 from . import _lib
 from ._pad import pad_last, pad_plan, pad_qk
-from .hip_pope_flash_attn import _freqs_strides
+from .hip_pope_flash_attn import _freqs_strides, _phase_grad
 
 
 def exists(v):
@@ -91,17 +91,15 @@ def sim_bwd_op(dsim: Tensor, q: Tensor, k: Tensor, freqs: Tensor, bias: Tensor, 
     q, k, dsim = _aligned(q), _aligned(k), _aligned(dsim.float())
     d = _desc(q, k, freqs, bias, split)
     d.flags |= _lib.deterministic_flag()   # torch.use_deterministic_algorithms(True): no fp32 atomics
-    # the library clears dfreqs / dbias before accumulating into them, over the positions n < Nk
-    # it addresses; rows of a longer freqs table get no gradient, so that gradient starts from zeros
+    # the library clears dfreqs / dbias before accumulating into them
     d.flags |= _lib.FLAG_ZERO_GRADS
     d.sim_s[:] = _lib.strides3(dsim)
     dq, dk = torch.empty_like(q), torch.empty_like(k)
     d.dq_s[:], d.dk_s[:] = _lib.strides3(dq), _lib.strides3(dk)
-    alloc_df = torch.zeros if freqs.shape[-2] > k.shape[2] else torch.empty
-    dfreqs = alloc_df(freqs.shape, device=q.device, dtype=torch.float32) if need_dfreqs else q.new_empty(0, dtype=torch.float32)
+    dfreqs, df_strides = _phase_grad(freqs, q.shape[0], q.shape[1], k.shape[2]) if need_dfreqs else (q.new_empty(0, dtype=torch.float32), None)
     dbias = torch.empty(bias.shape, device=q.device, dtype=torch.float32) if need_dbias else q.new_empty(0, dtype=torch.float32)
     if need_dfreqs:
-        d.df_s[:] = _freqs_strides(dfreqs)
+        d.df_s[:] = df_strides
     ws = _lib.workspace(_lib.OP_SIM_BWD, d, q.device)
     st = L.pope_sim_bwd(ctypes.byref(d), _lib.ptr(dsim), _lib.ptr(q), _lib.ptr(k), _lib.ptr(freqs), _lib.ptr(bias),
                         _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dfreqs) if need_dfreqs else None,

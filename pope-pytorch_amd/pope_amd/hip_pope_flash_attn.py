@@ -63,6 +63,21 @@ def _freqs_strides(freqs: Tensor, head_first: bool = True) -> tuple:
     raise ValueError(f"freqs must be 2-D, 3-D or 4-D, got shape {tuple(freqs.shape)}")
 
 
+def _phase_grad(freqs: Tensor, B: int, Hq: int, Nk: int):
+    """The gradient of freqs and its descriptor strides.  The library clears and fills the positions n < Nk of one
+    table per batch and head that the descriptor tells apart: any other entry (a longer table, more batches, a
+    broadcast extent) stays zero, and a broadcast extent's gradient is summed into its first entry, not written
+    past the tensor (grouped heads: more query heads than entries)."""
+    s = _freqs_strides(freqs)
+    whole = freqs.shape[-2] == Nk
+    if freqs.ndim >= 3:
+        whole = whole and freqs.shape[0] == (B if s[0] else 1)
+    if freqs.ndim == 4:
+        whole = whole and freqs.shape[1] == (Hq if s[1] else 1)
+    g = (torch.empty if whole else torch.zeros)(freqs.shape, device=freqs.device, dtype=torch.float32)
+    return g, tuple(0 if f == 0 and i < 2 else st for i, (f, st) in enumerate(zip(s, _freqs_strides(g))))
+
+
 def _prep_pope(freqs: Optional[Tensor], bias: Optional[Tensor]):
     if freqs is None or bias is None:
         return None, None
@@ -381,12 +396,8 @@ def _bwd_impl(do, q, k, v, o, lse, freqs, bias, mask, causal, softmax_scale, nee
     if o.shape != q.shape or do.shape != q.shape:
         raise ValueError(f"o {tuple(o.shape)} and do {tuple(do.shape)} must match q {tuple(q.shape)}")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    # the library clears dfreqs / dbias itself (POPE_FLAG_ZERO_GRADS) before accumulating, over the
-    # key positions n < Nk it addresses; rows of a longer freqs table get no gradient, so such a
-    # table's gradient starts from zeros
-    long_freqs = need_dfreqs and freqs.shape[-2] > k.shape[2]
-    alloc_df = torch.zeros if long_freqs else torch.empty
-    dfreqs = alloc_df(freqs.shape, device=q.device, dtype=torch.float32) if need_dfreqs else q.new_empty(0, dtype=torch.float32)
+    # the library clears dfreqs / dbias itself (POPE_FLAG_ZERO_GRADS) before accumulating
+    dfreqs, df_strides = _phase_grad(freqs, q.shape[0], q.shape[1], k.shape[2]) if need_dfreqs else (q.new_empty(0, dtype=torch.float32), None)
     dbias = torch.empty(bias.shape, device=q.device, dtype=torch.float32) if need_dbias else q.new_empty(0, dtype=torch.float32)
     deterministic = _lib.deterministic_flag()
     key = ("bwd", deterministic, q.shape, q.stride(), k.shape, k.stride(), v.shape, v.stride(), o.stride(), do.stride(),
@@ -401,7 +412,7 @@ def _bwd_impl(do, q, k, v, o, lse, freqs, bias, mask, causal, softmax_scale, nee
         d.do_s[:] = _lib.strides3(do)
         d.dq_s[:], d.dk_s[:], d.dv_s[:] = _lib.strides3(dq), _lib.strides3(dk), _lib.strides3(dv)
         if need_dfreqs:
-            d.df_s[:] = _freqs_strides(dfreqs)
+            d.df_s[:] = df_strides
         if exists(mask):
             d.mask_sb = mask.stride(0)
         # torch.use_deterministic_algorithms(True): dfreqs / dbias summed in a fixed order

@@ -135,3 +135,34 @@ def test_similarity_per_batch_positions_and_offset(cuda, allow_tf32):
         for a, b in zip([S] + [x.grad for x in t], [S_ref] + [x.grad for x in r]):
             rel = ((a.detach().double().cpu() - b.detach().double()).abs().max() / b.abs().max()).item()
             assert rel <= 1e-4, rel
+
+
+@pytest.mark.parametrize("deterministic", [False, True])
+@pytest.mark.parametrize("shape", ["batches", "heads", "longer"])
+@pytest.mark.parametrize("path", ["native", "op"])
+def test_gradient_of_broadcast_freqs(cuda, path, shape, deterministic):
+    """A table expanded over batches or heads, in a view longer than the keys or not, gets the gradient of the table
+    itself (fp32 sums in another order), with more query heads than the table has entries."""
+    import pope_amd
+    from pope_amd.hip_pope import sim_fwd_op
+    from pope_amd.hip_pope_flash_attn import flash_fwd_op
+    B, Hq, Hk, N, D, R = 3, 4, 2, 40, 64, 32
+    inp = make_pope_inputs(97, B, Hq, Hk, N, N, D, R, torch.bfloat16)
+    q, k, v, b, do = (inp[n] for n in ("q", "k", "v", "bias", "do"))
+    up = torch.randn(B, Hq, N, N, device="cuda")
+    view = {"batches": lambda t: t.expand(B, N, R), "heads": lambda t: t.expand(B, Hk, N, R),
+            "longer": lambda t: torch.cat([t, t]).expand(B, Hk, 2 * N, R)}[shape]
+    flash = (lambda f: pope_amd.flash_attn_with_pope(q, k, v, pos_emb=(f, b), causal=True)) if path == "native" else \
+        (lambda f: flash_fwd_op(q, k, v, f, b, None, True, D ** -0.5)[0])
+    sim = (lambda f: pope_amd.compute_attn_similarity(q.float(), k.float(), (f, b))) if path == "native" else \
+        (lambda f: sim_fwd_op(q.float(), k.float(), f, b, True))
+    torch.use_deterministic_algorithms(deterministic)
+    try:
+        for fn, grad in ((flash, do), (sim, up)):
+            base = inp["freqs"].detach().requires_grad_(True)
+            (want,) = torch.autograd.grad(fn(base), base, grad)
+            torch.empty(1 << 20, device="cuda").fill_(1e9)   # what an allocation may find
+            (got,) = torch.autograd.grad(fn(view(base)), base, grad)
+            torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-5 * want.abs().max().item())
+    finally:
+        torch.use_deterministic_algorithms(False)
