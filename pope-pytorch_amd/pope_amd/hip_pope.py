@@ -30,7 +30,7 @@ from torch import Tensor
 
 from . import _lib
 from ._pad import pad_last, pad_plan, pad_qk
-from .hip_pope_flash_attn import _freqs_strides, _phase_grad
+from .hip_pope_flash_attn import _check_freqs_extents, _freqs_strides, _phase_grad
 
 
 def exists(v):
@@ -172,6 +172,9 @@ def hip_compute_qk_similarity(q, k, freqs, bias, rotate_dim=None, allow_tf32=Tru
         raise ValueError(f"bias {tuple(bias.shape)} must be (1 or {k.shape[1]}, {R})")
     if freqs.shape[-2] < k.shape[2]:
         raise ValueError(f"freqs has {freqs.shape[-2]} positions, keys need {k.shape[2]}")
+    if k.shape[0] < q.shape[0] or k.shape[-1] < q.shape[-1]:   # read by q's extents
+        raise ValueError(f"incompatible q {tuple(q.shape)} and k {tuple(k.shape)}")
+    _check_freqs_extents(freqs, q.shape[0], q.shape[1])
     out_dtype = q.dtype
     qf, kf = q.float(), k.float()
     # head / rotate dims that are not multiples of 8: padded on the device (pope_amd._pad)

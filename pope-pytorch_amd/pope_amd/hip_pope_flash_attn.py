@@ -63,6 +63,14 @@ def _freqs_strides(freqs: Tensor, head_first: bool = True) -> tuple:
     raise ValueError(f"freqs must be 2-D, 3-D or 4-D, got shape {tuple(freqs.shape)}")
 
 
+def _check_freqs_extents(freqs: Tensor, B: int, Hq: int):
+    """The kernels step through a table's batches and heads by stride: fewer entries than the call has would be
+    read past the end (an extent of 1, or any with stride 0, broadcasts)."""
+    for i, (n, want, name) in enumerate(zip(freqs.shape[:-2], (B, Hq), ("batches", "heads"))):
+        if 1 < n < want and freqs.stride(i):
+            raise ValueError(f"freqs has {n} {name}, the call {want}")
+
+
 def _phase_grad(freqs: Tensor, B: int, Hq: int, Nk: int):
     """The gradient of freqs and its descriptor strides.  The library clears and fills the positions n < Nk of one
     table per batch and head that the descriptor tells apart: any other entry (a longer table, more batches, a
@@ -147,6 +155,7 @@ def _check_pope_shapes(q, k, freqs, bias):
             raise ValueError(f"freqs has {freqs.shape[-2]} positions, keys need {k.shape[2]}")
         if bias.shape[-1] != R or bias.shape[0] not in (1, k.shape[1]):
             raise ValueError(f"bias {tuple(bias.shape)} must be (1 or {k.shape[1]}, {R})")
+        _check_freqs_extents(freqs, B, Hq)
 
 
 def _check_views(q, k, v, mask, lse=None):

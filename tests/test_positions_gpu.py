@@ -166,3 +166,29 @@ def test_gradient_of_broadcast_freqs(cuda, path, shape, deterministic):
             torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-5 * want.abs().max().item())
     finally:
         torch.use_deterministic_algorithms(False)
+
+
+@pytest.mark.parametrize("R", [32, 20])   # 20: padded operands
+def test_tables_and_keys_with_too_few_entries_are_refused(cuda, R):
+    """They would be read past their end.  More entries than the call has are accepted, as before."""
+    import pope_amd
+    from pope_amd.hip_pope_flash_attn import flash_fwd_op
+    B, H, N, D = 3, 4, 16, 64
+    inp = make_pope_inputs(98, B, H, H, N, N, D, R, torch.bfloat16)
+    q, k, v, f, b = (inp[n] for n in ("q", "k", "v", "freqs", "bias"))
+    flash = lambda f: pope_amd.flash_attn_with_pope(q, k, v, pos_emb=(f, b))
+    sim = lambda f, k=k: pope_amd.compute_attn_similarity(q.float(), k.float(), (f, b))
+    for bad in (f.repeat(B - 1, 1, 1), f.repeat(B - 1, H, 1, 1), f.repeat(B, H - 1, 1, 1)):
+        for fn in (flash, sim):
+            with pytest.raises(ValueError):
+                fn(bad)
+    if R % 8 == 0:
+        with pytest.raises(ValueError):
+            flash_fwd_op(q, k, v, f.repeat(B - 1, 1, 1), b, None, False, 0.125)
+    for bad in (k[:1], k[:2], k[..., :32]):
+        with pytest.raises(ValueError):
+            sim(f, bad)
+    for fn in (flash, sim):
+        want = fn(f)
+        for good in (f[None], f.repeat(B + 1, 1, 1), f.expand(B, H, N, R), f.repeat(B, H, 1, 1)):
+            assert torch.equal(fn(good), want)
