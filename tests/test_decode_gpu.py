@@ -245,3 +245,61 @@ def test_decode_dead_splits_ignore_workspace_contents(cuda):
     finite = torch.isfinite(ref["lse"])
     assert torch.equal(torch.isfinite(l1.cpu()), finite)
     assert (l1.cpu()[finite] - ref["lse"][finite]).abs().max().item() <= TOL
+
+
+# The shortest cache of the decode kernel: 1024 keys, or fewer where a key's row is long (Nk * D >= 36 * 1024)
+THRESHOLDS = [   # D, R, shortest Nk, Hq, Hk, dtype
+    (128, 128, 288, 4, 2, torch.bfloat16),
+    (128, 64, 288, 8, 8, torch.float16),
+    (96, 96, 384, 6, 3, torch.bfloat16),
+    (64, 64, 576, 2, 2, torch.bfloat16),
+    (64, 32, 576, 12, 4, torch.float16),
+    (100, 100, 355, 2, 1, torch.bfloat16),     # padded to 104
+    (36, 20, 922, 3, 3, torch.float16),        # padded to 40
+    (32, 32, 1024, 4, 4, torch.bfloat16),
+]
+
+
+@pytest.mark.parametrize("case", THRESHOLDS, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
+def test_decode_threshold(cuda, case):
+    """Just below, at and above the shortest cache, with a masked end and a dead row: the public call and the op take
+    the same kernel, and either agrees with the oracle."""
+    import pope_amd
+    from pope_amd import _lib
+    from pope_amd._pad import pad_last, pad_plan, pad_qk
+    from pope_amd.hip_pope_flash_attn import flash_fwd_op
+    D, R, shortest, Hq, Hk, dtype = case
+    plan = pad_plan(D, R)
+    for Nk in (shortest - 1, shortest, shortest + 1):
+        inp = _decode_inputs(300 + Nk, 3, Hq, Hk, Nk, D, R, dtype, lengths=[Nk, Nk, Nk // 2 + 1], dead_row=True)
+        q, k, v, f, b = (inp[n] for n in ("q", "k", "v", "freqs", "bias"))
+        ref = oracle_attention(inp, False, grads=False)["o"]
+
+        def op():
+            if plan is None:
+                return flash_fwd_op(q, k, v, f, b, inp["mask"], False, D ** -0.5)[0]
+            padded = (pad_qk(q, plan), pad_qk(k, plan), pad_last(v, plan.Dp), pad_last(f, plan.R8), pad_last(b, plan.R8))
+            return flash_fwd_op(*padded, inp["mask"], False, D ** -0.5)[0][..., :D]
+
+        outs = []
+        for call in (lambda: pope_amd.flash_attn_with_pope(q, k, v, pos_emb=(f, b), mask=inp["mask"]), op):
+            _lib.profile_reset()
+            _lib.profile_enable(True)
+            outs.append(call())
+            torch.cuda.synchronize()
+            _lib.profile_enable(False)
+            ran = _lib.profile_read()
+            assert ("flash_decode_split" in ran) == (Nk >= shortest) and ("flash_fwd" in ran) == (Nk < shortest), Nk
+        assert torch.equal(*outs)
+        assert max_abs(outs[0], ref) <= TOL
+        assert outs[0][0].abs().max().item() == 0.0   # every key masked
+
+
+@pytest.mark.parametrize("Nk,D", [(288, 128), (400, 128), (700, 64), (1023, 64), (390, 96)])
+def test_decode_backward_of_short_caches(cuda, Nk, D):
+    """The backward prepares for itself after a decode forward."""
+    inp = _decode_inputs(500 + Nk, 2, 4, 2, Nk, D, D // 2, torch.bfloat16)
+    res = _run(inp, need_grads=True)
+    ref = oracle_attention(inp, False)
+    for n in ("o", "dq", "dk", "dv", "dbias"):
+        assert max_abs(res[n], ref[n]) <= TOL * (max(1.0, ref[n].abs().max().item()) if n == "dbias" else 1.0), n

@@ -162,3 +162,20 @@ def test_fp32_backward_with_split_reductions(cuda, B, Hq, Hk, Nq, Nk, D, R):
     want = [S.detach()] + list(torch.autograd.grad(S, refs, G.double()))
     for a, r in zip(got, want):
         assert (a.double().cpu() - r).abs().max().item() <= 1e-4 * r.abs().max().item()
+
+
+@pytest.mark.parametrize("D,R,Nk", [(64, 32, 2048), (128, 128, 1100), (160, 32, 999), (256, 256, 1025)])
+def test_split_forward_of_one_row(cuda, D, R, Nk):
+    """One query row through the split forward itself: head dims above 128, and per-head tables, which the decode
+    kernel does not take."""
+    from pope_amd import _lib
+    from pope_amd.hip_pope_flash_attn import flash_attn_head_first
+    inp = make_pope_inputs(8600 + D, 2, 2, 2, 1, Nk, D, R, torch.bfloat16, "dead_row")
+    ref = oracle_attention(inp, False, grads=False)
+    _lib.profile_reset()
+    _lib.profile_enable(True)
+    o = flash_attn_head_first(inp["q"], inp["k"], inp["v"], inp["freqs"].repeat(2, 2, 1, 1), inp["bias"], mask=inp["mask"])
+    torch.cuda.synchronize()
+    _lib.profile_enable(False)
+    assert "flash_merge" in _lib.profile_read()
+    assert excess_over(o, ref["o"], 2e-2) <= 0
