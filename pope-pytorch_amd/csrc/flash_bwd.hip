@@ -11,19 +11,16 @@ namespace pope {
 // A dK/dV job loops over the query heads of its group and the query steps, a dQ job over the key
 // steps; one workgroup runs per CU.  With grouped heads, or few batches x heads, the longest jobs
 // are longer than an even share of the work (per_cu) and CUs idle: 16 query heads on 4 kv heads,
-// 2,999 tokens, D 128 ran 96 dK/dV jobs of up to 188 steps, 478 us in flash_bwd.  Jobs split until
-// the longest is about 1.2 even shares, at least three 128-row steps each (measured 0.5, 0.65, 0.8,
-// 1.0, 1.3 shares: that case 238, 224, 237, 228, 228 us for kernel + merge; 4 heads x 2,048 tokens, D 64: 56, 56, 56,
-// 49, 46 against 73 unsplit).  The partial rows' traffic and the launch have to be worth it.
+// 2,999 tokens, D 128 run 96 dK/dV jobs of up to 188 steps unsplit, 499 us in flash_bwd.  Jobs split until
+// the longest is about 1.2 even shares, or three 128-row steps where that is longer; the number of splits
+// rounds up past a quarter, so a split can be as short as two steps.  (Measured 0.5, 0.65, 0.8, 1.0, 1.3
+// shares: that case 238, 224, 237, 228, 228 us for kernel + merge; 4 heads x 2,048 tokens, D 64: 56, 56, 56,
+// 49, 46 against 73 unsplit.)  The partial rows' traffic and the launch have to be worth it.
 //
 // A rotate dim that is no multiple of 32 takes the jobs' general epilogue, one wave at a time through
 // LDS; where the raw rows are few, writing them and the separate chain-rule launch are faster.
 FlashBwdSplit flash_bwd_split(int B, int Hq, int Hk, int Nq, int Nk, int R, int EP, int DV, bool causal) {
-  // BwdCfg's geometry
-  const bool big = EP + DV > 160;
-  const int job = big ? 128 : 256;
-  const bool wide128 = big && 2 * ((128 * EP + 128 * DV) * 2 + 64 * 16) <= 150 * 1024;
-  const int bm = big && !wide128 ? 64 : 128;
+  const int job = bwd_job(EP, DV), bm = bwd_step(EP, DV);
   const auto up = [](int x, int m) { return (x + m - 1) / m; };
   // lengths of the longest jobs in 128-row steps of a dK/dV job (a dQ step does 0.8 of its products)
   const double unit = bm / 128.0;

@@ -152,24 +152,28 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(FlashBwdParams p) {
 }
 
 // ---------------------------------------------------------------------------
+// Geometry of a job, shared with the host's split rule (flash_bwd_split).
+// Small rows: 8 waves (256 keys per dK/dV job, 256 queries per dQ job) and 128-row steps, one
+// workgroup per CU (two waves per SIMD).  Wide rows need up to 512 registers per lane: 4 waves,
+// one per SIMD; 128-row steps in a two-slot ring where two such slots fit the LDS (C4's E = 192, D = 96:
+// 326 against 331 us with 64-row steps in three slots), else 64-row steps in three.
+constexpr bool bwd_big(int EP, int DV) { return EP + DV > 160; }
+constexpr int bwd_waves(int EP, int DV) { return bwd_big(EP, DV) ? 4 : 8; }
+constexpr int bwd_job(int EP, int DV) { return 32 * bwd_waves(EP, DV); }   // keys (dK/dV) or queries (dQ)
+constexpr bool bwd_two_slots(int EP, int DV) { return bwd_big(EP, DV) && 2 * (128 * (EP + DV) * 2 + 64 * 16) <= 150 * 1024; }
+constexpr int bwd_step(int EP, int DV) { return bwd_big(EP, DV) && !bwd_two_slots(EP, DV) ? 64 : 128; }   // rows of a step
+
 template <int EP, int DV>
 struct BwdCfg {
-  // Small rows: 8 waves (256 keys per dK/dV job, 256 queries per dQ job) and 128-row steps, one
-  // workgroup per CU (two waves per SIMD).  Wide rows need up to 512 registers per lane: 4 waves,
-  // one per SIMD; 128-row steps in a two-slot ring where two such slots fit (C4's E = 192, D = 96:
-  // 326 against 331 us with 64-row steps in three slots), else 64-row steps in three.
-  static constexpr bool kBig = EP + DV > 160;
   // The widest rows read their score and dP operands through a ring of eight instead of all at
   // once: with all of them in registers these kernels spilled, and every reload of a spilled
   // register waits for the tile loads in flight behind it.
   static constexpr bool kChunked = EP + DV > 320;
-  static constexpr int NW = kBig ? 4 : 8;                    // waves per workgroup
+  static constexpr int NW = bwd_waves(EP, DV);               // waves per workgroup
   static constexpr int THREADS = 64 * NW;
-  static constexpr int JOB = 32 * NW;                        // keys (dK/dV) or queries (dQ) per job
-  // wide rows: 128-row steps in a two-slot ring when two such slots fit the LDS, else 64-row steps in three
-  static constexpr bool kWide128 = kBig && 2 * ((128 * EP + 128 * DV) * 2 + 64 * 16) <= 150 * 1024;
-  static constexpr int BM = (kBig && !kWide128) ? 64 : 128;  // query rows per dK/dV step, keys per dQ step
-  static constexpr int SLOTS = kWide128 ? 2 : 3;
+  static constexpr int JOB = bwd_job(EP, DV);
+  static constexpr int BM = bwd_step(EP, DV);                // query rows per dK/dV step, keys per dQ step
+  static constexpr int SLOTS = bwd_two_slots(EP, DV) ? 2 : 3;
   static constexpr int KS = EP / 16, DS = DV / 16, EB = EP / 32, DB = DV / 32;
   static constexpr int EPU = EP / 8, DVU = DV / 8;
   static constexpr int XT = BM * EP, YT = BM * DV;            // elements of the two tiles of a slot

@@ -52,9 +52,11 @@ constexpr int kThreads = 512;   // 8 waves
 
 __device__ __forceinline__ u32x4 ld16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
 
+constexpr int fwd_tile_keys(int EP, int DV) { return EP + DV <= 192 && DV <= 64 ? 64 : 32; }
+
 template <int EP, int DV>
 struct FwdCfg {
-  static constexpr int BN = (EP + DV <= 192 && DV <= 64) ? 64 : 32;   // keys per tile
+  static constexpr int BN = fwd_tile_keys(EP, DV);                    // keys per tile
   static constexpr int KB = BN / 32;                                  // 32-key blocks per tile
   static constexpr int KS = EP / 16;                                  // 16-wide k steps of S
   static constexpr int NDB = DV / 32;                                 // 32-row blocks of O^T
@@ -565,7 +567,7 @@ hipError_t dispatch(const FlashFwdParams& p, hipStream_t s) {
 
 }  // namespace
 
-int flash_fwd_step_keys(int EP, int DV) { return EP + DV <= 192 && DV <= 64 ? 128 : 64; }   // 2 FwdCfg::BN
+int flash_fwd_step_keys(int EP, int DV) { return 2 * fwd_tile_keys(EP, DV); }
 
 hipError_t launch_flash_fwd(const FlashFwdParams& p, int dtype, hipStream_t s) {
   return dtype == 2 ? dispatch<BF16>(p, s) : dispatch<F16>(p, s);

@@ -667,20 +667,17 @@ hipError_t fwd_t(const FlashFwdParams& p, hipStream_t s) {
 
 // Column chunks per row block (each chunk recomputes the scores), as few as the registers hold: one
 // at 256 features, two at 384 / 512.
-template <int EP>
-constexpr int kv_chunks() { return EP <= 256 ? 1 : 2; }
-template <int EP>
-constexpr int q_chunks() { return EP <= 256 ? 1 : 2; }
+constexpr int wide_chunks(int EP) { return EP <= 256 ? 1 : 2; }
 
 template <typename T, int EP, int DV>
 hipError_t bwd_t(const FlashBwdParams& p, hipStream_t s) {
-  constexpr int CK = kv_chunks<EP>(), CQ = q_chunks<EP>();
-  const dim3 gk((p.NkP / (128 / CK)) * p.B * p.Hk * p.kv_splits), gq((p.NqP / (128 / CQ)) * p.B * p.Hq * p.q_splits);
-  hipError_t e = p.kv_splits > 1 ? launch_named("flash_wide_kv", wide_kv_kernel<T, EP, DV, CK, true>, gk, dim3(256), s, p)
-                                 : launch_named("flash_wide_kv", wide_kv_kernel<T, EP, DV, CK, false>, gk, dim3(256), s, p);
+  constexpr int CH = wide_chunks(EP);
+  const dim3 gk((p.NkP / (128 / CH)) * p.B * p.Hk * p.kv_splits), gq((p.NqP / (128 / CH)) * p.B * p.Hq * p.q_splits);
+  hipError_t e = p.kv_splits > 1 ? launch_named("flash_wide_kv", wide_kv_kernel<T, EP, DV, CH, true>, gk, dim3(256), s, p)
+                                 : launch_named("flash_wide_kv", wide_kv_kernel<T, EP, DV, CH, false>, gk, dim3(256), s, p);
   if (e != hipSuccess) return e;
-  e = p.q_splits > 1 ? launch_named("flash_wide_q", wide_q_kernel<T, EP, DV, CQ, true>, gq, dim3(256), s, p)
-                     : launch_named("flash_wide_q", wide_q_kernel<T, EP, DV, CQ, false>, gq, dim3(256), s, p);
+  e = p.q_splits > 1 ? launch_named("flash_wide_q", wide_q_kernel<T, EP, DV, CH, true>, gq, dim3(256), s, p)
+                     : launch_named("flash_wide_q", wide_q_kernel<T, EP, DV, CH, false>, gq, dim3(256), s, p);
   if (e != hipSuccess) return e;
   FlashBwdParams c = p;   // both sides' raw rows; dV from the splits, or written already
   if (c.kv_splits == 1) c.wv = nullptr;
@@ -701,10 +698,10 @@ int wide_splits(int64_t n, int steps) {
 
 // Job splits of a wide backward (raw rows in any case: raw_kv and raw_q stay false).
 FlashBwdSplit flash_wide_bwd_split(int B, int Hq, int Hk, int Nq, int Nk, int EP, bool causal) {
-  const int jk = EP <= 256 ? 128 : 64, jq = jk;   // rows per workgroup: 128 / chunks
+  const int rows = 128 / wide_chunks(EP);   // per workgroup
   FlashBwdSplit r{1, 1, false, false};
-  r.kv = wide_splits((int64_t)((Nk + jk - 1) / jk) * B * Hk, Hq / Hk * ((Nq + 31) / 32));
-  r.q = wide_splits((int64_t)((Nq + jq - 1) / jq) * B * Hq, ((causal ? std::min(Nq, Nk) : Nk) + 31) / 32);
+  r.kv = wide_splits((int64_t)((Nk + rows - 1) / rows) * B * Hk, Hq / Hk * ((Nq + 31) / 32));
+  r.q = wide_splits((int64_t)((Nq + rows - 1) / rows) * B * Hq, ((causal ? std::min(Nq, Nk) : Nk) + 31) / 32);
   return r;
 }
 
