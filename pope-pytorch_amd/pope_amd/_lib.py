@@ -142,18 +142,12 @@ def host():
 _PLAIN = (torch.Tensor, torch.nn.Parameter, type(None))
 
 
-_PRE_DISPATCH = torch._C.DispatchKey.PreDispatch
-
-
 def eager(*ts) -> bool:
     """Whether a call on these tensors can take the native call layer in place of the torch.library ops: no
     tracing (torch.compile, torch.jit.trace, make_fx before dispatch), no dispatch mode (fake tensors, make_fx,
     operator-recording checkpointing), no functorch transform and no tensor subclass, each of which works on
     the ops."""
-    return (not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
-            and torch._C._len_torch_dispatch_stack() == 0
-            and not torch._C._dispatch_tls_is_dispatch_key_included(_PRE_DISPATCH)
-            and torch._C._functorch.peek_interpreter_stack() is None and all(type(t) in _PLAIN for t in ts))
+    return not torch.compiler.is_compiling() and host().untraced() and all(type(t) in _PLAIN for t in ts)
 
 
 def last_error() -> str:

@@ -24,6 +24,8 @@ def test_tracing_and_modes_take_the_ops():
     make_fx(fn)(x)
     make_fx(fn, pre_dispatch=True)(x)
     torch.vmap(fn)(x)
+    torch.func.grad(lambda t: fn(t).sum())(x)
+    torch.func.jvp(fn, (x,), (x,))
     with FakeTensorMode() as mode:
         fn(mode.from_tensor(x))
-    assert seen == [False] * 5
+    assert seen == [False] * 7
