@@ -114,6 +114,33 @@ pope_desc desc_of(const Tensor& q, const Tensor& k, const Tensor& freqs, const T
   return d;
 }
 
+// Whether nothing on this thread traces, records or transforms torch's operators: no torch.jit.trace, no dispatch mode
+// (the pre-dispatch ones have a stack of their own) and no functorch transform.  One call in place of four from
+// Python: the guard takes 1.2 us for a call's six tensors; with two of these checks, from Python, it took 1.3.
+bool untraced() {
+  using c10::DispatchKey;
+  return !torch::jit::tracer::isTracing() && c10::impl::TorchDispatchModeTLS::stack_len() == 0 &&
+         !c10::impl::tls_is_dispatch_key_included(DispatchKey::PreDispatch) &&
+         !c10::impl::tls_is_dispatch_key_included(DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
+// Whether a backward has to run on the torch.library ops: its gradients come from a tracer, a mode or a transform
+// (batched gradients, a vectorised Jacobian) that a launch through raw pointers would pass by.
+bool on_ops(at::TensorList grads) {
+  if (!untraced()) return true;
+  for (const Tensor& g : grads)
+    if (g.defined() && (!g.has_storage() || g.unsafeGetTensorImpl()->is_python_dispatch())) return true;
+  return false;
+}
+
+// A registered op of pope_amd (its Python modules are imported before anything here runs).
+template <typename Sig>
+c10::TypedOperatorHandle<Sig> op(const char* name) {
+  return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Sig>();
+}
+using Grads4 = std::tuple<Tensor, Tensor, Tensor, Tensor>;
+using Grads5 = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor>;
+
 // Every operand on q's GPU: the kernels read raw pointers.
 void check_device(const Tensor& q, std::initializer_list<const Tensor*> ts) {
   TORCH_CHECK(q.is_cuda(), "pope_amd runs on GPU tensors only");
@@ -186,6 +213,14 @@ variable_list pad_rows(at::TensorList ts, const std::vector<PadCols>& cols, bool
 
 bool tracked(at::TensorList ts);
 
+// The gradients' move with torch's operators, for backwards on the ops.
+Tensor pad_row_ops(const Tensor& t, const PadCols& c, bool pad) {
+  const auto part = [&](int64_t from, int64_t n) { return t.narrow(-1, from, n); };
+  if (!pad) return at::cat({part(0, c.split), part(c.split + c.gap, c.cols - c.split)}, -1);
+  return at::cat({at::constant_pad_nd(part(0, c.split), {0, c.gap}),
+                  at::constant_pad_nd(part(c.split, c.cols - c.split), {0, c.width - c.cols - c.gap})}, -1);
+}
+
 // Gradients under create_graph: differentiating them again raises, as it does through the torch.library
 // ops (whose backward ops have no autograd formula), instead of treating them as constants.
 variable_list once_differentiable(variable_list grads, const char* what) {
@@ -230,7 +265,12 @@ struct PadFn : torch::autograd::Function<PadFn> {
       }
     variable_list r(grads.size() + 3);
     if (ts.empty()) return r;
-    variable_list out = pad_rows(ts, cols, !ctx->saved_data["pad"].toBool());
+    const bool pad = !ctx->saved_data["pad"].toBool();
+    if (on_ops(ts)) {
+      for (size_t j = 0; j < ts.size(); ++j) r[at_[j]] = pad_row_ops(ts[j], cols[j], pad);
+      return r;
+    }
+    variable_list out = pad_rows(ts, cols, pad);
     // the node before this one may have marked its gradients as not differentiable: so are the moved ones
     if (std::any_of(ts.begin(), ts.end(), [](const Tensor& t) { return t.requires_grad(); }))
       out = once_differentiable(std::move(out), "padding");
@@ -378,8 +418,23 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
     return x;
   }
 
+  static variable_list backward_ops(AutogradContext* ctx, const variable_list& sv, Tensor dout) {
+    if (const int64_t cols = ctx->saved_data["cols"].toInt(); cols < sv[0].size(3))
+      dout = pad_row_ops(dout, {cols, 0, cols, sv[0].size(3), 0}, true);
+    const auto maybe = [](const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
+    const bool need_df = sv[3].defined() && ctx->needs_input_grad(3), need_db = sv[4].defined() && ctx->needs_input_grad(4);
+    using O = const std::optional<Tensor>&;
+    const auto [dq, dk, dv, df, db] =
+        op<Grads5(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, O, O, O, bool,
+                  double, bool, bool, O)>("pope_amd::flash_bwd")
+            .call(dout, sv[0], sv[1], sv[2], sv[6], sv[7], maybe(sv[3]), maybe(sv[4]), maybe(sv[5]),
+                  ctx->saved_data["causal"].toBool(), ctx->saved_data["scale"].toDouble(), need_df, need_db, maybe(sv[8]));
+    return {dq, dk, dv, need_df ? df : Tensor(), need_db ? db : Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list sv = ctx->get_saved_variables();
+    if (on_ops(grads)) return backward_ops(ctx, sv, grads[0]);
     const Tensor q = unit_feature(sv[0]), k = unit_feature(sv[1]), v = unit_feature(sv[2]), freqs = sv[3], bias = sv[4],
                  mask = sv[5], o = unit_feature(sv[6]), fwd_ws = sv[8];
     const Tensor lse = sv[7].contiguous();
@@ -501,12 +556,18 @@ struct SimFn : torch::autograd::Function<SimFn> {
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list sv = ctx->get_saved_variables();
+    const bool need_df = ctx->needs_input_grad(2) && sv[2].size(-1) > 0;
+    const bool need_db = ctx->needs_input_grad(3) && sv[3].size(-1) > 0;
+    if (on_ops(grads)) {
+      const auto [dq, dk, df, db] =
+          op<Grads4(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, bool, bool, bool)>("pope_amd::sim_bwd")
+              .call(grads[0], sv[0], sv[1], sv[2], sv[3], need_df, need_db, ctx->saved_data["split"].toBool());
+      return {dq, dk, need_df ? df : Tensor(), need_db ? db : Tensor(), Tensor()};
+    }
     const Tensor q = rows4(sv[0]), k = rows4(sv[1]), freqs = sv[2], bias = sv[3];
     const Tensor dsim = rows4(grads[0].to(at::kFloat));
     TORCH_CHECK_VALUE(dsim.dim() == 4 && dsim.size(0) == q.size(0) && dsim.size(1) == q.size(1) &&
                           dsim.size(2) == q.size(2) && dsim.size(3) == k.size(2), "dsim ", dsim.sizes(), " does not fit the similarity");
-    const bool need_df = ctx->needs_input_grad(2) && freqs.size(-1) > 0;
-    const bool need_db = ctx->needs_input_grad(3) && bias.size(-1) > 0;
     pope_desc d = desc_of(q, k, freqs, bias);
     d.flags = (ctx->saved_data["split"].toBool() ? POPE_FLAG_SPLIT_BF16 : 0) | deterministic_flag() | POPE_FLAG_ZERO_GRADS;
     strides3(d.sim_s, dsim);
@@ -583,8 +644,15 @@ struct PolarFn : torch::autograd::Function<PolarFn> {
       return g.defined() ? g.to(at::kFloat).contiguous()
                          : at::zeros({x.size(0), x.size(1), x.size(2), E}, x.options().dtype(at::kFloat).requires_grad(false));
     };
-    const Tensor gq = grad(grads[0], q), gk = grad(grads[1], k);
     const bool need_df = ctx->needs_input_grad(2), need_db = ctx->needs_input_grad(3);
+    const bool ops = on_ops(grads);
+    const Tensor gq = grad(grads[0], q), gk = grad(grads[1], k);
+    if (ops) {
+      const auto [dq, dk, df, db] =
+          op<Grads4(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, bool, bool, bool)>(
+              "pope_amd::polar_bwd").call(gq, gk, q, k, freqs, bias, need_df, need_db, cplx);
+      return {dq, dk, need_df ? df : Tensor(), need_db ? db : Tensor(), Tensor()};
+    }
     pope_desc d = desc_of(q, k, freqs, bias);
     d.flags = (cplx ? POPE_FLAG_COMPLEX : 0) | deterministic_flag();
     const Tensor dq = at::empty_like(q), dk = at::empty_like(k);
@@ -622,16 +690,6 @@ std::pair<Tensor, Tensor> polar_padded(const Tensor& q, const Tensor& k, const T
   const PadCols c{2 * R, 2 * (R8 - R), D + R, Dp + R8, 0};
   const variable_list r = padded({qh, kh}, {c, c}, false);
   return {r[0], r[1]};
-}
-
-// Whether nothing on this thread traces, records or transforms torch's operators: no torch.jit.trace, no dispatch mode
-// (the pre-dispatch ones have a stack of their own) and no functorch transform.  One call in place of four from
-// Python: the guard takes 1.2 us for a call's six tensors; with two of these checks, from Python, it took 1.3.
-bool untraced() {
-  using c10::DispatchKey;
-  return !torch::jit::tracer::isTracing() && c10::impl::TorchDispatchModeTLS::stack_len() == 0 &&
-         !c10::impl::tls_is_dispatch_key_included(DispatchKey::PreDispatch) &&
-         !c10::impl::tls_is_dispatch_key_included(DispatchKey::FuncTorchDynamicLayerFrontMode);
 }
 
 }  // namespace

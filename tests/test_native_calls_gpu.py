@@ -211,3 +211,25 @@ def test_the_ops_give_only_the_wanted_gradients(cuda, wanted):
             loss = sum(t.square().sum() for t in (out if isinstance(out, tuple) else (out,)))
             grads.append(torch.autograd.grad(loss, [t for t in leaves if t.requires_grad]))
         _same(*grads)
+
+
+@pytest.mark.filterwarnings("ignore")   # vmap's per-sample fallback of the ops
+@pytest.mark.parametrize("R", [16, 12])   # 12: padded operands
+@pytest.mark.parametrize("name", ["sim", "polar", "flash_bf16", "flash_fp32"])
+def test_transformed_backwards_run_on_the_ops(cuda, name, R):
+    """The backward of an eager call under batched gradients (what a vectorised Jacobian does) and under make_fx: the
+    node goes through the torch.library op, which those work on, and gives the same gradients."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    fn = {"sim": _sim, "polar": lambda *t: _polar(*t)[1], "flash_bf16": _flash(torch.bfloat16), "flash_fp32": _flash(torch.float32)}[name]
+    inp = make_pope_inputs(72, 1, 2, 1, 16, 16, 32, R, torch.float32)
+    leaves = [inp[n].detach().requires_grad_(True) for n in ("q", "k", "freqs", "bias")]
+    out = fn(*leaves)
+    wanted = leaves if name != "polar" else leaves[1:]
+    G = torch.randn(3, *out.shape, device="cuda").to(out.dtype)
+    back = lambda g, **kw: torch.autograd.grad(out, wanted, g, retain_graph=True, **kw)
+    want = [back(g) for g in G]
+    batched = back(G, is_grads_batched=True)
+    traced = make_fx(back)(G[0])
+    for i in range(3):
+        _same([t[i] for t in batched], want[i])
+        _same(traced(G[i]), want[i])
