@@ -315,8 +315,8 @@ void check_flash(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor
                     "incompatible q ", q.sizes(), " and k ", k.sizes());
   if (freqs.defined()) {
     TORCH_CHECK_VALUE(freqs.size(-2) >= k.size(2), "freqs has ", freqs.size(-2), " positions, keys need ", k.size(2));
-    // fewer batches or heads than the call has would be read past the end
-    for (int64_t i = 0; i + 2 < freqs.dim() && i < 2; ++i)
+    // fewer batches or heads than the call has would be read past the end (the library refuses per-head tables of grouped heads)
+    for (int64_t i = 0; i + 2 < freqs.dim() && i < (q.size(1) == k.size(1) ? 2 : 1); ++i)
       TORCH_CHECK_VALUE(freqs.size(i) == 1 || freqs.size(i) >= q.size(i) || freqs.stride(i) == 0, "freqs has ", freqs.size(i),
                         i ? " heads" : " batches", ", the call ", q.size(i));
     TORCH_CHECK_VALUE(bias.size(-1) == freqs.size(-1) && (bias.size(0) == 1 || bias.size(0) == k.size(1)), "bias ",

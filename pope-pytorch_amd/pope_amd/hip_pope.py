@@ -174,7 +174,7 @@ def hip_compute_qk_similarity(q, k, freqs, bias, rotate_dim=None, allow_tf32=Tru
         raise ValueError(f"freqs has {freqs.shape[-2]} positions, keys need {k.shape[2]}")
     if k.shape[0] < q.shape[0] or k.shape[-1] < q.shape[-1]:   # read by q's extents
         raise ValueError(f"incompatible q {tuple(q.shape)} and k {tuple(k.shape)}")
-    _check_freqs_extents(freqs, q.shape[0], q.shape[1])
+    _check_freqs_extents(freqs, q.shape[0], q.shape[1], k.shape[1])
     out_dtype = q.dtype
     qf, kf = q.float(), k.float()
     # head / rotate dims that are not multiples of 8: padded on the device (pope_amd._pad)

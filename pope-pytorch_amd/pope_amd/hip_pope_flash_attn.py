@@ -63,10 +63,11 @@ def _freqs_strides(freqs: Tensor, head_first: bool = True) -> tuple:
     raise ValueError(f"freqs must be 2-D, 3-D or 4-D, got shape {tuple(freqs.shape)}")
 
 
-def _check_freqs_extents(freqs: Tensor, B: int, Hq: int):
+def _check_freqs_extents(freqs: Tensor, B: int, Hq: int, Hk: int):
     """The kernels step through a table's batches and heads by stride: fewer entries than the call has would be
-    read past the end (an extent of 1, or any with stride 0, broadcasts)."""
-    for i, (n, want, name) in enumerate(zip(freqs.shape[:-2], (B, Hq), ("batches", "heads"))):
+    read past the end (an extent of 1, or any with stride 0, broadcasts; per-head tables of grouped heads are
+    refused by the library)."""
+    for i, (n, want, name) in enumerate(zip(freqs.shape[:-2], (B, Hq if Hq == Hk else 1), ("batches", "heads"))):
         if 1 < n < want and freqs.stride(i):
             raise ValueError(f"freqs has {n} {name}, the call {want}")
 
@@ -155,7 +156,7 @@ def _check_pope_shapes(q, k, freqs, bias):
             raise ValueError(f"freqs has {freqs.shape[-2]} positions, keys need {k.shape[2]}")
         if bias.shape[-1] != R or bias.shape[0] not in (1, k.shape[1]):
             raise ValueError(f"bias {tuple(bias.shape)} must be (1 or {k.shape[1]}, {R})")
-        _check_freqs_extents(freqs, B, Hq)
+        _check_freqs_extents(freqs, B, Hq, k.shape[1])
 
 
 def _check_views(q, k, v, mask, lse=None):

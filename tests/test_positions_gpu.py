@@ -192,3 +192,5 @@ def test_tables_and_keys_with_too_few_entries_are_refused(cuda, R):
         want = fn(f)
         for good in (f[None], f.repeat(B + 1, 1, 1), f.expand(B, H, N, R), f.repeat(B, H, 1, 1)):
             assert torch.equal(fn(good), want)
+    with pytest.raises(RuntimeError, match="per-head freqs"):   # grouped heads
+        pope_amd.flash_attn_with_pope(q, k[:, :2], v[:, :2], pos_emb=(f.repeat(B, 2, 1, 1), b[:2]))
