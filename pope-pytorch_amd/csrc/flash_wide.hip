@@ -18,7 +18,7 @@
 // exclusive or from one base per tile, masks are applied on a side branch, and a head's jobs stay on
 // one XCD.  What bounds the kernels: one operand read from LDS per product (1 KB per 32 cycles and
 // SIMD), and the softmax of a wave's only row block, which nothing overlaps.  At (2, 8, 2048, 256),
-// R 256, causal bf16 (two chunks): forward 205 -> 117 us, dK/dV 649 -> 168 (921 TFLOP/s of products),
+// R 256, causal bf16 (two chunks): forward 205 -> 144 us, dK/dV 649 -> 168 (921 TFLOP/s of products),
 // dQ 510 -> 167; before, every product group waited on reloads of spilled registers behind tile
 // loads that missed the XCD's L2.
 // Memory stays linear in the sequence length: no score matrix is stored.  Same workspace preparation as the narrow path
@@ -74,7 +74,8 @@ __device__ __forceinline__ int res_row(int r, int hf) { return 8 * (r >> 2) + 4 
 
 // Growth of a row's running max (log2 units) that the forward absorbs without rescaling its
 // accumulators: probabilities reach at most 2^lazy_max.  None at 512 features: the row's largest
-// probability is exactly 1 there and adds no 16-bit rounding of its own.
+// probability is exactly 1 there and adds no 16-bit rounding of its own (o's error against 64 bits
+// 0.00239, with a growth of 8 absorbed 0.00241; the forward of the header's case 144 us against 117).
 template <int EP>
 constexpr float lazy_max() { return EP < 512 ? 8.f : 0.f; }
 
@@ -153,7 +154,7 @@ struct WideAddr {
 };
 
 // Operand reads kept in flight ahead of the product that takes them: as many of eight as leave the
-// kernel without spills (a reload waits for every tile load in flight behind it).
+// kernel's loop without spills (a reload waits for every tile load in flight behind it).
 template <int EP>
 constexpr int fwd_ring() { return EP >= 512 ? 6 : 8; }
 constexpr int kKvRing = 4, kQRing = 8;

@@ -11,8 +11,8 @@
 
 namespace pope {
 
-// blockIdx.y: the table (the fp32 similarity's key and query tables go in one launch: 2 x 4.4 -> 4.6 us
-// at 1,024 rows of 64).
+// blockIdx.y: the table (the fp32 similarity's key and query tables go in one launch: 2 x 4.3 -> 5.2 us
+// at 1,024 rows of 64, 8 heads).
 __global__ __launch_bounds__(256) void phase_table_kernel(TableParams p0, TableParams p1) {
   const TableParams& p = blockIdx.y ? p1 : p0;
   // four consecutive entries of one row per thread (R is a multiple of 8): four independent

@@ -225,7 +225,7 @@ hipError_t launch_t(const PolarParams& p, bool bwd, hipStream_t s) {
   const auto blocks = [&](const Side& sd, int iters) {
     return (int64_t)((sd.N + rpb * iters - 1) / (rpb * iters)) * p.B * sd.H;
   };
-  // row groups per workgroup: up to 8 while about eight workgroups per CU remain
+  // row groups per workgroup: up to 8 while four workgroups per CU remain
   int iters = 1;
   while (iters < 8 && blocks(q, 2 * iters) + blocks(k, 2 * iters) >= 1024) iters *= 2;
   const int64_t nq = blocks(q, iters), nk = blocks(k, iters);

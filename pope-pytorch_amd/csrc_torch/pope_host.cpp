@@ -331,7 +331,8 @@ bool decode_groups(int64_t Hq, int64_t D) {
   return false;
 }
 
-// The same decision as hip_pope_flash_attn._decode_eligible.
+// The same decision as hip_pope_flash_attn._decode_eligible (tests/test_decode_gpu.py compares them around the
+// shortest caches).
 bool decode_eligible(const pope_desc& d, int64_t min_keys) {
   if (d.Nq != 1 || d.causal || (d.Nk < min_keys && (int64_t)d.Nk * d.D < 36 * min_keys) || d.D > 128 || !decode_groups(d.Hq, d.D)) return false;
   if (d.R && (d.f_s[1] != 0 || d.f_s[0] % 4 || d.f_s[2] % 4)) return false;

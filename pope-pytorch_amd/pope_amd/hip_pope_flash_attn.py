@@ -261,9 +261,11 @@ def _decode_head_groups(Hq: int, D: int) -> int:
 
 def _decode_eligible(q, k, v, freqs, causal) -> bool:
     """Whether the forward runs the split-K decode kernel (pope_flash_decode): one non-causal query
-    row against a cache of at least _DECODE_MIN_KEYS keys (fewer for wider heads), within the decode kernel's head-dim and 32-bit index
-    limits.  The forward op and its fake implementation both decide with this predicate, so the
-    workspace they return has the same size (empty for decode)."""
+    row against a cache of at least _DECODE_MIN_KEYS keys (fewer for wider heads), within the decode
+    kernel's head-dim and 32-bit index limits.  The forward op and its fake implementation both decide
+    with this predicate, so the workspace they return has the same size (empty for decode);
+    decode_eligible of the native call layer is the same rule (tests/test_decode_gpu.py compares them
+    around the shortest caches)."""
     B, Hq, Nq, D = q.shape
     Nk = k.shape[2]
     R = freqs.shape[-1] if exists(freqs) else 0
