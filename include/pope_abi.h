@@ -53,7 +53,8 @@ enum pope_flags {
   /* The workspace holds the preparation (expanded K/Q rows, phase tables, key visibility)
    * written by a pope_flash_fwd call with the same descriptor, q, k, freqs, bias and mask,
    * and not modified since: the backward reuses it instead of recomputing it.  The flash
-   * forward and backward workspaces have the same size and layout. */
+   * backward's workspace begins with the forward's layout; it is larger in deterministic mode and,
+   * without partials (pope_flash_bwd_split), for head dims above 128. */
   POPE_FLAG_PREPARED = 1,
   /* dfreqs / dbias are overwritten (cleared by the library before it accumulates into them)
    * instead of accumulated into. */
