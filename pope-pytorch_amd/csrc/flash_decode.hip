@@ -81,15 +81,17 @@ __device__ __forceinline__ QwIn query_weight_in(const DecodeParams& p, int b, in
 }
 // The query weight word, scale * log2 e folded in: rotated dims the fp16 pair
 // (a cos(F_q - b), a sin(F_q - b)) with a = softplus(q) and F_q = F[Nk - 1]; pass-through dims
-// the fp32 weight q.
-__device__ __forceinline__ uint32_t query_weight_of(const DecodeParams& p, int d, QwIn in) {
+// the fp32 weight q.  Both times `unit` (a power of two); `big` is set where a leaves fp16's range.
+constexpr float kF16Max = 65504.f;
+__device__ __forceinline__ uint32_t query_weight_of(const DecodeParams& p, int d, QwIn in, float unit, int& big) {
   if (d < p.R) {
     float sn, cs;
     sincos_acc(in.f - in.bb, &sn, &cs);
     const float a = softplus_f(in.qv) * p.scale_log2;
-    return __builtin_bit_cast(uint32_t, f16x2{(_Float16)(a * cs), (_Float16)(a * sn)});
+    big |= fabsf(a) > kF16Max;
+    return __builtin_bit_cast(uint32_t, f16x2{(_Float16)(a * unit * cs), (_Float16)(a * unit * sn)});
   }
-  return __builtin_bit_cast(uint32_t, in.qv * p.scale_log2);
+  return __builtin_bit_cast(uint32_t, in.qv * p.scale_log2 * unit);
 }
 
 // Split kernel.  A workgroup (4 waves) owns one (batch, split of S keys) for one group of query
@@ -137,6 +139,7 @@ __global__ __launch_bounds__(kThreads, 2) void decode_split_kernel(DecodeParams 
   __shared__ __attribute__((aligned(16))) uint32_t tab_s[S * TS];
   __shared__ __attribute__((aligned(16))) uint32_t qw_s[kQwMax];
   __shared__ uint8_t vis_s[S];
+  __shared__ float unit_s[kQwMax / 8];   // score units per head, where some weight left fp16's range
   __shared__ float sp_s[T::kCode == 2 ? kSpN : 1];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -251,20 +254,38 @@ __global__ __launch_bounds__(kThreads, 2) void decode_split_kernel(DecodeParams 
     }
   }
   // query weights of the workgroup's heads (after the rows: their registers are free again)
+  int big = 0;
 #pragma unroll
   for (int k = 0; k < kQwPre; ++k) {
     const int i = tid + k * kThreads;
-    if (i < HG * D) qw_s[i] = query_weight_of(p, i % D, qin[k]);
+    if (i < HG * D) qw_s[i] = query_weight_of(p, i % D, qin[k], 1.f, big);
   }
   for (int i = tid + kQwPre * kThreads; i < HG * D; i += kThreads)
-    qw_s[i] = query_weight_of(p, i % D, query_weight_in<T>(p, b, h_lo + i / D, i % D));
+    qw_s[i] = query_weight_of(p, i % D, query_weight_in<T>(p, b, h_lo + i / D, i % D), 1.f, big);
   if constexpr (T::kCode == 2) {
     for (int i = tid; i < kSpN; i += kThreads) {
       const float t = __builtin_bit_cast(float, (uint32_t)(i + kSpLo) << 16);
       sp_s[i] = __builtin_amdgcn_logf(1.f + __builtin_amdgcn_exp2f(-t * kLog2e));
     }
   }
-  __syncthreads();
+  const bool units = __syncthreads_or(big);
+  if (units) {   // bf16 queries beyond fp16's range: the weights of such a head in units of a power of two.
+    // (The test and the units cost ordinary calls 0 to 2% of this kernel: 8 x 32 heads over 8, 2,048 keys, D 128
+    // 57.5 -> 58.2 us, 1 x 32 over 8, 4,001 keys 18.8 -> 19.4, 2 x 16, 4,096 keys, D 32 13.7 -> 13.0.)
+    POPE_COLD_PATH();
+    for (int h = h_lo + wave; h < h_hi; h += kWaves) {
+      float amax = 0.f;
+      for (int d = lane; d < R; d += 64)
+        amax = fmaxf(amax, fabsf(softplus_f(query_weight_in<T>(p, b, h, d).qv) * p.scale_log2));
+      amax = rows_max<1>(amax);
+      const bool scaled = amax > kF16Max && amax < INFINITY;
+      const int e = scaled ? __builtin_amdgcn_frexp_expf(amax) - 15 : 0;   // amax 2^-e < 2^15
+      for (int d = lane; d < D; d += 64)
+        qw_s[(h - h_lo) * D + d] = query_weight_of(p, d, query_weight_in<T>(p, b, h, d), ldexpf(1.f, -e), big);
+      if (lane == 0) unit_s[h - h_lo] = ldexpf(1.f, e);
+    }
+    __syncthreads();
+  }
 
   // Head h of this wave; with `next` the K rows of head h + kWaves are loaded as soon as the K
   // side of h is done and its V rows as soon as the V side is (the last head of the wave,
@@ -326,12 +347,14 @@ __global__ __launch_bounds__(kThreads, 2) void decode_split_kernel(DecodeParams 
 #pragma unroll
     for (int u = 1; u < kLoads; ++u) m = fmaxf(m, sc[u]);
     m = rows_max<LPK>(m);
-    const float mu = m == -INFINITY ? 0.f : m;
+    // the scores' unit folded into the exponentials' arguments
+    const float unit = units ? __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, unit_s[h - h_lo]))) : 1.f;
+    const float mu = m == -INFINITY ? 0.f : m * unit;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     float l = 0.f;
 #pragma unroll
     for (int u = 0; u < kLoads; ++u) {
-      const float pv = __builtin_amdgcn_exp2f(sc[u] - mu);   // 0 when masked
+      const float pv = __builtin_amdgcn_exp2f(fmaf(sc[u], unit, -mu));   // 0 when masked
       float x[8];
       unpack8<T>(vb[u], x);
 #pragma unroll
@@ -351,7 +374,7 @@ __global__ __launch_bounds__(kThreads, 2) void decode_split_kernel(DecodeParams 
         if (d0 + q < D) p.part_o[row * D + d0 + q] = acc[q];
     }
     if (lane == 0) {
-      p.part_ml[row * 2] = m;
+      p.part_ml[row * 2] = m * unit;
       p.part_ml[row * 2 + 1] = l;
     }
   };

@@ -303,3 +303,33 @@ def test_decode_backward_of_short_caches(cuda, Nk, D):
     ref = oracle_attention(inp, False)
     for n in ("o", "dq", "dk", "dv", "dbias"):
         assert max_abs(res[n], ref[n]) <= TOL * (max(1.0, ref[n].abs().max().item()) if n == "dbias" else 1.0), n
+
+
+@pytest.mark.parametrize("Nk,D,R", [(300, 128, 128), (600, 64, 32), (600, 64, 64), (2000, 96, 96), (1100, 32, 16)])
+@pytest.mark.parametrize("value", [4e5, 1e6, 1e20])
+def test_decode_queries_beyond_fp16(cuda, Nk, D, R, value):
+    """bf16 queries whose weights leave fp16's range keep their order: one key scores highest by far (all phases zero,
+    so scores are sums of products of magnitudes) and its value row is the output.  The other heads, in the same
+    workgroup, give the bits they give beside ordinary queries."""
+    from pope_amd import _lib
+    import pope_amd
+    inp = _decode_inputs(600 + Nk, 2, 6, 3, Nk, D, R, torch.bfloat16)
+    inp["freqs"].zero_()
+    inp["bias"].zero_()
+    inp["k"].clamp_(max=2.5)
+    inp["k"][:, 0, 7, :R] = 5.0   # key 7 of kv head 0, visible in every batch
+    run = lambda: pope_amd.flash_attn_with_pope(inp["q"], inp["k"], inp["v"], pos_emb=(inp["freqs"], inp["bias"]), mask=inp["mask"])
+    plain = run()
+    inp["q"][1, 0, 0, :R] = value
+    _lib.profile_reset()
+    _lib.profile_enable(True)
+    o = run()
+    torch.cuda.synchronize()
+    _lib.profile_enable(False)
+    assert "flash_decode_split" in _lib.profile_read()
+    ref = oracle_attention(inp, False, grads=False)["o"]
+    assert torch.equal(o[1, 0, 0], inp["v"][1, 0, 7])
+    assert max_abs(o, ref) <= TOL
+    keep = torch.ones(2, 6, dtype=torch.bool, device="cuda")
+    keep[1, 0] = False
+    assert torch.equal(o[keep], plain[keep])
